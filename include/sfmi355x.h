@@ -68,9 +68,14 @@ extern "C" {
                                  Runs as six joint histograms, one per invariant.                 */
 
 /* precision */
-#define SF_PREC_FP64 0        /* binary64 pair arithmetic in the reference's order, bins certified
-                                 from the exact keys and values (the reference's rules near every
-                                 decision point): the drop-in (counts bit-exact)                 */
+#define SF_PREC_FP64 0        /* binary64 pair arithmetic, bins certified from the exact keys and
+                                 values (the reference's rules near every decision point): the
+                                 drop-in (counts bit-exact).  Every 1D operator, the single pass and
+                                 the joint du_L and du_L^2 form a pair's value from differences of
+                                 positions and velocities (within a few 2^-53 of the velocities of
+                                 the reference's sequence, which evaluates the pairs whose value is
+                                 not certain or is small against them); other joint operators
+                                 follow the reference's sequence for every pair.               */
 #define SF_PREC_MIXED 1       /* binary32 pair arithmetic, binary64 re-binning of pairs near any
                                  bin edge (counts bit-exact), binary64 accumulation              */
 #define SF_PREC_MIXED_FIXED 2 /* as SF_PREC_MIXED, but a joint histogram whose value edges are

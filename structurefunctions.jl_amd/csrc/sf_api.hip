@@ -199,6 +199,7 @@ struct Plan {
   bool J = false, mixed = false, sload = false, sp = false, fx = false;
   int block = 256, tj = 256, copies = 1, grid = 1, ncell_max = 1, n_items = 0;
   int strip = 0;            // B-strip launch (fields per strip), 0: off
+  int qcap64 = 0;           // binary64 kernel: LDS queue entries per workgroup
   int n_items64 = 0;        // B-strip: the per-slice items the binary64 kernel runs instead
   int64_t total_pts = 0, max_n = 0, total_pairs = 0, cap = 0;
   Params P{};
@@ -597,7 +598,7 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   // value axis
   s.v_uniform = 0;
   s.v_negzero = 0;
-  s.v0 = 0; s.vinv = 0; s.v0f = 0; s.vinvf = 0; s.vtc = 0; s.vslack = 0; s.vabs = 0;
+  s.v0 = 0; s.vinv = 0; s.v0f = 0; s.vinvf = 0; s.vtc = 0; s.vslack = 0; s.vabs = 0; s.vtcu = 0; s.veps2 = 0;
   s.v_fx = 0; s.vwf = 0; s.vsf = 0; s.fxc1 = 0; s.fxc0 = 0; s.plane = 0; s.vsmall = 0; s.gz = 0;
   s.v_log = 0; s.vk0 = 0; s.vl0f = 0; s.vlinvf = 0;
   if (p.n_val > 0) {
@@ -617,11 +618,17 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
         s.vinvf = (float)(1.0L / w);
         // exact product of two binary32 numbers, rounded once: within 2^-24 |v0 / w| of
         // -v0f / w, which the slack's 4u (1 + |v0 / w|) term covers
+        // 1 / w and of a binary64 value to binary32)
         s.vtc = (float)(-(double)s.v0f * (double)s.vinvf);
         // slack in t units: edge non-uniformity + rounding of v0 and 1/w in binary32
         const long double u = ldexpl(1.0L, -24);
         s.vslack = round_up_f(dev + 4.0L * u * (1.0L + fabsl((long double)v0 / w)) + 4.0L * u * nv + 1e-6L +
                               rule_slack(p.val_rule) / w);
+        // one margin for every value in range (|t| < nv + 1): 16u |t| covers the rounding of the
+        // multiply-add, of the value and of the sums vtc + margin and t - floor(t)
+        const long double eps = (long double)s.vslack + 24.0L * u * (nv + 2) + 4.0L * u * fabsl((long double)s.vtc);
+        s.vtcu = (float)((long double)s.vtc + eps);
+        s.veps2 = round_up_f(2.0L * eps);
         // fixed-point joint cells need every value of bin g within [-1/64, 1 + 1/64] widths of
         // the binary32 grid point fmaf(g, vwf, v0f)
         if (dev < 1.0L / 64) {
@@ -1001,14 +1008,18 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     prep[s].N = sl[s].N;
     prep[s].pt_off = pl.total_pts;
     prep[s].perm = nullptr;
-    prep[s].mul = mixed ? interleave_mul(sl[s].N) : 0;
+    // (the binary64 kernel's spherical records: joint histograms only, whose atomics the order
+    // spreads; 1D ones keep their lane-group copies and adjacent rows, see tile_row)
+    prep[s].mul = (mixed || (G == kSphere && J)) ? interleave_mul(sl[s].N) : 0;
     pl.total_pts += sl[s].N;
     pl.max_n = std::max<int64_t>(pl.max_n, sl[s].N);
     pl.total_pairs += pairs_of(sl[s].N);
   }
   PLBUF(pl.rec64, ((size_t)pl.total_pts * S64 + 16));
   // + one record (F32 <= 16): the binary32 pair loop requests the record after its last column
-  if (mixed) PLBUF(pl.rec32, ((size_t)pl.total_pts * F32 + 16));
+  // (sphere: the binary64 kernel's records, kF64Rec doubles per point, share the buffer)
+  static_assert(kF64Rec * 2 == rec_f32(kSphere, 2) && kF64Rec * 2 == rec_f32(kSphere, 3), "record sizes");
+  if (mixed || G == kSphere) PLBUF(pl.rec32, ((size_t)pl.total_pts * F32 + 16));
 
   // ---- tables
   std::vector<Slice> sdesc(n);
@@ -1117,10 +1128,17 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   pl.mcopies = mcop;
   const SmemLayout L0 = smem_layout(p0.n_dist, p0.n_val, ncell_max, stage_bytes, copies, nmom, pl.fx, 0, strip,
                                     jlayout, pl.n1d, mcop);
-  // the binary64 kernel keeps one copy of a joint histogram
-  // (the binary64 kernel reads its column records with scalar loads: no LDS stage)
+  // the binary64 kernel keeps one copy of a joint histogram, and queues the pairs it evaluates by
+  // the reference's sequence: kRareQueue entries per wave, fewer (or none: such pairs are then
+  // evaluated as they come) where the LDS does not hold them
+  // (it reads its column records with scalar loads: no LDS stage)
+  int qcap64 = kRareQueue * (block / 64);
+  while (qcap64 > 0 && (size_t)smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, J ? 1 : copies, nmom, 0, qcap64, 0,
+                                           jlayout).total > ctx->max_smem)
+    qcap64 = qcap64 > block / 64 ? qcap64 / 2 : 0;
   const SmemLayout L64 = smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, J ? 1 : copies, nmom, 0, 0, 0,
                                      jlayout);
+  pl.qcap64 = qcap64;
   if ((size_t)std::max(L0.total, L64.total) > ctx->max_smem)
     return ctx->fail(SF_E_UNSUPPORTED,
                      "histogram of %d cells needs %d bytes of LDS; the device allows %zu per workgroup",
@@ -1129,7 +1147,9 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     return strip ? strip_occupancy(G, D, hist_opk(Pk), blk, bytes)
                  : hist_occupancy(G, D, J, mixed, hist_opk(Pk), sload, pl.fx, blk, bytes);
   };
-  int bpc = occupancy(block, (size_t)L0.total);
+  int bpc = occupancy(block, (size_t)(mixed ? L0.total
+                                            : smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, copies, nmom, 0, qcap64,
+                                                          0, jlayout).total));
   if (bpc < 1) bpc = 1;
   if (!t_block && pl.fx && bpc * block < 1024) {
     // registers allow only one 768-thread workgroup per CU: use 1024 threads instead
@@ -1377,8 +1397,8 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
   if (!use_mixed) {  // the binary64 kernel keeps binary64 sums and 32-bit counts, no queue
     P.fx = 0;
     if (P.n_val > 0) P.copies = 1;
-    P.qcap = 0;
-    P.qw = 0;
+    P.qcap = pl.qcap64;
+    P.qw = pl.qcap64 / (pl.block / 64);
     P.flush_limit = 0x7fffffffLL;
     if (pl.strip) {  // one slice at a time
       P.strip = 0;

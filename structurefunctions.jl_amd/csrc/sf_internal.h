@@ -29,6 +29,8 @@ enum Geom : int { kFlat = 0, kSphere = 1 };
 inline constexpr __host__ __device__ int rec_d64(int G, int D) { return (G == kFlat) ? ((D == 2) ? 4 : 6) : 12; }
 inline constexpr __host__ __device__ int rec_f32(int G, int D) { return (G == kFlat && D == 2) ? 12 : 16; }
 inline constexpr __host__ __device__ int rec_id(int G, int D) { return (G == kFlat) ? 4 * D + 1 : 15; }
+//   binary64 kernel, sphere (pair64f): P0 P1 P2 2 U0 2 U1 2 U2 ur {2^-12 |u|, id}  (8 doubles)
+inline constexpr int kF64Rec = 8;
 template <int G, int D> struct Rec {
   static constexpr int d64 = rec_d64(G, D);
   static constexpr int f32 = rec_f32(G, D);
@@ -72,6 +74,8 @@ struct Slice {
   float v0f, vinvf;   // binary32 value guess
   float vtc;          // -v0f * vinvf rounded to binary32: t = fmaf(v, vinvf, vtc)
   float vslack;       // binary32 value-axis slack in units of t (edge non-uniformity + rounding)
+  // the same with one margin for every value in range: vtcu = vtc + margin, veps2 = 2 margin
+  float vtcu, veps2;
   float vabs;         // binary32 value-axis absolute slack of searched edges (LinearBinEdges rule)
   int32_t v_fx;       // value edges uniform to 1/64 of a bin: fixed-point joint accumulation allowed
   // fixed-point joint accumulation: a value v of value bin g (0-based) is stored as the integer
@@ -242,6 +246,9 @@ inline constexpr int kCell32Max = 1024;
 // largest re-bin queue staged in LDS per workgroup (entries, split evenly between its waves);
 // the host shrinks it where the LDS it takes would cost a workgroup per CU
 inline constexpr int kQueueCap = 8192;
+// binary64 kernel: queued pairs per wave (8 bytes each) evaluated together by the reference's
+// sequence (64: every lane takes one)
+inline constexpr int kRareQueue = 64;
 // LDS queue header: one fill counter per wave (at most 16 waves of 64 lanes)
 inline constexpr int kQueueHead = 64;
 // largest global re-bin queue (entries of 16 bytes: 4 GiB); a call needing more is redone with
@@ -272,7 +279,9 @@ inline __host__ __device__ SmemLayout smem_layout(int n_dist, int n_val, int nce
   // nothing to add (never flushed); a B-strip launch keeps one histogram per field
   const int one = (n_val > 0) ? joint_layout(n_dist, n_val, jlayout).slots : n_dist;
   const int nh = one * copies * (strip > 1 ? strip : 1) + kDummySlots;
+  // the key table comes first: its reads then take their offset from the instruction
   int o = 0;
+  L.tab = o; o += 16 * ((n_val > 0 && ncell_max < kCell32Max) ? kCell32Max : ncell_max);
   L.hs = o; o += 8 * nh * nmom;
   L.hc = o; o += fx ? 0 : 4 * ((nh + 3) & ~3);  // fixed-point cells carry their count
   const int nz = fx ? kZeroBins * n_dist + kDummySlots : 0;
@@ -282,7 +291,6 @@ inline __host__ __device__ SmemLayout smem_layout(int n_dist, int n_val, int nce
   const int nm = n1d > 0 ? n_dist * mcopies + kDummySlots : 0;
   L.ms = o; o += 8 * nm * fused_pad(n1d);
   L.mc = o; o += 4 * ((nm + 3) & ~3);
-  L.tab = o; o += 16 * ((n_val > 0 && ncell_max < kCell32Max) ? kCell32Max : ncell_max);
   L.dE = o; o += 8 * ((n_dist + 2) & ~1);
   L.vE = o; o += 8 * ((n_val + 2) & ~1);
   L.vE32 = o; o += 4 * ((n_val + 4) & ~3);

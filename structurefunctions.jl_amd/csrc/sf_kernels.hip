@@ -3,10 +3,11 @@
 // Kernels
 //   prep64<G,D>      per-point binary64 records (sphere: sincosd once per point, not per pair)
 //   prep32<G,D>      per-point binary32 records for the mixed kernel
-//   hist64<G,D,J>    persistent upper-triangle tile kernel, binary64 pair arithmetic written in
-//                    the reference's operation order: counts bit-identical to SerialBackend
-//                    (bins certified from the exact key and value, the reference's rules where a
-//                    key or value is within the margin of a decision point)
+//   hist64<G,D,J>    persistent upper-triangle tile kernel, binary64 pair arithmetic in difference
+//                    form (pair64f; some joint operators in the reference's operation order):
+//                    counts bit-identical to SerialBackend (bins certified from the exact key and
+//                    value, the reference's sequence and rules where a key or value is within the
+//                    margin of a decision point)
 //   hist32<G,D,J>    same schedule, binary32 pair arithmetic; a pair whose distance key or value
 //                    lies within the binary32 error bound of a bin edge (or is degenerate) is
 //                    appended to a queue instead of being binned
@@ -22,13 +23,20 @@
 // accumulators with global atomics when it changes slice, before its 32-bit counts could wrap,
 // and when it runs out of items.
 //
-// All files of this library are compiled with -ffp-contract=off: the binary64 path must perform
+// All files of this library are compiled with -ffp-contract=off: the exact path must perform
 // exactly the operations of the reference (src/HelperFunctions.jl, src/StructureFunctionTypes.jl,
-// src/BinEdges.jl) with no fused multiply-adds.  The binary32 path asks for fma explicitly.
+// src/BinEdges.jl) with no fused multiply-adds.  The other paths ask for fma explicitly.
 #include <hip/hip_runtime.h>
 
 #include "sf_internal.h"
 #include "sfmath.h"
+
+// The file is compiled in five parts (SF_PART, see the Makefile) so that a build uses several
+// cores: part 0 holds the O(N) kernels and the launchers, parts 1 .. 4 the pair kernels of flat
+// D = 2, flat D = 3, sphere D = 2 and sphere D = 3.
+#ifndef SF_PART
+#error "compile with -DSF_PART=0 .. 4"
+#endif
 
 namespace sfk {
 
@@ -298,6 +306,7 @@ DEV T sp_invariant(int t, T duL, T dn2) {
 }
 
 DEV int cell32(float key, const Slice &s);
+DEV unsigned cell32_off(float key, const Slice &s);
 
 // CERT (sphere): the distance bin is read from the chord^2 cell table of the binary32 kernel
 // (lo, hi, blo: ambiguity interval and bin count per cell) with the binary64 chord^2 |q - p|^2,
@@ -517,6 +526,32 @@ __global__ void prep32(const PrepSlice *ps, const double *rec64, float *rec32) {
   o[Rec<G, D>::id] = __int_as_float((int)src);
 }
 
+// Spherical records of the binary64 kernel's pair (kF64Rec doubles per point): the unit position P,
+// twice the tangent velocity U = u_e E + u_n N in R^3 and the radial component, so that the pair
+// needs neither the local frame nor the (east, north) components (twice: the pair divides by
+// |p + q| |q - p| = 2 sin); the last word holds 2^-12 times an upper bound of the velocity norm
+// (binary32) and the point's index in the caller's order.
+template <int D>
+__global__ void prep64s(const PrepSlice *ps, const double *rec64, double *recf) {
+  const PrepSlice s = ps[blockIdx.y];
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= s.N) return;
+  constexpr int S = Rec<kSphere, D>::d64;
+  const int64_t src = s.perm ? (int64_t)s.perm[i] : (s.mul ? (i * s.mul) % s.N : i);
+  const double *r = rec64 + (s.pt_off + src) * S;
+  double *o = recf + (s.pt_off + i) * kF64Rec;
+  const double ue = r[8], un = r[9];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) o[k] = r[k];
+  o[3] = 2.0 * (ue * r[3] + un * r[5]);
+  o[4] = 2.0 * (ue * r[4] + un * r[6]);
+  o[5] = 2.0 * (un * r[7]);
+  o[6] = r[10];
+  const double n2 = ue * ue + un * un + (D == 3 ? r[10] * r[10] : 0.0);
+  const float nrm = round_up_f(__builtin_sqrt(n2) * (1.0 + 1e-12));
+  o[7] = __hiloint2double((int)src, __float_as_int(0x1p-12f * nrm));
+}
+
 // =============================================================================================
 // persistent histogram kernels
 // =============================================================================================
@@ -535,6 +570,7 @@ struct Smem {
   char *stage;
   int ncell_h;
   int copies;     // 1D: lane-group copies; joint: copies by lane halves (1 or 2)
+  int lcop;       // 1D: log2 of copies (slots by shift: an integer multiply takes 4 times as long)
   bool joint;
   int nd, nslots;
   int jv, jd, jslots;  // joint slot of (d, v) in one copy: v jv + d jd; a copy holds jslots slots
@@ -551,6 +587,7 @@ struct Smem {
   double *ms;
   unsigned *mc;
   int n1d, mcop, mstr, mscr;
+  int lmcop;                // log2 of mcop
   int qcap;                 // re-bin queue staged in LDS: entries in all
   int qw;                   // entries per wave: wave w owns q[w qw, (w + 1) qw) and fill qn[w]
   unsigned *qn;
@@ -567,6 +604,7 @@ DEV Smem carve(char *base, const Params &P, int stage_bytes) {
   m.fx = P.fx != 0;
   m.ncell_h = P.n_dist * (P.n_val > 0 ? P.n_val : 1);
   m.copies = P.copies;
+  m.lcop = __ffs(P.copies) - 1;
   m.joint = P.n_val > 0;
   m.nd = P.n_dist;
   const JointLayout JL = joint_layout(P.n_dist, P.n_val, P.jlayout);
@@ -587,6 +625,7 @@ DEV Smem carve(char *base, const Params &P, int stage_bytes) {
   m.mc = (unsigned *)(base + L.mc);
   m.n1d = P.n1d;
   m.mcop = P.mcopies > 0 ? P.mcopies : 1;
+  m.lmcop = __ffs(m.mcop) - 1;
   m.mstr = P.n_dist * m.mcop + kDummySlots;
   m.mscr = P.n_dist * m.mcop + (int)__lane_id();
   m.tab = (Cell *)(base + L.tab);
@@ -644,7 +683,7 @@ DEV void flush_multi(const Smem &m, const Params &P, int slice_id) {
 // LDS slot of output cell c = db0 + n_dist * vb0 (0-based bins) for this lane
 DEV int hslot(const Smem &m, int db0, int vb0) {
   if (m.joint) return vb0 * m.jv + db0 * m.jd + m.coff;
-  return db0 * m.copies + (__lane_id() & (m.copies - 1));
+  return (db0 << m.lcop) + (int)(__lane_id() & (m.copies - 1));
 }
 
 // one pair into LDS slot h: the value, or (single pass) the four moments of (du_L, |du|^2) in the
@@ -780,8 +819,44 @@ DEV void load_tables(const Smem &m, const Params &P, const Slice &s, bool fast32
   }
 }
 
+// Exclusive prefix sum of n (< 64) over the active lanes of the wave, from one ballot per bit;
+// *total receives the sum.  Works with any set of active lanes.
+DEV unsigned wave_prefix(unsigned n, unsigned *total) {
+  const unsigned long long lt = (1ull << __lane_id()) - 1ull;
+  unsigned tot = 0, pre = 0;
+#pragma unroll
+  for (int b = 0; b < 6; ++b) {
+    const unsigned long long bal = __ballot((n >> b) & 1u);
+    tot += (unsigned)__popcll(bal) << b;
+    pre += (unsigned)__popcll(bal & lt) << b;
+  }
+  *total = tot;
+  return pre;
+}
+
+// One atomic add of `total` for the whole wave, by its first active lane; returns the old value
+// to every lane.
+template <typename T>
+DEV T wave_reserve(T *counter, T total) {
+  const int leader = __ffsll((long long)__ballot(1)) - 1;
+  T base = 0;
+  if ((int)__lane_id() == leader) base = atomicAdd(counter, total);
+  return __shfl(base, leader);
+}
+
+// the wave's index in its workgroup, in an SGPR
+DEV int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+
+// Orders the wave's LDS accesses to its queue segment: entries written by one lane are read by
+// another lane of the same wave.
+DEV void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------------------------------------
-// hist64: binary64 exact pair arithmetic for every pair
+// hist64: binary64 pair arithmetic
 // ---------------------------------------------------------------------------------------------
 template <int G, int D, bool J, int OPK, bool MASK>
 DEV void pair64(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j,
@@ -796,7 +871,7 @@ DEV void pair64(const Params &P, const Slice &s, const Smem &m, const double *ri
     c = exact_cell<G, D, J, OPK>(P, s, ri, rj, m.tab, m.dE, m.vE, v, nullptr, nullptr, bins);
   // the slot from the bins (no division of c), and a pair that is not counted goes to the lane's
   // scratch slot (never flushed): the update is unconditional, the loop body has no branch here
-  int h = J ? bins[1] * m.jv + bins[0] * m.jd + m.coff : bins[0] * m.copies + (int)(__lane_id() & (m.copies - 1));
+  int h = J ? bins[1] * m.jv + bins[0] * m.jd + m.coff : (bins[0] << m.lcop) + (int)(__lane_id() & (m.copies - 1));
   h = c >= 0 ? h : m.scr;
   if constexpr (OPK == 3) hist_add_sp(m, h, v[0], v[1]);
   else hist_add(m, h, v[0]);
@@ -858,6 +933,13 @@ DEV int tile_row() {
 // margin of a value decision point, by the exact rules.  Flat keys that are not above 2^-100
 // (coincident points, NaN) also take the exact rules.  A pair that is not counted updates the
 // lane's scratch slot.
+// the binary64 launches that take the difference form (pair64f): every 1D operator and the single
+// pass, and the joint du_L and du_L^2; the other joint operators keep the reference's sequence
+inline constexpr bool fast64(bool J, int opk) { return !J || opk == 1 || opk == 2; }
+// doubles per point of the records it reads: the flat binary64 records, or prep64s's
+template <int G, int D>
+inline constexpr int rec_pair64 = (G == kFlat) ? Rec<G, D>::d64 : kF64Rec;
+
 struct Pending64 {
   int h;
   double v, w;  // value (single pass: du_L) and |du|^2 (single pass)
@@ -882,9 +964,9 @@ DEV void pair64p(const Params &P, const Slice &s, const Smem &m, const double *A
     r2 = sdot<D>(dx, dx);
     key = (float)r2;
   }
-  const int c = cell32(key, s);
-  const float2 lh = m.lohi[c];
-  const int blo = m.blo[c].x;
+  const unsigned c = cell32_off(key, s);
+  const float2 lh = *(const float2 *)((const char *)m.lohi + c);
+  const int blo = ((const int2 *)((const char *)m.blo + c))->x;
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (OPK == 3) hist_add_sp(m, pa.h, pa.v, pa.w);
   else hist_add(m, pa.h, pa.v);
@@ -974,7 +1056,7 @@ DEV void pair64p(const Params &P, const Slice &s, const Smem &m, const double *A
   const bool add = (!MASK || j > i) & ok & ((unsigned)(db - 1) < (unsigned)P.n_dist) &
                    (!J || (unsigned)(vb - 1) < (unsigned)P.n_val);
   const int h = J ? (vb - 1) * m.jv + (db - 1) * m.jd + m.coff
-                  : (db - 1) * m.copies + (int)(__lane_id() & (m.copies - 1));
+                  : ((db - 1) << m.lcop) + (int)(__lane_id() & (m.copies - 1));
   pa.h = add ? h : m.scr;
   pa.v = v;
   pa.w = w;
@@ -1008,10 +1090,320 @@ DEV void run_cols64p(const Params &P, const Slice &s, const Smem &m, const doubl
   else run_cols64pv<G, D, J, OPK, MASK, false>(P, s, m, ri, i, j0, j1, rec);
 }
 
+// ---------------------------------------------------------------------------------------------
+// The binary64 pair in difference form (every 1D operator, and the joint du_L and du_L^2).
+//
+//   flat    du_L = du.dx / |dx|,  du_T = (du x dx)_z / |dx|      from du = u_j - u_i, dx = x_j - x_i
+//   sphere  du_L = d.dU / sin,    du_T = (p x d).dU / sin        from d = q - p, dU = U_j - U_i,
+//           sin^2 = |d|^2 |p + q|^2 / 4   (U_A is tangent at p and U_B at q, so the reference's
+//           t_B.U_B - t_A.U_A is d.(U_B - U_A) / sin exactly)
+//
+// All of it in binary64, 1 / |dx| and 1 / sin from the hardware's estimate with one third-order
+// step (its error is the last multiply-add's rounding).  The reference's sequence forms the frame
+// of every pair (on the sphere two tangent vectors, four projections on the local bases, a square
+// root and a division: 92 binary64 operations); this one takes 19 and the reciprocal square root,
+// and its rounding errors are no larger: differences of nearby points are exact here, where the
+// reference subtracts two projections of the full velocities.
+//
+// What bounds it: the vector ALU, where a binary64 add or multiply-add takes 4.5 cycles per wave,
+// a binary32 multiply-add 4 and a binary32 add 2.5 (so splitting values into binary32 pairs saves
+// nothing), and, for joint histograms, the LDS unit (a binary64 atomic on scattered slots takes 23
+// cycles per wave and CU).
+//
+// Bins are certified as in pair64p; what is not certain goes through exact_cell, the reference's
+// own sequence: a key in a cell's ambiguity interval, nearly coincident or
+// nearly antipodal points, a non-finite value, and, for joint histograms, a value within its
+// margin of a value edge or small against the velocities (|du_L| below 2^-12 of their norms on
+// the sphere, of |du| on the flat geometry).  The last rule keeps every joint cell within rounding
+// of the reference's sequence relative to its own sum: two sequences agree to a few 2^-53 of the
+// velocities, so a larger value agrees to 2^-38 of itself, which also keeps the value bins'
+// margins (2^-22 and more, relative) valid.
+//
+// Those pairs (5e-4 of the spherical joint workload's) are not evaluated where they are found:
+// the loop collects flags, every 32 columns the flagged pairs are appended to the wave's segment
+// of an LDS queue, and a full segment is evaluated by the wave with all its lanes (rare64).  A
+// branch in the loop ran the exact sequence for one lane or two at a time, and its registers made
+// the loop spill: N = 100003, 14.2 ms against 22.6 before the difference form.
+// ---------------------------------------------------------------------------------------------
+DEV double rsqrt64(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-(x * y), y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+
+template <int D>
+DEV double fdot(const double *a, const double *b) {
+  double s = a[0] * b[0];
+#pragma unroll
+  for (int k = 1; k < D; ++k) s = __builtin_fma(a[k], b[k], s);
+  return s;
+}
+
+// operator value from du_L, du_T (signed transverse), ||du||^2 - du_L^2 and ||du||^2
+template <int OPK>
+DEV double op64(const Params &P, int D, double L, double T, double tn2, double n2) {
+  if constexpr (OPK == 1) return L;
+  else if constexpr (OPK == 2) return L * L;
+  else if constexpr (OPK == 5) return L * L * L;
+  else if constexpr (OPK == 6) return T;
+  else if constexpr (OPK == 7) return tn2;
+  else if constexpr (OPK == 8) return T * T * T;
+  else {
+    switch (P.op) {
+      case 0: {
+        double ex = 1.0;
+        if (P.nl != 0) ex = ipow(L, P.nl);
+        if (P.nt != 0) ex = ex * (P.nt == 2 ? tn2 : ipow(T, P.nt));
+        return ex;
+      }
+      case 1: return n2;
+      case 2: return L * n2;
+      case 3: return tn2 / (double)(D - 1);
+      case 4: return L * (tn2 / (double)(D - 1));
+      default: return P.nl == 2 ? n2 : ipow(__builtin_sqrt(n2), P.nl);
+    }
+  }
+}
+
+// exact_cell on the caller's points i and j of the slice (any order), from the binary64 records
+template <int G, int D, bool J, int OPK>
+DEV int exact_points(const Params &P, const Slice &s, const Smem &m, int i, int j, double *v, int *bins) {
+  constexpr int S = Rec<G, D>::d64;
+  const int lo = i < j ? i : j, hi = i < j ? j : i;
+  double A[S], B[S];
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    A[k] = P.rec64[(s.pt_off + lo) * S + k];
+    B[k] = P.rec64[(s.pt_off + hi) * S + k];
+  }
+  return exact_cell<G, D, J, (OPK <= 4 ? OPK : 0)>(P, s, A, B, P.cells + s.tab_off, m.dE, m.vE, v, nullptr,
+                                                   nullptr, bins);
+}
+
+// whether a searched value edge next to 0-based bin g lies within 2^-34 (relative) of v: the two
+// sequences' values of a pair agree to 2^-37 there
+DEV bool near_value_edge(double v, const double *E, int nE, int g) {
+  const double tol = 0x1p-34 * __builtin_fabs(v);
+  bool near = !(__builtin_fabs(v) < __builtin_inf());
+  if (g >= 0 && g < nE) near = near | !(__builtin_fabs(v - E[g]) > tol);
+  if (g + 1 >= 0 && g + 1 < nE) near = near | !(__builtin_fabs(v - E[g + 1]) > tol);
+  return near;
+}
+
+template <int G, int D, bool J, int OPK, bool MASK, bool VU>
+DEV bool pair64f(const Params &P, const Slice &s, const Smem &m, const double *A, int i, int j,
+                 const double *B, double *rn, const double *next, Pending64 &pa) {
+  constexpr int S = rec_pair64<G, D>;
+  constexpr int W = (G == kFlat) ? D : 3;  // space the differences live in
+  constexpr int UO = (G == kFlat) ? D : 3; // first velocity word of a record
+  constexpr bool SP = (OPK == 3);
+  constexpr bool needT = (OPK == 0) || (OPK >= 6) || (SP && G == kSphere);
+  constexpr bool needN2 = (OPK == 0) || (OPK == 7) || SP;
+  double d[W], du[W];
+#pragma unroll
+  for (int k = 0; k < W; ++k) d[k] = B[k] - A[k];
+  const double key64 = fdot<W>(d, d);
+  const float key = (float)key64;
+  const unsigned c = cell32_off(key, s);
+  const float2 lh = *(const float2 *)((const char *)m.lohi + c);
+  const int bm1 = ((const int2 *)((const char *)m.blo + c))->y;
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (SP) hist_add_sp(m, pa.h, pa.v, pa.w);
+  else hist_add(m, pa.h, pa.v);
+  asm volatile("" ::"v"(lh.x), "v"(lh.y), "v"(bm1) : "memory");
+  // outside [lo, hi] a key is above the edge exactly when key >= lo
+  const bool ge = key >= lh.x;
+  bool rare = ge & (key <= lh.y);
+  int db0 = ge ? bm1 + 1 : bm1;
+  rare = rare | !(key > 0x1p-100f);
+  double e2 = 0.0;
+  if constexpr (G == kSphere) {
+    double e[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) e[k] = B[k] + A[k];
+    e2 = fdot<3>(e, e);
+    rare = rare | !(e2 > 0x1p-24);
+  }
+#pragma unroll
+  for (int k = 0; k < W; ++k) du[k] = B[UO + k] - A[UO + k];
+  double dw = 0.0;
+  if constexpr (G == kSphere && D == 3) dw = B[6] - A[6];
+  float nj = 0.f;
+  if constexpr (G == kSphere && J) nj = __int_as_float(__double2loint(B[7]));
+  load_rec64<S>(next, rn);
+  __builtin_amdgcn_sched_barrier(0);
+  // (sphere: 2 sin = sqrt(key e2), and the records hold 2 U)
+  const double y = rsqrt64((G == kFlat) ? key64 : key64 * e2);
+  const double L = fdot<W>(d, du) * y;
+  double T = 0.0, tn2 = 0.0, n2 = 0.0;
+  if constexpr (G == kFlat) {
+    if constexpr (needN2) {
+      n2 = fdot<D>(du, du);
+      tn2 = n2 - L * L;
+    }
+    if constexpr (needT && OPK != 7) {
+      const double cz = __builtin_fma(du[1], d[0], -(du[0] * d[1]));
+      T = cz * (D == 2 ? y : rsqrt64(__builtin_fma(d[1], d[1], d[0] * d[0])));
+    }
+  } else if constexpr (needT) {
+    const double w[3] = {__builtin_fma(A[1], d[2], -(A[2] * d[1])), __builtin_fma(A[2], d[0], -(A[0] * d[2])),
+                         __builtin_fma(A[0], d[1], -(A[1] * d[0]))};
+    T = fdot<3>(w, du) * y;
+    tn2 = T * T;
+    if constexpr (D == 3) tn2 = __builtin_fma(dw, dw, tn2);
+    n2 = __builtin_fma(L, L, tn2);
+  }
+  double v = SP ? L : op64<OPK>(P, D, L, T, tn2, n2);
+  int vb0 = 0;
+  if constexpr (J) {
+    const float Lf = __builtin_fabsf((float)L);
+    if constexpr (G == kSphere) {
+      const float ni = __int_as_float(__double2loint(A[7]));
+      rare = rare | !(Lf > ni + nj);
+    } else {
+      float q = __builtin_fabsf((float)du[0]) + __builtin_fabsf((float)du[1]);
+      if constexpr (D == 3) q += __builtin_fabsf((float)du[2]);
+      rare = rare | !(Lf > 0x1p-12f * q);
+    }
+    if constexpr (VU) {  // s.v_uniform, chosen once per column range
+      // t + eps with the margin eps of the largest value that can be in range: a value outside
+      // the edges has a larger error (relative 2^-20), but stays outside.  Uncertain when a value
+      // edge lies within eps of t (NaN fails the comparison too).
+      const float t = __builtin_fmaf((float)v, s.vinvf, s.vtcu);
+      const float gh = __builtin_floorf(t);
+      rare = rare | !(t - gh >= s.veps2);
+      vb0 = (int)gh;
+    } else {
+      vb0 = (s.vrule.on ? lin_rule_bin(s.vrule, v, P.n_val) : val_bin64(v, m.vE, P.n_val + 1, s)) - 1;
+      // searched edges: a value close to one takes the reference's own value
+      rare = rare | near_value_edge(v, m.vE, P.n_val + 1, vb0);
+    }
+  } else if constexpr (SP) {
+    rare = rare | !(__builtin_fabs(L) < __builtin_inf()) | !(n2 < __builtin_inf());
+  } else {
+    rare = rare | !(__builtin_fabs(v) < __builtin_inf());
+  }
+  bool add = !rare & ((unsigned)db0 < (unsigned)P.n_dist);
+  if constexpr (J) add = add & ((unsigned)vb0 < (unsigned)P.n_val);
+  if constexpr (MASK) {
+    add = add & (j > i);
+    rare = rare & (j > i);
+  }
+  const int h = J ? vb0 * m.jv + db0 * m.jd + m.coff
+                  : (db0 << m.lcop) + (int)(__lane_id() & (m.copies - 1));
+  pa.h = add ? h : m.scr;
+  pa.v = v;
+  pa.w = n2;
+  return rare;
+}
+
+// Append the pairs (i, jl - t) whose bit t is set in dm to the wave's segment of the LDS queue.
+// Returns false, with nothing appended, when the segment has no room for all of them.
+DEV bool push_rare(const Smem &m, unsigned dm, int i, int jl) {
+  if (__ballot(dm != 0u) == 0ull) return true;
+  unsigned tot;
+  const unsigned pre = wave_prefix((unsigned)__popc(dm), &tot);
+  unsigned *fillp = m.qn + wave_index();
+  const unsigned fill = m.qw ? (unsigned)__builtin_amdgcn_readfirstlane((int)*fillp) : 0u;
+  if (fill + tot > (unsigned)m.qw) return false;
+  int2 *seg = m.q + wave_index() * m.qw + fill + pre;
+  unsigned e = 0;
+  while (dm) {
+    const int t = __ffs((int)dm) - 1;
+    dm &= dm - 1u;
+    seg[e++] = make_int2(i, jl - t);
+  }
+  *fillp = fill + tot;  // every active lane stores the same value
+  return true;
+}
+
+// Evaluate the wave's queued pairs, and then each lane's own pairs (i, jl - t) of dm, by the
+// reference's sequence, and add them to the workgroup's histogram.
+template <int G, int D, bool J, int OPK>
+DEV void rare64(const Params &P, const Slice &s, const Smem &m, const double *rec, unsigned dm, int i, int jl) {
+  const unsigned long long act = __ballot(1);
+  const unsigned na = (unsigned)__popcll(act);
+  unsigned k = (unsigned)__popcll(act & ((1ull << __lane_id()) - 1ull));
+  unsigned *fillp = m.qn + wave_index();
+  const unsigned fill = m.qw ? (unsigned)__builtin_amdgcn_readfirstlane((int)*fillp) : 0u;
+  if (fill == 0u && __ballot(dm != 0u) == 0ull) return;
+  wave_lds_sync();
+  const int2 *seg = m.q + wave_index() * m.qw;
+  for (;;) {
+    int2 e = make_int2(-1, 0);
+    if (k < fill) {
+      e = seg[k];
+      k += na;
+    } else if (dm) {
+      e = make_int2(i, jl - (__ffs((int)dm) - 1));
+      dm &= dm - 1u;
+    }
+    if (__ballot(e.x >= 0) == 0ull) break;
+    if (e.x >= 0) {
+      if constexpr (G == kSphere) {  // record indices to the caller's
+        e.x = __double2hiint(rec[(s.pt_off + e.x) * kF64Rec + 7]);
+        e.y = __double2hiint(rec[(s.pt_off + e.y) * kF64Rec + 7]);
+      }
+      double v[2] = {0.0, 0.0};
+      int bins[2] = {0, 0};
+      if (exact_points<G, D, J, OPK>(P, s, m, e.x, e.y, v, bins) >= 0) {
+        const int h = J ? bins[1] * m.jv + bins[0] * m.jd + m.coff
+                        : (bins[0] << m.lcop) + (int)(__lane_id() & (m.copies - 1));
+        if constexpr (OPK == 3) hist_add_sp(m, h, v[0], v[1]);
+        else hist_add(m, h, v[0]);
+      }
+    }
+  }
+  wave_lds_sync();
+  if (m.qw) *fillp = 0u;
+}
+
+// Columns j .. j1 - 1 of one row with pair64f, in groups of 32 (the flags are shifted in, so bit
+// t of dm flags column jl - t); two record buffers alternate (the request past the last column
+// reads at most one record beyond the slice, as in run_cols64).  Returns j1, or the first column
+// not done when a group's flagged pairs did not fit the queue: they are then left in dm, their
+// last column in jl.
+template <int G, int D, bool J, int OPK, bool MASK, bool VU>
+DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j, int j1,
+                    const double *__restrict__ rec, unsigned &dm_out, int &jl) {
+  constexpr int S = rec_pair64<G, D>;
+  // the slice offset is wave-uniform by construction; say so, so that the column addresses stay in
+  // SGPRs
+  const uint64_t po = (uint64_t)s.pt_off;
+  const int64_t off = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(po >> 32)) << 32) |
+                                (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)po));
+  const double *cp = rec + (off + __builtin_amdgcn_readfirstlane(j)) * S;
+  double ra[S], rb[S];
+  load_rec64<S>(cp, ra);
+  Pending64 pa{m.scr, 0.0, 0.0};
+  unsigned dm = 0u;
+  while (j < j1) {
+    const int je = min(j1, j + 32);
+    dm = 0u;
+    for (; j + 1 < je; j += 2, cp += 2 * S) {
+      dm = (dm << 1) | (unsigned)pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, cp + S, pa);
+      dm = (dm << 1) | (unsigned)pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * S, pa);
+    }
+    // an odd count only occurs in the last group (the others hold 32 columns)
+    if (j < je) {
+      dm = (dm << 1) | (unsigned)pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, cp + S, pa);
+      ++j;
+    }
+    jl = je - 1;
+    if (!push_rare(m, dm, i, jl)) break;
+    dm = 0u;
+  }
+  if constexpr (OPK == 3) hist_add_sp(m, pa.h, pa.v, pa.w);
+  else hist_add(m, pa.h, pa.v);
+  dm_out = dm;
+  return j;
+}
+
 template <int G, int D, bool J, int OPK>
 __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restrict__ rec) {
   extern __shared__ __align__(16) char smem_raw[];
-  constexpr int S = Rec<G, D>::d64;
+  constexpr bool FAST = fast64(J, OPK);
+  constexpr int S = FAST ? rec_pair64<G, D> : Rec<G, D>::d64;
   const Smem m = carve<J>(smem_raw, P, P.stage_bytes);
   __shared__ int s_item;
   const int B = blockDim.x;
@@ -1019,6 +1411,7 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
   Slice s{};
   unsigned long long since_flush = 0;
   zero_hist(m);
+  if ((threadIdx.x & 63) == 0 && m.qcap > 0) m.qn[threadIdx.x >> 6] = 0u;
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) s_item = atomicAdd(P.counter, 1);
@@ -1029,15 +1422,19 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
     const unsigned long long work = (unsigned long long)B * (unsigned long long)(w.j1 - w.j0);
     if (w.slice != cur || since_flush + work > (unsigned long long)P.flush_limit) {
       if (cur >= 0) {
+        if (FAST && w.slice != cur) {
+          rare64<G, D, J, OPK>(P, s, m, rec, 0u, 0, 0);
+          __syncthreads();
+        }
         flush_hist(m, P, s);
         __syncthreads();
       }
       if (w.slice != cur) {
         cur = w.slice;
         s = P.slices[cur];
-        // sphere and flat point fields: the binary32 key table of certified distance bins (the
+        // the binary32 key table of certified distance bins (the
         // binary64 key table is read from global memory by the rare pairs that need it)
-        load_tables(m, P, s, G == kSphere || !P.bl);
+        load_tables(m, P, s, FAST || G == kSphere || !P.bl);
       }
       since_flush = 0;
       __syncthreads();  // tables and cleared histogram visible before the item's pairs
@@ -1049,7 +1446,25 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
 #pragma unroll
     for (int k = 0; k < S; ++k) ri[k] = iv ? rec[(s.pt_off + i) * S + k] : 0.0;
     if (iv) {
-      if (G == kSphere || !P.bl) {
+      if constexpr (FAST) {
+        // the columns up to the tile's last row need the j > i mask, the others do not; the
+        // value-bin lookup (uniform or exact) is chosen per column range, not per pair
+        const int jm = min(w.j1, w.i0 + B);
+        for (int j = w.j0; j < w.j1;) {
+          unsigned dm = 0u;
+          int jl = 0;
+          const bool mask = j < jm;
+          const int je = mask ? jm : w.j1;
+          if (J && s.v_uniform) {
+            j = mask ? run_cols64f<G, D, J, OPK, true, true>(P, s, m, ri, i, j, je, rec, dm, jl)
+                     : run_cols64f<G, D, J, OPK, false, true>(P, s, m, ri, i, j, je, rec, dm, jl);
+          } else {
+            j = mask ? run_cols64f<G, D, J, OPK, true, false>(P, s, m, ri, i, j, je, rec, dm, jl)
+                     : run_cols64f<G, D, J, OPK, false, false>(P, s, m, ri, i, j, je, rec, dm, jl);
+          }
+          if (__ballot(dm != 0u)) rare64<G, D, J, OPK>(P, s, m, rec, dm, i, jl);
+        }
+      } else if (G == kSphere || !P.bl) {
         if (w.j0 < w.i0 + B) run_cols64p<G, D, J, OPK, true>(P, s, m, ri, i, w.j0, w.j1, rec);
         else run_cols64p<G, D, J, OPK, false>(P, s, m, ri, i, w.j0, w.j1, rec);
       } else {
@@ -1058,6 +1473,7 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
       }
     }
   }
+  if (FAST && cur >= 0) rare64<G, D, J, OPK>(P, s, m, rec, 0u, 0, 0);
   __syncthreads();
   if (cur >= 0) flush_hist(m, P, s);
 }
@@ -1084,6 +1500,18 @@ DEV int cell32(float key, const Slice &s) {
   return r;
 }
 
+
+// the same as a byte offset into the table's 8-byte entries.  The clamped offset is masked rather
+// than shifted: the mask shows the compiler a small non-negative offset, so that it folds the
+// tables' constant addresses into the reads.
+DEV unsigned cell32_off(float key, const Slice &s) {
+  static_assert(kCell32Max * 8 == 0x2000, "mask of the table's byte offsets");
+  const int bits = __float_as_int(key);
+  const int c = (bits >> (20 - s.M32)) - 8 * s.base32;
+  int r;
+  asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(c), "s"(8 * s.ncell32 - 1));
+  return (unsigned)r & 0x1ff8u;
+}
 
 // value-axis bin from a binary32 value with absolute error bound dv = dva * dvb; sets amb when
 // undecidable.  For uniform edges (VU) dva carries the factor 1 / bin width (the bound in bin
@@ -1468,7 +1896,7 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
   if constexpr (MULTI) {
     // the fused 1D outputs of a certain, in-range distance bin (whatever the joint value bin)
     const bool add1 = upper & !amb & db_ok;
-    const int h1 = add1 ? db0 * m.mcop + (int)(__lane_id() & (m.mcop - 1)) : m.mscr;
+    const int h1 = add1 ? (db0 << m.lmcop) + (int)(__lane_id() & (m.mcop - 1)) : m.mscr;
     atomicAdd(&m.mc[h1], 1u);
     double *const mp = m.ms + h1;
 #pragma unroll
@@ -1489,7 +1917,7 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
     asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(hv) : "v"(vb0), "s"(m.jv), "v"(m.coff));
     asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(h) : "v"(db0), "s"(m.jd), "v"(hv));
   } else {
-    h = db0 * m.copies + (__lane_id() & (m.copies - 1));
+    h = (db0 << m.lcop) + (int)(__lane_id() & (m.copies - 1));
   }
   if constexpr (FX) {
     // a value below a quarter bin width goes to the binary64 cell of its (distance, value) bin
@@ -1516,42 +1944,6 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
   // it implies comes after this pair's arithmetic, not right after the request.
   if constexpr (SL && F == 16) asm volatile("" ::"s"(rn[13]), "s"(rn[14]), "s"(rn[15]));
   return defer;
-}
-
-// Exclusive prefix sum of n (< 64) over the active lanes of the wave, from one ballot per bit;
-// *total receives the sum.  Works with any set of active lanes.
-DEV unsigned wave_prefix(unsigned n, unsigned *total) {
-  const unsigned long long lt = (1ull << __lane_id()) - 1ull;
-  unsigned tot = 0, pre = 0;
-#pragma unroll
-  for (int b = 0; b < 6; ++b) {
-    const unsigned long long bal = __ballot((n >> b) & 1u);
-    tot += (unsigned)__popcll(bal) << b;
-    pre += (unsigned)__popcll(bal & lt) << b;
-  }
-  *total = tot;
-  return pre;
-}
-
-// One atomic add of `total` for the whole wave, by its first active lane; returns the old value
-// to every lane.
-template <typename T>
-DEV T wave_reserve(T *counter, T total) {
-  const int leader = __ffsll((long long)__ballot(1)) - 1;
-  T base = 0;
-  if ((int)__lane_id() == leader) base = atomicAdd(counter, total);
-  return __shfl(base, leader);
-}
-
-// the wave's index in its workgroup, in an SGPR
-DEV int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
-
-// Orders the wave's LDS accesses to its queue segment: entries written by one lane are read by
-// another lane of the same wave.
-DEV void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Move the first `fill` entries of the wave's LDS segment to the global queue: one reservation
@@ -1898,7 +2290,7 @@ DEV void run_chunk_strip(const Params &P, const Slice &s, const Smem &m, const f
       const bool defer = upper & amb & (amb_d | db_ok);
       if (add) {
         // one count for the pair (every field of the strip shares the bin); one sum per field
-        const int h = (db - 1) * m.copies + slot0;
+        const int h = ((db - 1) << m.lcop) + slot0;
         atomicAdd(&m.hc[h], 1u);
 #pragma unroll
         for (int b = 0; b < kStripMax; ++b)
@@ -2195,6 +2587,7 @@ __global__ void __launch_bounds__(256) recheck_multi(Params P) {
   }
 }
 
+#if SF_PART == 0
 __global__ void merge_out(const double *src_s, const unsigned long long *src_c, double *dst_s,
                           unsigned long long *dst_c, int64_t n) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2272,6 +2665,8 @@ __global__ void zero_multi(ZeroSet z) {
   if (k < z.n[b]) z.p[b][k] = 0;
 }
 
+#endif  // SF_PART == 0
+
 }  // namespace sfk
 
 // =============================================================================================
@@ -2279,31 +2674,19 @@ __global__ void zero_multi(ZeroSet z) {
 // =============================================================================================
 namespace sfk {
 
-struct PrepSliceHost;
+// the kernels of one (geometry, D): histogram, B-strip, re-bin and fused re-bin entry points
+struct KernelTable {
+  const void *(*hist)(bool J, bool mixed, int opk, bool sload, bool fx);
+  const void *(*strip)(int opk);
+  const void *(*recheck)(bool J, bool sp);
+  const void *(*recheck_multi)(bool J);
+};
+KernelTable table_flat2();
+KernelTable table_flat3();
+KernelTable table_sphere2();
+KernelTable table_sphere3();
 
-template <int G, int D>
-static hipError_t prep_impl(bool mixed, int geom_code, const void *ps, int n_slices, int64_t max_n,
-                            double *rec64, float *rec32, hipStream_t st) {
-  if (max_n <= 0) return hipSuccess;
-  const int T = 256;
-  dim3 grid((unsigned)((max_n + T - 1) / T), (unsigned)n_slices);
-  prep64<G, D><<<grid, T, 0, st>>>((const PrepSlice *)ps, geom_code, rec64);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !mixed) return e;
-  prep32<G, D><<<grid, T, 0, st>>>((const PrepSlice *)ps, rec64, rec32);
-  return hipGetLastError();
-}
-
-hipError_t launch_prep(int G, int D, bool mixed, int geom_code, const void *ps, int n_slices,
-                       int64_t max_n, double *rec64, float *rec32, hipStream_t st) {
-  if (G == kFlat) {
-    return D == 2 ? prep_impl<kFlat, 2>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st)
-                  : prep_impl<kFlat, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st);
-  }
-  return D == 2 ? prep_impl<kSphere, 2>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st)
-                : prep_impl<kSphere, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st);
-}
-
+#if SF_PART > 0
 template <int G, int D, bool J, bool SL, bool FX>
 static const void *hist32_fn(int opk) {
   // fused outputs: scalar-loaded columns only
@@ -2342,6 +2725,10 @@ static const void *hist_fn(bool mixed, int opk, bool sload, bool fx) {
   if (mixed) return sload ? hist32_fx<G, D, J, true>(fx, opk) : hist32_fx<G, D, J, false>(fx, opk);
   if constexpr (!J) {
     if (opk == 3) return (const void *)&hist64<G, D, false, 3>;
+    if (opk == 5) return (const void *)&hist64<G, D, false, 5>;
+    if (opk == 6) return (const void *)&hist64<G, D, false, 6>;
+    if (opk == 7) return (const void *)&hist64<G, D, false, 7>;
+    if (opk == 8) return (const void *)&hist64<G, D, false, 8>;
   } else {
     if (opk == 4) return (const void *)&hist64<G, D, true, 4>;
   }
@@ -2350,13 +2737,82 @@ static const void *hist_fn(bool mixed, int opk, bool sload, bool fx) {
   return (const void *)&hist64<G, D, J, 0>;
 }
 
-static const void *pick_hist(int G, int D, bool J, bool mixed, int opk, bool sl, bool fx) {
-  if (G == kFlat) {
-    if (D == 2) return J ? hist_fn<kFlat, 2, true>(mixed, opk, sl, fx) : hist_fn<kFlat, 2, false>(mixed, opk, sl, fx);
-    return J ? hist_fn<kFlat, 3, true>(mixed, opk, sl, fx) : hist_fn<kFlat, 3, false>(mixed, opk, sl, fx);
+template <int G, int D>
+static const void *strip_fn(int opk) {
+  if (opk == 1) return (const void *)&hist32s<G, D, 1>;
+  if (opk == 2) return (const void *)&hist32s<G, D, 2>;
+  return (const void *)&hist32s<G, D, 0>;
+}
+
+template <int G, int D>
+static const void *recheck_fn(bool J, bool sp) {
+  if (J) return sp ? (const void *)&recheck<G, D, true, true> : (const void *)&recheck<G, D, true, false>;
+  return sp ? (const void *)&recheck<G, D, false, true> : (const void *)&recheck<G, D, false, false>;
+}
+
+template <int G, int D>
+static const void *recheck_multi_fn(bool J) {
+  return J ? (const void *)&recheck_multi<G, D, true> : (const void *)&recheck_multi<G, D, false>;
+}
+
+template <int G, int D>
+static const void *hist_of(bool J, bool mixed, int opk, bool sload, bool fx) {
+  return J ? hist_fn<G, D, true>(mixed, opk, sload, fx) : hist_fn<G, D, false>(mixed, opk, sload, fx);
+}
+template <int G, int D>
+static KernelTable table_of() {
+  return KernelTable{&hist_of<G, D>, &strip_fn<G, D>, &recheck_fn<G, D>, &recheck_multi_fn<G, D>};
+}
+#if SF_PART == 1
+KernelTable table_flat2() { return table_of<kFlat, 2>(); }
+#elif SF_PART == 2
+KernelTable table_flat3() { return table_of<kFlat, 3>(); }
+#elif SF_PART == 3
+KernelTable table_sphere2() { return table_of<kSphere, 2>(); }
+#elif SF_PART == 4
+KernelTable table_sphere3() { return table_of<kSphere, 3>(); }
+#endif
+#else  // SF_PART == 0
+struct PrepSliceHost;
+
+static KernelTable table(int G, int D) {
+  if (G == kFlat) return D == 2 ? table_flat2() : table_flat3();
+  return D == 2 ? table_sphere2() : table_sphere3();
+}
+
+
+template <int G, int D>
+static hipError_t prep_impl(bool mixed, int geom_code, const void *ps, int n_slices, int64_t max_n,
+                            double *rec64, float *rec32, hipStream_t st) {
+  if (max_n <= 0) return hipSuccess;
+  const int T = 256;
+  dim3 grid((unsigned)((max_n + T - 1) / T), (unsigned)n_slices);
+  prep64<G, D><<<grid, T, 0, st>>>((const PrepSlice *)ps, geom_code, rec64);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if (!mixed) {
+    // the binary64 kernel's spherical records take the binary32 records' place (same size)
+    if constexpr (G == kSphere) {
+      if (rec32) prep64s<D><<<grid, T, 0, st>>>((const PrepSlice *)ps, rec64, (double *)rec32);
+    }
+    return hipGetLastError();
   }
-  if (D == 2) return J ? hist_fn<kSphere, 2, true>(mixed, opk, sl, fx) : hist_fn<kSphere, 2, false>(mixed, opk, sl, fx);
-  return J ? hist_fn<kSphere, 3, true>(mixed, opk, sl, fx) : hist_fn<kSphere, 3, false>(mixed, opk, sl, fx);
+  prep32<G, D><<<grid, T, 0, st>>>((const PrepSlice *)ps, rec64, rec32);
+  return hipGetLastError();
+}
+
+hipError_t launch_prep(int G, int D, bool mixed, int geom_code, const void *ps, int n_slices,
+                       int64_t max_n, double *rec64, float *rec32, hipStream_t st) {
+  if (G == kFlat) {
+    return D == 2 ? prep_impl<kFlat, 2>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st)
+                  : prep_impl<kFlat, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st);
+  }
+  return D == 2 ? prep_impl<kSphere, 2>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st)
+                : prep_impl<kSphere, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st);
+}
+
+static const void *pick_hist(int G, int D, bool J, bool mixed, int opk, bool sl, bool fx) {
+  return table(G, D).hist(J, mixed, opk, sl, fx);
 }
 
 static int opk_of(const Params &P) {
@@ -2383,17 +2839,7 @@ int hist_occupancy(int G, int D, bool J, bool mixed, int opk, bool sload, bool f
 
 int hist_opk(const Params &P) { return opk_of(P); }
 
-template <int G, int D>
-static const void *strip_fn(int opk) {
-  if (opk == 1) return (const void *)&hist32s<G, D, 1>;
-  if (opk == 2) return (const void *)&hist32s<G, D, 2>;
-  return (const void *)&hist32s<G, D, 0>;
-}
-
-static const void *pick_strip(int G, int D, int opk) {
-  if (G == kFlat) return D == 2 ? strip_fn<kFlat, 2>(opk) : strip_fn<kFlat, 3>(opk);
-  return D == 2 ? strip_fn<kSphere, 2>(opk) : strip_fn<kSphere, 3>(opk);
-}
+static const void *pick_strip(int G, int D, int opk) { return table(G, D).strip(opk); }
 
 int strip_occupancy(int G, int D, int opk, int block, size_t smem) {
   const void *f = pick_strip(G, D, opk);
@@ -2409,26 +2855,16 @@ hipError_t launch_hist(int G, int D, bool J, bool mixed, bool sload, const Param
                                          : pick_hist(G, D, J, mixed, opk_of(P), sload, mixed && P.fx);
   (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   Params Pc = P;
-  const void *rec = mixed ? (const void *)P.rec32 : (const void *)P.rec64;
+  const int opk = opk_of(P);
+  const bool f64s = !mixed && G == kSphere && fast64(J, opk);  // prep64s's records
+  const void *rec = (mixed || f64s) ? (const void *)P.rec32 : (const void *)P.rec64;
   void *args[] = {&Pc, &rec};
   return hipLaunchKernel(f, dim3(grid), dim3(block), args, smem, st);
 }
 
-template <int G, int D>
-static const void *recheck_fn(bool J, bool sp) {
-  if (J) return sp ? (const void *)&recheck<G, D, true, true> : (const void *)&recheck<G, D, true, false>;
-  return sp ? (const void *)&recheck<G, D, false, true> : (const void *)&recheck<G, D, false, false>;
-}
-
-template <int G, int D>
-static const void *recheck_multi_fn(bool J) {
-  return J ? (const void *)&recheck_multi<G, D, true> : (const void *)&recheck_multi<G, D, false>;
-}
-
 hipError_t launch_recheck(int G, int D, bool J, const Params &P, int grid, hipStream_t st) {
   if (P.n1d > 0) {
-    const void *f = G == kFlat ? (D == 2 ? recheck_multi_fn<kFlat, 2>(J) : recheck_multi_fn<kFlat, 3>(J))
-                               : (D == 2 ? recheck_multi_fn<kSphere, 2>(J) : recheck_multi_fn<kSphere, 3>(J));
+    const void *f = table(G, D).recheck_multi(J);
     Params Pc = P;
     void *args[] = {&Pc};
     const size_t nh = J ? (size_t)P.n_dist * P.n_val : 0;
@@ -2437,9 +2873,7 @@ hipError_t launch_recheck(int G, int D, bool J, const Params &P, int grid, hipSt
     return hipLaunchKernel(f, dim3(grid), dim3(256), args, smem, st);
   }
   const bool sp = P.nmom > 1 || sp2d(P.op, P.n_val);
-  const void *f;
-  if (G == kFlat) f = D == 2 ? recheck_fn<kFlat, 2>(J, sp) : recheck_fn<kFlat, 3>(J, sp);
-  else f = D == 2 ? recheck_fn<kSphere, 2>(J, sp) : recheck_fn<kSphere, 3>(J, sp);
+  const void *f = table(G, D).recheck(J, sp);
   Params Pc = P;
   void *args[] = {&Pc};
   const int nh = P.n_dist * (P.n_val > 0 ? P.n_val : 1);
@@ -2497,5 +2931,7 @@ hipError_t launch_zero_multi(int count, void *const *p, const int64_t *bytes, hi
   zero_multi<<<dim3((unsigned)((nmax + 255) / 256), (unsigned)count), 256, 0, st>>>(z);
   return hipGetLastError();
 }
+
+#endif  // SF_PART
 
 }  // namespace sfk
