@@ -562,6 +562,14 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   if (P32.ehi <= P32.elo) P32.ehi = P32.elo + 1;
   const int n32 = P32.ncell();  // <= kCell32Max: at most 252 binades, M chosen to fit
   T.tab32.resize(n32);
+  // Nearly coincident points: the binary32 records carry positions as hi + lo (2^-48 relative), a
+  // direction error of 2^-48 / separation that below a separation of 2^-22 (sphere: radians; flat:
+  // times max|x|) would outgrow the value bound's margin and the reference's own binary64 accuracy
+  // (2^-53 / separation); below 1e-30 products of tiny differences underflow.  Nearly antipodal
+  // points, within 2^-10 rad: sin(separation) and the error bound's 1 / sin lose their accuracy.
+  const float close = flat ? round_up_f(std::max(1e-30L, ldexpl((long double)xmax * (long double)xmax, -44)))
+                           : 0x1p-44f;
+  const float anti = 4.0f - 0x1p-20f;
   for (int c = 0; c < n32; ++c) {
     const float Fc = (c == 0) ? -INFINITY : (float)P32.low(c);
     const float Fn = (c + 1 >= n32) ? INFINITY : (float)P32.low(c + 1);
@@ -585,6 +593,27 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
       cl.lo = -INFINITY;
       cl.hi = INFINITY;
     }
+    // keys that the kernels leave to the exact sequence wherever a bin holds them: those of nearly
+    // coincident points (below `close`) and on the sphere of nearly antipodal ones
+    if (Fc < close) {
+      if (nint == 0) {
+        if (below > 0 && below < nE) {
+          cl.lo = -INFINITY;
+          cl.hi = close;
+          cl.blo = below - 1;
+        }
+      } else if (nint == 1 && hi[which] <= close) {  // an edge at or near zero
+        cl.lo = -INFINITY;
+        cl.hi = close;
+      } else if (!(nint == 1 && below == 0 && lo[which] > close)) {  // (else nothing counted below the edge)
+        cl.lo = -INFINITY;
+        cl.hi = INFINITY;
+      }
+    }
+    if (!flat && below + nint > 0 && below < nE && Fn > anti && Fc < 8.0f) {
+      cl.lo = nint == 0 ? anti : std::min(cl.lo, anti);
+      cl.hi = INFINITY;
+    }
   }
   Slice &s = T.desc;
   s.drule = lin_rule_of(p.dist_rule);
@@ -598,7 +627,7 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   // value axis
   s.v_uniform = 0;
   s.v_negzero = 0;
-  s.v0 = 0; s.vinv = 0; s.v0f = 0; s.vinvf = 0; s.vtc = 0; s.vslack = 0; s.vabs = 0; s.vtcu = 0; s.veps2 = 0;
+  s.v0 = 0; s.vinv = 0; s.v0f = 0; s.vinvf = 0; s.vtc = 0; s.vslack = 0; s.vabs = 0; s.vslackt = 0; s.vtcu = 0; s.veps2 = 0;
   s.v_fx = 0; s.vwf = 0; s.vsf = 0; s.fxc1 = 0; s.fxc0 = 0; s.plane = 0; s.vsmall = 0; s.gz = 0;
   s.v_log = 0; s.vk0 = 0; s.vl0f = 0; s.vlinvf = 0;
   if (p.n_val > 0) {
@@ -624,6 +653,7 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
         const long double u = ldexpl(1.0L, -24);
         s.vslack = round_up_f(dev + 4.0L * u * (1.0L + fabsl((long double)v0 / w)) + 4.0L * u * nv + 1e-6L +
                               rule_slack(p.val_rule) / w);
+        s.vslackt = round_up_f((long double)s.vslack + 4.8e-7L * (nv + 2));
         // one margin for every value in range (|t| < nv + 1): 16u |t| covers the rounding of the
         // multiply-add, of the value and of the sums vtc + margin and t - floor(t)
         const long double eps = (long double)s.vslack + 24.0L * u * (nv + 2) + 4.0L * u * fabsl((long double)s.vtc);

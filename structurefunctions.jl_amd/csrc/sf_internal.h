@@ -74,7 +74,8 @@ struct Slice {
   float v0f, vinvf;   // binary32 value guess
   float vtc;          // -v0f * vinvf rounded to binary32: t = fmaf(v, vinvf, vtc)
   float vslack;       // binary32 value-axis slack in units of t (edge non-uniformity + rounding)
-  // the same with one margin for every value in range: vtcu = vtc + margin, veps2 = 2 margin
+  float vslackt;      // vslack and the rounding of t and of the two offsets, for every value in range
+  // the same with one margin for every value in range (binary64 kernel): vtcu = vtc + margin, veps2 = 2 margin
   float vtcu, veps2;
   float vabs;         // binary32 value-axis absolute slack of searched edges (LinearBinEdges rule)
   int32_t v_fx;       // value edges uniform to 1/64 of a bin: fixed-point joint accumulation allowed

@@ -703,7 +703,8 @@ DEV void hist_add_sp(const Smem &m, int h, T duL, T dn2) {
   atomicAdd(&m.hc[h], 1u);
 }
 
-DEV void flush_hist(const Smem &m, const Params &P, const Slice &s) {
+DEV void flush_hist(const Smem &m, const Params &P, const Slice &s, int cur) {
+  const int64_t out_off = P.slices[cur].out_off;  // (read here: not held over the pair loops)
   // output cell c of the slice is out_off + c, or every sixth cell for a 2D single-pass plane
   const int64_t ostride = sp2d(P.op, P.n_val) ? kSpRows : 1;
   if (m.fx) {
@@ -727,7 +728,7 @@ DEV void flush_hist(const Smem &m, const Params &P, const Slice &s) {
         // division
         const float cg = __builtin_fmaf(-(float)vb0, s.fxc1, s.fxc0);
         const double v = ((double)sq + (double)n * (8388608.0 - (double)cg)) / (double)s.vsf;
-        const int64_t o = s.out_off + ostride * c;
+        const int64_t o = out_off + ostride * c;
         atomicAdd(&P.counts[o], n);
         atomicAdd(&P.sums[o], v);
       }
@@ -739,7 +740,7 @@ DEV void flush_hist(const Smem &m, const Params &P, const Slice &s) {
       m.zs[c] = 0.0;
       const int db0 = c / kZeroBins, vb0 = s.gz + c % kZeroBins;
       if (n && vb0 >= 0 && vb0 < P.n_val) {
-        const int64_t o = s.out_off + ostride * (db0 + m.nd * vb0);
+        const int64_t o = out_off + ostride * (db0 + m.nd * vb0);
         atomicAdd(&P.counts[o], (unsigned long long)n);
         atomicAdd(&P.sums[o], v);
       }
@@ -762,7 +763,7 @@ DEV void flush_hist(const Smem &m, const Params &P, const Slice &s) {
         }
       }
       if (n) {
-        const int64_t o = s.out_off + (int64_t)kSpRows * c;
+        const int64_t o = out_off + (int64_t)kSpRows * c;
         atomicAdd(&P.counts[o], n);
 #pragma unroll
         for (int q = 0; q < 4; ++q) atomicAdd(&P.sums[o + sp_row(q)], v[q]);
@@ -792,8 +793,8 @@ DEV void flush_hist(const Smem &m, const Params &P, const Slice &s) {
       }
     }
     if (n) {
-      atomicAdd(&P.counts[s.out_off + ostride * c], n);
-      atomicAdd(&P.sums[s.out_off + ostride * c], v);
+      atomicAdd(&P.counts[out_off + ostride * c], n);
+      atomicAdd(&P.sums[out_off + ostride * c], v);
     }
   }
 }
@@ -818,6 +819,26 @@ DEV void load_tables(const Smem &m, const Params &P, const Slice &s, bool fast32
     }
   }
 }
+
+// ---------------------------------------------------------------------------------------------
+// Lane masks.  A pair's conditions are combined as 64-bit masks on the scalar unit: a bool that is
+// combined from several compares and then turned into a mask (a ballot, a flag shifted into a bit
+// mask) costs two vector instructions each time, and the pair loops are bound by those.
+// ---------------------------------------------------------------------------------------------
+typedef unsigned long long lanes_t;
+// the builtins take the compiler's predicate codes
+DEV lanes_t lanes_lt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 4); }    // a < b
+DEV lanes_t lanes_nlt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 11); }  // !(a < b)
+DEV lanes_t lanes_ngt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 13); }  // !(a > b)
+DEV lanes_t lanes_nge(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 12); }  // !(a >= b)
+DEV lanes_t lanes_nlt(double a, double b) { return __builtin_amdgcn_fcmp(a, b, 11); }
+DEV lanes_t lanes_nge(double a, double b) { return __builtin_amdgcn_fcmp(a, b, 12); }
+DEV lanes_t lanes_below(int a, int b) { return __builtin_amdgcn_uicmp((unsigned)a, (unsigned)b, 36); }  // 0 <= a < b
+DEV lanes_t lanes_gt(int a, int b) { return __builtin_amdgcn_sicmp(a, b, 38); }
+// this lane's bit of a mask
+DEV bool lane_of(lanes_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+// dm shifted left by one with the lane's flag in bit 0 (one add with the mask as carry)
+DEV unsigned shift_flag(unsigned dm, lanes_t f) { return dm + dm + (lane_of(f) ? 1u : 0u); }
 
 // Exclusive prefix sum of n (< 64) over the active lanes of the wave, from one ballot per bit;
 // *total receives the sum.  Works with any set of active lanes.
@@ -919,6 +940,31 @@ DEV int tile_row() {
   const int B = blockDim.x;
   const int t = threadIdx.x;
   return (!J || (B & 63)) ? t : (t & 63) * (B >> 6) + (t >> 6);
+}
+
+// A lane's row of the work item: its index (kNoRow past the slice's last point) and the record to
+// load for it.  Lanes without a row stay active and load the last record: their pairs all fail j > i,
+// and the tile's column ranges are evaluated with that mask.  (Masking the lanes off instead had
+// the compiler spill a value inside the masked region and reload it outside, with garbage in the
+// masked lanes.)
+inline constexpr int kNoRow = 0x7fffffff;
+struct Row {
+  int i;          // row, or kNoRow
+  int64_t rec;    // record index within the slice
+  bool any;       // some lane of the wave has a row (wave-uniform)
+  int jm;         // columns below jm need the j > i mask
+};
+template <bool J>
+DEV Row item_row(const Item &w, const Slice &s) {
+  const int B = blockDim.x;
+  const int i = w.i0 + tile_row<J>();
+  Row r;
+  r.i = i < s.N ? i : kNoRow;
+  r.rec = i < s.N ? i : s.N - 1;
+  r.any = __ballot(i < s.N) != 0ull;
+  const bool full = (int64_t)w.i0 + B <= __builtin_amdgcn_readfirstlane((int)s.N);
+  r.jm = full ? min(w.j1, w.i0 + B) : w.j1;
+  return r;
 }
 
 // Sphere, and flat point fields (not the batch-leading pairs): the same pairs as pair64 /
@@ -1111,8 +1157,8 @@ DEV void run_cols64p(const Params &P, const Slice &s, const Smem &m, const doubl
 // cycles per wave and CU).
 //
 // Bins are certified as in pair64p; what is not certain goes through exact_cell, the reference's
-// own sequence: a key in a cell's ambiguity interval, nearly coincident or
-// nearly antipodal points, a non-finite value, and, for joint histograms, a value within its
+// own sequence: a key in a cell's ambiguity interval (which the table extends to nearly coincident
+// and nearly antipodal points), a non-finite value, and, for joint histograms, a value within its
 // margin of a value edge or small against the velocities (|du_L| below 2^-12 of their norms on
 // the sphere, of |du| on the flat geometry).  The last rule keeps every joint cell within rounding
 // of the reference's sequence relative to its own sum: two sequences agree to a few 2^-53 of the
@@ -1191,7 +1237,7 @@ DEV bool near_value_edge(double v, const double *E, int nE, int g) {
 }
 
 template <int G, int D, bool J, int OPK, bool MASK, bool VU>
-DEV bool pair64f(const Params &P, const Slice &s, const Smem &m, const double *A, int i, int j,
+DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double *A, int i, int j,
                  const double *B, double *rn, const double *next, Pending64 &pa) {
   constexpr int S = rec_pair64<G, D>;
   constexpr int W = (G == kFlat) ? D : 3;  // space the differences live in
@@ -1211,18 +1257,16 @@ DEV bool pair64f(const Params &P, const Slice &s, const Smem &m, const double *A
   if constexpr (SP) hist_add_sp(m, pa.h, pa.v, pa.w);
   else hist_add(m, pa.h, pa.v);
   asm volatile("" ::"v"(lh.x), "v"(lh.y), "v"(bm1) : "memory");
-  // outside [lo, hi] a key is above the edge exactly when key >= lo
-  const bool ge = key >= lh.x;
-  bool rare = ge & (key <= lh.y);
-  int db0 = ge ? bm1 + 1 : bm1;
-  rare = rare | !(key > 0x1p-100f);
+  // a key outside [lo, hi] is above the edge exactly when it is not below lo; a NaN key is uncertain
+  const lanes_t ge = lanes_nlt(key, lh.x);
+  lanes_t rare = ge & lanes_ngt(key, lh.y);
+  const int db0 = lane_of(ge) ? bm1 + 1 : bm1;
   double e2 = 0.0;
   if constexpr (G == kSphere) {
     double e[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) e[k] = B[k] + A[k];
     e2 = fdot<3>(e, e);
-    rare = rare | !(e2 > 0x1p-24);
   }
 #pragma unroll
   for (int k = 0; k < W; ++k) du[k] = B[UO + k] - A[UO + k];
@@ -1259,11 +1303,11 @@ DEV bool pair64f(const Params &P, const Slice &s, const Smem &m, const double *A
     const float Lf = __builtin_fabsf((float)L);
     if constexpr (G == kSphere) {
       const float ni = __int_as_float(__double2loint(A[7]));
-      rare = rare | !(Lf > ni + nj);
+      rare |= lanes_ngt(Lf, ni + nj);
     } else {
       float q = __builtin_fabsf((float)du[0]) + __builtin_fabsf((float)du[1]);
       if constexpr (D == 3) q += __builtin_fabsf((float)du[2]);
-      rare = rare | !(Lf > 0x1p-12f * q);
+      rare |= lanes_ngt(Lf, 0x1p-12f * q);
     }
     if constexpr (VU) {  // s.v_uniform, chosen once per column range
       // t + eps with the margin eps of the largest value that can be in range: a value outside
@@ -1271,27 +1315,28 @@ DEV bool pair64f(const Params &P, const Slice &s, const Smem &m, const double *A
       // edge lies within eps of t (NaN fails the comparison too).
       const float t = __builtin_fmaf((float)v, s.vinvf, s.vtcu);
       const float gh = __builtin_floorf(t);
-      rare = rare | !(t - gh >= s.veps2);
+      rare |= lanes_nge(t - gh, s.veps2);
       vb0 = (int)gh;
     } else {
       vb0 = (s.vrule.on ? lin_rule_bin(s.vrule, v, P.n_val) : val_bin64(v, m.vE, P.n_val + 1, s)) - 1;
       // searched edges: a value close to one takes the reference's own value
-      rare = rare | near_value_edge(v, m.vE, P.n_val + 1, vb0);
+      rare |= __builtin_amdgcn_ballot_w64(near_value_edge(v, m.vE, P.n_val + 1, vb0));
     }
   } else if constexpr (SP) {
-    rare = rare | !(__builtin_fabs(L) < __builtin_inf()) | !(n2 < __builtin_inf());
+    rare |= lanes_nlt(__builtin_fabs(L), __builtin_inf()) | lanes_nlt(n2, __builtin_inf());
   } else {
-    rare = rare | !(__builtin_fabs(v) < __builtin_inf());
+    rare |= lanes_nlt(__builtin_fabs(v), __builtin_inf());
   }
-  bool add = !rare & ((unsigned)db0 < (unsigned)P.n_dist);
-  if constexpr (J) add = add & ((unsigned)vb0 < (unsigned)P.n_val);
+  lanes_t add = ~rare & lanes_below(db0, P.n_dist);
+  if constexpr (J) add &= lanes_below(vb0, P.n_val);
   if constexpr (MASK) {
-    add = add & (j > i);
-    rare = rare & (j > i);
+    const lanes_t upper = lanes_gt(j, i);
+    add &= upper;
+    rare &= upper;
   }
   const int h = J ? vb0 * m.jv + db0 * m.jd + m.coff
                   : (db0 << m.lcop) + (int)(__lane_id() & (m.copies - 1));
-  pa.h = add ? h : m.scr;
+  pa.h = lane_of(add) ? h : m.scr;
   pa.v = v;
   pa.w = n2;
   return rare;
@@ -1381,12 +1426,12 @@ DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double
     const int je = min(j1, j + 32);
     dm = 0u;
     for (; j + 1 < je; j += 2, cp += 2 * S) {
-      dm = (dm << 1) | (unsigned)pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, cp + S, pa);
-      dm = (dm << 1) | (unsigned)pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * S, pa);
+      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, cp + S, pa));
+      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * S, pa));
     }
     // an odd count only occurs in the last group (the others hold 32 columns)
     if (j < je) {
-      dm = (dm << 1) | (unsigned)pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, cp + S, pa);
+      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, cp + S, pa));
       ++j;
     }
     jl = je - 1;
@@ -1426,7 +1471,7 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
           rare64<G, D, J, OPK>(P, s, m, rec, 0u, 0, 0);
           __syncthreads();
         }
-        flush_hist(m, P, s);
+        flush_hist(m, P, s, cur);
         __syncthreads();
       }
       if (w.slice != cur) {
@@ -1440,56 +1485,44 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
       __syncthreads();  // tables and cleared histogram visible before the item's pairs
     }
     since_flush += work;
-    const int i = w.i0 + tile_row<J>();
-    const bool iv = i < s.N;
-    double ri[S];
-#pragma unroll
-    for (int k = 0; k < S; ++k) ri[k] = iv ? rec[(s.pt_off + i) * S + k] : 0.0;
-    if (iv) {
+    const Row row = item_row<J>(w, s);
+    if (row.any) {
+      double ri[S];
+      load_rec64<S>(rec + (s.pt_off + row.rec) * S, ri);
       if constexpr (FAST) {
-        // the columns up to the tile's last row need the j > i mask, the others do not; the
-        // value-bin lookup (uniform or exact) is chosen per column range, not per pair
-        const int jm = min(w.j1, w.i0 + B);
+        // the value-bin lookup (uniform or exact) is chosen per column range, not per pair
         for (int j = w.j0; j < w.j1;) {
           unsigned dm = 0u;
           int jl = 0;
-          const bool mask = j < jm;
-          const int je = mask ? jm : w.j1;
+          const bool mask = j < row.jm;
+          const int je = mask ? row.jm : w.j1;
           if (J && s.v_uniform) {
-            j = mask ? run_cols64f<G, D, J, OPK, true, true>(P, s, m, ri, i, j, je, rec, dm, jl)
-                     : run_cols64f<G, D, J, OPK, false, true>(P, s, m, ri, i, j, je, rec, dm, jl);
+            j = mask ? run_cols64f<G, D, J, OPK, true, true>(P, s, m, ri, row.i, j, je, rec, dm, jl)
+                     : run_cols64f<G, D, J, OPK, false, true>(P, s, m, ri, row.i, j, je, rec, dm, jl);
           } else {
-            j = mask ? run_cols64f<G, D, J, OPK, true, false>(P, s, m, ri, i, j, je, rec, dm, jl)
-                     : run_cols64f<G, D, J, OPK, false, false>(P, s, m, ri, i, j, je, rec, dm, jl);
+            j = mask ? run_cols64f<G, D, J, OPK, true, false>(P, s, m, ri, row.i, j, je, rec, dm, jl)
+                     : run_cols64f<G, D, J, OPK, false, false>(P, s, m, ri, row.i, j, je, rec, dm, jl);
           }
-          if (__ballot(dm != 0u)) rare64<G, D, J, OPK>(P, s, m, rec, dm, i, jl);
+          if (__ballot(dm != 0u)) rare64<G, D, J, OPK>(P, s, m, rec, dm, row.i, jl);
         }
       } else if (G == kSphere || !P.bl) {
-        if (w.j0 < w.i0 + B) run_cols64p<G, D, J, OPK, true>(P, s, m, ri, i, w.j0, w.j1, rec);
-        else run_cols64p<G, D, J, OPK, false>(P, s, m, ri, i, w.j0, w.j1, rec);
+        if (w.j0 < row.jm) run_cols64p<G, D, J, OPK, true>(P, s, m, ri, row.i, w.j0, row.jm, rec);
+        if (row.jm < w.j1) run_cols64p<G, D, J, OPK, false>(P, s, m, ri, row.i, max(row.jm, w.j0), w.j1, rec);
       } else {
-        if (w.j0 < w.i0 + B) run_cols64<G, D, J, OPK, true>(P, s, m, ri, i, w.j0, w.j1, rec);
-        else run_cols64<G, D, J, OPK, false>(P, s, m, ri, i, w.j0, w.j1, rec);
+        if (w.j0 < row.jm) run_cols64<G, D, J, OPK, true>(P, s, m, ri, row.i, w.j0, row.jm, rec);
+        if (row.jm < w.j1) run_cols64<G, D, J, OPK, false>(P, s, m, ri, row.i, max(row.jm, w.j0), w.j1, rec);
       }
     }
   }
   if (FAST && cur >= 0) rare64<G, D, J, OPK>(P, s, m, rec, 0u, 0, 0);
   __syncthreads();
-  if (cur >= 0) flush_hist(m, P, s);
+  if (cur >= 0) flush_hist(m, P, s, cur);
 }
 
 // ---------------------------------------------------------------------------------------------
 // hist32: binary32 pair arithmetic with certified binning, uncertain pairs queued
 // ---------------------------------------------------------------------------------------------
 DEV float frsq(float x) { return __builtin_amdgcn_rsqf(x); }
-
-// Nearly coincident points go to the binary64 re-bin: the binary32 records carry positions as
-// hi + lo (2^-48 relative), a direction error of 2^-48 / separation that below a separation of
-// 2^-22 (sphere: radians; flat: times max|x|) would outgrow the value bound's margin and the
-// reference's own binary64 accuracy (2^-53 / separation).  Smallest sin^2(sigma) (sphere) and
-// squared distance (flat) evaluated in binary32:
-inline constexpr float kCloseS2 = 0x1p-44f;
-DEV float close_key(const Slice &s) { return __builtin_fmaxf(1e-30f, 0x1p12f * s.xerr * s.xerr); }
 
 DEV int cell32(float key, const Slice &s) {
   const int bits = __float_as_int(key);
@@ -1518,26 +1551,25 @@ DEV unsigned cell32_off(float key, const Slice &s) {
 // widths is then one multiply-add away).  Returns the 0-based value bin g (valid bins 0 .. nE-2;
 // anything else is out of range) and g as a float in gf.
 template <bool VU>
-DEV int val_bin32(float v, float dva, float dvb, const Slice &s, const float *E32, int nE, bool &amb,
+DEV int val_bin32(float v, float dva, float dvb, const Slice &s, const float *E32, int nE, lanes_t &amb,
                   float &gf) {
   if constexpr (VU) {  // uniform value edges (s.v_uniform; chosen once per column range)
     // t = v / w - v0 / w in one fma (its product exact, one rounding)
     const float t = __builtin_fmaf(v, s.vinvf, s.vtc);
-    // error of t: value bound (1/w > 0), host slack (edge non-uniformity, rounding of v0, 1/w and
-    // -v0 / w), and the rounding of the fma and the two offsets below (a few ulp of |t|).  Undecidable iff an integer lies in (t - eps, t + eps].  Far outside the edges
-    // (|t| >= 2^21) eps exceeds 1, so such values are undecidable too (and re-binned); the
-    // float-to-int conversion saturates, so no clamp is needed.  A non-finite v is undecidable
-    // without a test of its own: t = +-Inf makes eps infinite and t - eps or t + eps NaN, and a
-    // NaN fails the comparison below.
-    const float eps = __builtin_fmaf(dva, dvb, __builtin_fmaf(4.8e-7f, __builtin_fabsf(t), s.vslack));
+    // error of t: value bound (1/w > 0) and host slack (edge non-uniformity, rounding of v0, 1/w
+    // and -v0 / w, and the rounding of the fma and the two offsets below for the largest |t| that
+    // can be in range; a value outside the edges has a larger error, but stays outside).
+    // Undecidable iff an integer lies in (t - eps, t + eps]; a NaN fails the comparison below.  The
+    // float-to-int conversion saturates, so no clamp is needed.
+    const float eps = __builtin_fmaf(dva, dvb, s.vslackt);
     // floor(t - eps) != floor(t + eps) exactly when t - eps < floor(t + eps) (NaN: undecidable)
     const float gh = __builtin_floorf(t + eps);
-    amb = amb || !(t - eps >= gh);
+    amb |= lanes_nge(t - eps, gh);
     gf = gh;
     return (int)gh;
   }
   // a non-finite value is undecidable here; the lookup below still runs, its bin is ignored
-  amb = amb || !(__builtin_fabsf(v) < __builtin_inff());
+  amb |= lanes_nlt(__builtin_fabsf(v), __builtin_inff());
   int lo = 0;
   if (s.v_log) {
     // log-spaced edges (positive from edge vk0 on): the first edge >= v guessed from log2(v),
@@ -1556,8 +1588,10 @@ DEV int val_bin32(float v, float dva, float dvb, const Slice &s, const float *E3
   }
   // nearest edges must be farther than the error bound (edges rounded to binary32: slack)
   const float gap = __builtin_fmaf(dva, dvb, __builtin_fmaf(s.vslack, __builtin_fabsf(v), s.vabs)) + 1e-37f;
-  if (lo > 0 && v - E32[lo - 1] <= gap) amb = true;
-  if (lo < nE && E32[lo] - v <= gap) amb = true;
+  bool near = false;
+  if (lo > 0 && v - E32[lo - 1] <= gap) near = true;
+  if (lo < nE && E32[lo] - v <= gap) near = true;
+  amb |= __builtin_amdgcn_ballot_w64(near);
   gf = (float)(lo - 1);
   return lo - 1;
 }
@@ -1637,6 +1671,26 @@ struct PendingAdd {
   unsigned q;  // fixed-point joint cells: the quantized value
 };
 
+// Fixed-point joint cells: a lane's pending small value (see pair32) and its bins (distance bin in
+// the high half, value bin in the low); occ has the bits of the lanes that hold one.
+struct SmallAdd {
+  float v;
+  unsigned b;
+  lanes_t occ;
+};
+
+// Add the pending small values to their binary64 cells.
+DEV void flush_small(const Slice &s, const Smem &m, SmallAdd &sa) {
+  if (lane_of(sa.occ)) {
+    // the clamp keeps the cell in range; the host's choice of gz puts every such bin inside it
+    const int k = min(max((int)(sa.b & 0xffffu) - s.gz, 0), kZeroBins - 1);
+    const int z = (int)(sa.b >> 16) * kZeroBins + k;
+    atomicAdd(&m.zs[z], (double)sa.v);
+    atomicAdd(&m.zc[z], 1u);
+  }
+  sa.occ = 0ull;
+}
+
 // One pair (i, j): certified distance bin from the binary32 key, operator value, certified value
 // bin, and the deferred update.  rj is column j's record; the record of column j + 1 (if
 // j + 1 < j_end) is requested into rn.  The body has no branch on the pair's own state: every
@@ -1644,8 +1698,8 @@ struct PendingAdd {
 // Returns whether the pair is undecidable in binary32 and must be re-binned in binary64; the
 // caller collects these flags and queues the pairs every few columns (queue_deferred).
 template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool VU, bool SL>
-DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri, int i, int j,
-                const float *rj, float *rn, const float4 *next, bool has_next, PendingAdd &pa) {
+DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *ri, int i, int j,
+                const float *rj, float *rn, const float4 *next, bool has_next, PendingAdd &pa, SmallAdd &sa) {
   constexpr int F = Rec<G, D>::f32;
   // OPK 3 (single pass) and 4 (a plane of its 2D form) need du_L and |du|^2; on the sphere
   // |du|^2 = du_L^2 + |du_T|^2
@@ -1658,8 +1712,7 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
   constexpr int NF = OPK == 9 ? 1 : (OPK == 10 ? 2 : (OPK == 11 ? 4 : (OPK == 12 ? 6 : kMaxFused)));
   constexpr bool needN2 = (OPK == 0) || MULTI || SP || SP2;
   const int nb = P.n_dist;
-  const bool upper = !MASK || j > i;
-  bool amb, amb_d;
+  lanes_t amb, amb_d;
   float key, L = 0.f, T = 0.f, tn2 = 0.f, n2 = 0.f, amp = 1.0f, umax;
   int db0;  // 0-based distance bin
   // ---- distance key and certified bin
@@ -1696,11 +1749,12 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
     // operations): the next column's record is requested only after this point, because a
     // scalar load still in flight would make the wait for the table read wait for it as well
     asm volatile("" ::"v"(lh.x), "v"(lh.y), "v"(bm1) : "memory");
-    // two compares: a key that is not in [lo, hi] is above the edge exactly when key >= lo (a
-    // NaN key fails both: not ambiguous here, bin blo, and degenerate by the tests below)
-    const bool ge = key >= lh.x;
-    amb_d = ge & (key <= lh.y);
-    db0 = ge ? bm1 + 1 : bm1;
+    // two compares: a key that is not in [lo, hi] is above the edge exactly when it is not below lo
+    // (a NaN key is ambiguous).  Nearly coincident and nearly antipodal points lie in the table's
+    // intervals: no test of their own.
+    const lanes_t ge = lanes_nlt(key, lh.x);
+    amb_d = ge & lanes_ngt(key, lh.y);
+    db0 = lane_of(ge) ? bm1 + 1 : bm1;
   }
   // scalar-load variant: the request is unconditional (past the last column it reads the record
   // array's one-record tail pad) and pinned here, so that the scheduler does not sink it towards
@@ -1712,8 +1766,8 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
     load_rec<F>(next, 0, rn);
   }
   amb = amb_d;
-  const bool db_ok = (unsigned)db0 < (unsigned)nb;
-  bool vb_ok = true;
+  const lanes_t db_ok = lanes_below(db0, nb);
+  lanes_t vb_ok = ~0ull;
   float v = 0.f;
   int vb0 = 0;
   // value bound inputs (joint histograms): largest |component| of the velocity difference, the
@@ -1757,7 +1811,6 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
         tn2 = __builtin_fmaf(cz, cz, __builtin_fmaf(cy, cy, cx * cx)) * (rinv * rinv);
       }
     }
-    amb = amb || !(key > close_key(s));
   } else {
     // geodesic frame (HelperFunctions.jl:186-200): t_A = (d - (p.d) p)/sin, t_B = (d + (p.d) q)/sin
     // with d = q - p, sin^2(sigma) = |p x d|^2.  U_A is tangent at p and U_B at q, so
@@ -1771,7 +1824,6 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
     w[1] = __builtin_fmaf(ri[2], d[0], -ri[0] * d[2]);
     w[2] = __builtin_fmaf(ri[0], d[1], -ri[1] * d[0]);
     const float s2 = __builtin_fmaf(w[2], w[2], __builtin_fmaf(w[1], w[1], w[0] * w[0]));
-    amb = amb || !(s2 > kCloseS2);
     const float inv_s = frsq(s2);
     L = __builtin_fmaf(d[2], dU[2], __builtin_fmaf(d[1], dU[1], d[0] * dU[0])) * inv_s;
     float dw = 0.f;
@@ -1806,8 +1858,8 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
   if constexpr (SP) {
     // moments are formed at the accumulation; all four must be finite in binary32
     const float L2 = L * L;
-    amb = amb || !(n2 < __builtin_inff()) || !(__builtin_fabsf(L * n2) < __builtin_inff()) ||
-          !(__builtin_fabsf(L * L2) < __builtin_inff());
+    amb |= lanes_nlt(n2, __builtin_inff()) | lanes_nlt(__builtin_fabsf(L * n2), __builtin_inff()) |
+           lanes_nlt(__builtin_fabsf(L * L2), __builtin_inff());
   } else if constexpr (SP2) {
     v = sp_invariant(s.plane, L, n2);
   } else if constexpr (MULTI) {
@@ -1855,10 +1907,10 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
     // matters in units of a (tiny) bin, so re-bin in binary64.  Order 1 needs no test: a bound
     // that underflows is below 2^-126 bin widths, far inside the slack, and a NaN fails the
     // value-bin test by itself.
-    if constexpr (!(OPK == 1 || OPK == 6)) amb = amb || !(umax >= 0x1p-30f);
+    if constexpr (!(OPK == 1 || OPK == 6)) amb |= lanes_nge(umax, 0x1p-30f);
     float gf;
     vb0 = val_bin32<VU>(v, dva, ampv, s, m.vE32, P.n_val + 1, amb, gf);
-    vb_ok = (unsigned)vb0 < (unsigned)P.n_val;
+    vb_ok = lanes_below(vb0, P.n_val);
     if constexpr (FX) {
       // offset within the value bin in units of 2^-22 bin widths, biased, rounded to nearest:
       // v vsf + c_g with c_g ~ 2^23 + kFxBias - a_g vsf (one fma, exact before its rounding)
@@ -1867,7 +1919,7 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
       pa.q = __float_as_uint(__builtin_fmaf(v, s.vsf, __builtin_fmaf(-gf, s.fxc1, s.fxc0)));
     }
   } else if constexpr (!SP) {
-    amb = amb || !(__builtin_fabsf(v) < __builtin_inff());
+    amb |= lanes_nlt(__builtin_fabsf(v), __builtin_inff());
   }
   // fused 1D outputs: every value must be finite in binary32 (else the pair is re-binned)
   // fused 1D outputs: NF values per pair, unconditionally (outputs past P.n1d have a = b = 0)
@@ -1882,21 +1934,22 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
       // loop, 2 NF indices would hold SGPRs of their own (at NF = 8 they spilled to VGPR lanes,
       // read back with a v_readlane per lookup)
       int ia, ib;
-      asm volatile("s_bfe_u32 %0, %1, %2" : "=s"(ia) : "s"(P.mab_a), "i"((4 * k) | (4 << 16)));
-      asm volatile("s_bfe_u32 %0, %1, %2" : "=s"(ib) : "s"(P.mab_b), "i"((4 * k) | (4 << 16)));
+      asm volatile("s_bfe_u32 %0, %1, %2" : "=s"(ia) : "s"(P.mab_a), "i"((4 * k) | (4 << 16)) : "scc");
+      asm volatile("s_bfe_u32 %0, %1, %2" : "=s"(ib) : "s"(P.mab_b), "i"((4 * k) | (4 << 16)) : "scc");
       mv[k] = X[ia] * X[ib];
       mag += __builtin_fabsf(mv[k]);
     }
-    amb = amb || !(mag < __builtin_inff());
+    amb |= lanes_nlt(mag, __builtin_inff());
   }
   // binned here: certain and in range; queued: undecidable and not certainly out of range.  A
   // fused call without a joint output bins through its 1D histograms only.
-  const bool add = upper & !amb & db_ok & vb_ok & !(MULTI && !J);
-  const bool defer = upper & amb & (amb_d | db_ok);
+  const lanes_t upper = MASK ? lanes_gt(j, i) : ~0ull;
+  const lanes_t add1 = upper & ~amb & db_ok;
+  const lanes_t add = (MULTI && !J) ? 0ull : add1 & vb_ok;
+  const lanes_t defer = upper & amb & (amb_d | db_ok);
   if constexpr (MULTI) {
     // the fused 1D outputs of a certain, in-range distance bin (whatever the joint value bin)
-    const bool add1 = upper & !amb & db_ok;
-    const int h1 = add1 ? (db0 << m.lmcop) + (int)(__lane_id() & (m.mcop - 1)) : m.mscr;
+    const int h1 = lane_of(add1) ? (db0 << m.lmcop) + (int)(__lane_id() & (m.mcop - 1)) : m.mscr;
     atomicAdd(&m.mc[h1], 1u);
     double *const mp = m.ms + h1;
 #pragma unroll
@@ -1920,21 +1973,19 @@ DEV bool pair32(const Params &P, const Slice &s, const Smem &m, const float *ri,
     h = (db0 << m.lcop) + (int)(__lane_id() & (m.copies - 1));
   }
   if constexpr (FX) {
-    // a value below a quarter bin width goes to the binary64 cell of its (distance, value) bin
-    // at once (few lanes, so a branch): the fixed-point error (up to 2^-22 bin widths) would not
-    // be small relative to it.  The other pairs take the deferred fixed-point update.  The clamp
-    // keeps the cell in range; the host's choice of gz already puts every such bin inside it
-    // (a range test in its place measured 0.8 % slower)
-    const int k = min(max(vb0 - s.gz, 0), kZeroBins - 1);
-    const bool small = add & (__builtin_fabsf(v) < s.vsmall);
-    if (small) {
-      const int z = db0 * kZeroBins + k;
-      atomicAdd(&m.zs[z], (double)v);
-      atomicAdd(&m.zc[z], 1u);
-    }
-    pa.h = (add & !small) ? h : m.scr;
+    // a value below a quarter bin width goes to the binary64 cell of its (distance, value) bin:
+    // the fixed-point error (up to 2^-22 bin widths) would not be small relative to it.  About 1 %
+    // of the lanes have one, so half of the waves: each lane keeps its value until some lane has a
+    // second one (every 18 pairs or so), and then all of them are added at once.  The other pairs
+    // take the deferred fixed-point update.
+    const lanes_t small = add & lanes_lt(__builtin_fabsf(v), s.vsmall);
+    if (small & sa.occ) flush_small(s, m, sa);
+    sa.v = lane_of(small) ? v : sa.v;
+    sa.b = lane_of(small) ? ((unsigned)db0 << 16) | (unsigned)vb0 : sa.b;
+    sa.occ |= small;
+    pa.h = lane_of(add & ~small) ? h : m.scr;
   } else {
-    pa.h = add ? h : m.scr;
+    pa.h = lane_of(add) ? h : m.scr;
   }
   pa.v = SP ? L : v;
   pa.w = n2;
@@ -2030,6 +2081,7 @@ DEV void run_chunk32_vu(const Params &P, const Slice &s, const Smem &m, const fl
   const float4 *cp = col + (j_begin - col_j0) * R;
   load_rec<F>(cp, 0, ra);
   PendingAdd pa{m.scr, 0.f, 0.f, 0u};
+  SmallAdd sa{0.f, 0u, 0ull};
   int j = j_begin;
   // groups of 32 columns: the flags are shifted in, so bit t of dm flags pair (i, je - 1 - t)
   // for the re-bin queue (one shift-add per pair)
@@ -2038,19 +2090,20 @@ DEV void run_chunk32_vu(const Params &P, const Slice &s, const Smem &m, const fl
     const int je = min(j_end, jg + 32);
     unsigned dm = 0u;
     for (; j + 1 < je; j += 2, cp += 2 * R) {
-      dm = (dm << 1) | (unsigned)pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j, ra, rb, cp + R, true, pa);
-      dm = (dm << 1) |
-           (unsigned)pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * R, j + 2 < j_end, pa);
+      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j, ra, rb, cp + R, true, pa, sa));
+      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * R, j + 2 < j_end,
+                                                                  pa, sa));
     }
     // an odd count only occurs in the last group (the others hold 32 columns)
     if (j < je) {
-      dm = (dm << 1) | (unsigned)pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j, ra, rb, cp + R, false, pa);
+      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j, ra, rb, cp + R, false, pa, sa));
       ++j;
     }
     queue_deferred(P, m, dm, i, je - 1, slice_id, 0, -1);
   }
   if constexpr (FX) {
     atomicAdd(&m.hq[pa.h], (1ull << kFxShift) | (unsigned long long)pa.q);
+    if (sa.occ) flush_small(s, m, sa);
   } else if constexpr (OPK == 3) {
     hist_add_sp(m, pa.h, pa.v, pa.w);
   } else {
@@ -2097,7 +2150,7 @@ __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, 
     const unsigned long long work = (unsigned long long)B * (unsigned long long)(w.j1 - w.j0);
     if (w.slice != cur || since_flush + work > (unsigned long long)P.flush_limit) {
       if (cur >= 0) {
-        flush_hist(m, P, s);
+        flush_hist(m, P, s, cur);
         if constexpr (OPK >= 9) flush_multi(m, P, cur);
         __syncthreads();
       }
@@ -2111,22 +2164,21 @@ __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, 
       since_flush = 0;
     }
     since_flush += work;
-    const int i = w.i0 + tile_row<J>();
-    const bool iv = i < s.N;
+    const Row row = item_row<J>(w, s);
     float ri[F];
 #pragma unroll
-    for (int k = 0; k < F; ++k) ri[k] = iv ? rec[(s.pt_off + i) * F + k] : 0.0f;
+    for (int k = 0; k < F; ++k) ri[k] = rec[(s.pt_off + row.rec) * F + k];
     if constexpr (SLOAD) {
-      if (iv) {
+      if (row.any) {
         // the slice offset is wave-uniform by construction; say so, so that column addresses
         // stay in SGPRs (the pointer itself keeps its global address space: scalar loads)
         const uint64_t po = (uint64_t)s.pt_off;
         const int64_t off = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(po >> 32)) << 32) |
                                       (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)po));
         const float4 *col = (const float4 *)(rec + off * F);
-        const int jm = min(w.j1, w.i0 + B);  // columns that can still be <= some row of the tile
-        if (w.j0 < jm) run_chunk32<G, D, J, OPK, true, FX, true>(P, s, m, ri, i, w.j0, jm, col, 0, cur);
-        if (jm < w.j1) run_chunk32<G, D, J, OPK, false, FX, true>(P, s, m, ri, i, max(jm, w.j0), w.j1, col, 0, cur);
+        if (w.j0 < row.jm) run_chunk32<G, D, J, OPK, true, FX, true>(P, s, m, ri, row.i, w.j0, row.jm, col, 0, cur);
+        if (row.jm < w.j1)
+          run_chunk32<G, D, J, OPK, false, FX, true>(P, s, m, ri, row.i, max(row.jm, w.j0), w.j1, col, 0, cur);
       }
     } else {
       for (int jb = w.j0; jb < w.j1; jb += P.tj) {
@@ -2136,10 +2188,10 @@ __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, 
         float4 *dst = (float4 *)m.stage;
         for (int k = threadIdx.x; k < cnt * (F / 4); k += B) dst[k] = src[k];
         __syncthreads();
-        if (iv) {
+        if (row.any) {
           const float4 *col = (const float4 *)m.stage;
-          if (jb < w.i0 + B) run_chunk32<G, D, J, OPK, true, FX, false>(P, s, m, ri, i, jb, jb + cnt, col, jb, cur);
-          else run_chunk32<G, D, J, OPK, false, FX, false>(P, s, m, ri, i, jb, jb + cnt, col, jb, cur);
+          if (jb < row.jm) run_chunk32<G, D, J, OPK, true, FX, false>(P, s, m, ri, row.i, jb, jb + cnt, col, jb, cur);
+          else run_chunk32<G, D, J, OPK, false, FX, false>(P, s, m, ri, row.i, jb, jb + cnt, col, jb, cur);
         }
       }
     }
@@ -2147,7 +2199,7 @@ __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, 
   __syncthreads();
   if (cur >= 0) {
     queue_wave_flush(P, m, cur);
-    flush_hist(m, P, s);
+    flush_hist(m, P, s, cur);
     if constexpr (OPK >= 9) flush_multi(m, P, cur);
   }
 }
@@ -2217,19 +2269,18 @@ DEV void run_chunk_strip(const Params &P, const Slice &s, const Smem &m, const f
       const int c = cell32(key, s);
       const float2 lh = m.lohi[c];
       const int blo = m.blo[c].x;
-      const bool amb_d = (key >= lh.x) & (key <= lh.y);
-      const int db = (key > lh.y) ? blo + 1 : blo;
+      const bool ge = !(key < lh.x);  // as in pair32: a NaN key is ambiguous
+      const bool amb_d = ge & !(key > lh.y);
+      const int db = ge ? blo + 1 : blo;
       const bool db_ok = (unsigned)(db - 1) < (unsigned)nb;
       bool amb = amb_d;
       if constexpr (G == kFlat) {
         rinv = frsq(key);
-        amb = amb || !(key > close_key(s));
       } else {
         w[0] = __builtin_fmaf(ri[1], d[2], -ri[2] * d[1]);
         w[1] = __builtin_fmaf(ri[2], d[0], -ri[0] * d[2]);
         w[2] = __builtin_fmaf(ri[0], d[1], -ri[1] * d[0]);
         const float s2 = __builtin_fmaf(w[2], w[2], __builtin_fmaf(w[1], w[1], w[0] * w[0]));
-        amb = amb || !(s2 > kCloseS2);
         inv_s = frsq(s2);
       }
       float vals[kStripMax];
@@ -2362,18 +2413,17 @@ __global__ void __launch_bounds__(1024) hist32s(Params P, const float *__restric
       since_flush = 0;
     }
     since_flush += work;
-    const int i = w.i0 + (int)threadIdx.x;
-    const bool iv = i < s.N;
+    const Row row = item_row<false>(w, s);
     float ri[SR::pos];
 #pragma unroll
-    for (int k = 0; k < SR::pos; ++k) ri[k] = iv ? rec[(s.pt_off + i) * F + k] : 0.0f;
+    for (int k = 0; k < SR::pos; ++k) ri[k] = rec[(s.pt_off + row.rec) * F + k];
     float rv[kStripMax][SR::VS];
 #pragma unroll
     for (int b = 0; b < kStripMax; ++b) {
 #pragma unroll
       for (int k = 0; k < SR::VS; ++k) {
         rv[b][k] = 0.f;
-        if (iv && b < nf && k < SR::vel) rv[b][k] = rec[(P.slices[cur + b].pt_off + i) * F + SR::voff + k];
+        if (b < nf && k < SR::vel) rv[b][k] = rec[(P.slices[cur + b].pt_off + row.rec) * F + SR::voff + k];
       }
     }
     for (int jb = w.j0; jb < w.j1; jb += P.tj) {
@@ -2397,9 +2447,9 @@ __global__ void __launch_bounds__(1024) hist32s(Params P, const float *__restric
         }
       }
       __syncthreads();
-      if (iv) {
-        if (jb < w.i0 + B) run_chunk_strip<G, D, OPK, true>(P, s, m, ri, rv, nf, i, jb, cnt, cur);
-        else run_chunk_strip<G, D, OPK, false>(P, s, m, ri, rv, nf, i, jb, cnt, cur);
+      if (row.any) {
+        if (jb < row.jm) run_chunk_strip<G, D, OPK, true>(P, s, m, ri, rv, nf, row.i, jb, cnt, cur);
+        else run_chunk_strip<G, D, OPK, false>(P, s, m, ri, rv, nf, row.i, jb, cnt, cur);
       }
     }
   }
