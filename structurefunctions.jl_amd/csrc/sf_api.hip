@@ -43,7 +43,7 @@ hipError_t launch_eval_math(int fn, int64_t n, const double *a, const double *b,
                             hipStream_t st);
 hipError_t cull_workspace_bytes(int64_t N, size_t *bytes);
 hipError_t launch_cull(const double *x, int64_t N, int W, int D, int geom, int rows, void *ws,
-                       int32_t *perm, double *info, hipStream_t st);
+                       int32_t *perm, double *info, float *gbox, hipStream_t st);
 int hist_occupancy(int G, int D, bool J, bool mixed, int opk, bool sload, bool fx, int block,
                    size_t smem);
 int hist_opk(const Params &P);
@@ -218,8 +218,10 @@ struct Plan {
   DevBuf<Pending> pending;
   DevBuf<PrepSliceHost> prep;
   DevBuf<int> flag;
+  DevBuf<float> gboxes;   // boxes of the column groups of culled slices
   DevBuf<int32_t> perm;   // spatial order of the binary32 records (tile culling)
   bool culled = false;    // some work items were dropped by tile culling
+  bool near = false;      // some slice's column groups are culled per wave
   Arena *arena = nullptr;  // set: every buffer is taken from this region (no device allocation)
   // fused outputs: 1D operators evaluated with the main (joint) one, their accumulators and the
   // caller's outputs they merge into
@@ -240,6 +242,7 @@ struct Plan {
     counter.release(); pcount.release(); pending.release(); prep.release(); flag.release();
     items64.release();
     perm.release();
+    gboxes.release();
     msums.release();
     mcounts.release();
   }
@@ -867,7 +870,7 @@ struct CullInfo {
 // Spatial order and tile boxes of one slice, computed on the device (launch_cull): the record
 // order goes to perm (device, N entries); ci.active says whether culling is worth it.
 int cull_prepare(sf_ctx *ctx, const sf_problem &p, const double *dx, double xmax, int rows,
-                 hipStream_t st, CullInfo &ci, int32_t *perm) {
+                 hipStream_t st, CullInfo &ci, int32_t *perm, float *gbox) {
   ci.active = false;
   const int64_t N = p.N;
   const double emax = p.dist_edges[p.n_dist];
@@ -892,7 +895,7 @@ int cull_prepare(sf_ctx *ctx, const sf_problem &p, const double *dx, double xmax
   HIPCHK(ctx->cull_ws.ensure(wsb));
   HIPCHK(ctx->cull_info.ensure((size_t)(8 + 6 * ntile)));
   const int geom = flat ? 0 : (p.geometry == SF_GEOM_SPHERE_DEG ? 1 : 2);
-  HIPCHK(launch_cull(dx, N, p.W, p.D, geom, rows, ctx->cull_ws.p, perm, ctx->cull_info.p, st));
+  HIPCHK(launch_cull(dx, N, p.W, p.D, geom, rows, ctx->cull_ws.p, perm, ctx->cull_info.p, gbox, st));
   std::vector<double> info((size_t)(8 + 6 * ntile));
   HIPCHK(hipMemcpyAsync(info.data(), ctx->cull_info.p, sizeof(double) * info.size(), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
@@ -1066,6 +1069,8 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     d.out_off = planes ? (int64_t)(s / kSpRows) * ncell + s % kSpRows : (int64_t)s * ncell;
     d.plane = planes ? s % kSpRows : 0;
     d.xerr = flat ? round_up_f(ldexpl((long double)xmax[s], -28)) : 0.0f;
+    d.grp_off = 0;
+    d.clim2 = 0.0f;
     d.strip_n = (strip && s % strip == 0) ? std::min(strip, n - s) : 0;
     d.tab_off = (int32_t)cells.size();
     cells.insert(cells.end(), T.tab64.begin(), T.tab64.end());
@@ -1214,14 +1219,25 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   if (pl.fx) jchunk = std::max(1, std::min<int>(jchunk, (int)(kFxFlushLimit / block)));
   // spatial sort and tile culling (binary32 kernel, one-shot calls): column chunks of one tile
   std::vector<CullInfo> cinfo(n);
-  pl.culled = false;
+  pl.culled = pl.near = false;
   if (cull && mixed && !strip) {
     // the record order of slice s lands at pl.perm + pt_off (used only where culling is active)
     PLBUF(pl.perm, ((size_t)pl.total_pts));
+    int64_t groups = 0;
     for (int s = 0; s < n; ++s) {
-      const int rc = cull_prepare(ctx, sl[s], dx[s], xmax[s], block, st, cinfo[s], pl.perm.p + prep[s].pt_off);
+      sdesc[s].grp_off = (int32_t)groups;
+      groups += (sl[s].N + kGroup - 1) / kGroup;
+    }
+    PLBUF(pl.gboxes, ((size_t)groups * 6));
+    for (int s = 0; s < n; ++s) {
+      const int rc = cull_prepare(ctx, sl[s], dx[s], xmax[s], block, st, cinfo[s], pl.perm.p + prep[s].pt_off,
+                                  pl.gboxes.p + (size_t)sdesc[s].grp_off * 6);
       if (rc) return rc;
-      if (cinfo[s].active) prep[s].perm = pl.perm.p + prep[s].pt_off;
+      if (!cinfo[s].active) continue;
+      pl.near = true;
+      prep[s].perm = pl.perm.p + prep[s].pt_off;
+      // squared limit for the binary32 gaps of the group boxes (three squares and their sum)
+      sdesc[s].clim2 = round_up_f((long double)cinfo[s].limit * cinfo[s].limit * (1.0L + 1e-5L) + 1e-30L);
     }
   }
   PLBUF(pl.prep, (n));
@@ -1339,6 +1355,7 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   P.counter = pl.counter.p;
   P.rec64 = pl.rec64.p;
   P.rec32 = pl.rec32.p;
+  P.gboxes = pl.near ? pl.gboxes.p : nullptr;
   P.cells = pl.cells.p;
   P.dedges = pl.dedges.p;
   P.vedges = pl.vedges.p;

@@ -165,6 +165,30 @@ __global__ void __launch_bounds__(kCullBlock) cull_tiles(const double *kc, const
   if (t < 6) boxes[(size_t)blockIdx.x * 6 + t] = red[t][0];
 }
 
+// boxes (lo[3], hi[3]) of groups of 32 consecutive records, rounded outwards to binary32: two
+// groups per wave
+__global__ void __launch_bounds__(kCullBlock) cull_groups(const double *kc, const int32_t *perm, int64_t N,
+                                                          float *gbox) {
+  const int64_t k = (int64_t)blockIdx.x * kCullBlock + threadIdx.x;
+  const int64_t i = perm[k < N ? k : N - 1];
+  float lo[3], hi[3];
+  for (int c = 0; c < 3; ++c) {
+    const double v = kc[3 * i + c];
+    lo[c] = __double2float_rd(v);
+    hi[c] = __double2float_ru(v);
+  }
+  for (int o = 16; o > 0; o >>= 1)
+    for (int c = 0; c < 3; ++c) {
+      lo[c] = fminf(lo[c], __shfl_xor(lo[c], o));
+      hi[c] = fmaxf(hi[c], __shfl_xor(hi[c], o));
+    }
+  if ((threadIdx.x & 31) == 0 && k < N)
+    for (int c = 0; c < 3; ++c) {
+      gbox[6 * (k / 32) + c] = lo[c];
+      gbox[6 * (k / 32) + 3 + c] = hi[c];
+    }
+}
+
 struct CullWs {
   double *kc, *part;
   uint32_t *key_in, *key_out;
@@ -213,9 +237,10 @@ hipError_t cull_workspace_bytes(int64_t N, size_t *bytes) {
 // x: the slice's positions (device, point-major, W per point); geom 0 flat, 1 sphere in degrees,
 // 2 sphere in radians.  Writes the record order to perm (N entries) and to info the slice box
 // (8 doubles: lo[3], hi[3], non-finite count, largest |coordinate|) followed by one box per tile
-// (6 doubles each, ceil(N / rows) tiles).  ws: cull_workspace_bytes(N) bytes of device memory.
+// (6 doubles each, ceil(N / rows) tiles), and to gbox one box per kGroup records (6 floats each).  ws: cull_workspace_bytes(N) bytes of device memory.
 hipError_t launch_cull(const double *x, int64_t N, int W, int D, int geom, int rows, void *ws,
-                       int32_t *perm, double *info, hipStream_t st) {
+                       int32_t *perm, double *info, float *gbox, hipStream_t st) {
+  static_assert(kGroup == 32, "cull_groups reduces over half waves");
   if (N < 1 || N > 0x7fffffffLL || rows < 1) return hipErrorInvalidValue;
   CullWs w;
   hipError_t e = cull_ws_layout(N, (char *)ws, w);
@@ -235,6 +260,9 @@ hipError_t launch_cull(const double *x, int64_t N, int W, int D, int geom, int r
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(cull_tiles, dim3(ntile), dim3(kCullBlock), 0, st, (const double *)w.kc,
                      (const int32_t *)perm, N, rows, info + 8);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  hipLaunchKernelGGL(cull_groups, dim3(nblk), dim3(kCullBlock), 0, st, (const double *)w.kc,
+                     (const int32_t *)perm, N, gbox);
   return hipGetLastError();
 }
 

@@ -92,6 +92,8 @@ struct Slice {
   int32_t gz;
   int32_t plane;      // single pass, 2D form: invariant (0..5) whose joint histogram this slice holds
   float xerr;         // flat: 2^-28 max|x| (binary32 value bound: reference's direction error)
+  int32_t grp_off;    // tile culling: first box of the slice in gboxes
+  float clim2;        // ... and the squared distance beyond which two boxes hold no counted pair; 0: off
   int32_t strip_n;    // B-strip launch: fields of the strip this slice leads (0: not a leader)
   // value edges log-spaced from edge vk0 on (binary32 lookup guesses the bin from log2 v):
   // log2(edge vk0 + m) ~ vl0f + m / vlinvf
@@ -118,6 +120,7 @@ struct Params {
   int32_t *counter;        // work-queue head (zeroed before launch)
   const double *rec64;     // binary64 records
   const float *rec32;      // binary32 records
+  const float *gboxes;     // culled slices: a box (lo[3], hi[3]) per kGroup records, rounded outwards
   const Cell *cells;       // cell tables (binary64 tables and binary32 tables)
   const double *dedges;    // exact distance-key edges
   const double *vedges;    // value edges (binary64)
@@ -244,6 +247,8 @@ inline constexpr int kZeroSetMax = 8;  // buffers cleared by one zero_multi laun
 // takes a constant offset), for 1D ones right after the largest table of the launch (their LDS
 // decides how many workgroups fit: 16 KB of table region cost them 12 %)
 inline constexpr int kCell32Max = 1024;
+// records per box of a culled slice (a column group of the binary32 pair loop)
+inline constexpr int kGroup = 32;
 // largest re-bin queue staged in LDS per workgroup (entries, split evenly between its waves);
 // the host shrinks it where the LDS it takes would cost a workgroup per CU
 inline constexpr int kQueueCap = 8192;

@@ -954,10 +954,11 @@ struct Row {
   bool any;       // some lane of the wave has a row (wave-uniform)
   int jm;         // columns below jm need the j > i mask
 };
+// near: a wave's rows side by side (a slice whose column groups are culled per wave)
 template <bool J>
-DEV Row item_row(const Item &w, const Slice &s) {
+DEV Row item_row(const Item &w, const Slice &s, bool near = false) {
   const int B = blockDim.x;
-  const int i = w.i0 + tile_row<J>();
+  const int i = w.i0 + (near ? (int)threadIdx.x : tile_row<J>());
   Row r;
   r.i = i < s.N ? i : kNoRow;
   r.rec = i < s.N ? i : s.N - 1;
@@ -2121,6 +2122,30 @@ DEV void run_chunk32(const Params &P, const Slice &s, const Smem &m, const float
     run_chunk32_vu<G, D, J, OPK, MASK, FX, false, SL>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
 }
 
+// Column groups (kGroup records) of an item that can hold a counted pair of the wave's rows: bit t
+// of the mask stands for the group at jb + t kGroup.  Lane t compares the box of group t with the
+// box of the wave's 64 rows (side by side in the slice's spatial order); 64 groups per call.  The
+// boxes are rounded outwards to binary32 and the limit carries a margin, so no counted pair is
+// lost.  Workgroup tiles alone left 75 evaluated pairs for one counted at N = 262144 points of the
+// sphere and a reach of 0.05 rad; with them the call went from 3.24 to 1.45 ms.
+DEV lanes_t near_groups(const Params &P, const Slice &s, const Item &w, int jb) {
+  const int r0 = w.i0 + (int)(threadIdx.x & ~63u);
+  const int last = (int)((s.N - 1) / kGroup);
+  const float *bx = P.gboxes + (int64_t)s.grp_off * 6;
+  const float *a0 = bx + 6 * min(r0 / kGroup, last);
+  const float *a1 = bx + 6 * min(r0 / kGroup + 1, last);
+  const int g = jb / kGroup + (int)__lane_id();
+  const float *b = bx + 6 * min(g, last);
+  float d2 = 0.f;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const float lo = __builtin_fminf(a0[k], a1[k]), hi = __builtin_fmaxf(a0[3 + k], a1[3 + k]);
+    const float gap = __builtin_fmaxf(0.f, __builtin_fmaxf(b[k] - hi, lo - b[3 + k]));
+    d2 = __builtin_fmaf(gap, gap, d2);
+  }
+  return __builtin_amdgcn_ballot_w64(g * kGroup < w.j1 && d2 <= s.clim2);
+}
+
 // SLOAD: column records are read straight from global memory with wave-uniform addresses, which
 // the compiler turns into scalar loads (SGPR operands, scalar cache) -- no LDS staging, no
 // barriers inside an item.  Otherwise columns are staged through LDS in chunks of P.tj.
@@ -2128,7 +2153,10 @@ DEV void run_chunk32(const Params &P, const Slice &s, const Smem &m, const float
 // per CU, which their small LDS footprint allows; the few values this spills are per-item ones
 // (the fused ones spill a few SGPR-held values of the pair loop too, and still gain: the 256
 // ragged 2D slices' du_L^2 and joint du_L from one launch, 73.7 -> 57.6 ms).
-template <int G, int D, bool J, int OPK, bool SLOAD, bool FX>
+// NEAR: the launch has slices whose column groups are culled per wave (near_groups).  A kernel of
+// its own, because the runs' loop costs launches without culling 4 % of a 1D single pass
+// (N = 32768, sphere: 8.05 against 8.37 ms).
+template <int G, int D, bool J, int OPK, bool SLOAD, bool FX, bool NEAR = false>
 __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, const float *__restrict__ rec) {
   extern __shared__ __align__(16) char smem_raw[];
   constexpr int F = Rec<G, D>::f32;
@@ -2164,7 +2192,8 @@ __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, 
       since_flush = 0;
     }
     since_flush += work;
-    const Row row = item_row<J>(w, s);
+    const bool culled = NEAR && __builtin_amdgcn_readfirstlane(__float_as_int(s.clim2)) != 0;
+    const Row row = item_row<J>(w, s, culled);
     float ri[F];
 #pragma unroll
     for (int k = 0; k < F; ++k) ri[k] = rec[(s.pt_off + row.rec) * F + k];
@@ -2176,9 +2205,27 @@ __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, 
         const int64_t off = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(po >> 32)) << 32) |
                                       (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)po));
         const float4 *col = (const float4 *)(rec + off * F);
-        if (w.j0 < row.jm) run_chunk32<G, D, J, OPK, true, FX, true>(P, s, m, ri, row.i, w.j0, row.jm, col, 0, cur);
-        if (row.jm < w.j1)
-          run_chunk32<G, D, J, OPK, false, FX, true>(P, s, m, ri, row.i, max(row.jm, w.j0), w.j1, col, 0, cur);
+        auto run = [&](int ja, int je) {
+          const int jm = min(row.jm, je);
+          if (ja < jm) run_chunk32<G, D, J, OPK, true, FX, true>(P, s, m, ri, row.i, ja, jm, col, 0, cur);
+          if (jm < je)
+            run_chunk32<G, D, J, OPK, false, FX, true>(P, s, m, ri, row.i, max(jm, ja), je, col, 0, cur);
+        };
+        if constexpr (NEAR) {
+          // the runs of neighbouring groups that the wave's rows can reach, or all columns
+          for (int jb = w.j0; jb < w.j1; jb += culled ? 64 * kGroup : w.j1 - w.j0) {
+            lanes_t near = culled ? near_groups(P, s, w, jb) : 1ull;
+            while (near) {
+              const int t = __builtin_ctzll(near);
+              const lanes_t rest = near >> t;  // starts with a run of set bits
+              const int n = ~rest ? __builtin_ctzll(~rest) : 64;
+              near = t + n < 64 ? (rest >> n) << (t + n) : 0ull;
+              run(jb + t * kGroup, culled ? min(w.j1, jb + (t + n) * kGroup) : w.j1);
+            }
+          }
+        } else {
+          run(w.j0, w.j1);
+        }
       }
     } else {
       for (int jb = w.j0; jb < w.j1; jb += P.tj) {
@@ -2726,7 +2773,7 @@ namespace sfk {
 
 // the kernels of one (geometry, D): histogram, B-strip, re-bin and fused re-bin entry points
 struct KernelTable {
-  const void *(*hist)(bool J, bool mixed, int opk, bool sload, bool fx);
+  const void *(*hist)(bool J, bool mixed, int opk, bool sload, bool fx, bool near);
   const void *(*strip)(int opk);
   const void *(*recheck)(bool J, bool sp);
   const void *(*recheck_multi)(bool J);
@@ -2737,42 +2784,43 @@ KernelTable table_sphere2();
 KernelTable table_sphere3();
 
 #if SF_PART > 0
-template <int G, int D, bool J, bool SL, bool FX>
+template <int G, int D, bool J, bool SL, bool FX, bool NR>
 static const void *hist32_fn(int opk) {
   // fused outputs: scalar-loaded columns only
-  if (opk == 9) return (const void *)&hist32<G, D, J, 9, true, FX>;
-  if (opk == 10) return (const void *)&hist32<G, D, J, 10, true, FX>;
-  if (opk == 11) return (const void *)&hist32<G, D, J, 11, true, FX>;
-  if (opk == 12) return (const void *)&hist32<G, D, J, 12, true, FX>;
-  if (opk == 13) return (const void *)&hist32<G, D, J, 13, true, FX>;
+  if (opk == 9) return (const void *)&hist32<G, D, J, 9, true, FX, NR>;
+  if (opk == 10) return (const void *)&hist32<G, D, J, 10, true, FX, NR>;
+  if (opk == 11) return (const void *)&hist32<G, D, J, 11, true, FX, NR>;
+  if (opk == 12) return (const void *)&hist32<G, D, J, 12, true, FX, NR>;
+  if (opk == 13) return (const void *)&hist32<G, D, J, 13, true, FX, NR>;
   if constexpr (!J) {
-    if (opk == 3) return (const void *)&hist32<G, D, false, 3, SL, false>;
+    if (opk == 3) return (const void *)&hist32<G, D, false, 3, SL, false, NR>;
     if constexpr (SL) {  // 1D, scalar-loaded columns (the default): L^3, T, T^2, T^3
-      if (opk == 5) return (const void *)&hist32<G, D, false, 5, true, false>;
-      if (opk == 6) return (const void *)&hist32<G, D, false, 6, true, false>;
-      if (opk == 7) return (const void *)&hist32<G, D, false, 7, true, false>;
-      if (opk == 8) return (const void *)&hist32<G, D, false, 8, true, false>;
+      if (opk == 5) return (const void *)&hist32<G, D, false, 5, true, false, NR>;
+      if (opk == 6) return (const void *)&hist32<G, D, false, 6, true, false, NR>;
+      if (opk == 7) return (const void *)&hist32<G, D, false, 7, true, false, NR>;
+      if (opk == 8) return (const void *)&hist32<G, D, false, 8, true, false, NR>;
     }
   } else {
-    if (opk == 4) return (const void *)&hist32<G, D, true, 4, SL, FX>;
+    if (opk == 4) return (const void *)&hist32<G, D, true, 4, SL, FX, NR>;
   }
-  if (opk == 1) return (const void *)&hist32<G, D, J, 1, SL, FX>;
-  if (opk == 2) return (const void *)&hist32<G, D, J, 2, SL, FX>;
-  return (const void *)&hist32<G, D, J, 0, SL, FX>;
+  if (opk == 1) return (const void *)&hist32<G, D, J, 1, SL, FX, NR>;
+  if (opk == 2) return (const void *)&hist32<G, D, J, 2, SL, FX, NR>;
+  return (const void *)&hist32<G, D, J, 0, SL, FX, NR>;
 }
 
-template <int G, int D, bool J, bool SL>
+template <int G, int D, bool J, bool SL, bool NR>
 static const void *hist32_fx(bool fx, int opk) {
   // fixed-point cells exist for joint histograms only
   if constexpr (J) {
-    if (fx) return hist32_fn<G, D, true, SL, true>(opk);
+    if (fx) return hist32_fn<G, D, true, SL, true, NR>(opk);
   }
-  return hist32_fn<G, D, J, SL, false>(opk);
+  return hist32_fn<G, D, J, SL, false, NR>(opk);
 }
 
 template <int G, int D, bool J>
-static const void *hist_fn(bool mixed, int opk, bool sload, bool fx) {
-  if (mixed) return sload ? hist32_fx<G, D, J, true>(fx, opk) : hist32_fx<G, D, J, false>(fx, opk);
+static const void *hist_fn(bool mixed, int opk, bool sload, bool fx, bool near) {
+  if (mixed && near && sload) return hist32_fx<G, D, J, true, true>(fx, opk);
+  if (mixed) return sload ? hist32_fx<G, D, J, true, false>(fx, opk) : hist32_fx<G, D, J, false, false>(fx, opk);
   if constexpr (!J) {
     if (opk == 3) return (const void *)&hist64<G, D, false, 3>;
     if (opk == 5) return (const void *)&hist64<G, D, false, 5>;
@@ -2806,8 +2854,8 @@ static const void *recheck_multi_fn(bool J) {
 }
 
 template <int G, int D>
-static const void *hist_of(bool J, bool mixed, int opk, bool sload, bool fx) {
-  return J ? hist_fn<G, D, true>(mixed, opk, sload, fx) : hist_fn<G, D, false>(mixed, opk, sload, fx);
+static const void *hist_of(bool J, bool mixed, int opk, bool sload, bool fx, bool near) {
+  return J ? hist_fn<G, D, true>(mixed, opk, sload, fx, near) : hist_fn<G, D, false>(mixed, opk, sload, fx, near);
 }
 template <int G, int D>
 static KernelTable table_of() {
@@ -2861,8 +2909,8 @@ hipError_t launch_prep(int G, int D, bool mixed, int geom_code, const void *ps, 
                 : prep_impl<kSphere, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st);
 }
 
-static const void *pick_hist(int G, int D, bool J, bool mixed, int opk, bool sl, bool fx) {
-  return table(G, D).hist(J, mixed, opk, sl, fx);
+static const void *pick_hist(int G, int D, bool J, bool mixed, int opk, bool sl, bool fx, bool near) {
+  return table(G, D).hist(J, mixed, opk, sl, fx, near);
 }
 
 static int opk_of(const Params &P) {
@@ -2880,7 +2928,7 @@ static int opk_of(const Params &P) {
 
 int hist_occupancy(int G, int D, bool J, bool mixed, int opk, bool sload, bool fx, int block,
                    size_t smem) {
-  const void *f = pick_hist(G, D, J, mixed, opk, sload, fx);
+  const void *f = pick_hist(G, D, J, mixed, opk, sload, fx, false);
   (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   int nb = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, block, smem) != hipSuccess) return 1;
@@ -2902,7 +2950,7 @@ int strip_occupancy(int G, int D, int opk, int block, size_t smem) {
 hipError_t launch_hist(int G, int D, bool J, bool mixed, bool sload, const Params &P, int grid,
                        int block, size_t smem, hipStream_t st) {
   const void *f = (mixed && P.strip > 1) ? pick_strip(G, D, opk_of(P))
-                                         : pick_hist(G, D, J, mixed, opk_of(P), sload, mixed && P.fx);
+                                         : pick_hist(G, D, J, mixed, opk_of(P), sload, mixed && P.fx, P.gboxes != nullptr);
   (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   Params Pc = P;
   const int opk = opk_of(P);
