@@ -2263,12 +2263,14 @@ __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, 
 template <int G, int D>
 struct StripRec {
   // the strip's LDS stage per column: positions (flat x_hi, x_lo; sphere P_hi, P_lo) and per field
-  // the velocity (flat u_hi, u_lo; sphere U_hi, U_lo, u_r hi/lo), each padded to whole float4s
+  // the velocity (flat u_hi, u_lo; sphere U_hi, U_lo, the norm's bound, u_r hi/lo), each padded to
+  // whole float4s
   static constexpr int pos = (G == kFlat) ? 2 * D : 6;      // floats of the position part
   static constexpr int PS = (pos + 3) / 4 * 4;
   static constexpr int voff = (G == kFlat) ? 2 * D : 6;     // velocity part's offset in a record
-  static constexpr int vel = (G == kFlat) ? 2 * D : (D == 3 ? 8 : 6);
+  static constexpr int vel = (G == kFlat) ? 2 * D : (D == 3 ? 9 : 6);
   static constexpr int VS = (vel + 3) / 4 * 4;
+  static_assert(PS + kStripMax * VS <= kStripMax * Rec<G, D>::f32, "the strip's LDS stage holds kStripMax records a column");
 };
 
 template <int N4>
@@ -2373,7 +2375,7 @@ DEV void run_chunk_strip(const Params &P, const Slice &s, const Smem &m, const f
               T = __builtin_fmaf(w[2], dU[2], __builtin_fmaf(w[1], dU[1], w[0] * dU[0])) * inv_s;
               tn2 = T * T;
               if constexpr (D == 3) {
-                const float dw = (rjb[6] - rib[6]) + (rjb[7] - rib[7]);
+                const float dw = (rjb[7] - rib[7]) + (rjb[8] - rib[8]);
                 tn2 = __builtin_fmaf(dw, dw, tn2);
               }
               n2 = __builtin_fmaf(L, L, tn2);
