@@ -37,6 +37,7 @@ hipError_t launch_merge_checked(const double *src_s, const unsigned long long *s
                                 const unsigned long long *pcount, int64_t cap, int *flag,
                                 hipStream_t st);
 hipError_t launch_zero(void *p, int64_t bytes, hipStream_t st);
+hipError_t launch_absmax(int count, const double *const *x, const int64_t *n, double *out, hipStream_t st);
 hipError_t launch_zero_multi(int count, void *const *p, const int64_t *bytes, hipStream_t st);
 hipError_t launch_derive_sp(double *s, unsigned long long *c, int64_t nbins, hipStream_t st);
 hipError_t launch_eval_math(int fn, int64_t n, const double *a, const double *b, double *out,
@@ -110,6 +111,68 @@ struct DevBuf {
   }
 };
 
+// Page-locked host memory for one kind of transfer, kept by a context.  `done` follows the last
+// copy out of it: the buffer is not written before that copy has ended.
+struct Stage {
+  char *p = nullptr;
+  size_t cap = 0;
+  hipEvent_t done = nullptr;
+  bool busy = false;
+  hipError_t acquire(size_t n) {
+    if (busy) {
+      const hipError_t e = hipEventSynchronize(done);
+      if (e != hipSuccess) return e;
+      busy = false;
+    }
+    if (n <= cap && p) return hipSuccess;
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    cap = 0;
+    const size_t want = std::max<size_t>(n, 1 << 16);
+    const hipError_t e = hipHostMalloc((void **)&p, want, hipHostMallocDefault);
+    if (e == hipSuccess) cap = want;
+    return e;
+  }
+  // copies the first n bytes to the device and marks the buffer busy until that has happened
+  hipError_t send(void *dst, size_t n, hipStream_t st) {
+    hipError_t e = hipSuccess;
+    if (!done) e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipMemcpyAsync(dst, p, n, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) {
+      busy = true;
+      e = hipEventRecord(done, st);
+      if (e != hipSuccess) {  // no event to wait for: wait here
+        busy = false;
+        (void)hipStreamSynchronize(st);
+      }
+    }
+    return e;
+  }
+  void release() {
+    if (busy) (void)hipEventSynchronize(done);
+    if (p) (void)hipHostFree(p);
+    if (done) (void)hipEventDestroy(done);
+    p = nullptr;
+    cap = 0;
+    done = nullptr;
+    busy = false;
+  }
+};
+// Larger transfers go from and to pageable memory: the copy through a staging buffer would cost
+// more than the driver's handling of a pageable one, and the kept memory stays bounded.
+inline constexpr size_t kStageMax = 1 << 20;
+
+// largest |v| (NaN ignored): several running maxima, because one is a chain of dependent compares
+double abs_max(const double *v, int64_t n) {
+  double m[8] = {};
+  int64_t k = 0;
+  for (; k + 8 <= n; k += 8)
+    for (int l = 0; l < 8; ++l) m[l] = std::max(m[l], fabs(v[k + l]));
+  for (; k < n; ++k) m[0] = std::max(m[0], fabs(v[k]));
+  for (int l = 1; l < 8; ++l) m[0] = std::max(m[0], m[l]);
+  return m[0];
+}
+
 bool jl_isless(double a, double b) {
   if (a != a) return false;
   if (b != b) return true;
@@ -146,11 +209,14 @@ struct Partition {
   int M;
   int elo, ehi;
   int ncell() const { return (ehi - elo) << M; }
-  // real lower bound of cell c (c = 0 also stands for everything below)
-  long double low(int c) const {
+  // lower bound of cell c (c = 0 also stands for everything below): (1 + m / 2^M) 2^e, exact
+  double low(int c) const {
     const int e = elo + (c >> M);
-    const int m = c & ((1 << M) - 1);
-    return ldexpl(1.0L + (long double)m / (long double)(1 << M), e);
+    const uint64_t m = (uint64_t)(c & ((1 << M) - 1));
+    const uint64_t bits = ((uint64_t)(e + 1023) << 52) | (m << (52 - M));
+    double v;
+    memcpy(&v, &bits, sizeof v);
+    return v;
   }
 };
 
@@ -205,19 +271,19 @@ struct Plan {
   Params P{};
   DevBuf<double> rec64;
   DevBuf<float> rec32;
-  DevBuf<Slice> slices;
-  DevBuf<Item> items;
-  DevBuf<Cell> cells;
-  DevBuf<double> dedges, vedges;
-  DevBuf<float> vedges32;
-  DevBuf<double> acc_s;
-  DevBuf<unsigned long long> acc_c;
-  DevBuf<int> counter;
-  DevBuf<unsigned long long> pcount;
-  DevBuf<Item> items64;
+  DevBuf<char> tables;  // slices, items, tables, edges and record sources: one upload
+  const PrepSliceHost *prep = nullptr;
+  const Item *items64 = nullptr;
+  // accumulators: sums, counts, the re-bin queue's count, the work counter and the overflow flag,
+  // in one piece (one clear; a host call reads sums, counts and queue count in one copy)
+  DevBuf<char> acc;
+  double *acc_s = nullptr;
+  unsigned long long *acc_c = nullptr;
+  unsigned long long *pcount = nullptr;
+  int *counter = nullptr;
+  int *flag = nullptr;
+  size_t acc_bytes = 0;
   DevBuf<Pending> pending;
-  DevBuf<PrepSliceHost> prep;
-  DevBuf<int> flag;
   DevBuf<float> gboxes;   // boxes of the column groups of culled slices
   DevBuf<int32_t> perm;   // spatial order of the binary32 records (tile culling)
   bool culled = false;    // some work items were dropped by tile culling
@@ -237,10 +303,7 @@ struct Plan {
   void release() {
     if (graph) (void)hipGraphExecDestroy(graph);
     graph = nullptr;
-    rec64.release(); rec32.release(); slices.release(); items.release(); cells.release();
-    dedges.release(); vedges.release(); vedges32.release(); acc_s.release(); acc_c.release();
-    counter.release(); pcount.release(); pending.release(); prep.release(); flag.release();
-    items64.release();
+    rec64.release(); rec32.release(); tables.release(); acc.release(); pending.release();
     perm.release();
     gboxes.release();
     msums.release();
@@ -300,6 +363,9 @@ struct sf_ctx {
   std::map<TuneKey, Tuning> tuned;
   // device buffers: host-input staging and the plan reused by one-shot calls
   DevBuf<double> d_x, d_u;
+  DevBuf<char> d_out;   // host calls of several outputs: their device sums and counts
+  DevBuf<double> d_max;  // coordinate magnitudes (partial maxima)
+  Stage up_xu, up_tab, down;  // host calls' inputs, every call's tables, read-backs
   Plan oneshot;
   // the allocation-free entry: its plan (buffers borrowed from the scratch array) and this
   // device's address of the array
@@ -514,17 +580,12 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   Partition P64 = make_partition(k64, 1024, 6);
   const int n64 = P64.ncell();
   T.tab64.resize(n64);
+  int b64 = 0;  // edges below the cell: they ascend, and so do the cells
   for (int c = 0; c < n64; ++c) {
-    const long double lowl = (c == 0) ? 0.0L : P64.low(c);
-    const double low = (double)lowl;  // cell bounds are exact binary64 values
-    int b = 0;
-    if (c == 0) {
-      // keys below the window: only non-positive edges are below them
-      for (int k = 0; k < nE; ++k) if (T.dedges[k] <= 0.0) b = k + 1;
-    } else {
-      for (int k = 0; k < nE; ++k) if (T.dedges[k] < low) b = k + 1;
-    }
-    T.tab64[c].bx = b;
+    const double low = P64.low(c);  // cell bounds are exact binary64 values
+    // (keys below the window, c = 0: only non-positive edges are below them)
+    while (b64 < nE && (c == 0 ? T.dedges[b64] <= 0.0 : T.dedges[b64] < low)) ++b64;
+    T.tab64[c].bx = b64;
     T.tab64[c].lo = INFINITY;
     T.tab64[c].hi = INFINITY;
     T.tab64[c].blo = 0;
@@ -573,16 +634,32 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   const float close = flat ? round_up_f(std::max(1e-30L, ldexpl((long double)xmax * (long double)xmax, -44)))
                            : 0x1p-44f;
   const float anti = 4.0f - 0x1p-20f;
-  for (int c = 0; c < n32; ++c) {
-    const float Fc = (c == 0) ? -INFINITY : (float)P32.low(c);
-    const float Fn = (c + 1 >= n32) ? INFINITY : (float)P32.low(c + 1);
-    int nint = 0, which = -1, below = 0;
-    for (int k = 0; k < nE; ++k) {
-      if (C[k] == -INFINITY || hi[k] < Fc) { ++below; continue; }  // -Inf: below every key
-      if (lo[k] >= Fn) continue;
-      ++nint;
-      which = k;
+  // per cell: the edges whose intervals end below it, and the number (and the index, where it is
+  // one) of those that meet it, from each edge's first and last cell
+  std::vector<float> F(n32 + 1);
+  for (int c = 0; c < n32; ++c) F[c] = (float)P32.low(c);
+  F[0] = -INFINITY;
+  F[n32] = INFINITY;
+  std::vector<int> dbelow(n32 + 1, 0), dmeet(n32 + 1, 0), dwhich(n32 + 1, 0);
+  for (int k = 0; k < nE; ++k) {
+    if (C[k] == -INFINITY) { ++dbelow[0]; continue; }  // -Inf: below every key
+    const int c0 = (int)(std::partition_point(F.begin() + 1, F.end(), [&](float Fn) { return lo[k] >= Fn; }) -
+                         (F.begin() + 1));
+    const int c1 = (int)(std::partition_point(F.begin(), F.begin() + n32, [&](float Fc) { return !(hi[k] < Fc); }) -
+                         F.begin());
+    ++dbelow[c1];
+    if (c0 < c1) {
+      ++dmeet[c0];
+      --dmeet[c1];
+      dwhich[c0] += k;
+      dwhich[c1] -= k;
     }
+  }
+  for (int c = 0, below = 0, nint = 0, which = 0; c < n32; ++c) {
+    const float Fc = F[c], Fn = F[c + 1];
+    below += dbelow[c];
+    nint += dmeet[c];
+    which += dwhich[c];
     Cell &cl = T.tab32[c];
     cl.bx = 0;
     cl.blo = below;
@@ -704,6 +781,21 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   }
 }
 
+// whether build_tables gives both slices of a batch (validate_batch: one geometry, operator and bin
+// counts) the same tables
+bool same_tables(const sf_problem &a, double xa, const sf_problem &b, double xb) {
+  auto rule = [](const sf_bin_rule *r, const sf_bin_rule *q) {
+    return r == q || (r && q && r->kind == q->kind && r->padded == q->padded && r->n == q->n &&
+                      r->first_edge == q->first_edge && r->last_edge == q->last_edge &&
+                      r->inv_step == q->inv_step && r->step_val == q->step_val);
+  };
+  auto edges = [](const double *e, const double *f, int n) {
+    return e == f || memcmp(e, f, sizeof(double) * n) == 0;
+  };
+  return xa == xb && rule(a.dist_rule, b.dist_rule) && edges(a.dist_edges, b.dist_edges, a.n_dist + 1) &&
+         (a.n_val == 0 || (rule(a.val_rule, b.val_rule) && edges(a.val_edges, b.val_edges, a.n_val + 1)));
+}
+
 int64_t pairs_of(int64_t n) { return n > 1 ? n * (n - 1) / 2 : 0; }
 
 // output cells per slice: (n_dist), (n_dist, n_val), or (6, n_dist) for the single pass
@@ -762,6 +854,11 @@ extern "C" void sf_destroy(sf_ctx *ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   ctx->d_x.release();
   ctx->d_u.release();
+  ctx->d_out.release();
+  ctx->d_max.release();
+  ctx->up_xu.release();
+  ctx->up_tab.release();
+  ctx->down.release();
   ctx->oneshot.release();
   ctx->noalloc.release();
   ctx->fused.release();
@@ -1060,9 +1157,13 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   std::vector<double> dedges, vedges;
   std::vector<float> vedges32;
   int ncell_max = 1;
+  SliceTables T;
   for (int s = 0; s < n; ++s) {
-    SliceTables T;
-    build_tables(sl[s], xmax[s], T);
+    // (slices of one call mostly bin by the same edges: a table is built where they differ)
+    if (s == 0 || !same_tables(sl[s - 1], xmax[s - 1], sl[s], xmax[s])) {
+      T = SliceTables();
+      build_tables(sl[s], xmax[s], T);
+    }
     Slice d = T.desc;
     d.N = sl[s].N;
     d.pt_off = prep[s].pt_off;
@@ -1240,9 +1341,6 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
       sdesc[s].clim2 = round_up_f((long double)cinfo[s].limit * cinfo[s].limit * (1.0L + 1e-5L) + 1e-30L);
     }
   }
-  PLBUF(pl.prep, (n));
-  HIPCHK(hipMemcpyAsync(pl.prep.p, prep.data(), sizeof(PrepSliceHost) * n, hipMemcpyHostToDevice, st));
-
   std::vector<int> order(n);
   for (int s = 0; s < n; ++s) order[s] = s;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return sl[a].N > sl[b].N; });
@@ -1299,34 +1397,55 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   pl.copies = copies;
   pl.sload = sload;
 
-  // ---- upload
-  PLBUF(pl.slices, (n));
-  PLBUF(pl.items, (items.size()));
-  PLBUF(pl.cells, (cells.size()));
-  PLBUF(pl.dedges, (dedges.size()));
-  PLBUF(pl.vedges, (vedges.size()));
-  PLBUF(pl.vedges32, (vedges32.size()));
-  PLBUF(pl.acc_s, ((size_t)pl.nout * ncell));
-  PLBUF(pl.acc_c, ((size_t)pl.nout * ncell));
+  // ---- upload: every table in one copy
+  struct Part {
+    const void *src;
+    size_t bytes, off;
+  };
+  Part parts[] = {{sdesc.data(), sizeof(Slice) * n, 0},
+                  {items.data(), sizeof(Item) * items.size(), 0},
+                  {cells.data(), sizeof(Cell) * cells.size(), 0},
+                  {dedges.data(), sizeof(double) * dedges.size(), 0},
+                  {vedges.data(), sizeof(double) * vedges.size(), 0},
+                  {vedges32.data(), sizeof(float) * vedges32.size(), 0},
+                  {prep.data(), sizeof(PrepSliceHost) * n, 0},
+                  {items64.data(), sizeof(Item) * items64.size(), 0}};
+  size_t total = 0;
+  for (Part &q : parts) {
+    q.off = total;
+    total = (total + q.bytes + 255) & ~(size_t)255;
+  }
+  PLBUF(pl.tables, total);
+  {
+    // from page-locked memory, without waiting for it (the allocation-free entry keeps none)
+    const bool pinned = !pl.arena && total <= kStageMax;
+    std::vector<char> own(pinned ? 0 : total);
+    if (pinned) HIPCHK(ctx->up_tab.acquire(total));
+    char *h = pinned ? ctx->up_tab.p : own.data();
+    for (const Part &q : parts)
+      if (q.bytes) memcpy(h + q.off, q.src, q.bytes);
+    if (pinned) {
+      HIPCHK(ctx->up_tab.send(pl.tables.p, total, st));
+    } else {
+      HIPCHK(hipMemcpyAsync(pl.tables.p, h, total, hipMemcpyHostToDevice, st));
+      HIPCHK(hipStreamSynchronize(st));
+    }
+  }
+  char *tb = pl.tables.p;
+  pl.prep = (const PrepSliceHost *)(tb + parts[6].off);
+  pl.items64 = (const Item *)(tb + parts[7].off);
+  const size_t acells = (size_t)pl.nout * ncell;
+  pl.acc_bytes = 16 * acells + 4 * sizeof(unsigned long long) + 8 * sizeof(int);
+  PLBUF(pl.acc, pl.acc_bytes);
+  pl.acc_s = (double *)pl.acc.p;
+  pl.acc_c = (unsigned long long *)(pl.acc_s + acells);
+  pl.pcount = pl.acc_c + acells;
+  pl.counter = (int *)(pl.pcount + 4);
+  pl.flag = pl.counter + 4;
   if (pl.n1d) {
     PLBUF(pl.msums, ((size_t)pl.n1d * pl.nout * p0.n_dist));
     PLBUF(pl.mcounts, ((size_t)pl.n1d * pl.nout * p0.n_dist));
   }
-  PLBUF(pl.counter, (4));
-  PLBUF(pl.pcount, (4));
-  PLBUF(pl.flag, (4));
-  HIPCHK(hipMemcpyAsync(pl.slices.p, sdesc.data(), sizeof(Slice) * n, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(pl.items.p, items.data(), sizeof(Item) * items.size(), hipMemcpyHostToDevice, st));
-  if (strip) {
-    PLBUF(pl.items64, (items64.size()));
-    HIPCHK(hipMemcpyAsync(pl.items64.p, items64.data(), sizeof(Item) * items64.size(), hipMemcpyHostToDevice, st));
-  }
-  HIPCHK(hipMemcpyAsync(pl.cells.p, cells.data(), sizeof(Cell) * cells.size(), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(pl.dedges.p, dedges.data(), sizeof(double) * dedges.size(), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(pl.vedges.p, vedges.data(), sizeof(double) * vedges.size(), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(pl.vedges32.p, vedges32.data(), sizeof(float) * vedges32.size(), hipMemcpyHostToDevice, st));
-  // host vectors go out of scope: make the asynchronous copies complete first
-  HIPCHK(hipStreamSynchronize(st));
 
   pl.cap = 0;
   if (mixed) {
@@ -1348,22 +1467,22 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
 
   Params &P = pl.P;
   P = Params{};
-  P.slices = pl.slices.p;
-  P.items = pl.items.p;
+  P.slices = (const Slice *)(tb + parts[0].off);
+  P.items = (const Item *)(tb + parts[1].off);
   P.n_items = pl.n_items;
   P.block_rows = block;
-  P.counter = pl.counter.p;
+  P.counter = pl.counter;
   P.rec64 = pl.rec64.p;
   P.rec32 = pl.rec32.p;
   P.gboxes = pl.near ? pl.gboxes.p : nullptr;
-  P.cells = pl.cells.p;
-  P.dedges = pl.dedges.p;
-  P.vedges = pl.vedges.p;
-  P.vedges32 = pl.vedges32.p;
-  P.sums = pl.acc_s.p;
-  P.counts = pl.acc_c.p;
+  P.cells = (const Cell *)(tb + parts[2].off);
+  P.dedges = (const double *)(tb + parts[3].off);
+  P.vedges = (const double *)(tb + parts[4].off);
+  P.vedges32 = (const float *)(tb + parts[5].off);
+  P.sums = pl.acc_s;
+  P.counts = pl.acc_c;
   P.pending = pl.pending.p;
-  P.pending_count = pl.pcount.p;
+  P.pending_count = pl.pcount;
   P.pending_cap = pl.cap;
   P.stats = nullptr;
   P.ncell_max = ncell_max;
@@ -1417,18 +1536,16 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
   sf_ctx *ctx = pl.ctx;
   if (pl.total_pairs == 0) return SF_OK;
   const int64_t ncells = (int64_t)pl.nout * pl.ncell;
-  HIPCHK(launch_prep(pl.G, pl.D, use_mixed, pl.geom_code, pl.prep.p, pl.n, pl.max_n, pl.rec64.p,
+  HIPCHK(launch_prep(pl.G, pl.D, use_mixed, pl.geom_code, pl.prep, pl.n, pl.max_n, pl.rec64.p,
                      pl.rec32.p, st));
   const int64_t mcells = (int64_t)pl.n1d * pl.nout * pl.P.n_dist;
   if (pl.n1d && !use_mixed)  // fused outputs exist in the binary32 kernel only
     return ctx->fail(SF_E_UNSUPPORTED, "internal: fused outputs launched on the binary64 kernel");
   {
-    // accumulators, the work counter, the re-bin queue count and the overflow flag: one launch
-    void *zp[kZeroSetMax] = {pl.acc_s.p, pl.acc_c.p, pl.counter.p, pl.pcount.p, pl.flag.p};
-    int64_t zb[kZeroSetMax] = {(int64_t)sizeof(double) * ncells, (int64_t)sizeof(unsigned long long) * ncells,
-                               (int64_t)sizeof(int) * 4, (int64_t)sizeof(unsigned long long) * 4,
-                               (int64_t)sizeof(int) * 4};
-    int nz = 5;
+    // accumulators, queue count, work counter and overflow flag, and the fused ones: one launch
+    void *zp[kZeroSetMax] = {pl.acc.p};
+    int64_t zb[kZeroSetMax] = {(int64_t)pl.acc_bytes};
+    int nz = 1;
     if (pl.n1d) {
       zp[nz] = pl.msums.p;
       zb[nz++] = (int64_t)sizeof(double) * mcells;
@@ -1449,7 +1566,7 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
     P.flush_limit = 0x7fffffffLL;
     if (pl.strip) {  // one slice at a time
       P.strip = 0;
-      P.items = pl.items64.p;
+      P.items = pl.items64;
       P.n_items = pl.n_items64;
     }
   }
@@ -1464,24 +1581,26 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
   // 2.7e8 queued pairs: 22.6 / 16.7 / 19.6 ms with one / four / eight per CU)
   if (use_mixed) HIPCHK(launch_recheck(pl.G, pl.D, pl.J, P, 4 * ctx->n_cu, st));
   if (ev) HIPCHK(hipEventRecord(ev[2], st));
-  // (a fused call without a joint output passes no out_s / out_c)
+  // (a fused call without a joint output passes no out_s / out_c, a host call reads acc)
   if (out_s)
-    HIPCHK(launch_merge_checked(pl.acc_s.p, pl.acc_c.p, out_s, out_c, ncells,
-                                use_mixed ? pl.pcount.p : nullptr, pl.cap, pl.flag.p, st));
+    HIPCHK(launch_merge_checked(pl.acc_s, pl.acc_c, out_s, out_c, ncells,
+                                use_mixed ? pl.pcount : nullptr, pl.cap, pl.flag, st));
   const int64_t per = (int64_t)pl.nout * pl.P.n_dist;
   for (int k = 0; k < pl.n1d; ++k)
     HIPCHK(launch_merge_checked(pl.msums.p + k * per, pl.mcounts.p + k * per, pl.mdst_s[k], pl.mdst_c[k], per,
-                                pl.pcount.p, pl.cap, pl.flag.p, st));
-  if (pl.sp) HIPCHK(launch_derive_sp(out_s, out_c, (int64_t)pl.nout * pl.P.n_dist, st));
+                                pl.pcount, pl.cap, pl.flag, st));
+  if (pl.sp && out_s) HIPCHK(launch_derive_sp(out_s, out_c, (int64_t)pl.nout * pl.P.n_dist, st));
   if (ev) HIPCHK(hipEventRecord(ev[3], st));
   return SF_OK;
 }
 
 // One-shot: build (into the context's cached plan, reusing its buffers), launch, and on a
-// re-bin queue overflow redo the call with the binary64 kernel.
+// re-bin queue overflow redo the call with the binary64 kernel.  h_acc (host calls; out_s and out_c
+// are null then): receives the accumulators (sums, then counts) instead of a merge, read with the
+// queue's count in one copy.
 int run_batch(sf_ctx *ctx, int n, const sf_problem *sl, const double *const *dx,
               const double *const *du, const double *xmax, double *out_s,
-              unsigned long long *out_c, hipStream_t st) {
+              unsigned long long *out_c, hipStream_t st, std::vector<char> *h_acc = nullptr) {
   Plan &pl = ctx->oneshot;
   int rc = plan_build(ctx, pl, n, sl, dx, du, xmax, st, true);
   if (rc) return rc;
@@ -1496,10 +1615,25 @@ int run_batch(sf_ctx *ctx, int n, const sf_problem *sl, const double *const *dx,
     if (!ctx->ev[k]) HIPCHK(hipEventCreate(&ctx->ev[k]));
   rc = plan_launch(pl, pl.mixed, out_s, out_c, st, ctx->ev);
   if (rc) return rc;
-  if (pl.mixed) {
-    unsigned long long pc = 0;
-    HIPCHK(hipMemcpyAsync(&pc, pl.pcount.p, sizeof(pc), hipMemcpyDeviceToHost, st));
+  unsigned long long pc = 0;
+  const size_t acells = 16 * (size_t)pl.nout * pl.ncell;  // bytes of sums and counts
+  auto fetch = [&]() -> int {
+    const size_t from = h_acc ? 0 : acells, bytes = acells + sizeof(pc) - from;
+    const bool pinned = bytes <= kStageMax;
+    if (pinned) HIPCHK(ctx->down.acquire(bytes));
+    if (h_acc) h_acc->resize(bytes);
+    char *h = pinned ? ctx->down.p : h_acc->data();
+    HIPCHK(hipMemcpyAsync(h, pl.acc.p + from, bytes, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    if (h_acc && pinned) memcpy(h_acc->data(), h, bytes);
+    memcpy(&pc, h + (acells - from), sizeof(pc));
+    return SF_OK;
+  };
+  if (pl.mixed || h_acc) {
+    rc = fetch();
+    if (rc) return rc;
+  }
+  if (pl.mixed) {
     ctx->stats[1] = (int64_t)pc;
     if ((int64_t)pc > pl.cap && (int64_t)pc <= kQueueMax) {
       // the merge was skipped: the queue now knows its size, so grow it and run the binary32
@@ -1511,8 +1645,8 @@ int run_batch(sf_ctx *ctx, int n, const sf_problem *sl, const double *const *dx,
       pl.P.pending_cap = pl.cap;
       rc = plan_launch(pl, true, out_s, out_c, st, ctx->ev);
       if (rc) return rc;
-      HIPCHK(hipMemcpyAsync(&pc, pl.pcount.p, sizeof(pc), hipMemcpyDeviceToHost, st));
-      HIPCHK(hipStreamSynchronize(st));
+      rc = fetch();
+      if (rc) return rc;
       ctx->stats[1] = (int64_t)pc;
     }
     if ((int64_t)pc > pl.cap) {
@@ -1524,9 +1658,90 @@ int run_batch(sf_ctx *ctx, int n, const sf_problem *sl, const double *const *dx,
       }
       rc = plan_launch(pl, false, out_s, out_c, st, ctx->ev);
       if (rc) return rc;
+      if (h_acc && (rc = fetch())) return rc;
     }
   }
   ctx->ev_pending = true;
+  return SF_OK;
+}
+
+// Coordinate magnitudes max|x| (times scale) of a batch of device slices, for the binary32 kernels'
+// margins; zero where no binary32 kernel on flat points needs them.  Partial maxima are reduced on the
+// device (a read-back of x cost 0.25 ms of a 2.3 ms call at N = 65536, 2D) into d_part: at least
+// kMaxParts doubles a slice, or null for a buffer of the context's.
+int coord_max(sf_ctx *ctx, int n, const sf_problem *sl, hipStream_t st, double scale, std::vector<double> &xmax,
+              double *d_part = nullptr) {
+  xmax.assign((size_t)n, 0.0);
+  if (sl[0].precision == SF_PREC_FP64 || sl[0].geometry != SF_GEOM_FLAT) return SF_OK;
+  std::vector<const double *> x;
+  std::vector<int64_t> len;
+  for (int s = 0; s < n; ++s)
+    if (sl[s].N > 0) {
+      x.push_back(sl[s].x);
+      len.push_back((int64_t)sl[s].W * sl[s].N);
+    }
+  if (x.empty()) return SF_OK;
+  const size_t np = x.size() * kMaxParts;
+  const bool pinned = !d_part && sizeof(double) * np <= kStageMax;
+  if (!d_part) {
+    HIPCHK(ctx->d_max.ensure(np));
+    d_part = ctx->d_max.p;
+  }
+  std::vector<double> own(pinned ? 0 : np);
+  if (pinned) HIPCHK(ctx->down.acquire(sizeof(double) * np));
+  double *h = pinned ? (double *)ctx->down.p : own.data();
+  HIPCHK(launch_absmax((int)x.size(), x.data(), len.data(), d_part, st));
+  HIPCHK(hipMemcpyAsync(h, d_part, sizeof(double) * np, hipMemcpyDeviceToHost, st));
+  HIPCHK(hipStreamSynchronize(st));
+  size_t k = 0;
+  for (int s = 0; s < n; ++s)
+    if (sl[s].N > 0) {
+      xmax[s] = scale * abs_max(h + k, kMaxParts);
+      k += kMaxParts;
+    }
+  return SF_OK;
+}
+
+// whether host slice s has the positions of the slice before it (auxiliary axes share them)
+bool shares_x(const sf_problem *sl, int s) {
+  return s > 0 && sl[s].x == sl[s - 1].x && sl[s].N == sl[s - 1].N && sl[s].W == sl[s - 1].W;
+}
+
+// Host slices' x and u to the device (ctx->d_x, ctx->d_u): small ones together through page-locked
+// memory, shared positions once.
+int send_inputs(sf_ctx *ctx, int n, const sf_problem *sl, hipStream_t st, std::vector<const double *> &px,
+                std::vector<const double *> &pu) {
+  int64_t tx = 0, tu = 0;
+  for (int s = 0; s < n; ++s) {
+    tx += shares_x(sl, s) ? 0 : (int64_t)sl[s].W * sl[s].N;
+    tu += (int64_t)sl[s].D * sl[s].N;
+  }
+  const bool pinned = sizeof(double) * (size_t)(tx + tu) <= kStageMax;
+  if (pinned) {
+    HIPCHK(ctx->d_x.ensure((size_t)(tx + tu) + 2));
+    HIPCHK(ctx->up_xu.acquire(sizeof(double) * (size_t)(tx + tu)));
+  } else {
+    HIPCHK(ctx->d_x.ensure((size_t)tx + 2));
+    HIPCHK(ctx->d_u.ensure((size_t)tu + 2));
+  }
+  double *h = (double *)ctx->up_xu.p;
+  int64_t ox = 0, ou = 0;
+  for (int s = 0; s < n; ++s) {
+    const bool same = shares_x(sl, s);
+    const int64_t nx = same ? 0 : (int64_t)sl[s].W * sl[s].N, nu = (int64_t)sl[s].D * sl[s].N;
+    px[s] = same ? px[s - 1] : ctx->d_x.p + ox;
+    pu[s] = pinned ? ctx->d_x.p + tx + ou : ctx->d_u.p + ou;
+    if (pinned) {
+      if (nx) memcpy(h + ox, sl[s].x, sizeof(double) * nx);
+      if (nu) memcpy(h + tx + ou, sl[s].u, sizeof(double) * nu);
+    } else {
+      if (nx) HIPCHK(hipMemcpyAsync(ctx->d_x.p + ox, sl[s].x, sizeof(double) * nx, hipMemcpyHostToDevice, st));
+      if (nu) HIPCHK(hipMemcpyAsync(ctx->d_u.p + ou, sl[s].u, sizeof(double) * nu, hipMemcpyHostToDevice, st));
+    }
+    ox += nx;
+    ou += nu;
+  }
+  if (pinned && tx + tu > 0) HIPCHK(ctx->up_xu.send(ctx->d_x.p, sizeof(double) * (size_t)(tx + tu), st));
   return SF_OK;
 }
 
@@ -1540,48 +1755,19 @@ int host_entry(sf_ctx *ctx, int n, const sf_problem *sl, double *sums, uint64_t 
   hipStream_t st = ctx->stream;
   const sf_problem &p0 = sl[0];
   const int ncell = out_cells(p0);
-  int64_t tx = 0, tu = 0;
-  for (int s = 0; s < n; ++s) {
-    tx += (int64_t)sl[s].W * sl[s].N;
-    tu += (int64_t)sl[s].D * sl[s].N;
-  }
-  HIPCHK(ctx->d_x.ensure((size_t)tx + 2));
-  HIPCHK(ctx->d_u.ensure((size_t)tu + 2));
   std::vector<const double *> px(n), pu(n);
   std::vector<double> xmax(n, 0.0);
-  int64_t ox = 0, ou = 0;
-  for (int s = 0; s < n; ++s) {
-    const int64_t nx = (int64_t)sl[s].W * sl[s].N, nu = (int64_t)sl[s].D * sl[s].N;
-    if (nx) HIPCHK(hipMemcpyAsync(ctx->d_x.p + ox, sl[s].x, sizeof(double) * nx, hipMemcpyHostToDevice, st));
-    if (nu) HIPCHK(hipMemcpyAsync(ctx->d_u.p + ou, sl[s].u, sizeof(double) * nu, hipMemcpyHostToDevice, st));
-    px[s] = ctx->d_x.p + ox;
-    pu[s] = ctx->d_u.p + ou;
-    double m = 0;
-    for (int64_t k = 0; k < nx; ++k) m = std::max(m, fabs(sl[s].x[k]));
-    xmax[s] = m;
-    ox += nx;
-    ou += nu;
-  }
-  // outputs: accumulate into zeroed device staging, then add on the host
-  DevBuf<double> os;
-  DevBuf<unsigned long long> oc;
-  HIPCHK(os.ensure((size_t)n * ncell));
-  HIPCHK(oc.ensure((size_t)n * ncell));
-  HIPCHK(launch_zero(os.p, sizeof(double) * (int64_t)n * ncell, st));
-  HIPCHK(launch_zero(oc.p, sizeof(unsigned long long) * (int64_t)n * ncell, st));
-  rc = run_batch(ctx, n, sl, px.data(), pu.data(), xmax.data(), os.p, oc.p, st);
-  if (rc) { os.release(); oc.release(); return rc; }
-  std::vector<double> hs((size_t)n * ncell);
-  std::vector<unsigned long long> hc((size_t)n * ncell);
-  hipError_t e1 = hipMemcpyAsync(hs.data(), os.p, sizeof(double) * hs.size(), hipMemcpyDeviceToHost, st);
-  hipError_t e2 = hipMemcpyAsync(hc.data(), oc.p, sizeof(unsigned long long) * hc.size(), hipMemcpyDeviceToHost, st);
-  hipError_t e3 = hipStreamSynchronize(st);
-  os.release();
-  oc.release();
-  if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess)
-    return ctx->fail(SF_E_DEVICE, "device to host copy failed: %s",
-                     hipGetErrorString(e3 != hipSuccess ? e3 : (e1 != hipSuccess ? e1 : e2)));
-  for (size_t k = 0; k < hs.size(); ++k) {
+  rc = send_inputs(ctx, n, sl, st, px, pu);
+  if (rc) return rc;
+  for (int s = 0; s < n; ++s) xmax[s] = shares_x(sl, s) ? xmax[s - 1] : abs_max(sl[s].x, (int64_t)sl[s].W * sl[s].N);
+  std::vector<char> acc;
+  rc = run_batch(ctx, n, sl, px.data(), pu.data(), xmax.data(), nullptr, nullptr, st, &acc);
+  if (rc) return rc;
+  const size_t cells = (size_t)n * ncell;
+  if (acc.empty()) acc.assign(16 * cells, 0);  // no pairs: nothing was launched
+  const double *hs = (const double *)acc.data();
+  const uint64_t *hc = (const uint64_t *)(hs + cells);
+  for (size_t k = 0; k < cells; ++k) {
     sums[k] += hs[k];
     counts[k] += hc[k];
   }
@@ -1613,20 +1799,13 @@ extern "C" int sf_hist_batch_device(sf_ctx *ctx, int32_t n, const sf_problem *sl
   HIPCHK(hipSetDevice(ctx->device));
   hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
   std::vector<const double *> px(n), pu(n);
-  std::vector<double> xmax(n, 0.0);
+  std::vector<double> xmax;
   for (int s = 0; s < n; ++s) {
     px[s] = sl[s].x;
     pu[s] = sl[s].u;
-    // coordinate magnitude for the binary32 margin: read x back (O(N)) only for the mixed flat path
-    if (sl[s].precision != SF_PREC_FP64 && sl[s].geometry == SF_GEOM_FLAT && sl[s].N > 0) {
-      std::vector<double> hx((size_t)sl[s].W * sl[s].N);
-      HIPCHK(hipMemcpyAsync(hx.data(), sl[s].x, sizeof(double) * hx.size(), hipMemcpyDeviceToHost, st));
-      HIPCHK(hipStreamSynchronize(st));
-      double m = 0;
-      for (double v : hx) m = std::max(m, fabs(v));
-      xmax[s] = m;
-    }
   }
+  rc = coord_max(ctx, n, sl, st, 1.0, xmax);
+  if (rc) return rc;
   return run_batch(ctx, n, sl, px.data(), pu.data(), xmax.data(), d_sums,
                    (unsigned long long *)d_counts, st);
 }
@@ -1712,22 +1891,6 @@ int fused_setup(sf_ctx *ctx, int32_t n, const sf_problem *sl, int32_t n_out, con
   return SF_OK;
 }
 
-// coordinate magnitudes of flat slices (the binary32 kernels' margins), read from the device
-int slice_xmax(sf_ctx *ctx, int n, const sf_problem *sl, hipStream_t st, double scale, std::vector<double> &xmax) {
-  xmax.assign((size_t)n, 0.0);
-  for (int s = 0; s < n; ++s) {
-    if (sl[s].geometry == SF_GEOM_FLAT && sl[s].N > 0) {
-      std::vector<double> hx((size_t)sl[s].W * sl[s].N);
-      HIPCHK(hipMemcpyAsync(hx.data(), sl[s].x, sizeof(double) * hx.size(), hipMemcpyDeviceToHost, st));
-      HIPCHK(hipStreamSynchronize(st));
-      double m = 0;
-      for (double v : hx) m = std::max(m, fabs(v));
-      xmax[s] = scale * m;
-    }
-  }
-  return SF_OK;
-}
-
 extern "C" int sf_hist_multi_device(sf_ctx *ctx, int32_t n, const sf_problem *sl, int32_t n_out,
                                     const sf_output *outs, double *const *d_sums, uint64_t *const *d_counts,
                                     void *stream) {
@@ -1764,7 +1927,7 @@ extern "C" int sf_hist_multi_device(sf_ctx *ctx, int32_t n, const sf_problem *sl
     px[s] = sl[s].x;
     pu[s] = sl[s].u;
   }
-  rc = slice_xmax(ctx, n, sl, st, 1.0, xmax);
+  rc = coord_max(ctx, n, sl, st, 1.0, xmax);
   if (rc) return rc;
   rc = plan_build(ctx, pl, n, main.data(), px.data(), pu.data(), xmax.data(), st, true, &fs.ms);
   if (rc) return rc;
@@ -1783,7 +1946,7 @@ extern "C" int sf_hist_multi_device(sf_ctx *ctx, int32_t n, const sf_problem *sl
   for (int attempt = 0; attempt < 2; ++attempt) {
     rc = plan_launch(pl, true, js, jc, st, ctx->ev);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(&pc, pl.pcount.p, sizeof(pc), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(&pc, pl.pcount, sizeof(pc), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     ctx->stats[1] = (int64_t)pc;
     if ((int64_t)pc <= pl.cap || (int64_t)pc > kQueueMax) break;
@@ -1836,61 +1999,51 @@ extern "C" int sf_hist_multi(sf_ctx *ctx, int32_t n, const sf_problem *sl, int32
   if (n == 0) return SF_OK;
   HIPCHK(hipSetDevice(ctx->device));
   hipStream_t st = ctx->stream;
-  int64_t tx = 0, tu = 0;
-  for (int s = 0; s < n; ++s) {
-    tx += (int64_t)sl[s].W * sl[s].N;
-    tu += (int64_t)sl[s].D * sl[s].N;
-  }
-  HIPCHK(ctx->d_x.ensure((size_t)tx + 2));
-  HIPCHK(ctx->d_u.ensure((size_t)tu + 2));
+  std::vector<const double *> px(n), pu(n);
+  int rc = send_inputs(ctx, n, sl, st, px, pu);
+  if (rc) return rc;
   std::vector<sf_problem> dev(sl, sl + n);
-  int64_t ox = 0, ou = 0;
   for (int s = 0; s < n; ++s) {
-    const int64_t nx = (int64_t)sl[s].W * sl[s].N, nu = (int64_t)sl[s].D * sl[s].N;
-    if (nx) HIPCHK(hipMemcpyAsync(ctx->d_x.p + ox, sl[s].x, sizeof(double) * nx, hipMemcpyHostToDevice, st));
-    if (nu) HIPCHK(hipMemcpyAsync(ctx->d_u.p + ou, sl[s].u, sizeof(double) * nu, hipMemcpyHostToDevice, st));
-    dev[s].x = ctx->d_x.p + ox;
-    dev[s].u = ctx->d_u.p + ou;
-    ox += nx;
-    ou += nu;
+    dev[s].x = px[s];
+    dev[s].u = pu[s];
   }
-  std::vector<DevBuf<double>> os((size_t)n_out);
-  std::vector<DevBuf<unsigned long long>> oc((size_t)n_out);
+  // outputs: every output's sums, then every output's counts, in one kept buffer
+  std::vector<int64_t> cells((size_t)n_out);
+  size_t total = 0;
+  for (int k = 0; k < n_out; ++k) {
+    cells[k] = (int64_t)n * sl[0].n_dist * (outs[k].n_val > 0 ? outs[k].n_val : 1);
+    total += (size_t)cells[k];
+  }
+  const size_t bytes = 16 * total;
+  HIPCHK(ctx->d_out.ensure(bytes));
   std::vector<double *> ds((size_t)n_out);
   std::vector<uint64_t *> dc((size_t)n_out);
-  std::vector<int64_t> cells((size_t)n_out);
-  int rc = SF_OK;
-  for (int k = 0; k < n_out && !rc; ++k) {
-    cells[k] = (int64_t)n * sl[0].n_dist * (outs[k].n_val > 0 ? outs[k].n_val : 1);
-    if (os[k].ensure((size_t)cells[k]) != hipSuccess || oc[k].ensure((size_t)cells[k]) != hipSuccess)
-      rc = ctx->fail(SF_E_DEVICE, "output buffers");
-    else if (launch_zero(os[k].p, sizeof(double) * cells[k], st) != hipSuccess ||
-             launch_zero(oc[k].p, sizeof(unsigned long long) * cells[k], st) != hipSuccess)
-      rc = ctx->fail(SF_E_DEVICE, "output zeroing");
-    ds[k] = os[k].p;
-    dc[k] = (uint64_t *)oc[k].p;
-  }
-  if (!rc) rc = sf_hist_multi_device(ctx, n, dev.data(), n_out, outs, ds.data(), dc.data(), st);
-  for (int k = 0; k < n_out && !rc; ++k) {
-    std::vector<double> hs((size_t)cells[k]);
-    std::vector<unsigned long long> hc((size_t)cells[k]);
-    hipError_t e1 = hipMemcpyAsync(hs.data(), os[k].p, sizeof(double) * hs.size(), hipMemcpyDeviceToHost, st);
-    hipError_t e2 = hipMemcpyAsync(hc.data(), oc[k].p, sizeof(unsigned long long) * hc.size(), hipMemcpyDeviceToHost, st);
-    hipError_t e3 = hipStreamSynchronize(st);
-    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
-      rc = ctx->fail(SF_E_DEVICE, "device to host copy failed");
-      break;
-    }
-    for (int64_t c = 0; c < cells[k]; ++c) {
-      sums[k][c] += hs[c];
-      counts[k][c] += hc[c];
-    }
-  }
+  size_t off = 0;
   for (int k = 0; k < n_out; ++k) {
-    os[k].release();
-    oc[k].release();
+    ds[k] = (double *)ctx->d_out.p + off;
+    dc[k] = (uint64_t *)ctx->d_out.p + total + off;
+    off += (size_t)cells[k];
   }
-  return rc;
+  HIPCHK(launch_zero(ctx->d_out.p, (int64_t)bytes, st));
+  rc = sf_hist_multi_device(ctx, n, dev.data(), n_out, outs, ds.data(), dc.data(), st);
+  if (rc) return rc;
+  const bool pinned = bytes <= kStageMax;
+  std::vector<char> own(pinned ? 0 : bytes);
+  if (pinned) HIPCHK(ctx->down.acquire(bytes));
+  char *h = pinned ? ctx->down.p : own.data();
+  HIPCHK(hipMemcpyAsync(h, ctx->d_out.p, bytes, hipMemcpyDeviceToHost, st));
+  HIPCHK(hipStreamSynchronize(st));
+  const double *hs = (const double *)h;
+  const uint64_t *hc = (const uint64_t *)h + total;
+  off = 0;
+  for (int k = 0; k < n_out; ++k) {
+    for (int64_t c = 0; c < cells[k]; ++c) {
+      sums[k][c] += hs[off + c];
+      counts[k][c] += hc[off + c];
+    }
+    off += (size_t)cells[k];
+  }
+  return SF_OK;
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -1919,19 +2072,20 @@ extern "C" int sf_hist_batch_device_noalloc(sf_ctx *ctx, int32_t n, const sf_pro
   HIPCHK(hipSetDevice(ctx->device));
   hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
   std::vector<const double *> px(n), pu(n);
-  std::vector<double> xmax(n, 0.0);
+  std::vector<double> xmax;
   for (int s = 0; s < n; ++s) {
     px[s] = sl[s].x;
     pu[s] = sl[s].u;
-    if (sl[s].precision != SF_PREC_FP64 && sl[s].geometry == SF_GEOM_FLAT && sl[s].N > 0) {
-      std::vector<double> hx((size_t)sl[s].W * sl[s].N);
-      HIPCHK(hipMemcpyAsync(hx.data(), sl[s].x, sizeof(double) * hx.size(), hipMemcpyDeviceToHost, st));
-      HIPCHK(hipStreamSynchronize(st));
-      double m = 0;
-      for (double v : hx) m = std::max(m, fabs(v));
-      xmax[s] = m;
-    }
   }
+  // the partial maxima take the head of the scratch before the plan does (they are read back here;
+  // their bytes are fewer than those of the slices' descriptions)
+  static_assert(sizeof(double) * kMaxParts <= sizeof(Slice), "partial maxima of a slice");
+  if (sizeof(Slice) * (size_t)n > SF_NOALLOC_SCRATCH_BYTES)
+    return ctx->fail(SF_E_UNSUPPORTED,
+                     "%d slices need more device scratch than the allocation-free entry's %llu MiB; use "
+                     "sf_hist_batch_device", n, (unsigned long long)(SF_NOALLOC_SCRATCH_BYTES >> 20));
+  rc = coord_max(ctx, n, sl, st, 1.0, xmax, (double *)ctx->scratch_ptr);
+  if (rc) return rc;
   Plan &pl = ctx->noalloc;
   Arena arena{ctx->scratch_ptr, (size_t)SF_NOALLOC_SCRATCH_BYTES, 0};
   pl.arena = &arena;
@@ -1951,7 +2105,7 @@ extern "C" int sf_hist_batch_device_noalloc(sf_ctx *ctx, int32_t n, const sf_pro
   if (rc) return rc;
   if (pl.mixed) {
     unsigned long long pc = 0;
-    HIPCHK(hipMemcpyAsync(&pc, pl.pcount.p, sizeof(pc), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(&pc, pl.pcount, sizeof(pc), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     ctx->stats[1] = (int64_t)pc;
     // the queue overflowed its share of the scratch: the merge was skipped, redo in binary64
@@ -1987,20 +2141,14 @@ extern "C" int sf_plan_create(sf_ctx *ctx, int32_t n, const sf_problem *sl, sf_p
   HIPCHK(hipSetDevice(ctx->device));
   hipStream_t st = ctx->stream;
   std::vector<const double *> px(n), pu(n);
-  std::vector<double> xmax(n, 0.0);
+  std::vector<double> xmax;
   for (int s = 0; s < n; ++s) {
     px[s] = sl[s].x;
     pu[s] = sl[s].u;
-    if (sl[s].precision != SF_PREC_FP64 && sl[s].geometry == SF_GEOM_FLAT && sl[s].N > 0) {
-      // coordinate magnitude for the binary32 margin; later contents must stay within 2x of it
-      std::vector<double> hx((size_t)sl[s].W * sl[s].N);
-      HIPCHK(hipMemcpyAsync(hx.data(), sl[s].x, sizeof(double) * hx.size(), hipMemcpyDeviceToHost, st));
-      HIPCHK(hipStreamSynchronize(st));
-      double m = 0;
-      for (double v : hx) m = std::max(m, fabs(v));
-      xmax[s] = 2.0 * m;
-    }
   }
+  // coordinate magnitude for the binary32 margin; later contents must stay within 2x of it
+  rc = coord_max(ctx, n, sl, st, 2.0, xmax);
+  if (rc) return rc;
   sf_plan *plan = new sf_plan();
   plan->ctx = ctx;
   // no culling in plans: the positions behind x may change between executions
@@ -2084,7 +2232,7 @@ extern "C" int sf_plan_create_multi(sf_ctx *ctx, int32_t n, const sf_problem *sl
     pu[s] = sl[s].u;
   }
   // later contents must stay within 2x of the coordinate magnitude read now
-  rc = slice_xmax(ctx, n, sl, st, 2.0, xmax);
+  rc = coord_max(ctx, n, sl, st, 2.0, xmax);
   // no culling in plans: the positions behind x may change between executions
   if (!rc) rc = plan_build(ctx, plan->pl, n, plan->fs.main().data(), px.data(), pu.data(), xmax.data(), st, false,
                            &plan->fs.ms);
@@ -2159,7 +2307,7 @@ extern "C" int sf_plan_sync(sf_plan *plan, int32_t *redone) {
   HIPCHK(hipStreamSynchronize(plan->last_stream));
   if (!pl.mixed || pl.total_pairs == 0) return SF_OK;
   int flag = 0;
-  HIPCHK(hipMemcpy(&flag, pl.flag.p, sizeof(int), hipMemcpyDeviceToHost));
+  HIPCHK(hipMemcpy(&flag, pl.flag, sizeof(int), hipMemcpyDeviceToHost));
   if (flag && plan->n_out) {
     // a fused plan's last execute overflowed the re-bin queue and left every output untouched:
     // each output with the binary64 kernel

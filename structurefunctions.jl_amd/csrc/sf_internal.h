@@ -241,6 +241,8 @@ inline __host__ __device__ bool sp2d(int op, int n_val) { return op == 6 && n_va
 
 inline constexpr int kDummySlots = 64;
 inline constexpr int kZeroSetMax = 8;  // buffers cleared by one zero_multi launch
+inline constexpr int kMaxParts = 16;   // partial maxima of one slice's coordinates (absmax)
+inline constexpr int kMaxSet = 32;     // slices of one absmax launch
 // largest binary32 key table (cells); the host's partition never exceeds it.  In LDS the table's
 // (lo, hi) pairs start the region and its bin counts follow at the same 8-byte stride; for joint
 // histograms they sit kCell32Max * 8 bytes on, so that one address serves both reads (the second

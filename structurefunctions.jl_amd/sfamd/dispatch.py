@@ -154,16 +154,29 @@ def _problem(sf, x2, u2, dedges, vedges, metric, precision, keep, semantics=_nat
 
 
 def _slices(x, u, kind):
-    """Split auxiliary axes into (W,N)/(D,N) slices; returns (list of (x2,u2), aux shape)."""
+    """Split auxiliary axes into (W,N)/(D,N) slices, column-major; returns (list of (x2,u2), aux shape).
+    Shared positions are one array for every slice."""
     if kind == "point":
         return [(x, u)], ()
     aux = u.shape[2:]
     B = int(np.prod(aux))
-    uu = u.reshape(u.shape[0], u.shape[1], B, order="F")
+    us = _slice_major(u.reshape(u.shape[0], u.shape[1], B, order="F"))
     if kind == "shared":
-        return [(x, uu[:, :, b]) for b in range(B)], aux
-    xx = x.reshape(x.shape[0], x.shape[1], B, order="F")
-    return [(xx[:, :, b], uu[:, :, b]) for b in range(B)], aux
+        xc = np.asfortranarray(x)
+        return [(xc, us[b].T) for b in range(B)], aux
+    xs = _slice_major(x.reshape(x.shape[0], x.shape[1], B, order="F"))
+    return [(xs[b].T, us[b].T) for b in range(B)], aux
+
+
+def _slice_major(a):
+    """(D, N, B) as a C-contiguous (B, N, D), one component at a time: a gather per slice reads the
+    array B times (eight fields of 5003 points: 390 us, this 105 us)."""
+    t = np.ascontiguousarray(a.T) if a.flags.f_contiguous else None
+    if t is None:
+        t = np.empty(a.shape[::-1], dtype=a.dtype)
+        for d in range(a.shape[0]):
+            t[:, :, d] = a[d].T
+    return t
 
 
 def _semantics(kind):
