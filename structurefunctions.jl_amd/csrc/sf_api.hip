@@ -1308,12 +1308,21 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   // ---- work items: (slice, i-tile, j-chunk); slices in descending N
   int jchunk = t_jchunk;
   if (jchunk <= 0) {
-    const double target_items = 16.0 * max_blocks;
-    double per_item = (double)pl.total_pairs / target_items;  // pairs per item
-    int jc = (int)(per_item / block);
-    jc = std::max(jc, block);
-    jc = std::min(jc, 64 * block);
-    jchunk = (jc + block - 1) / block * block;
+    // Large calls: 16 items per resident workgroup, in whole tiles.  Smaller ones: an item's fixed
+    // cost against the workgroups that it leaves idle at the end, which is least at a width that goes
+    // with the root of the call's (row tile, column) count.  Measured, against one tile at least: host
+    // du_L^2 at N = 777 107 / 153 us (binary64; 10 items then; sphere 122 / 195), N = 4096 157 / 200;
+    // joint du_L at N = 16384 binary64 385 / 550.
+    // The planes of a 2D single pass: their pairs that share a cell serialize, so an item's time varies
+    // most, and narrow items pay at every size (sphere, N = 12000: 2.03 ms at 128 columns, 2.4 at 256,
+    // 6.9 at 1024; N = 3000: 0.50 ms, 0.56 at 32 columns).
+    const double cols = (double)pl.total_pairs / block;  // columns of all row tiles
+    const double large = std::min(std::max(cols / (16.0 * max_blocks), (double)block), 64.0 * block);
+    const double small = sp2d(p0.op, p0.n_val) ? std::max(128.0, cols / (64.0 * max_blocks))
+                                               : std::max(16.0, sqrt(cols) / 3.0);
+    const int jc = (int)std::min(large, small);
+    const int unit = jc >= block ? block : 16;
+    jchunk = (jc + unit - 1) / unit * unit;
   }
   // fixed-point cells: one item must stay below the flush limit (the LDS histogram is flushed
   // between items only)
