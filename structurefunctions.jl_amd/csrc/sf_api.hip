@@ -27,7 +27,7 @@ namespace sfk {
 // kernel launchers (sf_kernels.hip)
 hipError_t launch_prep(int G, int D, bool mixed, int geom_code, const void *prep_slices,
                        int n_slices, int64_t max_n, double *rec64, float *rec32, hipStream_t st);
-hipError_t launch_hist(int G, int D, bool J, bool mixed, bool sload, const Params &P, int grid,
+hipError_t launch_hist(int G, int D, bool J, bool mixed, bool sload, bool near, const Params &P, int grid,
                        int block, size_t smem, hipStream_t st);
 hipError_t launch_recheck(int G, int D, bool J, const Params &P, int grid, hipStream_t st);
 hipError_t launch_merge(const double *src_s, const unsigned long long *src_c, double *dst_s,
@@ -42,9 +42,11 @@ hipError_t launch_zero_multi(int count, void *const *p, const int64_t *bytes, hi
 hipError_t launch_derive_sp(double *s, unsigned long long *c, int64_t nbins, hipStream_t st);
 hipError_t launch_eval_math(int fn, int64_t n, const double *a, const double *b, double *out,
                             hipStream_t st);
-hipError_t cull_workspace_bytes(int64_t N, size_t *bytes);
-hipError_t launch_cull(const double *x, int64_t N, int W, int D, int geom, int rows, void *ws,
+size_t cull_workspace_bytes(int64_t N);
+hipError_t launch_cull(const double *x, int64_t N, int W, int D, int geom, double reach, int bits, void *ws,
                        int32_t *perm, double *info, float *gbox, hipStream_t st);
+hipError_t launch_cull_units(const float *gbox, int64_t N, double *info, double reach, int slice, Item *units,
+                             int64_t n, hipStream_t st);
 int hist_occupancy(int G, int D, bool J, bool mixed, int opk, bool sload, bool fx, int block,
                    size_t smem);
 int hist_opk(const Params &P);
@@ -284,10 +286,11 @@ struct Plan {
   int *flag = nullptr;
   size_t acc_bytes = 0;
   DevBuf<Pending> pending;
-  DevBuf<float> gboxes;   // boxes of the column groups of culled slices
+  DevBuf<float> gboxes;   // boxes of the record groups of culled slices
+  DevBuf<Item> units;     // culled slices' work units, slice after slice
+  int n_units = 0, near_grid = 1, jchunk = 1;
   DevBuf<int32_t> perm;   // spatial order of the binary32 records (tile culling)
-  bool culled = false;    // some work items were dropped by tile culling
-  bool near = false;      // some slice's column groups are culled per wave
+  bool culled = false;    // some slice is evaluated by its work units, not by items
   Arena *arena = nullptr;  // set: every buffer is taken from this region (no device allocation)
   // fused outputs: 1D operators evaluated with the main (joint) one, their accumulators and the
   // caller's outputs they merge into
@@ -306,6 +309,7 @@ struct Plan {
     rec64.release(); rec32.release(); tables.release(); acc.release(); pending.release();
     perm.release();
     gboxes.release();
+    units.release();
     msums.release();
     mcounts.release();
   }
@@ -947,31 +951,27 @@ extern "C" int sf_set_tuning(sf_ctx *ctx, int32_t block, int32_t j_chunk, int32_
 
 namespace {
 
-// ---- spatial sort and tile culling ----------------------------------------------------------
+// ---- spatial sort and culling ----------------------------------------------------------------
 // When every distance edge of a slice is finite, a pair farther apart than the last edge is not
 // counted.  Points are put in Morton (Z-curve) order of their key-space coordinates (flat: x;
-// sphere: the unit vector), so that a tile of consecutive points is spatially compact, and a
-// work item (row tile, column chunk) whose bounding boxes are farther apart than the last edge is
-// dropped.  Only the binary32 records are reordered (each keeps its caller index); the binary64
-// records, and with them every re-binned pair, stay in the caller's order.
-struct Box {
-  double lo[3], hi[3];
-};
-
+// sphere: the unit vector), so that consecutive points are spatially compact, and only those blocks
+// of 64 rows and one or two groups of kGroup columns are evaluated whose bounding boxes are not
+// farther apart than the last edge: the slice's work units, which the device lists (launch_cull).
+// Only the binary32 records are reordered (each keeps its caller index); the binary64 records, and
+// with them every re-binned pair, stay in the caller's order.
 struct CullInfo {
-  bool active = false;
-  double limit = 0;               // a pair of boxes farther apart than this holds no counted pair
-  std::vector<Box> tiles;         // bounding box of each `rows`-record tile, in record order
+  bool tried = false, active = false;
+  double reach = 0;       // largest counted distance in key-space units
+  int64_t units = 0;
 };
 
-// Spatial order and tile boxes of one slice, computed on the device (launch_cull): the record
-// order goes to perm (device, N entries); ci.active says whether culling is worth it.
-int cull_prepare(sf_ctx *ctx, const sf_problem &p, const double *dx, double xmax, int rows,
-                 hipStream_t st, CullInfo &ci, int32_t *perm, float *gbox) {
-  ci.active = false;
+// Starts the spatial order, group boxes and number of work units of one slice on the device
+// (launch_cull), where culling may be worth it: the record order goes to perm (device, N entries).
+int cull_start(sf_ctx *ctx, const sf_problem &p, const double *dx, double xmax, int rows, hipStream_t st, CullInfo &ci,
+               int32_t *perm, double *info_d, float *gbox) {
   const int64_t N = p.N;
   const double emax = p.dist_edges[p.n_dist];
-  if (N < 4 * (int64_t)rows || !(emax < INFINITY)) return SF_OK;
+  if (N < 4 * (int64_t)rows || N > (1LL << 30) || !(emax < INFINITY)) return SF_OK;
   const bool flat = p.geometry == SF_GEOM_FLAT;
   // largest distance in key-space units: flat |dx|; sphere chord 2 sin(theta / 2)
   double reach;
@@ -986,41 +986,34 @@ int cull_prepare(sf_ctx *ctx, const sf_problem &p, const double *dx, double xmax
   // at most 2 max|x| (when the caller measured it)
   if (!flat && reach >= 1.0) return SF_OK;
   if (flat && xmax > 0 && reach >= xmax) return SF_OK;
-  const int64_t ntile = (N + rows - 1) / rows;
-  size_t wsb = 0;
-  HIPCHK(cull_workspace_bytes(N, &wsb));
-  HIPCHK(ctx->cull_ws.ensure(wsb));
-  HIPCHK(ctx->cull_info.ensure((size_t)(8 + 6 * ntile)));
+  // 8 bits of the Morton key per axis where its cells (the extent's 1/256 at most) are a quarter of the
+  // reach or less: finer ones leave the boxes what they are (N = 262144 points of the sphere, reach
+  // 0.05 rad: 206e6 pairs evaluated, 204e6 with 10), and the sort takes two passes, not three
+  const double ext = flat ? 2.0 * xmax : 2.0;
+  const int bits = ext > 0 && ext <= 64.0 * reach ? 8 : 10;
   const int geom = flat ? 0 : (p.geometry == SF_GEOM_SPHERE_DEG ? 1 : 2);
-  HIPCHK(launch_cull(dx, N, p.W, p.D, geom, rows, ctx->cull_ws.p, perm, ctx->cull_info.p, gbox, st));
-  std::vector<double> info((size_t)(8 + 6 * ntile));
-  HIPCHK(hipMemcpyAsync(info.data(), ctx->cull_info.p, sizeof(double) * info.size(), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  if (info[6] != 0.0) return SF_OK;  // non-finite coordinates: no culling
-  // margin: relative 1e-6 plus the rounding of coordinates of magnitude cmax
-  ci.limit = reach * (1.0 + 1e-6) + 1e-13 * std::max(1.0, info[7]);
-  // worth it only if the reach is small against the extent
-  double ext = 0;
-  for (int k = 0; k < 3; ++k) ext = std::max(ext, info[3 + k] - info[k]);
-  if (!(ci.limit < 0.5 * ext)) return SF_OK;
-  ci.tiles.resize((size_t)ntile);
-  for (int64_t t = 0; t < ntile; ++t)
-    for (int k = 0; k < 3; ++k) {
-      ci.tiles[t].lo[k] = info[8 + 6 * t + k];
-      ci.tiles[t].hi[k] = info[8 + 6 * t + 3 + k];
-    }
-  ci.active = true;
+  HIPCHK(ctx->cull_ws.ensure(cull_workspace_bytes(N)));
+  HIPCHK(launch_cull(dx, N, p.W, p.D, geom, reach, bits, ctx->cull_ws.p, perm, info_d, gbox, st));
+  ci.tried = true;
+  ci.reach = reach;
   return SF_OK;
 }
 
-// true if no point of box a is within `limit` of a point of box b
-bool boxes_apart(const Box &a, const Box &b, double limit) {
-  double g2 = 0;
-  for (int k = 0; k < 3; ++k) {
-    const double g = std::max(0.0, std::max(b.lo[k] - a.hi[k], a.lo[k] - b.hi[k]));
-    g2 += g * g;
-  }
-  return g2 > limit * limit;
+// ci.active: whether culling is worth it, from launch_cull's info
+void cull_decide(const sf_problem &p, const double *info, int rows, CullInfo &ci) {
+  if (!ci.tried || p.N < 4 * (int64_t)rows) return;
+  if (info[6] != 0.0) return;  // non-finite coordinates: no culling
+  // worth it only if the reach is small against the extent
+  double ext = 0;
+  for (int k = 0; k < 3; ++k) ext = std::max(ext, info[3 + k] - info[k]);
+  if (!(info[9] < 0.5 * ext)) return;
+  // ... and units leave out half of the pairs at least: a full unit is 64 x 64 pairs, and whole row
+  // tiles over long column ranges take less per pair
+  uint64_t units;
+  memcpy(&units, &info[8], sizeof units);
+  if ((double)units * 4096.0 > 0.5 * (double)pairs_of(p.N) || units > (uint64_t)(1 << 30)) return;
+  ci.active = true;
+  ci.units = (int64_t)units;
 }
 
 // Stride of the binary32 record order: record k holds point (k * mul) mod N.  Points that the
@@ -1151,6 +1144,29 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   static_assert(kF64Rec * 2 == rec_f32(kSphere, 2) && kF64Rec * 2 == rec_f32(kSphere, 3), "record sizes");
   if (mixed || G == kSphere) PLBUF(pl.rec32, ((size_t)pl.total_pts * F32 + 16));
 
+  // ---- spatial sort and culling (binary32 kernel, one-shot calls): started here, so that the device
+  // works on it while the tables are built
+  std::vector<CullInfo> cinfo(n);
+  std::vector<int64_t> grp(n);  // first group box of each slice
+  bool cull_tried = false;
+  if (cull && mixed && !strip) {
+    int64_t groups = 0;
+    for (int s = 0; s < n; ++s) {
+      grp[s] = groups;
+      groups += (sl[s].N + kGroup - 1) / kGroup;
+    }
+    // the record order of slice s lands at pl.perm + pt_off (used only where culling is active)
+    PLBUF(pl.perm, ((size_t)pl.total_pts));
+    PLBUF(pl.gboxes, ((size_t)groups * 6));
+    HIPCHK(ctx->cull_info.ensure((size_t)n * kCullInfo));
+    for (int s = 0; s < n; ++s) {
+      const int rc = cull_start(ctx, sl[s], dx[s], xmax[s], J ? 768 : 256, st, cinfo[s], pl.perm.p + prep[s].pt_off,
+                                ctx->cull_info.p + (size_t)s * kCullInfo, pl.gboxes.p + (size_t)grp[s] * 6);
+      if (rc) return rc;
+      cull_tried = cull_tried || cinfo[s].tried;
+    }
+  }
+
   // ---- tables
   std::vector<Slice> sdesc(n);
   std::vector<Cell> cells;
@@ -1170,8 +1186,6 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     d.out_off = planes ? (int64_t)(s / kSpRows) * ncell + s % kSpRows : (int64_t)s * ncell;
     d.plane = planes ? s % kSpRows : 0;
     d.xerr = flat ? round_up_f(ldexpl((long double)xmax[s], -28)) : 0.0f;
-    d.grp_off = 0;
-    d.clim2 = 0.0f;
     d.strip_n = (strip && s % strip == 0) ? std::min(strip, n - s) : 0;
     d.tab_off = (int32_t)cells.size();
     cells.insert(cells.end(), T.tab64.begin(), T.tab64.end());
@@ -1327,50 +1341,51 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   // fixed-point cells: one item must stay below the flush limit (the LDS histogram is flushed
   // between items only)
   if (pl.fx) jchunk = std::max(1, std::min<int>(jchunk, (int)(kFxFlushLimit / block)));
-  // spatial sort and tile culling (binary32 kernel, one-shot calls): column chunks of one tile
-  std::vector<CullInfo> cinfo(n);
-  pl.culled = pl.near = false;
-  if (cull && mixed && !strip) {
-    // the record order of slice s lands at pl.perm + pt_off (used only where culling is active)
-    PLBUF(pl.perm, ((size_t)pl.total_pts));
-    int64_t groups = 0;
+  // culling, second part (scalar-loaded columns only): which slices, and their work units
+  pl.culled = false;
+  pl.n_units = 0;
+  if (cull_tried && sload) {
+    const size_t bytes = sizeof(double) * kCullInfo * (size_t)n;
+    const bool pinned = bytes <= kStageMax;
+    std::vector<double> own(pinned ? 0 : (size_t)n * kCullInfo);
+    if (pinned) HIPCHK(ctx->down.acquire(bytes));
+    double *info = pinned ? (double *)ctx->down.p : own.data();
+    HIPCHK(hipMemcpyAsync(info, ctx->cull_info.p, bytes, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    int64_t units = 0;
     for (int s = 0; s < n; ++s) {
-      sdesc[s].grp_off = (int32_t)groups;
-      groups += (sl[s].N + kGroup - 1) / kGroup;
-    }
-    PLBUF(pl.gboxes, ((size_t)groups * 6));
-    for (int s = 0; s < n; ++s) {
-      const int rc = cull_prepare(ctx, sl[s], dx[s], xmax[s], block, st, cinfo[s], pl.perm.p + prep[s].pt_off,
-                                  pl.gboxes.p + (size_t)sdesc[s].grp_off * 6);
-      if (rc) return rc;
+      cull_decide(sl[s], info + (size_t)s * kCullInfo, block, cinfo[s]);
+      if (units + cinfo[s].units > (1LL << 30)) cinfo[s].active = false;
       if (!cinfo[s].active) continue;
-      pl.near = true;
+      units += cinfo[s].units;
       prep[s].perm = pl.perm.p + prep[s].pt_off;
-      // squared limit for the binary32 gaps of the group boxes (three squares and their sum)
-      sdesc[s].clim2 = round_up_f((long double)cinfo[s].limit * cinfo[s].limit * (1.0L + 1e-5L) + 1e-30L);
+      pl.culled = true;
     }
+    pl.n_units = (int)units;
+    if (units > 0) {
+      PLBUF(pl.units, (size_t)units);
+      units = 0;
+      for (int s = 0; s < n; ++s) {
+        if (!cinfo[s].active || cinfo[s].units == 0) continue;
+        HIPCHK(launch_cull_units(pl.gboxes.p + (size_t)grp[s] * 6, sl[s].N, ctx->cull_info.p + (size_t)s * kCullInfo,
+                                 cinfo[s].reach, s, pl.units.p + units, cinfo[s].units, st));
+        units += cinfo[s].units;
+      }
+    }
+    const int waves = block / 64;
+    pl.near_grid = std::max(1, std::min(max_blocks, (pl.n_units + waves - 1) / waves));
   }
   std::vector<int> order(n);
   for (int s = 0; s < n; ++s) order[s] = s;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return sl[a].N > sl[b].N; });
   std::vector<Item> items, items64;
-  // fixed-point cells: a workgroup flushes its LDS histogram only between items, so one item may
-  // add at most kFxFlushLimit updates (block rows x its columns).  A culled item spans one column
-  // tile of `block` columns; at block 1024 that is 2^20 updates, so such tiles are split in halves
-  // (the tile of a column is still j0 / block).
-  int64_t jc_cull = block;
-  while (pl.fx && jc_cull > 1 && (int64_t)block * jc_cull > kFxFlushLimit) jc_cull >>= 1;
   for (int s : order) {
+    if (cinfo[s].active) continue;  // its work units are listed on the device
     const int64_t N = sl[s].N;
-    const CullInfo &ci = cinfo[s];
-    const int64_t jc = ci.active ? jc_cull : jchunk;
+    const int64_t jc = jchunk;
     const size_t first = items.size();
     for (int64_t i0 = 0; i0 < N - 1; i0 += block) {
       for (int64_t j0 = i0; j0 < N; j0 += jc) {
-        if (ci.active && j0 > i0 && boxes_apart(ci.tiles[i0 / block], ci.tiles[j0 / block], ci.limit)) {
-          pl.culled = true;
-          continue;
-        }
         Item it;
         it.slice = s;
         it.i0 = (int32_t)i0;
@@ -1396,12 +1411,13 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
         return ctx->fail(SF_E_DEVICE, "internal: work item of %d x %d pair updates exceeds the fixed-point flush limit",
                          block, it.j1 - it.j0);
   }
+  pl.n_items = (int)items.size();  // (none: every slice is culled)
   if (items.empty()) items.push_back(Item{0, 0, 0, 0});
   if (strip && items64.empty()) items64.push_back(Item{0, 0, 0, 0});
   pl.n_items64 = (int)items64.size();
-  pl.n_items = (int)items.size();
   pl.grid = std::max(1, std::min(pl.n_items, max_blocks));
   pl.block = block;
+  pl.jchunk = jchunk;
   pl.tj = tj;
   pl.copies = copies;
   pl.sload = sload;
@@ -1483,7 +1499,6 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   P.counter = pl.counter;
   P.rec64 = pl.rec64.p;
   P.rec32 = pl.rec32.p;
-  P.gboxes = pl.near ? pl.gboxes.p : nullptr;
   P.cells = (const Cell *)(tb + parts[2].off);
   P.dedges = (const double *)(tb + parts[3].off);
   P.vedges = (const double *)(tb + parts[4].off);
@@ -1584,7 +1599,14 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
   const SmemLayout L = smem_layout(P.n_dist, P.n_val, P.ncell_max, stage_mixed, P.copies, P.nmom, P.fx, P.qcap,
                                    P.strip, P.jlayout, P.n1d, P.mcopies);
   if (ev) HIPCHK(hipEventRecord(ev[0], st));
-  HIPCHK(launch_hist(pl.G, pl.D, pl.J, use_mixed, use_sload, P, pl.grid, pl.block, (size_t)L.total, st));
+  if (P.n_items > 0)
+    HIPCHK(launch_hist(pl.G, pl.D, pl.J, use_mixed, use_sload, false, P, pl.grid, pl.block, (size_t)L.total, st));
+  if (use_mixed && pl.n_units > 0) {  // culled slices: their work units instead of items
+    Params Pu = P;
+    Pu.items = pl.units.p;
+    Pu.n_items = pl.n_units;
+    HIPCHK(launch_hist(pl.G, pl.D, pl.J, true, true, true, Pu, pl.near_grid, pl.block, (size_t)L.total, st));
+  }
   if (ev) HIPCHK(hipEventRecord(ev[1], st));
   // four 256-thread workgroups per CU: the re-bin is a latency-bound gather (2D single pass,
   // 2.7e8 queued pairs: 22.6 / 16.7 / 19.6 ms with one / four / eight per CU)
@@ -1603,6 +1625,12 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
   return SF_OK;
 }
 
+// work items of a plan's launch; culled slices: the number of items that their units' pairs would fill
+int64_t work_items(const Plan &pl) {
+  const int64_t item = (int64_t)pl.block * pl.jchunk;
+  return pl.n_items + ((int64_t)pl.n_units * 4096 + item - 1) / item;
+}
+
 // One-shot: build (into the context's cached plan, reusing its buffers), launch, and on a
 // re-bin queue overflow redo the call with the binary64 kernel.  h_acc (host calls; out_s and out_c
 // are null then): receives the accumulators (sums, then counts) instead of a merge, read with the
@@ -1615,8 +1643,8 @@ int run_batch(sf_ctx *ctx, int n, const sf_problem *sl, const double *const *dx,
   if (rc) return rc;
   for (int k = 0; k < 8; ++k) ctx->stats[k] = 0;
   ctx->stats[0] = pl.total_pairs;
-  ctx->stats[2] = pl.n_items;
-  ctx->stats[3] = pl.grid;
+  ctx->stats[2] = work_items(pl);
+  ctx->stats[3] = std::max(pl.n_items > 0 ? pl.grid : 0, pl.n_units > 0 ? pl.near_grid : 0);
   ctx->stats[7] = pl.block;
   ctx->ev_pending = false;
   if (pl.total_pairs == 0) return SF_OK;
@@ -1942,8 +1970,8 @@ extern "C" int sf_hist_multi_device(sf_ctx *ctx, int32_t n, const sf_problem *sl
   if (rc) return rc;
   for (int k = 0; k < 8; ++k) ctx->stats[k] = 0;
   ctx->stats[0] = pl.total_pairs;
-  ctx->stats[2] = pl.n_items;
-  ctx->stats[3] = pl.grid;
+  ctx->stats[2] = work_items(pl);
+  ctx->stats[3] = std::max(pl.n_items > 0 ? pl.grid : 0, pl.n_units > 0 ? pl.near_grid : 0);
   ctx->stats[7] = pl.block;
   ctx->ev_pending = false;
   if (pl.total_pairs == 0) return SF_OK;
@@ -2104,8 +2132,8 @@ extern "C" int sf_hist_batch_device_noalloc(sf_ctx *ctx, int32_t n, const sf_pro
   if (rc) return rc;
   for (int k = 0; k < 8; ++k) ctx->stats[k] = 0;
   ctx->stats[0] = pl.total_pairs;
-  ctx->stats[2] = pl.n_items;
-  ctx->stats[3] = pl.grid;
+  ctx->stats[2] = work_items(pl);
+  ctx->stats[3] = std::max(pl.n_items > 0 ? pl.grid : 0, pl.n_units > 0 ? pl.near_grid : 0);
   ctx->stats[7] = pl.block;
   ctx->ev_pending = false;
   if (pl.total_pairs == 0) return SF_OK;

@@ -92,8 +92,6 @@ struct Slice {
   int32_t gz;
   int32_t plane;      // single pass, 2D form: invariant (0..5) whose joint histogram this slice holds
   float xerr;         // flat: 2^-28 max|x| (binary32 value bound: reference's direction error)
-  int32_t grp_off;    // tile culling: first box of the slice in gboxes
-  float clim2;        // ... and the squared distance beyond which two boxes hold no counted pair; 0: off
   int32_t strip_n;    // B-strip launch: fields of the strip this slice leads (0: not a leader)
   // value edges log-spaced from edge vk0 on (binary32 lookup guesses the bin from log2 v):
   // log2(edge vk0 + m) ~ vl0f + m / vlinvf
@@ -106,6 +104,7 @@ struct Item {
   int32_t i0;       // first row of the i-tile
   int32_t j0, j1;   // column range [j0, j1), j0 >= i0
 };
+// (a culled slice's work unit is an Item of one wave: 64 rows from i0 on, at most 64 columns)
 
 struct Pending {      // a pair the binary32 kernel could not bin with certainty (binary32 record indices)
   int32_t slice, i, j;
@@ -120,7 +119,6 @@ struct Params {
   int32_t *counter;        // work-queue head (zeroed before launch)
   const double *rec64;     // binary64 records
   const float *rec32;      // binary32 records
-  const float *gboxes;     // culled slices: a box (lo[3], hi[3]) per kGroup records, rounded outwards
   const Cell *cells;       // cell tables (binary64 tables and binary32 tables)
   const double *dedges;    // exact distance-key edges
   const double *vedges;    // value edges (binary64)
@@ -249,8 +247,10 @@ inline constexpr int kMaxSet = 32;     // slices of one absmax launch
 // takes a constant offset), for 1D ones right after the largest table of the launch (their LDS
 // decides how many workgroups fit: 16 KB of table region cost them 12 %)
 inline constexpr int kCell32Max = 1024;
-// records per box of a culled slice (a column group of the binary32 pair loop)
+// records per box of a culled slice (its work units hold one or two such groups of columns)
 inline constexpr int kGroup = 32;
+// words (8 bytes) of a slice's culling information: see launch_cull
+inline constexpr int kCullInfo = 11;
 // largest re-bin queue staged in LDS per workgroup (entries, split evenly between its waves);
 // the host shrinks it where the LDS it takes would cost a workgroup per CU
 inline constexpr int kQueueCap = 8192;

@@ -954,11 +954,10 @@ struct Row {
   bool any;       // some lane of the wave has a row (wave-uniform)
   int jm;         // columns below jm need the j > i mask
 };
-// near: a wave's rows side by side (a slice whose column groups are culled per wave)
 template <bool J>
-DEV Row item_row(const Item &w, const Slice &s, bool near = false) {
+DEV Row item_row(const Item &w, const Slice &s) {
   const int B = blockDim.x;
-  const int i = w.i0 + (near ? (int)threadIdx.x : tile_row<J>());
+  const int i = w.i0 + tile_row<J>();
   Row r;
   r.i = i < s.N ? i : kNoRow;
   r.rec = i < s.N ? i : s.N - 1;
@@ -2122,28 +2121,20 @@ DEV void run_chunk32(const Params &P, const Slice &s, const Smem &m, const float
     run_chunk32_vu<G, D, J, OPK, MASK, FX, false, SL>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
 }
 
-// Column groups (kGroup records) of an item that can hold a counted pair of the wave's rows: bit t
-// of the mask stands for the group at jb + t kGroup.  Lane t compares the box of group t with the
-// box of the wave's 64 rows (side by side in the slice's spatial order); 64 groups per call.  The
-// boxes are rounded outwards to binary32 and the limit carries a margin, so no counted pair is
-// lost.  Workgroup tiles alone left 75 evaluated pairs for one counted at N = 262144 points of the
-// sphere and a reach of 0.05 rad; with them the call went from 3.24 to 1.45 ms.
-DEV lanes_t near_groups(const Params &P, const Slice &s, const Item &w, int jb) {
-  const int r0 = w.i0 + (int)(threadIdx.x & ~63u);
-  const int last = (int)((s.N - 1) / kGroup);
-  const float *bx = P.gboxes + (int64_t)s.grp_off * 6;
-  const float *a0 = bx + 6 * min(r0 / kGroup, last);
-  const float *a1 = bx + 6 * min(r0 / kGroup + 1, last);
-  const int g = jb / kGroup + (int)__lane_id();
-  const float *b = bx + 6 * min(g, last);
-  float d2 = 0.f;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const float lo = __builtin_fminf(a0[k], a1[k]), hi = __builtin_fmaxf(a0[3 + k], a1[3 + k]);
-    const float gap = __builtin_fmaxf(0.f, __builtin_fmaxf(b[k] - hi, lo - b[3 + k]));
-    d2 = __builtin_fmaf(gap, gap, d2);
-  }
-  return __builtin_amdgcn_ballot_w64(g * kGroup < w.j1 && d2 <= s.clim2);
+// Columns [ja, je) for a wave's row with scalar-loaded column records; the ones below row.jm may lie
+// below some row
+template <int G, int D, bool J, int OPK, bool FX>
+DEV void run_cols32(const Params &P, const Slice &s, const Smem &m, const float *ri, const Row &row, int ja, int je,
+                    const float *rec, int slice_id) {
+  // the slice offset is wave-uniform by construction; say so, so that column addresses
+  // stay in SGPRs (the pointer itself keeps its global address space: scalar loads)
+  const uint64_t po = (uint64_t)s.pt_off;
+  const int64_t off = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(po >> 32)) << 32) |
+                                (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)po));
+  const float4 *col = (const float4 *)(rec + off * Rec<G, D>::f32);
+  const int jm = min(row.jm, je);
+  if (ja < jm) run_chunk32<G, D, J, OPK, true, FX, true>(P, s, m, ri, row.i, ja, jm, col, 0, slice_id);
+  if (jm < je) run_chunk32<G, D, J, OPK, false, FX, true>(P, s, m, ri, row.i, max(jm, ja), je, col, 0, slice_id);
 }
 
 // SLOAD: column records are read straight from global memory with wave-uniform addresses, which
@@ -2153,10 +2144,7 @@ DEV lanes_t near_groups(const Params &P, const Slice &s, const Item &w, int jb) 
 // per CU, which their small LDS footprint allows; the few values this spills are per-item ones
 // (the fused ones spill a few SGPR-held values of the pair loop too, and still gain: the 256
 // ragged 2D slices' du_L^2 and joint du_L from one launch, 73.7 -> 57.6 ms).
-// NEAR: the launch has slices whose column groups are culled per wave (near_groups).  A kernel of
-// its own, because the runs' loop costs launches without culling 4 % of a 1D single pass
-// (N = 32768, sphere: 8.05 against 8.37 ms).
-template <int G, int D, bool J, int OPK, bool SLOAD, bool FX, bool NEAR = false>
+template <int G, int D, bool J, int OPK, bool SLOAD, bool FX>
 __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, const float *__restrict__ rec) {
   extern __shared__ __align__(16) char smem_raw[];
   constexpr int F = Rec<G, D>::f32;
@@ -2192,41 +2180,12 @@ __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, 
       since_flush = 0;
     }
     since_flush += work;
-    const bool culled = NEAR && __builtin_amdgcn_readfirstlane(__float_as_int(s.clim2)) != 0;
-    const Row row = item_row<J>(w, s, culled);
+    const Row row = item_row<J>(w, s);
     float ri[F];
 #pragma unroll
     for (int k = 0; k < F; ++k) ri[k] = rec[(s.pt_off + row.rec) * F + k];
     if constexpr (SLOAD) {
-      if (row.any) {
-        // the slice offset is wave-uniform by construction; say so, so that column addresses
-        // stay in SGPRs (the pointer itself keeps its global address space: scalar loads)
-        const uint64_t po = (uint64_t)s.pt_off;
-        const int64_t off = (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(po >> 32)) << 32) |
-                                      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)po));
-        const float4 *col = (const float4 *)(rec + off * F);
-        auto run = [&](int ja, int je) {
-          const int jm = min(row.jm, je);
-          if (ja < jm) run_chunk32<G, D, J, OPK, true, FX, true>(P, s, m, ri, row.i, ja, jm, col, 0, cur);
-          if (jm < je)
-            run_chunk32<G, D, J, OPK, false, FX, true>(P, s, m, ri, row.i, max(jm, ja), je, col, 0, cur);
-        };
-        if constexpr (NEAR) {
-          // the runs of neighbouring groups that the wave's rows can reach, or all columns
-          for (int jb = w.j0; jb < w.j1; jb += culled ? 64 * kGroup : w.j1 - w.j0) {
-            lanes_t near = culled ? near_groups(P, s, w, jb) : 1ull;
-            while (near) {
-              const int t = __builtin_ctzll(near);
-              const lanes_t rest = near >> t;  // starts with a run of set bits
-              const int n = ~rest ? __builtin_ctzll(~rest) : 64;
-              near = t + n < 64 ? (rest >> n) << (t + n) : 0ull;
-              run(jb + t * kGroup, culled ? min(w.j1, jb + (t + n) * kGroup) : w.j1);
-            }
-          }
-        } else {
-          run(w.j0, w.j1);
-        }
-      }
+      if (row.any) run_cols32<G, D, J, OPK, FX>(P, s, m, ri, row, w.j0, w.j1, rec, cur);
     } else {
       for (int jb = w.j0; jb < w.j1; jb += P.tj) {
         const int cnt = min(P.tj, w.j1 - jb);
@@ -2248,6 +2207,76 @@ __global__ void __launch_bounds__(1024, (FX && SLOAD) ? 6 : 1) hist32(Params P, 
     queue_wave_flush(P, m, cur);
     flush_hist(m, P, s, cur);
     if constexpr (OPK >= 9) flush_multi(m, P, cur);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// hist32n: the work units of culled slices.  Few pairs are evaluated (6 for one counted at N = 262144
+// points of the sphere and a reach of 0.05 rad), unevenly spread: a workgroup's row tile shared out
+// by rows left its waves waiting for the one with most columns in reach two thirds of the time (825 us
+// where the pairs take 240).  So a unit is a wave's, of 64 rows and at most 64 columns, and wave w of W
+// takes units w, w + W, ...: about eleven each there, near enough the same time for every CU without
+// a shared counter.  The waves of a workgroup meet only where its histogram has to be written out:
+// before the slice changes and before the updates of a round could pass the flush limit.  Call:
+// 1279 -> 683 us.
+// ---------------------------------------------------------------------------------------------
+template <int G, int D, bool J, int OPK, bool FX>
+__global__ void __launch_bounds__(1024, FX ? 6 : 1) hist32n(Params P, const float *__restrict__ rec) {
+  extern __shared__ __align__(16) char smem_raw[];
+  constexpr int F = Rec<G, D>::f32;
+  const Smem m = carve<J>(smem_raw, P, 0);
+  __shared__ int s_slice;
+  const int B = blockDim.x, waves = B >> 6, lane = (int)__lane_id();
+  const int stride = (int)gridDim.x * waves;
+  // columns a wave may run between two flushes (a unit has at most 64; the limit allows 1023 and more)
+  const int budget = (int)(P.flush_limit / B);
+  int u = __builtin_amdgcn_readfirstlane((int)blockIdx.x * waves + (int)(threadIdx.x >> 6));
+  bool have = u < P.n_items;
+  Item w = P.items[have ? u : 0];
+  int cur = -1;
+  Slice s{};
+  zero_hist(m);
+  if ((threadIdx.x & 63) == 0 && m.qcap > 0) m.qn[threadIdx.x >> 6] = 0u;
+  for (;;) {
+    // the round's slice: the first of those the waves hold a unit of (units are listed slice by slice)
+    __syncthreads();
+    if (threadIdx.x == 0) s_slice = 0x7fffffff;
+    __syncthreads();
+    if (have && lane == 0) atomicMin(&s_slice, w.slice);
+    __syncthreads();
+    const int next = __builtin_amdgcn_readfirstlane(s_slice);
+    if (cur >= 0) {
+      flush_hist(m, P, s, cur);
+      if constexpr (OPK >= 9) flush_multi(m, P, cur);
+      if (next != cur) queue_wave_flush(P, m, cur);
+      __syncthreads();
+    }
+    if (next == 0x7fffffff) break;
+    if (next != cur) {
+      cur = next;
+      s = P.slices[cur];
+      load_tables(m, P, s, true);
+      __syncthreads();
+    }
+    int cols = 0;
+    while (have && w.slice == cur) {
+      cols += w.j1 - w.j0;
+      if (cols > budget) break;
+      const int i = w.i0 + lane;
+      Row row;
+      row.i = i < s.N ? i : kNoRow;
+      row.any = true;
+      row.rec = i < s.N ? i : (int)(s.N - 1);
+      row.jm = w.i0 + 64 <= __builtin_amdgcn_readfirstlane((int)s.N) ? min(w.j1, w.i0 + 64) : w.j1;
+      float ri[F];
+#pragma unroll
+      for (int k = 0; k < F; ++k) ri[k] = rec[(s.pt_off + row.rec) * F + k];
+      const Item c = w;
+      u += stride;
+      have = u < P.n_items;
+      w = P.items[have ? u : 0];
+      run_cols32<G, D, J, OPK, FX>(P, s, m, ri, row, c.j0, c.j1, rec, cur);
+    }
   }
 }
 
@@ -2803,7 +2832,8 @@ namespace sfk {
 
 // the kernels of one (geometry, D): histogram, B-strip, re-bin and fused re-bin entry points
 struct KernelTable {
-  const void *(*hist)(bool J, bool mixed, int opk, bool sload, bool fx, bool near);
+  const void *(*hist)(bool J, bool mixed, int opk, bool sload, bool fx);
+  const void *(*near)(bool J, int opk, bool fx);
   const void *(*strip)(int opk);
   const void *(*recheck)(bool J, bool sp);
   const void *(*recheck_multi)(bool J);
@@ -2814,43 +2844,42 @@ KernelTable table_sphere2();
 KernelTable table_sphere3();
 
 #if SF_PART > 0
-template <int G, int D, bool J, bool SL, bool FX, bool NR>
+template <int G, int D, bool J, bool SL, bool FX>
 static const void *hist32_fn(int opk) {
   // fused outputs: scalar-loaded columns only
-  if (opk == 9) return (const void *)&hist32<G, D, J, 9, true, FX, NR>;
-  if (opk == 10) return (const void *)&hist32<G, D, J, 10, true, FX, NR>;
-  if (opk == 11) return (const void *)&hist32<G, D, J, 11, true, FX, NR>;
-  if (opk == 12) return (const void *)&hist32<G, D, J, 12, true, FX, NR>;
-  if (opk == 13) return (const void *)&hist32<G, D, J, 13, true, FX, NR>;
+  if (opk == 9) return (const void *)&hist32<G, D, J, 9, true, FX>;
+  if (opk == 10) return (const void *)&hist32<G, D, J, 10, true, FX>;
+  if (opk == 11) return (const void *)&hist32<G, D, J, 11, true, FX>;
+  if (opk == 12) return (const void *)&hist32<G, D, J, 12, true, FX>;
+  if (opk == 13) return (const void *)&hist32<G, D, J, 13, true, FX>;
   if constexpr (!J) {
-    if (opk == 3) return (const void *)&hist32<G, D, false, 3, SL, false, NR>;
+    if (opk == 3) return (const void *)&hist32<G, D, false, 3, SL, false>;
     if constexpr (SL) {  // 1D, scalar-loaded columns (the default): L^3, T, T^2, T^3
-      if (opk == 5) return (const void *)&hist32<G, D, false, 5, true, false, NR>;
-      if (opk == 6) return (const void *)&hist32<G, D, false, 6, true, false, NR>;
-      if (opk == 7) return (const void *)&hist32<G, D, false, 7, true, false, NR>;
-      if (opk == 8) return (const void *)&hist32<G, D, false, 8, true, false, NR>;
+      if (opk == 5) return (const void *)&hist32<G, D, false, 5, true, false>;
+      if (opk == 6) return (const void *)&hist32<G, D, false, 6, true, false>;
+      if (opk == 7) return (const void *)&hist32<G, D, false, 7, true, false>;
+      if (opk == 8) return (const void *)&hist32<G, D, false, 8, true, false>;
     }
   } else {
-    if (opk == 4) return (const void *)&hist32<G, D, true, 4, SL, FX, NR>;
+    if (opk == 4) return (const void *)&hist32<G, D, true, 4, SL, FX>;
   }
-  if (opk == 1) return (const void *)&hist32<G, D, J, 1, SL, FX, NR>;
-  if (opk == 2) return (const void *)&hist32<G, D, J, 2, SL, FX, NR>;
-  return (const void *)&hist32<G, D, J, 0, SL, FX, NR>;
+  if (opk == 1) return (const void *)&hist32<G, D, J, 1, SL, FX>;
+  if (opk == 2) return (const void *)&hist32<G, D, J, 2, SL, FX>;
+  return (const void *)&hist32<G, D, J, 0, SL, FX>;
 }
 
-template <int G, int D, bool J, bool SL, bool NR>
+template <int G, int D, bool J, bool SL>
 static const void *hist32_fx(bool fx, int opk) {
   // fixed-point cells exist for joint histograms only
   if constexpr (J) {
-    if (fx) return hist32_fn<G, D, true, SL, true, NR>(opk);
+    if (fx) return hist32_fn<G, D, true, SL, true>(opk);
   }
-  return hist32_fn<G, D, J, SL, false, NR>(opk);
+  return hist32_fn<G, D, J, SL, false>(opk);
 }
 
 template <int G, int D, bool J>
-static const void *hist_fn(bool mixed, int opk, bool sload, bool fx, bool near) {
-  if (mixed && near && sload) return hist32_fx<G, D, J, true, true>(fx, opk);
-  if (mixed) return sload ? hist32_fx<G, D, J, true, false>(fx, opk) : hist32_fx<G, D, J, false, false>(fx, opk);
+static const void *hist_fn(bool mixed, int opk, bool sload, bool fx) {
+  if (mixed) return sload ? hist32_fx<G, D, J, true>(fx, opk) : hist32_fx<G, D, J, false>(fx, opk);
   if constexpr (!J) {
     if (opk == 3) return (const void *)&hist64<G, D, false, 3>;
     if (opk == 5) return (const void *)&hist64<G, D, false, 5>;
@@ -2863,6 +2892,34 @@ static const void *hist_fn(bool mixed, int opk, bool sload, bool fx, bool near) 
   if (opk == 1) return (const void *)&hist64<G, D, J, 1>;
   if (opk == 2) return (const void *)&hist64<G, D, J, 2>;
   return (const void *)&hist64<G, D, J, 0>;
+}
+
+// culled slices (scalar-loaded columns)
+template <int G, int D, bool J, bool FX>
+static const void *near_fn(int opk) {
+  if (opk == 9) return (const void *)&hist32n<G, D, J, 9, FX>;
+  if (opk == 10) return (const void *)&hist32n<G, D, J, 10, FX>;
+  if (opk == 11) return (const void *)&hist32n<G, D, J, 11, FX>;
+  if (opk == 12) return (const void *)&hist32n<G, D, J, 12, FX>;
+  if (opk == 13) return (const void *)&hist32n<G, D, J, 13, FX>;
+  if constexpr (!J) {
+    if (opk == 3) return (const void *)&hist32n<G, D, false, 3, false>;
+    if (opk == 5) return (const void *)&hist32n<G, D, false, 5, false>;
+    if (opk == 6) return (const void *)&hist32n<G, D, false, 6, false>;
+    if (opk == 7) return (const void *)&hist32n<G, D, false, 7, false>;
+    if (opk == 8) return (const void *)&hist32n<G, D, false, 8, false>;
+  } else {
+    if (opk == 4) return (const void *)&hist32n<G, D, true, 4, FX>;
+  }
+  if (opk == 1) return (const void *)&hist32n<G, D, J, 1, FX>;
+  if (opk == 2) return (const void *)&hist32n<G, D, J, 2, FX>;
+  return (const void *)&hist32n<G, D, J, 0, FX>;
+}
+
+template <int G, int D>
+static const void *near_of(bool J, int opk, bool fx) {
+  if (!J) return near_fn<G, D, false, false>(opk);
+  return fx ? near_fn<G, D, true, true>(opk) : near_fn<G, D, true, false>(opk);
 }
 
 template <int G, int D>
@@ -2884,12 +2941,12 @@ static const void *recheck_multi_fn(bool J) {
 }
 
 template <int G, int D>
-static const void *hist_of(bool J, bool mixed, int opk, bool sload, bool fx, bool near) {
-  return J ? hist_fn<G, D, true>(mixed, opk, sload, fx, near) : hist_fn<G, D, false>(mixed, opk, sload, fx, near);
+static const void *hist_of(bool J, bool mixed, int opk, bool sload, bool fx) {
+  return J ? hist_fn<G, D, true>(mixed, opk, sload, fx) : hist_fn<G, D, false>(mixed, opk, sload, fx);
 }
 template <int G, int D>
 static KernelTable table_of() {
-  return KernelTable{&hist_of<G, D>, &strip_fn<G, D>, &recheck_fn<G, D>, &recheck_multi_fn<G, D>};
+  return KernelTable{&hist_of<G, D>, &near_of<G, D>, &strip_fn<G, D>, &recheck_fn<G, D>, &recheck_multi_fn<G, D>};
 }
 #if SF_PART == 1
 KernelTable table_flat2() { return table_of<kFlat, 2>(); }
@@ -2939,8 +2996,8 @@ hipError_t launch_prep(int G, int D, bool mixed, int geom_code, const void *ps, 
                 : prep_impl<kSphere, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st);
 }
 
-static const void *pick_hist(int G, int D, bool J, bool mixed, int opk, bool sl, bool fx, bool near) {
-  return table(G, D).hist(J, mixed, opk, sl, fx, near);
+static const void *pick_hist(int G, int D, bool J, bool mixed, int opk, bool sl, bool fx) {
+  return table(G, D).hist(J, mixed, opk, sl, fx);
 }
 
 static int opk_of(const Params &P) {
@@ -2958,7 +3015,7 @@ static int opk_of(const Params &P) {
 
 int hist_occupancy(int G, int D, bool J, bool mixed, int opk, bool sload, bool fx, int block,
                    size_t smem) {
-  const void *f = pick_hist(G, D, J, mixed, opk, sload, fx, false);
+  const void *f = pick_hist(G, D, J, mixed, opk, sload, fx);
   (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   int nb = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, block, smem) != hipSuccess) return 1;
@@ -2977,10 +3034,12 @@ int strip_occupancy(int G, int D, int opk, int block, size_t smem) {
   return nb;
 }
 
-hipError_t launch_hist(int G, int D, bool J, bool mixed, bool sload, const Params &P, int grid,
+// near: P's items are the work units of culled slices
+hipError_t launch_hist(int G, int D, bool J, bool mixed, bool sload, bool near, const Params &P, int grid,
                        int block, size_t smem, hipStream_t st) {
-  const void *f = (mixed && P.strip > 1) ? pick_strip(G, D, opk_of(P))
-                                         : pick_hist(G, D, J, mixed, opk_of(P), sload, mixed && P.fx, P.gboxes != nullptr);
+  const void *f = near                     ? table(G, D).near(J, opk_of(P), P.fx != 0)
+                  : (mixed && P.strip > 1) ? pick_strip(G, D, opk_of(P))
+                                           : pick_hist(G, D, J, mixed, opk_of(P), sload, mixed && P.fx);
   (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   Params Pc = P;
   const int opk = opk_of(P);
