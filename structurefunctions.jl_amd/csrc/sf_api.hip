@@ -1294,8 +1294,13 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
                      "histogram of %d cells needs %d bytes of LDS; the device allows %zu per workgroup",
                      ncell, std::max(L0.total, L64.total), ctx->max_smem);
   auto occupancy = [&](int blk, size_t bytes) {
-    return strip ? strip_occupancy(G, D, hist_opk(Pk), blk, bytes)
-                 : hist_occupancy(G, D, J, mixed, hist_opk(Pk), sload, pl.fx, blk, bytes);
+    const int nb = strip ? strip_occupancy(G, D, hist_opk(Pk), blk, bytes)
+                         : hist_occupancy(G, D, J, mixed, hist_opk(Pk), sload, pl.fx, blk, bytes);
+    // LDS is handed out in units of 1280 bytes, which the runtime's figure leaves out (max_smem is a
+    // CU's: 128 of them): a re-bin queue sized to the last byte had cost a workgroup per CU (flat 3D
+    // du_L^2, 100 bins, N = 98304, 512 threads: 4.94 ms, now 4.24)
+    const size_t unit = ctx->max_smem / 128;
+    return std::min(nb, (int)(128 / std::max<size_t>(1, (bytes + unit - 1) / unit)));
   };
   int bpc = occupancy(block, (size_t)(mixed ? L0.total
                                             : smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, copies, nmom, 0, qcap64,
