@@ -64,6 +64,7 @@ struct Slice {
   int32_t M64, ncell64;
   int32_t M32, ncell32;
   int32_t base32;     // binary32 table: cell = (bits >> (23 - M32)) - base32
+  int32_t mir;        // sphere, mirrored table (cell32m): cells of either half; 0: plain
   int32_t tab_off;    // first Cell of this slice's table (binary64 keys)
   int32_t tab32_off;  // first Cell of this slice's binary32 (chord^2 / r^2) table
   int32_t dedge_off;  // exact distance-key edges (flat: e*e; sphere: e), n_dist + 1 doubles

@@ -28,6 +28,8 @@
 // src/BinEdges.jl) with no fused multiply-adds.  The other paths ask for fma explicitly.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "sf_internal.h"
 #include "sfmath.h"
 
@@ -307,6 +309,9 @@ DEV T sp_invariant(int t, T duL, T dn2) {
 
 DEV int cell32(float key, const Slice &s);
 DEV unsigned cell32_off(float key, const Slice &s);
+DEV int cell32m(float key, const Slice &s);
+template <int G>
+DEV int cell32_any(float key, const Slice &s);
 
 // CERT (sphere): the distance bin is read from the chord^2 cell table of the binary32 kernel
 // (lo, hi, blo: ambiguity interval and bin count per cell) with the binary64 chord^2 |q - p|^2,
@@ -400,7 +405,7 @@ DEV int exact_cell(const Params &P, const Slice &s, const double *A, const doubl
     if constexpr (CERT) {
       f = sphere_frame64_noangle(A, B);
       const float key = (float)sdot<3>(f.d, f.d);
-      const int c = cell32(key, s);
+      const int c = cell32_any<G>(key, s);
       const float2 lh = lohi[c];
       exact_dist = (key >= lh.x) & (key <= lh.y);
       db = (key > lh.y) ? blo_tab[c].x + 1 : blo_tab[c].x;
@@ -991,7 +996,7 @@ struct Pending64 {
   double v, w;  // value (single pass: du_L) and |du|^2 (single pass)
 };
 
-template <int G, int D, bool J, int OPK, bool MASK, bool VU>
+template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR>
 DEV void pair64p(const Params &P, const Slice &s, const Smem &m, const double *A, int i, int j,
                  const double *B, double *rn, const double *next, Pending64 &pa) {
   constexpr int S = Rec<G, D>::d64;
@@ -1010,7 +1015,7 @@ DEV void pair64p(const Params &P, const Slice &s, const Smem &m, const double *A
     r2 = sdot<D>(dx, dx);
     key = (float)r2;
   }
-  const unsigned c = cell32_off(key, s);
+  const unsigned c = MIR ? 8u * (unsigned)cell32m(key, s) : cell32_off(key, s);
   const float2 lh = *(const float2 *)((const char *)m.lohi + c);
   const int blo = ((const int2 *)((const char *)m.blo + c))->x;
   __builtin_amdgcn_sched_barrier(0);
@@ -1110,7 +1115,7 @@ DEV void pair64p(const Params &P, const Slice &s, const Smem &m, const double *A
 
 // Columns j0 .. j1 - 1 of one row with pair64p; two record buffers alternate (the request past
 // the last column reads at most one record beyond the slice, as in run_cols64).
-template <int G, int D, bool J, int OPK, bool MASK, bool VU>
+template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR>
 DEV void run_cols64pv(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j0, int j1,
                       const double *__restrict__ rec) {
   constexpr int S = Rec<G, D>::d64;
@@ -1120,20 +1125,25 @@ DEV void run_cols64pv(const Params &P, const Slice &s, const Smem &m, const doub
   Pending64 pa{m.scr, 0.0, 0.0};
   int j = j0;
   for (; j + 1 < j1; j += 2) {
-    pair64p<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, col + (int64_t)(j + 1) * S, pa);
-    pair64p<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j + 1, rb, ra, col + (int64_t)(j + 2) * S, pa);
+    pair64p<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, col + (int64_t)(j + 1) * S, pa);
+    pair64p<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j + 1, rb, ra, col + (int64_t)(j + 2) * S, pa);
   }
-  if (j < j1) pair64p<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, col + (int64_t)(j + 1) * S, pa);
+  if (j < j1) pair64p<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, col + (int64_t)(j + 1) * S, pa);
   if constexpr (OPK == 3) hist_add_sp(m, pa.h, pa.v, pa.w);
   else hist_add(m, pa.h, pa.v);
 }
 
-// the value-bin lookup (uniform or exact) is chosen once per column range, not per pair
+// the value-bin lookup (uniform or exact) and the key table's form are chosen once per column range,
+// not per pair
 template <int G, int D, bool J, int OPK, bool MASK>
 DEV void run_cols64p(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j0, int j1,
                      const double *__restrict__ rec) {
-  if (J && s.v_uniform) run_cols64pv<G, D, J, OPK, MASK, true>(P, s, m, ri, i, j0, j1, rec);
-  else run_cols64pv<G, D, J, OPK, MASK, false>(P, s, m, ri, i, j0, j1, rec);
+  auto run = [&](auto mir) {
+    if (J && s.v_uniform) run_cols64pv<G, D, J, OPK, MASK, J, mir.value>(P, s, m, ri, i, j0, j1, rec);
+    else run_cols64pv<G, D, J, OPK, MASK, false, mir.value>(P, s, m, ri, i, j0, j1, rec);
+  };
+  if (G == kSphere && s.mir) run(std::integral_constant<bool, G == kSphere>());
+  else run(std::false_type());
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1236,7 +1246,7 @@ DEV bool near_value_edge(double v, const double *E, int nE, int g) {
   return near;
 }
 
-template <int G, int D, bool J, int OPK, bool MASK, bool VU>
+template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR>
 DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double *A, int i, int j,
                  const double *B, double *rn, const double *next, Pending64 &pa) {
   constexpr int S = rec_pair64<G, D>;
@@ -1250,7 +1260,7 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
   for (int k = 0; k < W; ++k) d[k] = B[k] - A[k];
   const double key64 = fdot<W>(d, d);
   const float key = (float)key64;
-  const unsigned c = cell32_off(key, s);
+  const unsigned c = MIR ? 8u * (unsigned)cell32m(key, s) : cell32_off(key, s);
   const float2 lh = *(const float2 *)((const char *)m.lohi + c);
   const int bm1 = ((const int2 *)((const char *)m.blo + c))->y;
   __builtin_amdgcn_sched_barrier(0);
@@ -1408,7 +1418,7 @@ DEV void rare64(const Params &P, const Slice &s, const Smem &m, const double *re
 // reads at most one record beyond the slice, as in run_cols64).  Returns j1, or the first column
 // not done when a group's flagged pairs did not fit the queue: they are then left in dm, their
 // last column in jl.
-template <int G, int D, bool J, int OPK, bool MASK, bool VU>
+template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR>
 DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j, int j1,
                     const double *__restrict__ rec, unsigned &dm_out, int &jl) {
   constexpr int S = rec_pair64<G, D>;
@@ -1426,12 +1436,12 @@ DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double
     const int je = min(j1, j + 32);
     dm = 0u;
     for (; j + 1 < je; j += 2, cp += 2 * S) {
-      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, cp + S, pa));
-      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * S, pa));
+      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, cp + S, pa));
+      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * S, pa));
     }
     // an odd count only occurs in the last group (the others hold 32 columns)
     if (j < je) {
-      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU>(P, s, m, ri, i, j, ra, rb, cp + S, pa));
+      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, cp + S, pa));
       ++j;
     }
     jl = je - 1;
@@ -1490,19 +1500,22 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
       double ri[S];
       load_rec64<S>(rec + (s.pt_off + row.rec) * S, ri);
       if constexpr (FAST) {
-        // the value-bin lookup (uniform or exact) is chosen per column range, not per pair
+        // the value-bin lookup (uniform or exact) and the key table's form are chosen per column range,
+        // not per pair
         for (int j = w.j0; j < w.j1;) {
           unsigned dm = 0u;
           int jl = 0;
           const bool mask = j < row.jm;
           const int je = mask ? row.jm : w.j1;
-          if (J && s.v_uniform) {
-            j = mask ? run_cols64f<G, D, J, OPK, true, true>(P, s, m, ri, row.i, j, je, rec, dm, jl)
-                     : run_cols64f<G, D, J, OPK, false, true>(P, s, m, ri, row.i, j, je, rec, dm, jl);
-          } else {
-            j = mask ? run_cols64f<G, D, J, OPK, true, false>(P, s, m, ri, row.i, j, je, rec, dm, jl)
-                     : run_cols64f<G, D, J, OPK, false, false>(P, s, m, ri, row.i, j, je, rec, dm, jl);
-          }
+          auto run = [&](auto vu, auto mir) {
+            return mask ? run_cols64f<G, D, J, OPK, true, vu.value, mir.value>(P, s, m, ri, row.i, j, je, rec, dm, jl)
+                        : run_cols64f<G, D, J, OPK, false, vu.value, mir.value>(P, s, m, ri, row.i, j, je, rec, dm, jl);
+          };
+          auto run_vu = [&](auto mir) {
+            return (J && s.v_uniform) ? run(std::integral_constant<bool, J>(), mir) : run(std::false_type(), mir);
+          };
+          if (G == kSphere && s.mir) j = run_vu(std::integral_constant<bool, G == kSphere>());
+          else j = run_vu(std::false_type());
           if (__ballot(dm != 0u)) rare64<G, D, J, OPK>(P, s, m, rec, dm, row.i, jl);
         }
       } else if (G == kSphere || !P.bl) {
@@ -1544,6 +1557,28 @@ DEV unsigned cell32_off(float key, const Slice &s) {
   int r;
   asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(c), "s"(8 * s.ncell32 - 1));
   return (unsigned)r & 0x1ff8u;
+}
+
+// Mirrored table (sphere, s.mir cells a half): a key from 2 on is looked up by 4 - key, which is exact
+// there, downwards from the table's end.  Distance edges crowd in the key towards antipodal pairs
+// (chord^2 = 4 - delta^2 at an angle pi - delta) as they do towards zero, where the cells shrink with
+// the key: a linear axis of 100 bins up to pi had its last edges in common cells, and with them 3.9 % of
+// all pairs were left to the exact sequence.  Kernel time at N = 98304, du_L^2, 100 bins: binary32 34.4
+// -> 5.5 ms, binary64 27.1 -> 7.0; fixed-point joint du_L 35.9 -> 6.6; 20 bins 6.9 -> 4.9, 12.2 -> 6.9
+// and 8.2 -> 6.4.  The host takes it where cells hold several edges over a thousandth of the keys; the
+// five instructions it costs are kept out of the other launches' loop (chosen per column range, like
+// the value lookup).
+DEV int cell32m(float key, const Slice &s) {
+  const float k1 = 4.0f - key;
+  const int c = (__float_as_int(__builtin_fminf(key, k1)) >> (23 - s.M32)) - s.base32;
+  int r;
+  asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(c), "s"(s.mir - 1));
+  return key < k1 ? r : 2 * s.mir - 1 - r;
+}
+// either table, off the pair loops' main path
+template <int G>
+DEV int cell32_any(float key, const Slice &s) {
+  return (G == kSphere && s.mir) ? cell32m(key, s) : cell32(key, s);
 }
 
 // value-axis bin from a binary32 value with absolute error bound dv = dva * dvb; sets amb when
@@ -1697,7 +1732,7 @@ DEV void flush_small(const Slice &s, const Smem &m, SmallAdd &sa) {
 // pair is evaluated (out-of-range pairs are simply not counted), so the wave never splits.
 // Returns whether the pair is undecidable in binary32 and must be re-binned in binary64; the
 // caller collects these flags and queues the pairs every few columns (queue_deferred).
-template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool VU, bool SL>
+template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool VU, bool SL, bool MIR>
 DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *ri, int i, int j,
                 const float *rj, float *rn, const float4 *next, bool has_next, PendingAdd &pa, SmallAdd &sa) {
   constexpr int F = Rec<G, D>::f32;
@@ -1731,7 +1766,7 @@ DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *
     umax = ri[12] + rj[12];
   }
   {
-    const int c = cell32(key, s);
+    const int c = MIR ? cell32m(key, s) : cell32(key, s);
     const float2 lh = m.lohi[c];
     const int bm1 = m.blo[c].y;  // bin count below the cell's interval, minus one
     // the previous pair's update, unconditional (a lane with nothing pending holds its scratch
@@ -2070,7 +2105,7 @@ DEV void queue_wave_flush(const Params &P, const Smem &m, int slice_id, int fiel
   *fillp = 0u;
 }
 
-template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool VU, bool SL>
+template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool VU, bool SL, bool MIR>
 DEV void run_chunk32_vu(const Params &P, const Slice &s, const Smem &m, const float *ri, int i,
                         int j_begin, int j_end, const float4 *col, int col_j0, int slice_id) {
   constexpr int F = Rec<G, D>::f32;
@@ -2090,13 +2125,13 @@ DEV void run_chunk32_vu(const Params &P, const Slice &s, const Smem &m, const fl
     const int je = min(j_end, jg + 32);
     unsigned dm = 0u;
     for (; j + 1 < je; j += 2, cp += 2 * R) {
-      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j, ra, rb, cp + R, true, pa, sa));
-      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * R, j + 2 < j_end,
+      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL, MIR>(P, s, m, ri, i, j, ra, rb, cp + R, true, pa, sa));
+      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL, MIR>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * R, j + 2 < j_end,
                                                                   pa, sa));
     }
     // an odd count only occurs in the last group (the others hold 32 columns)
     if (j < je) {
-      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j, ra, rb, cp + R, false, pa, sa));
+      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL, MIR>(P, s, m, ri, i, j, ra, rb, cp + R, false, pa, sa));
       ++j;
     }
     queue_deferred(P, m, dm, i, je - 1, slice_id, 0, -1);
@@ -2111,14 +2146,19 @@ DEV void run_chunk32_vu(const Params &P, const Slice &s, const Smem &m, const fl
   }
 }
 
-// the value-edge lookup (uniform or searched) is chosen once per column range, not per pair
+// the value-edge lookup (uniform or searched) and the key table's form are chosen once per column
+// range, not per pair
 template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool SL>
 DEV void run_chunk32(const Params &P, const Slice &s, const Smem &m, const float *ri, int i,
                      int j_begin, int j_end, const float4 *col, int col_j0, int slice_id) {
-  if (FX || (J && s.v_uniform))
-    run_chunk32_vu<G, D, J, OPK, MASK, FX, true, SL>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
-  else
-    run_chunk32_vu<G, D, J, OPK, MASK, FX, false, SL>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
+  auto run = [&](auto mir) {
+    if (FX || (J && s.v_uniform))
+      run_chunk32_vu<G, D, J, OPK, MASK, FX, true, SL, mir.value>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
+    else
+      run_chunk32_vu<G, D, J, OPK, MASK, FX, false, SL, mir.value>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
+  };
+  if (G == kSphere && s.mir) run(std::integral_constant<bool, G == kSphere>());
+  else run(std::false_type());
 }
 
 // Columns [ja, je) for a wave's row with scalar-loaded column records; the ones below row.jm may lie
@@ -2344,7 +2384,7 @@ DEV void run_chunk_strip(const Params &P, const Slice &s, const Smem &m, const f
         for (int k = 0; k < 3; ++k) d[k] = (rj[k] - ri[k]) + (rj[3 + k] - ri[3 + k]);
         key = __builtin_fmaf(d[2], d[2], __builtin_fmaf(d[1], d[1], d[0] * d[0]));
       }
-      const int c = cell32(key, s);
+      const int c = cell32_any<G>(key, s);
       const float2 lh = m.lohi[c];
       const int blo = m.blo[c].x;
       const bool ge = !(key < lh.x);  // as in pair32: a NaN key is ambiguous
