@@ -636,10 +636,13 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   const float close = flat ? round_up_f(std::max(1e-30L, ldexpl((long double)xmax * (long double)xmax, -44)))
                            : 0x1p-44f;
   const float anti = 4.0f - 0x1p-20f;
+  double top = flat ? 0.0 : 4.0;  // largest key that matters (flat: that of the last finite edge)
+  for (int k = 0; flat && k < nE; ++k)
+    if (C[k] < INFINITY) top = std::max(top, (double)C[k]);
   // The table of n32 cells from their bounds: cell c holds keys in [Flo[c], Fhi[c]] at most (both
   // ascend).  Per cell: the edges whose intervals end below it, and the number (and the index, where
   // it is one) of those that meet it, from each edge's first and last cell.  Returns the length of
-  // key in [0, 4] whose cells hold several edges: on the sphere a quarter of it is the share of evenly
+  // key in [0, top] whose cells hold several edges: on the sphere a quarter of it is the share of evenly
   // spread pairs that will be re-binned.
   auto fill = [&](const std::vector<float> &Flo, const std::vector<float> &Fhi) {
     const int n32 = (int)Flo.size();
@@ -677,7 +680,7 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
       } else {
         cl.lo = -INFINITY;
         cl.hi = INFINITY;
-        crowded += std::max(0.0, std::min(4.0, (double)Fn) - std::max(0.0, (double)Fc));
+        crowded += std::max(0.0, std::min(top, (double)Fn) - std::max(0.0, (double)Fc));
       }
       // keys that the kernels leave to the exact sequence wherever a bin holds them: those of nearly
       // coincident points (below `close`) and on the sphere of nearly antipodal ones
@@ -703,14 +706,39 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
     }
     return crowded;
   };
+  // the length of key that fill would return for the plain table of P32's binades, M bits each
+  auto crowd_of = [&](int M) {
+    const Partition Q{M, P32.elo, P32.ehi};
+    auto cell = [&](float v) {
+      int32_t bits;
+      memcpy(&bits, &v, sizeof bits);
+      return std::min(std::max((bits >> (23 - M)) - ((Q.elo + 127) << M), 0), Q.ncell() - 1);
+    };
+    double len = 0.0;
+    int seen = -1, counted = -1;  // last cell that an edge so far meets, last one counted
+    for (int k = 0; k < nE; ++k) {
+      if (!(std::fabs(C[k]) < INFINITY)) continue;
+      const int c0 = cell(lo[k]), c1 = cell(hi[k]);
+      for (int c = std::max(c0, counted + 1); c <= std::min(seen, c1); ++c) {
+        len += std::max(0.0, std::min(top, c + 1 < Q.ncell() ? Q.low(c + 1) : top) - (c > 0 ? Q.low(c) : 0.0));
+        counted = c;
+      }
+      seen = std::max(seen, c1);
+    }
+    return len;
+  };
+  // the coarsest cells that keep the edges as far apart as the finest that fit: a wave's lanes then
+  // share more of them (reads of one cell are broadcasts, of two cells in one bank a conflict), and
+  // the LDS that they leave holds more copies of a 1D histogram, or another workgroup: du_L^2 over 64
+  // log bins, flat 2D, N = 65536, 112 cells for 896 and 32 copies for 16: kernel 1934 -> 1729 us
+  const double crowd = crowd_of(P32.M);
+  for (int M = 0; M < P32.M; ++M)
+    if (crowd_of(M) <= crowd) P32.M = M;
   const int np = P32.ncell();  // <= kCell32Max: at most 252 binades, M chosen to fit
-  std::vector<float> Flo(np), Fhi(np);
-  for (int c = 0; c < np; ++c) Flo[c] = (float)P32.low(c);
-  for (int c = 0; c + 1 < np; ++c) Fhi[c] = Flo[c + 1];
-  Flo[0] = -INFINITY;
-  Fhi[np - 1] = INFINITY;
+  std::vector<float> Flo(np, -INFINITY), Fhi(np, INFINITY);
+  for (int c = 1; c < np; ++c) Fhi[c - 1] = Flo[c] = (float)P32.low(c);
+  (void)fill(Flo, Fhi);
   int mir = 0;
-  const double crowd = fill(Flo, Fhi);
   // (its five instructions a pair cost 4 %, a share of 0.8 % re-binned 40 % and more)
   if (!flat && crowd > 0.004) {
     // mirrored table (cell32m): `mir` cells for keys below 2, the rest by m = 4 - key below 2 downwards.
@@ -1252,7 +1280,8 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
         vedges32.push_back((float)sl[s].val_edges[k]);
       }
     }
-    ncell_max = std::max(ncell_max, std::max(d.ncell64, d.ncell32));
+    // (the binary64 table is read by the batch-leading flat operators without a difference form only)
+    ncell_max = std::max(ncell_max, flat && p0.semantics == SF_SEM_BATCH ? std::max(d.ncell64, d.ncell32) : d.ncell32);
     sdesc[s] = d;
   }
   if (vedges.empty()) { vedges.push_back(0.0); vedges32.push_back(0.0f); }
@@ -1362,6 +1391,15 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     // registers allow only one 768-thread workgroup per CU: use 1024 threads instead
     block = 1024;
     bpc = std::max(1, occupancy(block, (size_t)L0.total));
+  }
+  if (!J && !strip && pl.n1d == 0 && !tn.copies && copies == 16 && pl.total_pairs >= 100000000) {
+    // 32 copies where they cost no workgroup per CU: two lanes of a wave share one, not four, and a
+    // half wave's atomics never meet (N = 98304, 20 bins: flat 2D du_L^2 3.53 -> 3.29 ms, 3D 4.02 -> 3.94,
+    // sphere 4.57 -> 4.47; 64 bins, where five fit instead of six: 3.32 -> 3.44); in calls of a few
+    // hundred microseconds clearing and summing them costs as much (N = 4096: 144 us, 148 with 32)
+    const size_t need64 = (size_t)smem_layout(p0.n_dist, 0, ncell_max, 0, 32, nmom, 0, qcap64).total;
+    const size_t need = mixed ? (size_t)smem_layout(p0.n_dist, 0, ncell_max, stage_bytes, 32, nmom, 0, 0).total : need64;
+    if (std::max(need, need64) <= ctx->max_smem && occupancy(block, need) >= bpc) copies = 32;
   }
   // binary32 kernel: the LDS re-bin queue, as large as fits without costing a workgroup per CU
   // (0: every queued pair takes the global queue's atomic)
