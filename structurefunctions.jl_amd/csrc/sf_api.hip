@@ -1290,9 +1290,8 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   pl.fx = p0.precision == SF_PREC_MIXED_FIXED && J && !pl.sp;
   for (int s = 0; s < n && pl.fx; ++s) pl.fx = sdesc[s].v_uniform && sdesc[s].v_fx;
 
-  // ---- launch geometry: one histogram per workgroup; large joint histograms get 1024-thread
-  // workgroups (one per CU, 16 waves share the table), small 1D histograms 256-thread workgroups
-  // with per-lane interleaved copies (several workgroups per CU)
+  // ---- launch geometry: one histogram per workgroup; small 1D histograms get 256-thread workgroups with
+  // per-lane interleaved copies (several workgroups per CU)
   // launch shape: explicit tuning (sf_set_tuning) > autotuned entry for this key > defaults
   Params Pk{};
   Pk.op = p0.op;
@@ -1312,14 +1311,14 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     if (it != ctx->tuned.end()) tn = it->second;
   }
   const int t_block = tn.block, t_jchunk = tn.j_chunk, t_bpc = tn.bpc, t_variant = tn.variant;
-  // fixed-point joint: 768 threads, two workgroups per CU; other joint: 1024 threads, one per CU
+  // joint histograms: chosen below, when the LDS they need is known
   // 1D single pass: 512 threads (its 36-byte slots fill the LDS at two or three workgroups per CU;
   // more waves per workgroup then pay: flat 2D 595 against 492 Gpairs/s, sphere 644 against 529).
   // One-operator 1D kernels keep 256: 512 gained 5 % on flat 2D at N = 262144, nothing at 65536,
   // and lost on small slices (N = 4096: 51 against 88; the 256 ragged slices: 1019 against 1031)
   // Fused 1D outputs without a joint one: 512 threads (their histograms, 16 copies each, fill the
   // LDS at two or three workgroups per CU, like the single pass's)
-  int block = t_block ? t_block : (J ? (pl.fx ? 768 : 1024) : ((pl.sp || pl.n1d) ? 512 : 256));
+  int block = t_block ? t_block : (J || pl.sp || pl.n1d) ? 512 : 256;
   // column records staged per LDS chunk; the fixed-point joint launch keeps two workgroups per CU
   const int tj = std::min(block, (pl.fx || strip) ? 128 : 256);
   // column records: variant 1 stages them through LDS, variant 2 reads them with scalar loads
@@ -1363,13 +1362,15 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   // the reference's sequence: kRareQueue entries per wave, fewer (or none: such pairs are then
   // evaluated as they come) where the LDS does not hold them
   // (it reads its column records with scalar loads: no LDS stage)
-  int qcap64 = kRareQueue * (block / 64);
-  while (qcap64 > 0 && (size_t)smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, J ? 1 : copies, nmom, 0, qcap64, 0,
-                                           jlayout).total > ctx->max_smem)
-    qcap64 = qcap64 > block / 64 ? qcap64 / 2 : 0;
+  auto rare_queue = [&](int blk) {
+    int q = kRareQueue * (blk / 64);
+    while (q > 0 && (size_t)smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, J ? 1 : copies, nmom, 0, q, 0,
+                                        jlayout).total > ctx->max_smem)
+      q = q > blk / 64 ? q / 2 : 0;
+    return q;
+  };
   const SmemLayout L64 = smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, J ? 1 : copies, nmom, 0, 0, 0,
                                      jlayout);
-  pl.qcap64 = qcap64;
   if ((size_t)std::max(L0.total, L64.total) > ctx->max_smem)
     return ctx->fail(SF_E_UNSUPPORTED,
                      "histogram of %d cells needs %d bytes of LDS; the device allows %zu per workgroup",
@@ -1383,15 +1384,29 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     const size_t unit = ctx->max_smem / 128;
     return std::min(nb, (int)(128 / std::max<size_t>(1, (bytes + unit - 1) / unit)));
   };
-  int bpc = occupancy(block, (size_t)(mixed ? L0.total
-                                            : smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, copies, nmom, 0, qcap64,
-                                                          0, jlayout).total));
-  if (bpc < 1) bpc = 1;
-  if (!t_block && pl.fx && bpc * block < 1024) {
-    // registers allow only one 768-thread workgroup per CU: use 1024 threads instead
-    block = 1024;
-    bpc = std::max(1, occupancy(block, (size_t)L0.total));
+  auto resident = [&](int blk) {  // workgroups of blk threads per CU
+    return std::max(1, occupancy(blk, (size_t)(mixed ? L0.total
+                                                     : smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, copies, nmom, 0,
+                                                                   rare_queue(blk), 0, jlayout).total)));
+  };
+  if (!t_block && J) {
+    // joint histograms: the workgroup that leaves most waves on a CU, the smallest of those (more of
+    // them end and begin at different times, and share fewer slots).  Three of 512 threads against two of
+    // 768, fixed point, N = 98304, flat 2D: 4.71 / 4.93 ms at 40 x 64 bins, 4.91 / 5.06 at 20 x 32; two of
+    // 512 against one of 1024, sphere, N = 65536, 40 x 64 bins: binary64 3.64 / 4.04, binary32 3.10 /
+    // 3.34; fused, 40 x 48: 10.1 / 10.6.  64 x 96 bins keep two of 768 (fixed point) and one of 1024.
+    int most = 0;
+    for (const int blk : {512, 768, 1024}) {
+      const int threads = resident(blk) * blk;
+      if (threads > most) {
+        most = threads;
+        block = blk;
+      }
+    }
   }
+  const int qcap64 = rare_queue(block);
+  pl.qcap64 = qcap64;
+  int bpc = resident(block);
   if (!J && !strip && pl.n1d == 0 && !tn.copies && copies == 16 && pl.total_pairs >= 100000000) {
     // 32 copies where they cost no workgroup per CU: two lanes of a wave share one, not four, and a
     // half wave's atomics never meet (N = 98304, 20 bins: flat 2D du_L^2 3.53 -> 3.29 ms, 3D 4.02 -> 3.94,
