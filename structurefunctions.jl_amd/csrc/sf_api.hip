@@ -26,7 +26,8 @@
 namespace sfk {
 // kernel launchers (sf_kernels.hip)
 hipError_t launch_prep(int G, int D, bool mixed, int geom_code, const void *prep_slices,
-                       int n_slices, int64_t max_n, double *rec64, float *rec32, hipStream_t st);
+                       int n_slices, int64_t max_n, double *rec64, float *rec32, int nz, void *const *zp,
+                       const int64_t *zb, hipStream_t st);
 hipError_t launch_hist(int G, int D, bool J, bool mixed, bool sload, bool near, const Params &P, int grid,
                        int block, size_t smem, hipStream_t st);
 hipError_t launch_recheck(int G, int D, bool J, const Params &P, int grid, hipStream_t st);
@@ -38,7 +39,6 @@ hipError_t launch_merge_checked(const double *src_s, const unsigned long long *s
                                 hipStream_t st);
 hipError_t launch_zero(void *p, int64_t bytes, hipStream_t st);
 hipError_t launch_absmax(int count, const double *const *x, const int64_t *n, double *out, hipStream_t st);
-hipError_t launch_zero_multi(int count, void *const *p, const int64_t *bytes, hipStream_t st);
 hipError_t launch_derive_sp(double *s, unsigned long long *c, int64_t nbins, hipStream_t st);
 hipError_t launch_eval_math(int fn, int64_t n, const double *a, const double *b, double *out,
                             hipStream_t st);
@@ -1670,13 +1670,11 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
   sf_ctx *ctx = pl.ctx;
   if (pl.total_pairs == 0) return SF_OK;
   const int64_t ncells = (int64_t)pl.nout * pl.ncell;
-  HIPCHK(launch_prep(pl.G, pl.D, use_mixed, pl.geom_code, pl.prep, pl.n, pl.max_n, pl.rec64.p,
-                     pl.rec32.p, st));
   const int64_t mcells = (int64_t)pl.n1d * pl.nout * pl.P.n_dist;
   if (pl.n1d && !use_mixed)  // fused outputs exist in the binary32 kernel only
     return ctx->fail(SF_E_UNSUPPORTED, "internal: fused outputs launched on the binary64 kernel");
   {
-    // accumulators, queue count, work counter and overflow flag, and the fused ones: one launch
+    // records; accumulators, queue count, work counter and overflow flag, and the fused ones cleared
     void *zp[kZeroSetMax] = {pl.acc.p};
     int64_t zb[kZeroSetMax] = {(int64_t)pl.acc_bytes};
     int nz = 1;
@@ -1686,7 +1684,8 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
       zp[nz] = pl.mcounts.p;
       zb[nz++] = (int64_t)sizeof(unsigned long long) * mcells;
     }
-    HIPCHK(launch_zero_multi(nz, zp, zb, st));
+    HIPCHK(launch_prep(pl.G, pl.D, use_mixed, pl.geom_code, pl.prep, pl.n, pl.max_n, pl.rec64.p, pl.rec32.p, nz, zp, zb,
+                       st));
   }
   const bool use_sload = use_mixed && pl.sload;
   const int stage = (use_sload || !use_mixed) ? 0 : pl.tj * pl.F32 * 4;

@@ -239,7 +239,7 @@ inline __host__ __device__ JointLayout joint_layout(int n_dist, int n_val, int l
 inline __host__ __device__ bool sp2d(int op, int n_val) { return op == 6 && n_val > 0; }
 
 inline constexpr int kDummySlots = 64;
-inline constexpr int kZeroSetMax = 8;  // buffers cleared by one zero_multi launch
+inline constexpr int kZeroSetMax = 4;  // buffers cleared by prep64
 inline constexpr int kMaxParts = 16;   // partial maxima of one slice's coordinates (absmax)
 inline constexpr int kMaxSet = 32;     // slices of one absmax launch
 // largest binary32 key table (cells); the host's partition never exceeds it.  In LDS the table's

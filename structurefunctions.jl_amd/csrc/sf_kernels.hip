@@ -452,10 +452,22 @@ struct PrepSlice {
   int64_t mul;          // without perm: record k is point (k * mul) mod N (0: identity)
 };
 
+// prep64 clears a call's accumulators, counters and flags as well (a launch of its own for them was
+// 1.5 us of work in 8 us of the smallest calls' 98)
+struct ZeroSet {
+  unsigned long long *p[kZeroSetMax];
+  int64_t n[kZeroSetMax];
+};
+
 template <int G, int D>
-__global__ void prep64(const PrepSlice *ps, int geom_code, double *rec64) {
+__global__ void prep64(const PrepSlice *ps, int geom_code, double *rec64, ZeroSet z) {
   const PrepSlice s = ps[blockIdx.y];
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  {
+    const int64_t t = (int64_t)blockIdx.y * gridDim.x * blockDim.x + i, all = (int64_t)gridDim.y * gridDim.x * blockDim.x;
+    for (int b = 0; b < kZeroSetMax; ++b)
+      for (int64_t k = t; k < z.n[b]; k += all) z.p[b][k] = 0;
+  }
   if (i >= s.N) return;
   constexpr int S = Rec<G, D>::d64;
   double *r = rec64 + (s.pt_off + i) * S;
@@ -2821,18 +2833,6 @@ __global__ void zero_i32(int *p, int64_t n) {
   if (k < n) p[k] = 0;
 }
 
-// Several buffers cleared by one launch (one row of blocks per buffer): a call's accumulators,
-// counters and flags, one kernel instead of one per buffer.
-struct ZeroSet {
-  int *p[kZeroSetMax];
-  int64_t n[kZeroSetMax];  // 32-bit words
-};
-__global__ void zero_multi(ZeroSet z) {
-  const int b = blockIdx.y;
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < z.n[b]) z.p[b][k] = 0;
-}
-
 // max|x| of a batch of slices (NaN ignored), kMaxParts partial maxima per slice (one per block of a
 // grid row); the host reduces those.  Reading only: 1 MB (N = 65536, 2D) takes 4 us, where copying it
 // back for the host to scan took 0.25 ms.
@@ -3008,11 +3008,11 @@ static KernelTable table(int G, int D) {
 
 template <int G, int D>
 static hipError_t prep_impl(bool mixed, int geom_code, const void *ps, int n_slices, int64_t max_n,
-                            double *rec64, float *rec32, hipStream_t st) {
-  if (max_n <= 0) return hipSuccess;
+                            double *rec64, float *rec32, const ZeroSet &z, hipStream_t st) {
+  if (max_n <= 0) return hipErrorInvalidValue;  // (nothing would be cleared)
   const int T = 256;
   dim3 grid((unsigned)((max_n + T - 1) / T), (unsigned)n_slices);
-  prep64<G, D><<<grid, T, 0, st>>>((const PrepSlice *)ps, geom_code, rec64);
+  prep64<G, D><<<grid, T, 0, st>>>((const PrepSlice *)ps, geom_code, rec64, z);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (!mixed) {
@@ -3026,14 +3026,22 @@ static hipError_t prep_impl(bool mixed, int geom_code, const void *ps, int n_sli
   return hipGetLastError();
 }
 
+// nz buffers zp of zb bytes each (multiples of 8) are cleared by the way
 hipError_t launch_prep(int G, int D, bool mixed, int geom_code, const void *ps, int n_slices,
-                       int64_t max_n, double *rec64, float *rec32, hipStream_t st) {
-  if (G == kFlat) {
-    return D == 2 ? prep_impl<kFlat, 2>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st)
-                  : prep_impl<kFlat, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st);
+                       int64_t max_n, double *rec64, float *rec32, int nz, void *const *zp, const int64_t *zb,
+                       hipStream_t st) {
+  if (nz < 0 || nz > kZeroSetMax) return hipErrorInvalidValue;
+  ZeroSet z{};
+  for (int b = 0; b < nz; ++b) {
+    z.p[b] = (unsigned long long *)zp[b];
+    z.n[b] = zb[b] / 8;
   }
-  return D == 2 ? prep_impl<kSphere, 2>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st)
-                : prep_impl<kSphere, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, st);
+  if (G == kFlat) {
+    return D == 2 ? prep_impl<kFlat, 2>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, z, st)
+                  : prep_impl<kFlat, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, z, st);
+  }
+  return D == 2 ? prep_impl<kSphere, 2>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, z, st)
+                : prep_impl<kSphere, 3>(mixed, geom_code, ps, n_slices, max_n, rec64, rec32, z, st);
 }
 
 static const void *pick_hist(int G, int D, bool J, bool mixed, int opk, bool sl, bool fx) {
@@ -3158,20 +3166,6 @@ hipError_t launch_absmax(int count, const double *const *x, const int64_t *n, do
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
-}
-
-hipError_t launch_zero_multi(int count, void *const *p, const int64_t *bytes, hipStream_t st) {
-  if (count <= 0 || count > kZeroSetMax) return hipErrorInvalidValue;
-  ZeroSet z{};
-  int64_t nmax = 0;
-  for (int b = 0; b < count; ++b) {
-    z.p[b] = (int *)p[b];
-    z.n[b] = bytes[b] / 4;
-    nmax = nmax > z.n[b] ? nmax : z.n[b];
-  }
-  if (nmax <= 0) return hipSuccess;
-  zero_multi<<<dim3((unsigned)((nmax + 255) / 256), (unsigned)count), 256, 0, st>>>(z);
-  return hipGetLastError();
 }
 
 #endif  // SF_PART
