@@ -544,6 +544,7 @@ struct SliceTables {
   std::vector<Cell> tab64, tab32;
   std::vector<double> dedges;  // exact keys
   Slice desc{};
+  double crowd = 0;  // share of the keys whose table cells hold several edges: those pairs are re-binned
 };
 
 // binary64 decision points of a LinearBinEdges rule lie within this distance of the edge values
@@ -738,9 +739,10 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   std::vector<float> Flo(np, -INFINITY), Fhi(np, INFINITY);
   for (int c = 1; c < np; ++c) Fhi[c - 1] = Flo[c] = (float)P32.low(c);
   (void)fill(Flo, Fhi);
+  T.crowd = crowd / std::max(top, 1e-300);
   int mir = 0;
   // (its five instructions a pair cost 4 %, a share of 0.8 % re-binned 40 % and more)
-  if (!flat && crowd > 0.004) {
+  if (!flat && p.precision == SF_PREC_FP64 && crowd > 0.004) {
     // mirrored table (cell32m): `mir` cells for keys below 2, the rest by m = 4 - key below 2 downwards.
     // The smallest cells are those of the edge next to zero or next to 4 (keys within 2^-20 of 4 are
     // uncertain anyway: nearly antipodal).
@@ -1253,6 +1255,7 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   std::vector<double> dedges, vedges;
   std::vector<float> vedges32;
   int ncell_max = 1;
+  double crowd = 0.0;
   SliceTables T;
   for (int s = 0; s < n; ++s) {
     // (slices of one call mostly bin by the same edges: a table is built where they differ)
@@ -1260,6 +1263,7 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
       T = SliceTables();
       build_tables(sl[s], xmax[s], T);
     }
+    crowd = std::max(crowd, T.crowd);
     Slice d = T.desc;
     d.N = sl[s].N;
     d.pt_off = prep[s].pt_off;
@@ -1384,10 +1388,27 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     const size_t unit = ctx->max_smem / 128;
     return std::min(nb, (int)(128 / std::max<size_t>(1, (bytes + unit - 1) / unit)));
   };
+  // binary32 kernel: LDS bytes with a re-bin queue of q entries; and the entries that the queue needs
+  // where table cells hold several edges: room for four groups of 32 columns' worth of their pairs, of
+  // few such pairs for twelve.  A group that does not fit goes to the global queue by itself, and the
+  // waves of the device wait for one counter.  Linear axes up to pi on the sphere, N = 98304: 100 bins
+  // (3.9 % of the pairs) 34.4 -> 13.6 ms, 50 bins (0.8 %) 10.0 -> 7.3; twelve groups of 3.9 % cost 16.9.
+  auto bytes32 = [&](int q) {
+    return (size_t)smem_layout(p0.n_dist, p0.n_val, ncell_max, stage_bytes, copies, nmom, pl.fx, q, strip, jlayout,
+                               pl.n1d, mcop).total;
+  };
+  auto queue_need = [&](int blk) {
+    if (!mixed || !(crowd > 0.001)) return 0;
+    const double each = 2048.0 * crowd, wave = std::max(4.0 * each, std::min(12.0 * each, 160.0));
+    int q = 64;
+    while (q < wave * (blk / 64) && q < kQueueCap) q *= 2;
+    while (q > 0 && bytes32(q) > ctx->max_smem) q = q > 64 ? q / 2 : 0;
+    return q;
+  };
   auto resident = [&](int blk) {  // workgroups of blk threads per CU
-    return std::max(1, occupancy(blk, (size_t)(mixed ? L0.total
-                                                     : smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, copies, nmom, 0,
-                                                                   rare_queue(blk), 0, jlayout).total)));
+    return std::max(1, occupancy(blk, mixed ? bytes32(queue_need(blk))
+                                            : (size_t)smem_layout(p0.n_dist, p0.n_val, ncell_max, 0, copies, nmom, 0,
+                                                                  rare_queue(blk), 0, jlayout).total));
   };
   if (!t_block && J) {
     // joint histograms: the workgroup that leaves most waves on a CU, the smallest of those (more of
@@ -1416,15 +1437,12 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     const size_t need = mixed ? (size_t)smem_layout(p0.n_dist, 0, ncell_max, stage_bytes, 32, nmom, 0, 0).total : need64;
     if (std::max(need, need64) <= ctx->max_smem && occupancy(block, need) >= bpc) copies = 32;
   }
-  // binary32 kernel: the LDS re-bin queue, as large as fits without costing a workgroup per CU
+  // binary32 kernel: the LDS re-bin queue, as large as fits without costing a workgroup per CU more
   // (0: every queued pair takes the global queue's atomic)
   int qcap = 0;
   if (mixed) {
-    for (int q = kQueueCap; q >= 64 && qcap == 0; q >>= 1) {
-      const int t = smem_layout(p0.n_dist, p0.n_val, ncell_max, stage_bytes, copies, nmom, pl.fx, q, strip,
-                                jlayout, pl.n1d, mcop).total;
-      if ((size_t)t <= ctx->max_smem && occupancy(block, (size_t)t) >= bpc) qcap = q;
-    }
+    for (int q = kQueueCap; q >= 64 && qcap == 0; q >>= 1)
+      if (bytes32(q) <= ctx->max_smem && occupancy(block, bytes32(q)) >= bpc) qcap = q;
   }
   if (t_bpc) bpc = std::min(bpc, t_bpc);
   const int max_blocks = bpc * ctx->n_cu;

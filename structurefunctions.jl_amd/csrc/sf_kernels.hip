@@ -1571,15 +1571,16 @@ DEV unsigned cell32_off(float key, const Slice &s) {
   return (unsigned)r & 0x1ff8u;
 }
 
-// Mirrored table (sphere, s.mir cells a half): a key from 2 on is looked up by 4 - key, which is exact
-// there, downwards from the table's end.  Distance edges crowd in the key towards antipodal pairs
-// (chord^2 = 4 - delta^2 at an angle pi - delta) as they do towards zero, where the cells shrink with
-// the key: a linear axis of 100 bins up to pi had its last edges in common cells, and with them 3.9 % of
-// all pairs were left to the exact sequence.  Kernel time at N = 98304, du_L^2, 100 bins: binary32 34.4
-// -> 5.5 ms, binary64 27.1 -> 7.0; fixed-point joint du_L 35.9 -> 6.6; 20 bins 6.9 -> 4.9, 12.2 -> 6.9
-// and 8.2 -> 6.4.  The host takes it where cells hold several edges over a thousandth of the keys; the
-// five instructions it costs are kept out of the other launches' loop (chosen per column range, like
-// the value lookup).
+// Mirrored table (binary64 calls on the sphere, s.mir cells a half): a key from 2 on is looked up by
+// 4 - key, which is exact there, downwards from the table's end.  Distance edges crowd in the key towards
+// antipodal pairs (chord^2 = 4 - delta^2 at an angle pi - delta) as they do towards zero, where the
+// cells shrink with the key: a linear axis of 100 bins up to pi had its last edges in common cells,
+// and with them 3.9 % of all pairs were left to the reference's sequence.  du_L^2, N = 98304: 100 bins
+// 27.1 -> 7.0 ms, 20 bins 12.2 -> 6.9.  The host takes it where cells hold several edges over a
+// thousandth of the keys; the five instructions it costs are kept out of the other launches' loop
+// (chosen per column range, like the value lookup).  The binary32 kernels keep the plain table: the
+// pairs that it leaves to the re-bin have binary64 values, which near antipodal pairs (an error that
+// grows with 1 / sin) odd orders would miss: du_L^3 over 100 bins was off by 1e-8 (2-norm) without them.
 DEV int cell32m(float key, const Slice &s) {
   const float k1 = 4.0f - key;
   const int c = (__float_as_int(__builtin_fminf(key, k1)) >> (23 - s.M32)) - s.base32;
@@ -1744,7 +1745,7 @@ DEV void flush_small(const Slice &s, const Smem &m, SmallAdd &sa) {
 // pair is evaluated (out-of-range pairs are simply not counted), so the wave never splits.
 // Returns whether the pair is undecidable in binary32 and must be re-binned in binary64; the
 // caller collects these flags and queues the pairs every few columns (queue_deferred).
-template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool VU, bool SL, bool MIR>
+template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool VU, bool SL>
 DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *ri, int i, int j,
                 const float *rj, float *rn, const float4 *next, bool has_next, PendingAdd &pa, SmallAdd &sa) {
   constexpr int F = Rec<G, D>::f32;
@@ -1778,7 +1779,7 @@ DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *
     umax = ri[12] + rj[12];
   }
   {
-    const int c = MIR ? cell32m(key, s) : cell32(key, s);
+    const int c = cell32(key, s);
     const float2 lh = m.lohi[c];
     const int bm1 = m.blo[c].y;  // bin count below the cell's interval, minus one
     // the previous pair's update, unconditional (a lane with nothing pending holds its scratch
@@ -2117,7 +2118,7 @@ DEV void queue_wave_flush(const Params &P, const Smem &m, int slice_id, int fiel
   *fillp = 0u;
 }
 
-template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool VU, bool SL, bool MIR>
+template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool VU, bool SL>
 DEV void run_chunk32_vu(const Params &P, const Slice &s, const Smem &m, const float *ri, int i,
                         int j_begin, int j_end, const float4 *col, int col_j0, int slice_id) {
   constexpr int F = Rec<G, D>::f32;
@@ -2137,13 +2138,13 @@ DEV void run_chunk32_vu(const Params &P, const Slice &s, const Smem &m, const fl
     const int je = min(j_end, jg + 32);
     unsigned dm = 0u;
     for (; j + 1 < je; j += 2, cp += 2 * R) {
-      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL, MIR>(P, s, m, ri, i, j, ra, rb, cp + R, true, pa, sa));
-      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL, MIR>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * R, j + 2 < j_end,
+      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j, ra, rb, cp + R, true, pa, sa));
+      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * R, j + 2 < j_end,
                                                                   pa, sa));
     }
     // an odd count only occurs in the last group (the others hold 32 columns)
     if (j < je) {
-      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL, MIR>(P, s, m, ri, i, j, ra, rb, cp + R, false, pa, sa));
+      dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j, ra, rb, cp + R, false, pa, sa));
       ++j;
     }
     queue_deferred(P, m, dm, i, je - 1, slice_id, 0, -1);
@@ -2158,19 +2159,14 @@ DEV void run_chunk32_vu(const Params &P, const Slice &s, const Smem &m, const fl
   }
 }
 
-// the value-edge lookup (uniform or searched) and the key table's form are chosen once per column
-// range, not per pair
+// the value-edge lookup (uniform or searched) is chosen once per column range, not per pair
 template <int G, int D, bool J, int OPK, bool MASK, bool FX, bool SL>
 DEV void run_chunk32(const Params &P, const Slice &s, const Smem &m, const float *ri, int i,
                      int j_begin, int j_end, const float4 *col, int col_j0, int slice_id) {
-  auto run = [&](auto mir) {
-    if (FX || (J && s.v_uniform))
-      run_chunk32_vu<G, D, J, OPK, MASK, FX, true, SL, mir.value>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
-    else
-      run_chunk32_vu<G, D, J, OPK, MASK, FX, false, SL, mir.value>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
-  };
-  if (G == kSphere && s.mir) run(std::integral_constant<bool, G == kSphere>());
-  else run(std::false_type());
+  if (FX || (J && s.v_uniform))
+    run_chunk32_vu<G, D, J, OPK, MASK, FX, true, SL>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
+  else
+    run_chunk32_vu<G, D, J, OPK, MASK, FX, false, SL>(P, s, m, ri, i, j_begin, j_end, col, col_j0, slice_id);
 }
 
 // Columns [ja, je) for a wave's row with scalar-loaded column records; the ones below row.jm may lie
@@ -2396,7 +2392,7 @@ DEV void run_chunk_strip(const Params &P, const Slice &s, const Smem &m, const f
         for (int k = 0; k < 3; ++k) d[k] = (rj[k] - ri[k]) + (rj[3 + k] - ri[3 + k]);
         key = __builtin_fmaf(d[2], d[2], __builtin_fmaf(d[1], d[1], d[0] * d[0]));
       }
-      const int c = cell32_any<G>(key, s);
+      const int c = cell32(key, s);
       const float2 lh = m.lohi[c];
       const int blo = m.blo[c].x;
       const bool ge = !(key < lh.x);  // as in pair32: a NaN key is ambiguous

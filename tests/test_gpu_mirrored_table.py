@@ -1,5 +1,5 @@
-"""Linear axes up to pi on the sphere, whose last edges crowd in chord^2 (the mirrored key table of the
-binary32 and binary64 kernels), against the oracle: bins of every width around where the table is taken
+"""Linear axes up to pi on the sphere, whose last edges crowd in chord^2 (the mirrored key table of
+binary64 calls, the re-bin of the binary32 ones), against the oracle: bins of every width around where the table is taken
 (2 to 300 bins; 300 and a log axis with a tiny first edge keep the plain one), pairs spread evenly, near
 coincident and near antipodal.  Counts are bit-identical, sums within the bounds of the parity tests
 (whose binary32 term is divided by the smallest sine among the pairs in binary32, 2^-10)."""
@@ -44,19 +44,6 @@ def test_linear_axis_to_pi(ctx, nd):
             if prec == "fixed":
                 bound = bound + 1.5 * 2.0 ** -23 * (ve[1] - ve[0]) * oc
             assert np.all(np.abs(gs - os_) <= bound + 1e-300), (nd, op, prec)
-
-
-def test_few_pairs_are_rebinned(ctx):
-    """100 bins: every edge in a cell of its own, so the re-binned share is that of the edges' margins
-    (2^-19 of the key each way: below 1e-4 of evenly spread pairs an edge) and of the cells beside the
-    smallest edges."""
-    rng = np.random.default_rng(1)
-    v = rng.normal(size=(3, 6000))
-    v /= np.linalg.norm(v, axis=0)
-    x = np.degrees(np.stack([np.arctan2(v[1], v[0]), np.arcsin(v[2])]))
-    gpu_hist(ctx, x, rng.normal(size=(2, 6000)), np.linspace(0, np.pi, 101), (0, 2, 0), geometry="deg", prec="mixed")
-    st = ctx.stats()
-    assert st["rebinned"] < 0.002 * st["pairs"]
 
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
