@@ -289,7 +289,7 @@ struct Plan {
   DevBuf<float> gboxes;   // boxes of the record groups of culled slices
   DevBuf<Item> units;     // culled slices' work units, slice after slice
   int n_units = 0, near_grid = 1, jchunk = 1;
-  DevBuf<int32_t> perm;   // spatial order of the binary32 records (tile culling)
+  DevBuf<int32_t> perm;   // spatial order of the binary32 records (culling)
   bool culled = false;    // some slice is evaluated by its work units, not by items
   Arena *arena = nullptr;  // set: every buffer is taken from this region (no device allocation)
   // fused outputs: 1D operators evaluated with the main (joint) one, their accumulators and the
@@ -376,7 +376,7 @@ struct sf_ctx {
   Plan noalloc;
   char *scratch_ptr = nullptr;
   Plan fused;  // the fused-output entry's plan
-  // spatial sort and tile culling: device workspace and the slice/tile boxes read back
+  // spatial sort and culling: device workspace, and each slice's information (launch_cull)
   DevBuf<char> cull_ws;
   DevBuf<double> cull_info;
 

@@ -1,4 +1,4 @@
-// sf_cull.hip -- device preparation of spatial sort and tile culling (gfx950).
+// sf_cull.hip -- device preparation of spatial sort and culling (gfx950).
 //
 // For a slice whose largest distance edge is small against its extent, the binary32 records are
 // put in Morton (Z-curve) order of their key-space coordinates (flat: x; sphere: the unit

@@ -25,7 +25,7 @@ enum Geom : int { kFlat = 0, kSphere = 1 };
 //                 U = u_e E + u_n N is the tangent velocity in R^3, ur the radial component
 //                 (D = 3), P the unit position; |u| is an upper bound of the velocity norm;
 //                 id is the point's index in the caller's order (int32 bits): binary32 records
-//                 may be stored in a spatially sorted order (tile culling).
+//                 may be stored in a spatially sorted order (culling).
 inline constexpr __host__ __device__ int rec_d64(int G, int D) { return (G == kFlat) ? ((D == 2) ? 4 : 6) : 12; }
 inline constexpr __host__ __device__ int rec_f32(int G, int D) { return (G == kFlat && D == 2) ? 12 : 16; }
 inline constexpr __host__ __device__ int rec_id(int G, int D) { return (G == kFlat) ? 4 * D + 1 : 15; }
