@@ -1398,8 +1398,11 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
                                pl.n1d, mcop).total;
   };
   auto queue_need = [&](int blk) {
-    if (!mixed || !(crowd > 0.001)) return 0;
-    const double each = 2048.0 * crowd, wave = std::max(4.0 * each, std::min(12.0 * each, 160.0));
+    if (!mixed) return 0;
+    // (32 entries a wave at least: a size that leaves no room for a queue beside one workgroup more per CU
+    // had every queued pair wait for the global counter, fixed point, 48 x 80 bins 2.25 -> 4.27 ms)
+    const double each = crowd > 0.001 ? 2048.0 * crowd : 0.0;
+    const double wave = std::max(32.0, std::max(4.0 * each, std::min(12.0 * each, 160.0)));
     int q = 64;
     while (q < wave * (blk / 64) && q < kQueueCap) q *= 2;
     while (q > 0 && bytes32(q) > ctx->max_smem) q = q > 64 ? q / 2 : 0;
@@ -1434,7 +1437,8 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     // sphere 4.57 -> 4.47; 64 bins, where five fit instead of six: 3.32 -> 3.44); in calls of a few
     // hundred microseconds clearing and summing them costs as much (N = 4096: 144 us, 148 with 32)
     const size_t need64 = (size_t)smem_layout(p0.n_dist, 0, ncell_max, 0, 32, nmom, 0, qcap64).total;
-    const size_t need = mixed ? (size_t)smem_layout(p0.n_dist, 0, ncell_max, stage_bytes, 32, nmom, 0, 0).total : need64;
+    const size_t need = mixed ? (size_t)smem_layout(p0.n_dist, 0, ncell_max, stage_bytes, 32, nmom, 0,
+                                                        queue_need(block)).total : need64;
     if (std::max(need, need64) <= ctx->max_smem && occupancy(block, need) >= bpc) copies = 32;
   }
   // binary32 kernel: the LDS re-bin queue, as large as fits without costing a workgroup per CU more
