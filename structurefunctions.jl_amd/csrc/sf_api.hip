@@ -2299,6 +2299,13 @@ struct sf_plan {
   std::vector<unsigned long long *> last_mc;
 };
 
+// Waits for the upload that plan_build leaves running on st: a plan is executed on whatever stream the
+// caller names (and is captured into a graph there), which nothing else orders after st.
+static int plan_ready(sf_ctx *ctx, hipStream_t st) {
+  HIPCHK(hipStreamSynchronize(st));
+  return SF_OK;
+}
+
 extern "C" int sf_plan_create(sf_ctx *ctx, int32_t n, const sf_problem *sl, sf_plan **out) {
   if (!ctx || !out) return SF_E_ARG;
   *out = nullptr;
@@ -2321,6 +2328,7 @@ extern "C" int sf_plan_create(sf_ctx *ctx, int32_t n, const sf_problem *sl, sf_p
   plan->ctx = ctx;
   // no culling in plans: the positions behind x may change between executions
   rc = plan_build(ctx, plan->pl, n, sl, px.data(), pu.data(), xmax.data(), st, false);
+  if (!rc) rc = plan_ready(ctx, st);
   if (rc) {
     plan->pl.release();
     delete plan;
@@ -2404,6 +2412,7 @@ extern "C" int sf_plan_create_multi(sf_ctx *ctx, int32_t n, const sf_problem *sl
   // no culling in plans: the positions behind x may change between executions
   if (!rc) rc = plan_build(ctx, plan->pl, n, plan->fs.main().data(), px.data(), pu.data(), xmax.data(), st, false,
                            &plan->fs.ms);
+  if (!rc) rc = plan_ready(ctx, st);
   if (rc) {
     plan->pl.release();
     delete plan;
