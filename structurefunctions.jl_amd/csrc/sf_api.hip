@@ -544,7 +544,7 @@ struct SliceTables {
   std::vector<Cell> tab64, tab32;
   std::vector<double> dedges;  // exact keys
   Slice desc{};
-  double crowd = 0;  // share of the keys whose table cells hold several edges: those pairs are re-binned
+  double crowd = 0;  // share of the keys that the table leaves uncertain (the edges' own intervals aside)
 };
 
 // binary64 decision points of a LinearBinEdges rule lie within this distance of the edge values
@@ -643,11 +643,13 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   // The table of n32 cells from their bounds: cell c holds keys in [Flo[c], Fhi[c]] at most (both
   // ascend).  Per cell: the edges whose intervals end below it, and the number (and the index, where
   // it is one) of those that meet it, from each edge's first and last cell.  Returns the length of
-  // key in [0, top] whose cells hold several edges: on the sphere a quarter of it is the share of evenly
-  // spread pairs that will be re-binned.
+  // key in [0, top] that its cells leave uncertain, the edges' own intervals aside: those that hold
+  // several edges, or one edge beside the nearly coincident keys.
+  // On the sphere a quarter of it is the share of evenly spread pairs that will be re-binned.
   auto fill = [&](const std::vector<float> &Flo, const std::vector<float> &Fhi) {
     const int n32 = (int)Flo.size();
-    double crowded = 0.0;
+    double lost = 0.0;
+    auto length = [&](double a, double b) { return std::max(0.0, std::min(top, b) - std::max(0.0, a)); };
     T.tab32.resize(n32);
     std::vector<int> dbelow(n32 + 1, 0), dmeet(n32 + 1, 0), dwhich(n32 + 1, 0);
     for (int k = 0; k < nE; ++k) {
@@ -681,7 +683,7 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
       } else {
         cl.lo = -INFINITY;
         cl.hi = INFINITY;
-        crowded += std::max(0.0, std::min(top, (double)Fn) - std::max(0.0, (double)Fc));
+        lost += length(Fc, Fn);
       }
       // keys that the kernels leave to the exact sequence wherever a bin holds them: those of nearly
       // coincident points (below `close`) and on the sphere of nearly antipodal ones
@@ -698,43 +700,61 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
         } else if (!(nint == 1 && below == 0 && lo[which] > close)) {  // (else nothing counted below the edge)
           cl.lo = -INFINITY;
           cl.hi = INFINITY;
+          if (nint == 1 && Fn > close) lost += length(Fc, Fn);
         }
       }
-      if (!flat && below + nint > 0 && below < nE && Fn > anti && Fc < 8.0f) {
+      // (keys past the last edge are in no bin: an axis that ends below `anti` has none of the latter)
+      const int under = below + (nint == 1 && hi[which] < anti);
+      if (!flat && below + nint > 0 && under < nE && Fn > anti && Fc < 8.0f) {
         cl.lo = nint == 0 ? anti : std::min(cl.lo, anti);
         cl.hi = INFINITY;
       }
     }
-    return crowded;
+    return lost;
   };
   // the length of key that fill would return for the plain table of P32's binades, M bits each
-  auto crowd_of = [&](int M) {
+  auto lost_of = [&](int M) {
     const Partition Q{M, P32.elo, P32.ehi};
     auto cell = [&](float v) {
       int32_t bits;
       memcpy(&bits, &v, sizeof bits);
       return std::min(std::max((bits >> (23 - M)) - ((Q.elo + 127) << M), 0), Q.ncell() - 1);
     };
+    auto low = [&](int c) { return c > 0 ? Q.low(c) : 0.0; };
+    auto high = [&](int c) { return c + 1 < Q.ncell() ? std::min(top, Q.low(c + 1)) : top; };
+    const int cc = cell(close);
     double len = 0.0;
     int seen = -1, counted = -1;  // last cell that an edge so far meets, last one counted
+    int below_c = 0, n_c = 0, k_c = 0;  // edges below cell cc; in it, and the last of those
     for (int k = 0; k < nE; ++k) {
-      if (!(std::fabs(C[k]) < INFINITY)) continue;
+      if (!(std::fabs(C[k]) < INFINITY)) {
+        below_c += C[k] < 0;
+        continue;
+      }
       const int c0 = cell(lo[k]), c1 = cell(hi[k]);
       for (int c = std::max(c0, counted + 1); c <= std::min(seen, c1); ++c) {
-        len += std::max(0.0, std::min(top, c + 1 < Q.ncell() ? Q.low(c + 1) : top) - (c > 0 ? Q.low(c) : 0.0));
+        len += std::max(0.0, high(c) - low(c));
         counted = c;
       }
       seen = std::max(seen, c1);
+      below_c += c1 < cc;
+      if (c0 <= cc && cc <= c1) {
+        ++n_c;
+        k_c = k;
+      }
     }
+    if (n_c == 1 && low(cc) < close && hi[k_c] > close && (below_c > 0 || lo[k_c] <= close))
+      len += std::max(0.0, high(cc) - low(cc));
     return len;
   };
-  // the coarsest cells that keep the edges as far apart as the finest that fit: a wave's lanes then
-  // share more of them (reads of one cell are broadcasts, of two cells in one bank a conflict), and
+  // the coarsest cells that keep the edges as far apart as the finest that fit, and away from the nearly
+  // coincident keys (a leading -Inf edge and a second one at a power of two): a wave's lanes then share
+  // more of them (reads of one cell are broadcasts, of two cells in one bank a conflict), and
   // the LDS that they leave holds more copies of a 1D histogram, or another workgroup: du_L^2 over 64
   // log bins, flat 2D, N = 65536, 112 cells for 896 and 32 copies for 16: kernel 1934 -> 1729 us
-  const double crowd = crowd_of(P32.M);
+  const double crowd = lost_of(P32.M);
   for (int M = 0; M < P32.M; ++M)
-    if (crowd_of(M) <= crowd) P32.M = M;
+    if (lost_of(M) <= crowd) P32.M = M;
   const int np = P32.ncell();  // <= kCell32Max: at most 252 binades, M chosen to fit
   std::vector<float> Flo(np, -INFINITY), Fhi(np, INFINITY);
   for (int c = 1; c < np; ++c) Fhi[c - 1] = Flo[c] = (float)P32.low(c);
