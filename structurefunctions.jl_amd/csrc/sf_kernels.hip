@@ -558,11 +558,15 @@ __global__ void prep64s(const PrepSlice *ps, const double *rec64, double *recf) 
   const double *r = rec64 + (s.pt_off + src) * S;
   double *o = recf + (s.pt_off + i) * kF64Rec;
   const double ue = r[8], un = r[9];
+  // every operator of the reference takes the difference of the radial components too, times zero where
+  // it does not depend on it: a component that is not finite (or whose differences may not be) makes
+  // the others NaN, so that such a pair's value is not finite and the reference's sequence decides
+  const double z = (D == 3) ? 0.0 * (4.0 * r[10]) : 0.0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) o[k] = r[k];
-  o[3] = 2.0 * (ue * r[3] + un * r[5]);
-  o[4] = 2.0 * (ue * r[4] + un * r[6]);
-  o[5] = 2.0 * (un * r[7]);
+  o[3] = 2.0 * (ue * r[3] + un * r[5]) + z;
+  o[4] = 2.0 * (ue * r[4] + un * r[6]) + z;
+  o[5] = 2.0 * (un * r[7]) + z;
   o[6] = r[10];
   const double n2 = ue * ue + un * un + (D == 3 ? r[10] * r[10] : 0.0);
   const float nrm = round_up_f(__builtin_sqrt(n2) * (1.0 + 1e-12));
@@ -1308,7 +1312,10 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
       tn2 = n2 - L * L;
     }
     if constexpr (needT && OPK != 7) {
-      const double cz = __builtin_fma(du[1], d[0], -(du[0] * d[1]));
+      double cz = __builtin_fma(du[1], d[0], -(du[0] * d[1]));
+      // the transverse direction is horizontal; the reference's dot product still takes the third
+      // component times zero, NaN where that is not finite
+      if constexpr (D == 3) cz = __builtin_fma(du[2], 0.0, cz);
       T = cz * (D == 2 ? y : rsqrt64(__builtin_fma(d[1], d[1], d[0] * d[0])));
     }
   } else if constexpr (needT) {
