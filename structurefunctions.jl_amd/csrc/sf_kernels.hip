@@ -569,7 +569,9 @@ __global__ void prep64s(const PrepSlice *ps, const double *rec64, double *recf) 
   o[5] = 2.0 * (un * r[7]) + z;
   o[6] = r[10];
   const double n2 = ue * ue + un * un + (D == 3 ? r[10] * r[10] : 0.0);
-  const float nrm = round_up_f(__builtin_sqrt(n2) * (1.0 + 1e-12));
+  float nrm = round_up_f(__builtin_sqrt(n2) * (1.0 + 1e-12));
+  // zero for a zero velocity only
+  if (ue != 0.0 || un != 0.0 || (D == 3 && r[10] != 0.0)) nrm = nrm < 0x1p-100f ? 0x1p-100f : nrm;
   o[7] = __hiloint2double((int)src, __float_as_int(0x1p-12f * nrm));
 }
 
@@ -852,6 +854,10 @@ DEV lanes_t lanes_lt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 4);
 DEV lanes_t lanes_nlt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 11); }  // !(a < b)
 DEV lanes_t lanes_ngt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 13); }  // !(a > b)
 DEV lanes_t lanes_nge(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 12); }  // !(a >= b)
+DEV lanes_t lanes_eq(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 1); }
+DEV lanes_t lanes_eq(double a, double b) { return __builtin_amdgcn_fcmp(a, b, 1); }
+DEV lanes_t lanes_nan(float a) { return __builtin_amdgcn_fcmpf(a, a, 8); }
+DEV lanes_t lanes_nan(double a) { return __builtin_amdgcn_fcmp(a, a, 8); }
 DEV lanes_t lanes_nlt(double a, double b) { return __builtin_amdgcn_fcmp(a, b, 11); }
 DEV lanes_t lanes_nge(double a, double b) { return __builtin_amdgcn_fcmp(a, b, 12); }
 DEV lanes_t lanes_below(int a, int b) { return __builtin_amdgcn_uicmp((unsigned)a, (unsigned)b, 36); }  // 0 <= a < b
@@ -1196,6 +1202,17 @@ DEV void run_cols64p(const Params &P, const Slice &s, const Smem &m, const doubl
 // of an LDS queue, and a full segment is evaluated by the wave with all its lanes (rare64).  A
 // branch in the loop ran the exact sequence for one lane or two at a time, and its registers made
 // the loop spill: N = 100003, 14.2 ms against 22.6 before the difference form.
+//
+// Fields with masked points (velocities of zero, or NaN) have many such pairs, and one evaluation by
+// the reference's sequence takes as long as seven of these.  Where a group of columns has kManyRare
+// of them, the wave goes on with the form for such fields (MANY), for the next kManyCols columns:
+// it knows the value of a pair with equal velocities (zero, whose value bin is looked up once) and
+// of one with a NaN velocity (NaN, which no value bin holds), and that a NaN distance is in no bin.
+// Its six instructions a pair are kept out of the other form.  Joint du_L on the sphere, N = 60000, 64 x 96
+// bins, all points at rest: 50.7 ms without it, 4.7 with it (11.8 before the difference form; no point at
+// rest 3.8); 30 % at rest: 14.1, 4.0 (9.1); 10 % of the velocities NaN: 33.6, 4.0 (8.5); 1D du_L^2, 10 % NaN:
+// 23.9, 3.1 (7.4).  Fewer rare pairs than kManyRare in a group (2 % of it) are better queued: those of a
+// joint du_L^2 whose first edge is zero, 0.8 %, took 0.82 ms and 0.94 with this form (N = 30011).
 // ---------------------------------------------------------------------------------------------
 DEV double rsqrt64(double x) {
   const double y = __builtin_amdgcn_rsq(x);
@@ -1262,9 +1279,16 @@ DEV bool near_value_edge(double v, const double *E, int nE, int g) {
   return near;
 }
 
-template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR>
+inline constexpr int kManyRare = 48, kManyCols = 4096;
+// no value bin is known for a zero (an edge of -0.0 tells the zeros' signs apart)
+inline constexpr int kNoZeroBin = (int)0x80000000;
+
+// MANY (with MASK): the form for fields with masked points; only the pairs of the lanes in `want` are
+// evaluated, and zb is the value bin of zero.  Returns the lanes whose pair is left to the reference's
+// sequence: their key is uncertain, or they lie in a distance bin and their value is.
+template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR, bool MANY>
 DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double *A, int i, int j,
-                 const double *B, double *rn, const double *next, Pending64 &pa) {
+                 const double *B, double *rn, const double *next, Pending64 &pa, lanes_t want, int zb) {
   constexpr int S = rec_pair64<G, D>;
   constexpr int W = (G == kFlat) ? D : 3;  // space the differences live in
   constexpr int UO = (G == kFlat) ? D : 3; // first velocity word of a record
@@ -1285,7 +1309,7 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
   asm volatile("" ::"v"(lh.x), "v"(lh.y), "v"(bm1) : "memory");
   // a key outside [lo, hi] is above the edge exactly when it is not below lo; a NaN key is uncertain
   const lanes_t ge = lanes_nlt(key, lh.x);
-  lanes_t rare = ge & lanes_ngt(key, lh.y);
+  const lanes_t rare_d = ge & lanes_ngt(key, lh.y);
   const int db0 = lane_of(ge) ? bm1 + 1 : bm1;
   double e2 = 0.0;
   if constexpr (G == kSphere) {
@@ -1299,7 +1323,7 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
   double dw = 0.0;
   if constexpr (G == kSphere && D == 3) dw = B[6] - A[6];
   float nj = 0.f;
-  if constexpr (G == kSphere && J) nj = __int_as_float(__double2loint(B[7]));
+  if constexpr (G == kSphere && (J || MANY)) nj = __int_as_float(__double2loint(B[7]));
   load_rec64<S>(next, rn);
   __builtin_amdgcn_sched_barrier(0);
   // (sphere: 2 sin = sqrt(key e2), and the records hold 2 U)
@@ -1328,15 +1352,26 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
   }
   double v = SP ? L : op64<OPK>(P, D, L, T, tn2, n2);
   int vb0 = 0;
+  lanes_t rare_v = 0ull, nan = 0ull;
   if constexpr (J) {
     const float Lf = __builtin_fabsf((float)L);
+    lanes_t zero = 0ull;
     if constexpr (G == kSphere) {
-      const float ni = __int_as_float(__double2loint(A[7]));
-      rare |= lanes_ngt(Lf, ni + nj);
+      const float n = __int_as_float(__double2loint(A[7])) + nj;
+      rare_v = lanes_ngt(Lf, n);
+      if constexpr (MANY) {
+        zero = lanes_eq(n, 0.f);  // (both velocities are zero: prep64s)
+        nan = lanes_nan(n);
+      }
     } else {
       float q = __builtin_fabsf((float)du[0]) + __builtin_fabsf((float)du[1]);
       if constexpr (D == 3) q += __builtin_fabsf((float)du[2]);
-      rare |= lanes_ngt(Lf, 0x1p-12f * q);
+      rare_v = lanes_ngt(Lf, 0x1p-12f * q);
+      if constexpr (MANY) {
+        zero = lanes_eq(du[0], 0.0) & lanes_eq(du[1], 0.0);
+        if constexpr (D == 3) zero &= lanes_eq(du[2], 0.0);
+        nan = lanes_nan(q);
+      }
     }
     if constexpr (VU) {  // s.v_uniform, chosen once per column range
       // t + eps with the margin eps of the largest value that can be in range: a value outside
@@ -1344,22 +1379,43 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
       // edge lies within eps of t (NaN fails the comparison too).
       const float t = __builtin_fmaf((float)v, s.vinvf, s.vtcu);
       const float gh = __builtin_floorf(t);
-      rare |= lanes_nge(t - gh, s.veps2);
+      rare_v |= lanes_nge(t - gh, s.veps2);
       vb0 = (int)gh;
     } else {
       vb0 = (s.vrule.on ? lin_rule_bin(s.vrule, v, P.n_val) : val_bin64(v, m.vE, P.n_val + 1, s)) - 1;
       // searched edges: a value close to one takes the reference's own value
-      rare |= __builtin_amdgcn_ballot_w64(near_value_edge(v, m.vE, P.n_val + 1, vb0));
+      rare_v |= __builtin_amdgcn_ballot_w64(near_value_edge(v, m.vE, P.n_val + 1, vb0));
     }
-  } else if constexpr (SP) {
-    rare |= lanes_nlt(__builtin_fabs(L), __builtin_inf()) | lanes_nlt(n2, __builtin_inf());
+    if constexpr (MANY) {
+      zero = zb == kNoZeroBin ? 0ull : zero;
+      vb0 = lane_of(zero) ? zb : vb0;
+      rare_v &= ~(zero | nan);
+    }
   } else {
-    rare |= lanes_nlt(__builtin_fabs(v), __builtin_inf());
+    if constexpr (SP) rare_v = lanes_nlt(__builtin_fabs(L), __builtin_inf()) | lanes_nlt(n2, __builtin_inf());
+    else rare_v = lanes_nlt(__builtin_fabs(v), __builtin_inf());
+    if constexpr (MANY) {  // NaN velocities: the value is NaN in any sequence
+      if constexpr (G == kSphere) {
+        rare_v &= ~lanes_nan(__int_as_float(__double2loint(A[7])) + nj);
+      } else {
+        double q = __builtin_fabs(du[0]) + __builtin_fabs(du[1]);
+        if constexpr (D == 3) q += __builtin_fabs(du[2]);
+        rare_v &= ~lanes_nan(q);
+      }
+    }
   }
-  lanes_t add = ~rare & lanes_below(db0, P.n_dist);
-  if constexpr (J) add &= lanes_below(vb0, P.n_val);
+  const lanes_t in_d = lanes_below(db0, P.n_dist);
+  lanes_t rare = rare_d | (rare_v & in_d);
+  lanes_t add = ~rare & in_d;
+  if constexpr (J) add &= lanes_below(vb0, P.n_val) & ~nan;
+  if constexpr (MANY) {  // a NaN distance is in no bin
+    const lanes_t there = ~lanes_nan(key);
+    rare &= there;
+    add &= there;
+  }
   if constexpr (MASK) {
-    const lanes_t upper = lanes_gt(j, i);
+    lanes_t upper = lanes_gt(j, i);
+    if constexpr (MANY) upper &= want;
     add &= upper;
     rare &= upper;
   }
@@ -1436,10 +1492,11 @@ DEV void rare64(const Params &P, const Slice &s, const Smem &m, const double *re
 // t of dm flags column jl - t); two record buffers alternate (the request past the last column
 // reads at most one record beyond the slice, as in run_cols64).  Returns j1, or the first column
 // not done when a group's flagged pairs did not fit the queue: they are then left in dm, their
-// last column in jl.
-template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR>
+// last column in jl.  MANY: only the pairs whose bits are set in want, as those in dm, in every group
+// (a call with other bits than all ones holds one group).
+template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR, bool MANY>
 DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j, int j1,
-                    const double *__restrict__ rec, unsigned &dm_out, int &jl) {
+                    const double *__restrict__ rec, unsigned &dm_out, int &jl, unsigned want) {
   constexpr int S = rec_pair64<G, D>;
   // the slice offset is wave-uniform by construction; say so, so that the column addresses stay in
   // SGPRs
@@ -1450,17 +1507,32 @@ DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double
   double ra[S], rb[S];
   load_rec64<S>(cp, ra);
   Pending64 pa{m.scr, 0.0, 0.0};
+  int zb = kNoZeroBin;
+  if constexpr (MANY && J) {
+    if (!s.v_negzero)
+      zb = __builtin_amdgcn_readfirstlane(
+               s.vrule.on ? lin_rule_bin(s.vrule, 0.0, P.n_val) : val_bin64(0.0, m.vE, P.n_val + 1, s)) - 1;
+  }
   unsigned dm = 0u;
   while (j < j1) {
     const int je = min(j1, j + 32);
+    unsigned wb = MANY ? want << (32 - (je - j)) : 0u;  // the next column's bit on top
+    auto pair = [&](int jc, const double *B, double *rn, const double *next) {
+      lanes_t wl = ~0ull;
+      if constexpr (MANY) {
+        wl = __builtin_amdgcn_ballot_w64((int)wb < 0);
+        wb += wb;
+      }
+      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU, MIR, MANY>(P, s, m, ri, i, jc, B, rn, next, pa, wl, zb));
+    };
     dm = 0u;
     for (; j + 1 < je; j += 2, cp += 2 * S) {
-      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, cp + S, pa));
-      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j + 1, rb, ra, cp + 2 * S, pa));
+      pair(j, ra, rb, cp + S);
+      pair(j + 1, rb, ra, cp + 2 * S);
     }
     // an odd count only occurs in the last group (the others hold 32 columns)
     if (j < je) {
-      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, cp + S, pa));
+      pair(j, ra, rb, cp + S);
       ++j;
     }
     jl = je - 1;
@@ -1473,6 +1545,23 @@ DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double
   return j;
 }
 
+// run_cols64f for columns below row.jm (mask) or all above; the value-bin lookup (uniform or exact),
+// the key table's form and the form of the pair (many) are chosen per column range, not per pair
+template <int G, int D, bool J, int OPK>
+DEV int run_range64f(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j, int je, bool mask,
+                     bool many, unsigned want, const double *__restrict__ rec, unsigned &dm, int &jl) {
+  auto run = [&](auto vu, auto mir) {
+    if (many) return run_cols64f<G, D, J, OPK, true, vu.value, mir.value, true>(P, s, m, ri, i, j, je, rec, dm, jl, want);
+    return mask ? run_cols64f<G, D, J, OPK, true, vu.value, mir.value, false>(P, s, m, ri, i, j, je, rec, dm, jl, ~0u)
+                : run_cols64f<G, D, J, OPK, false, vu.value, mir.value, false>(P, s, m, ri, i, j, je, rec, dm, jl, ~0u);
+  };
+  auto run_vu = [&](auto mir) {
+    return (J && s.v_uniform) ? run(std::integral_constant<bool, J>(), mir) : run(std::false_type(), mir);
+  };
+  if (G == kSphere && s.mir) return run_vu(std::integral_constant<bool, G == kSphere>());
+  return run_vu(std::false_type());
+}
+
 template <int G, int D, bool J, int OPK>
 __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restrict__ rec) {
   extern __shared__ __align__(16) char smem_raw[];
@@ -1482,6 +1571,7 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
   __shared__ int s_item;
   const int B = blockDim.x;
   int cur = -1;
+  int many = 0;  // columns that the wave still runs in the form for fields with masked points
   Slice s{};
   unsigned long long since_flush = 0;
   zero_hist(m);
@@ -1519,23 +1609,26 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
       double ri[S];
       load_rec64<S>(rec + (s.pt_off + row.rec) * S, ri);
       if constexpr (FAST) {
-        // the value-bin lookup (uniform or exact) and the key table's form are chosen per column range,
-        // not per pair
         for (int j = w.j0; j < w.j1;) {
           unsigned dm = 0u;
           int jl = 0;
           const bool mask = j < row.jm;
-          const int je = mask ? row.jm : w.j1;
-          auto run = [&](auto vu, auto mir) {
-            return mask ? run_cols64f<G, D, J, OPK, true, vu.value, mir.value>(P, s, m, ri, row.i, j, je, rec, dm, jl)
-                        : run_cols64f<G, D, J, OPK, false, vu.value, mir.value>(P, s, m, ri, row.i, j, je, rec, dm, jl);
-          };
-          auto run_vu = [&](auto mir) {
-            return (J && s.v_uniform) ? run(std::integral_constant<bool, J>(), mir) : run(std::false_type(), mir);
-          };
-          if (G == kSphere && s.mir) j = run_vu(std::integral_constant<bool, G == kSphere>());
-          else j = run_vu(std::false_type());
-          if (__ballot(dm != 0u)) rare64<G, D, J, OPK>(P, s, m, rec, dm, row.i, jl);
+          int je = mask ? row.jm : w.j1;
+          if (many > 0) je = min(je, j + many);
+          const int jn = run_range64f<G, D, J, OPK>(P, s, m, ri, row.i, j, je, mask, many > 0, ~0u, rec, dm, jl);
+          if (__ballot(dm != 0u)) {
+            unsigned tot = 0u;
+            if (many <= 0) (void)wave_prefix((unsigned)__popc(dm), &tot);
+            if (tot >= kManyRare) {
+              many = kManyCols;
+              const unsigned want = dm;
+              (void)run_range64f<G, D, J, OPK>(P, s, m, ri, row.i, j + ((jl - j) & ~31), jl + 1, true, true, want, rec,
+                                               dm, jl);
+            }
+            rare64<G, D, J, OPK>(P, s, m, rec, dm, row.i, jl);
+          }
+          many -= jn - j;
+          j = jn;
         }
       } else if (G == kSphere || !P.bl) {
         if (w.j0 < row.jm) run_cols64p<G, D, J, OPK, true>(P, s, m, ri, row.i, w.j0, row.jm, rec);

@@ -1,0 +1,86 @@
+"""Fields with masked points (velocities of zero, NaN velocities, NaN positions): every share of them, in
+runs and scattered, against the oracle, and the time of such a call against that of the same call without
+masked points (their pairs must not be evaluated one by one by the exact sequence)."""
+import numpy as np
+import pytest
+
+import _oracle
+from test_gpu_parity import MAG, TOL, check, field, gpu_hist
+
+pytestmark = pytest.mark.gpu
+# value axes with an edge at zero, without one, with one of -0.0, and one that zero lies outside of
+AXES = {"even": np.linspace(-4, 4, 25), "odd": np.linspace(-4, 4, 24),
+        "negzero": np.concatenate([np.linspace(-4, -1, 5), [-0.0, 0.5, 1.5]]), "above": np.linspace(0.25, 5, 20)}
+
+
+def mask(x, u, kind, share, run, seed):
+    x, u = x.copy(), u.copy()
+    n = x.shape[1]
+    k = int(round(share * n))
+    at = np.arange(n // 3, n // 3 + k) % n if run else np.random.default_rng(seed).permutation(n)[:k]
+    if kind == "rest":
+        u[:, at] = 0.0
+    elif kind == "nan":
+        u[seed % 2, at] = np.nan
+    elif kind == "nowhere":
+        x[seed % x.shape[0], at] = np.nan if seed % 2 else -np.nan
+    return x, u
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed", "fixed"])
+@pytest.mark.parametrize("geometry,D", [("flat", 2), ("flat", 3), ("deg", 2), ("deg", 3)])
+@pytest.mark.parametrize("kind", ["rest", "nan", "nowhere"])
+def test_masked(ctx, geometry, D, kind, prec):
+    p = "mixed" if prec == "fixed" else prec
+    for k, (share, run) in enumerate([(0.1, False), (0.5, False), (0.4, True), (1.0, False)]):
+        x, u, edges = field(geometry, D, 700, 21 + k)
+        x, u = mask(x, u, kind, share, run, k)
+        cases = [((0, 1, 0), "even"), ((0, 2, 0), "even"), ((0, 1, 0), "odd"), ((0, 1, 0), "negzero"),
+                 ((0, 2, 0), "above"), ((1, 0, 0), "even"), ((0, 0, 1), "odd")]
+        if prec != "fixed":
+            cases += [((0, 2, 0), None), ((2, 0, 0), None), ((0, 0, 3), None), ((1, 0, 0), None)]
+        for op, ve in cases:
+            ve = None if ve is None else AXES[ve]
+            # (fixed-point cells need equal bins; others fall back to the strict ones)
+            os_, oc, oa, og = _oracle.hist(x, u, edges, op=op, geometry=geometry, vedges=ve, nthreads=8, with_mag=True)
+            gs, gc = gpu_hist(ctx, x, u, edges, op, geometry=geometry, vedges=ve, prec=prec)
+            og = np.where(np.isfinite(og), og, 0.0)
+            mag = MAG[p] + (16 * 2.0 ** -53 / 1e-4 if prec == "fp64" else 0.0)
+            if prec == "fixed":  # 2^-22 value bins a pair
+                og = og + oc * (ve[1] - ve[0] if ve is not None else 0.0) * 2.0 ** -22 / mag
+            check(gs, gc, os_, oc, oa, TOL[p], f"{geometry} D={D} {kind} {share} {op} {prec}", og=og, mag=mag)
+
+
+@pytest.mark.parametrize("geometry", ["flat", "deg"])
+def test_masked_and_back(ctx, geometry):
+    """More columns than the form for such fields runs in one go, masked ones at the start, joint with the
+    binary64 kernel: in and out of that form."""
+    x, u, edges = field(geometry, 2, 9000, 3)
+    u[:, :1500] = 0.0
+    u[:, 1500:2000] = np.nan
+    os_, oc, oa, og = _oracle.hist(x, u, edges, op=(0, 1, 0), geometry=geometry, vedges=AXES["even"], nthreads=8,
+                                   with_mag=True)
+    gs, gc = gpu_hist(ctx, x, u, edges, (0, 1, 0), geometry=geometry, vedges=AXES["even"], prec="fp64")
+    og = np.where(np.isfinite(og), og, 0.0)
+    check(gs, gc, os_, oc, oa, TOL["fp64"], geometry, og=og, mag=16 * 2.0 ** -53 / 1e-4)
+
+
+@pytest.mark.parametrize("geometry", ["flat", "deg"])
+@pytest.mark.parametrize("kind,op,joint", [("rest", (0, 1, 0), True), ("nan", (0, 1, 0), True), ("nan", (0, 2, 0), False),
+                                           ("nowhere", (0, 1, 0), True), ("nowhere", (0, 2, 0), False)])
+def test_masked_time(ctx, geometry, kind, op, joint):
+    """Kernel time, binary64: at most three times that of the unmasked field (one by one: five to thirteen)."""
+    x, u, edges = field(geometry, 2, 30000, 5)
+    ve = AXES["even"] if joint else None
+
+    def best(x, u):
+        t = []
+        for _ in range(4):
+            gpu_hist(ctx, x, u, edges, op, geometry=geometry, vedges=ve, prec="fp64")
+            t.append(ctx.stats()["hist_ns"])
+        return min(t)
+
+    plain = best(x, u)
+    for share in (0.3, 1.0):
+        xm, um = mask(x, u, kind, share, False, 1)
+        assert best(xm, um) <= 3 * plain
