@@ -520,12 +520,15 @@ __global__ void prep32(const PrepSlice *ps, const double *rec64, float *rec32) {
   const double *r = rec64 + (s.pt_off + src) * S;
   float *o = rec32 + (s.pt_off + i) * F;
   for (int k = 0; k < F; ++k) o[k] = 0.0f;
+  // a third component that is not finite (or whose differences may not be) makes the others NaN, as in
+  // prep64s: the pair's value is then not finite, and the pair is re-binned
+  const double z = (D == 3) ? 0.0 * (4.0 * r[G == kFlat ? 5 : 10]) : 0.0;
   if (G == kFlat) {
     double n2 = 0.0;
 #pragma unroll
     for (int k = 0; k < D; ++k) {
       split2(r[k], &o[k], &o[D + k]);
-      split2(r[D + k], &o[2 * D + k], &o[3 * D + k]);
+      split2(r[D + k] + z, &o[2 * D + k], &o[3 * D + k]);
       n2 += r[D + k] * r[D + k];
     }
     o[4 * D] = round_up_f(__builtin_sqrt(n2) * (1.0 + 1e-12));
@@ -535,7 +538,7 @@ __global__ void prep32(const PrepSlice *ps, const double *rec64, float *rec32) {
     const double ue = r[8], un = r[9];
     const double E[3] = {r[3], r[4], 0.0}, Nn[3] = {r[5], r[6], r[7]};
 #pragma unroll
-    for (int k = 0; k < 3; ++k) split2(ue * E[k] + un * Nn[k], &o[6 + k], &o[9 + k]);
+    for (int k = 0; k < 3; ++k) split2(ue * E[k] + un * Nn[k] + z, &o[6 + k], &o[9 + k]);
     const double n2 = ue * ue + un * un + (D == 3 ? r[10] * r[10] : 0.0);
     o[12] = round_up_f(__builtin_sqrt(n2) * (1.0 + 1e-12));
     split2(r[10], &o[13], &o[14]);

@@ -21,7 +21,7 @@ def mask(x, u, kind, share, run, seed):
     if kind == "rest":
         u[:, at] = 0.0
     elif kind == "nan":
-        u[seed % 2, at] = np.nan
+        u[seed % u.shape[0], at] = np.nan
     elif kind == "nowhere":
         x[seed % x.shape[0], at] = np.nan if seed % 2 else -np.nan
     return x, u

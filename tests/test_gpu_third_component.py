@@ -1,6 +1,6 @@
 """A third velocity component that is not finite: every operator of the reference takes it (times zero
 where the value does not depend on it), so a bin's sum is NaN or infinite where one of its pairs has such a
-point.  Binary64 kernel, against the oracle's pairs."""
+point.  Against the oracle's pairs."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("bad", [np.nan, np.inf, -1e308])
 @pytest.mark.parametrize("op", [(0, 1, 0), (0, 2, 0), (0, 3, 0), (0, 0, 1), (0, 0, 2), (0, 0, 3), (0, 1, 1), (1, 0, 0),
                                 (2, 0, 0)])
-def test_third_component(ctx, geometry, bad, op):
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_third_component(ctx, geometry, bad, op, prec):
     x, u, edges = field(geometry, 3, 90, 31)
     n = 90
     u[2, 17] = bad
@@ -30,7 +31,7 @@ def test_third_component(ctx, geometry, bad, op):
                 if ok and 1 <= db < len(edges):
                     want[db - 1] += v
                     cnt[db - 1] += 1
-    gs, gc = gpu_hist(ctx, x, u, edges, op, geometry=geometry, prec="fp64")
+    gs, gc = gpu_hist(ctx, x, u, edges, op, geometry=geometry, prec=prec)
     gs, gc = gs.reshape(-1), gc.reshape(-1)
     assert np.array_equal(gc, cnt)
     assert np.array_equal(np.isnan(gs), np.isnan(want)) and np.array_equal(np.isinf(gs), np.isinf(want))
