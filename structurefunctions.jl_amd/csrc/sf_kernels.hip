@@ -624,7 +624,7 @@ struct Smem {
 template <bool JT>
 DEV Smem carve(char *base, const Params &P, int stage_bytes) {
   const SmemLayout L = smem_layout(P.n_dist, P.n_val, P.ncell_max, stage_bytes, P.copies, P.nmom, P.fx,
-                                   P.qcap, P.strip, P.jlayout, P.n1d, P.mcopies);
+                                   P.qcap, P.strip, P.jlayout, P.nf, P.mcopies);
   Smem m;
   m.nmom = P.nmom;
   m.fx = P.fx != 0;
@@ -857,6 +857,8 @@ DEV lanes_t lanes_lt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 4);
 DEV lanes_t lanes_nlt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 11); }  // !(a < b)
 DEV lanes_t lanes_ngt(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 13); }  // !(a > b)
 DEV lanes_t lanes_nge(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 12); }  // !(a >= b)
+DEV lanes_t lanes_ge(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 3); }    // a >= b
+DEV lanes_t lanes_le(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 5); }    // a <= b
 DEV lanes_t lanes_eq(float a, float b) { return __builtin_amdgcn_fcmpf(a, b, 1); }
 DEV lanes_t lanes_eq(double a, double b) { return __builtin_amdgcn_fcmp(a, b, 1); }
 DEV lanes_t lanes_nan(float a) { return __builtin_amdgcn_fcmpf(a, a, 8); }
@@ -1288,7 +1290,7 @@ inline constexpr int kNoZeroBin = (int)0x80000000;
 
 // MANY (with MASK): the form for fields with masked points; only the pairs of the lanes in `want` are
 // evaluated, and zb is the value bin of zero.  Returns the lanes whose pair is left to the reference's
-// sequence: their key is uncertain, or they lie in a distance bin and their value is.
+// sequence.
 template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR, bool MANY>
 DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double *A, int i, int j,
                  const double *B, double *rn, const double *next, Pending64 &pa, lanes_t want, int zb) {
@@ -1408,17 +1410,12 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
     }
   }
   const lanes_t in_d = lanes_below(db0, P.n_dist);
-  lanes_t rare = rare_d | (rare_v & in_d);
+  lanes_t rare = rare_d | (MANY ? rare_v & in_d : rare_v);
   lanes_t add = ~rare & in_d;
   if constexpr (J) add &= lanes_below(vb0, P.n_val) & ~nan;
-  if constexpr (MANY) {  // a NaN distance is in no bin
-    const lanes_t there = ~lanes_nan(key);
-    rare &= there;
-    add &= there;
-  }
   if constexpr (MASK) {
     lanes_t upper = lanes_gt(j, i);
-    if constexpr (MANY) upper &= want;
+    if constexpr (MANY) upper &= want & ~lanes_nan(key);  // (a NaN distance is in no bin)
     add &= upper;
     rare &= upper;
   }
@@ -1862,6 +1859,10 @@ DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *
   constexpr bool MULTI = (OPK >= 9);
   constexpr int NF = OPK == 9 ? 1 : (OPK == 10 ? 2 : (OPK == 11 ? 4 : (OPK == 12 ? 6 : kMaxFused)));
   constexpr bool needN2 = (OPK == 0) || MULTI || SP || SP2;
+  // operators that do not take the distance: |du|^2, and on the flat geometry the horizontal transverse
+  // component (fused outputs of such operators alone take the kernel of kMaxFused outputs, see plan_build)
+  constexpr bool NAN_KEY = OPK == 0 || (MULTI && NF == kMaxFused) ||
+                           (G == kFlat && (SP2 || (D == 3 && (OPK == 6 || OPK == 8))));
   const int nb = P.n_dist;
   lanes_t amb, amb_d;
   float key, L = 0.f, T = 0.f, tn2 = 0.f, n2 = 0.f, amp = 1.0f, umax;
@@ -1900,11 +1901,14 @@ DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *
     // operations): the next column's record is requested only after this point, because a
     // scalar load still in flight would make the wait for the table read wait for it as well
     asm volatile("" ::"v"(lh.x), "v"(lh.y), "v"(bm1) : "memory");
-    // two compares: a key that is not in [lo, hi] is above the edge exactly when it is not below lo
-    // (a NaN key is ambiguous).  Nearly coincident and nearly antipodal points lie in the table's
-    // intervals: no test of their own.
-    const lanes_t ge = lanes_nlt(key, lh.x);
-    amb_d = ge & lanes_ngt(key, lh.y);
+    // two compares: a key that is not in [lo, hi] is above the edge exactly when key >= lo.  Nearly
+    // coincident and nearly antipodal points lie in the table's intervals: no test of their own.
+    // A NaN key (a NaN position) belongs to no bin.  What its sign finds in the table, below the first
+    // edge or above the last, is none on most axes; on the others the value, NaN as well, leaves the pair
+    // to the re-bin.  Where the value may not be NaN (NAN_KEY), the key is tested: both compares fail.
+    const lanes_t ge = lanes_ge(key, lh.x), le = lanes_le(key, lh.y);
+    amb_d = ge & le;
+    amb = NAN_KEY ? amb_d | ~(ge | le) : amb_d;
     db0 = lane_of(ge) ? bm1 + 1 : bm1;
   }
   // scalar-load variant: the request is unconditional (past the last column it reads the record
@@ -1916,7 +1920,6 @@ DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *
   } else if (has_next) {
     load_rec<F>(next, 0, rn);
   }
-  amb = amb_d;
   const lanes_t db_ok = lanes_below(db0, nb);
   lanes_t vb_ok = ~0ull;
   float v = 0.f;
@@ -2567,7 +2570,7 @@ DEV void run_chunk_strip(const Params &P, const Slice &s, const Smem &m, const f
         }
       }
       const bool add = upper & !amb & db_ok;
-      const bool defer = upper & amb & (amb_d | db_ok);
+      const bool defer = upper & amb & (amb_d | db_ok) & (key == key);  // (a NaN distance is in no bin)
       if (add) {
         // one count for the pair (every field of the strip shares the bin); one sum per field
         const int h = ((db - 1) << m.lcop) + slot0;
@@ -3148,7 +3151,7 @@ static const void *pick_hist(int G, int D, bool J, bool mixed, int opk, bool sl,
 }
 
 static int opk_of(const Params &P) {
-  if (P.n1d > 0) return fused_opk(P.n1d);
+  if (P.n1d > 0) return fused_opk(P.nf);
   if (sp2d(P.op, P.n_val)) return 4;
   if (P.nmom > 1) return 3;
   if (P.op == 0 && P.nl == 1 && P.nt == 0) return 1;

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import _oracle
+from sfamd import _native
 from test_gpu_parity import MAG, TOL, check, field, gpu_hist
 
 pytestmark = pytest.mark.gpu
@@ -65,22 +66,62 @@ def test_masked_and_back(ctx, geometry):
     check(gs, gc, os_, oc, oa, TOL["fp64"], geometry, og=og, mag=16 * 2.0 ** -53 / 1e-4)
 
 
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("geometry", ["flat", "deg"])
 @pytest.mark.parametrize("kind,op,joint", [("rest", (0, 1, 0), True), ("nan", (0, 1, 0), True), ("nan", (0, 2, 0), False),
-                                           ("nowhere", (0, 1, 0), True), ("nowhere", (0, 2, 0), False)])
-def test_masked_time(ctx, geometry, kind, op, joint):
-    """Kernel time, binary64: at most three times that of the unmasked field (one by one: five to thirteen)."""
+                                           ("nowhere", (0, 1, 0), True), ("nowhere", (0, 2, 0), False),
+                                           ("nowhere", (1, 0, 0), False)])
+def test_masked_time(ctx, geometry, kind, op, joint, prec):
+    """Kernel time, binary64: at most three times that of the unmasked field (one by one: five to thirteen).
+    Binary32: no pair of a NaN position is queued for the re-bin."""
     x, u, edges = field(geometry, 2, 30000, 5)
     ve = AXES["even"] if joint else None
 
     def best(x, u):
         t = []
         for _ in range(4):
-            gpu_hist(ctx, x, u, edges, op, geometry=geometry, vedges=ve, prec="fp64")
+            gpu_hist(ctx, x, u, edges, op, geometry=geometry, vedges=ve, prec=prec)
             t.append(ctx.stats()["hist_ns"])
-        return min(t)
+        return min(t), ctx.stats()["rebinned"]
 
-    plain = best(x, u)
+    plain, queued = best(x, u)
     for share in (0.3, 1.0):
         xm, um = mask(x, u, kind, share, False, 1)
-        assert best(xm, um) <= 3 * plain
+        t, q = best(xm, um)
+        if prec == "fp64":
+            assert t <= 3 * plain
+        elif kind == "nowhere":
+            assert q <= queued
+
+
+@pytest.mark.parametrize("geometry,D", [("flat", 2), ("flat", 3), ("deg", 2)])
+@pytest.mark.parametrize("ops", [[(1, 0, 0)], [(0, 2, 0), (1, 0, 0)], [(1, 0, 0), (0, 0, 1), (0, 0, 3)], [(0, 0, 0)]])
+def test_masked_fused(ctx, geometry, D, ops):
+    """Fused outputs of a field with NaN positions of either sign, on axes with closed and open ends, with
+    outputs that take the distance and that do not."""
+    x, u, edges = field(geometry, D, 500, 41)
+    x, u = mask(x, u, "nowhere", 0.2, False, 1)
+    x[0, ::7] *= -1.0
+    x[0, 3::11] = -np.nan
+    axes = [edges, np.concatenate([edges, [np.inf]]), np.concatenate([[-np.inf, 0.0], edges, [np.inf]])]
+    for de in axes:
+        p = _native.SfProblem()
+        xc, uc = np.asfortranarray(x), np.asfortranarray(u)
+        p.D, p.W, p.N = uc.shape[0], xc.shape[0], 500
+        p.x, p.u = xc.ctypes.data, uc.ctypes.data
+        p.geometry, p.radius = _oracle.GEOM[geometry], 1.0
+        p.n_dist, p.dist_edges = len(de) - 1, de.ctypes.data
+        p.precision, p.count_bits = 1, 64
+        outs = []
+        for op in ops:
+            o = _native.SfOutput()
+            o.op, o.nl, o.nt = op
+            outs.append(o)
+        sums = [np.zeros(len(de) - 1) for _ in ops]
+        counts = [np.zeros(len(de) - 1, dtype=np.uint64) for _ in ops]
+        ctx.hist_multi([p], outs, sums, counts)
+        for k, op in enumerate(ops):
+            os_, oc, oa, og = _oracle.hist(x, u, de, op=op, geometry=geometry, nthreads=4, with_mag=True)
+            check(sums[k], counts[k], os_, oc, oa, TOL["mixed"], f"{geometry} {op}", og=og, mag=MAG["mixed"])
+            gs, gc = gpu_hist(ctx, x, u, de, op, geometry=geometry, prec="mixed")
+            check(gs.reshape(-1), gc.reshape(-1), os_, oc, oa, TOL["mixed"], f"{geometry} {op}", og=og, mag=MAG["mixed"])
