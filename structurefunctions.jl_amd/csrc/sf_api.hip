@@ -566,6 +566,19 @@ LinRule lin_rule_of(const sf_bin_rule *r) {
   return L;
 }
 
+// the kernels' lin_rule_bin
+int lin_rule_bin_host(const LinRule &r, double x, int nb) {
+  const double c = -r.f * r.inv;
+  const double t = std::fma(x, r.inv, c), n = (double)r.n;
+  const double fi = std::fmin(std::fmax(std::floor(t) + 1.0, 1.0), n);
+  int k = (int)fi + (std::fma(fi - 1.0, r.step, r.f) < x ? 1 : 0);
+  if (x <= r.f) k = 1;
+  if (x > r.l) k = (int)r.n + 1;
+  if (!r.padded) --k;
+  if (r.padded && x <= -INFINITY) k = 0;
+  return x != x ? nb + 1 : k;
+}
+
 void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   const int nE = p.n_dist + 1;
   const bool flat = p.geometry == SF_GEOM_FLAT;
@@ -813,6 +826,7 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   // value axis
   s.v_uniform = 0;
   s.v_negzero = 0;
+  s.vzero = kNoZeroBin;
   s.v0 = 0; s.vinv = 0; s.v0f = 0; s.vinvf = 0; s.vtc = 0; s.vslack = 0; s.vabs = 0; s.vslackt = 0; s.vtcu = 0; s.veps2 = 0;
   s.v_fx = 0; s.vwf = 0; s.vsf = 0; s.fxc1 = 0; s.fxc0 = 0; s.plane = 0; s.vsmall = 0; s.gz = 0;
   s.v_log = 0; s.vk0 = 0; s.vl0f = 0; s.vlinvf = 0;
@@ -820,6 +834,12 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
     const int nv = p.n_val;
     const double *E = p.val_edges;
     for (int k = 0; k <= nv; ++k) if (E[k] == 0.0 && signbit(E[k])) s.v_negzero++;
+    if (!s.v_negzero && !(p.op == SF_OP_PROJECTED && p.nl == 0 && p.nt == 0)) {
+      s.vzero = -1;
+      if (s.vrule.on) s.vzero += lin_rule_bin_host(s.vrule, 0.0, nv);
+      else
+        for (int k = 0; k <= nv; ++k) s.vzero += E[k] < 0.0;
+    }
     const double v0 = E[0], v1 = E[nv];
     if (v0 > -INFINITY && v1 < INFINITY && v1 > v0) {
       const long double w = ((long double)v1 - v0) / nv;
@@ -1303,6 +1323,8 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     Slice d = T.desc;
     d.N = sl[s].N;
     d.pt_off = prep[s].pt_off;
+    for (int k = 0; k < pl.n1d; ++k)  // (a fused output of another value than zero at rest)
+      if (multi->op[k] == SF_OP_PROJECTED && multi->nl[k] == 0 && multi->nt[k] == 0) d.vzero = kNoZeroBin;
     d.out_off = planes ? (int64_t)(s / kSpRows) * ncell + s % kSpRows : (int64_t)s * ncell;
     d.plane = planes ? s % kSpRows : 0;
     d.xerr = flat ? round_up_f(ldexpl((long double)xmax[s], -28)) : 0.0f;

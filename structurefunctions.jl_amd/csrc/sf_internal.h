@@ -54,6 +54,9 @@ struct LinRule {
   int32_t padded;          // InfPaddedBinEdges around the range
 };
 
+// Slice::vzero: no bin is known (an edge of -0.0 tells the zeros' signs apart, or some value is not zero)
+inline constexpr int kNoZeroBin = (int)0x80000000;
+
 struct Slice {
   LinRule drule;      // distance axis rule (flat point-field kernels: applied to sqrt(r^2))
   LinRule vrule;      // value axis rule
@@ -71,6 +74,7 @@ struct Slice {
   int32_t vedge_off;  // value edges, n_val + 1 doubles (and float copies at the same offset)
   int32_t v_uniform;  // value edges uniform enough for the guess-then-walk lookup
   int32_t v_negzero;  // count of -0.0 value edges (Julia isless places +0.0 above them)
+  int32_t vzero;      // 0-based value bin of a pair of equal velocities (value zero), or kNoZeroBin
   double v0, vinv;    // value guess t = (v - v0) * vinv
   float v0f, vinvf;   // binary32 value guess
   float vtc;          // -v0f * vinvf rounded to binary32: t = fmaf(v, vinvf, vtc)
