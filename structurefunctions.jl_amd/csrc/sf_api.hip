@@ -72,6 +72,7 @@ namespace {
 struct Arena {
   char *base = nullptr;
   size_t cap = 0, used = 0;
+  bool split = false;  // a call that did not fit, but would in parts (see plan_build)
 };
 
 template <typename T>
@@ -265,6 +266,7 @@ struct Plan {
   int n = 0, G = 0, D = 0, geom_code = 0, ncell = 0, S64 = 0, F32 = 0;
   int nout = 0;  // output slices (n is the internal slice count: six per slice for 2D single pass)
   bool J = false, mixed = false, sload = false, sp = false, fx = false;
+  bool rec_f = false;      // its binary64 kernel reads prep64s's records, which lie in rec32
   int block = 256, tj = 256, copies = 1, grid = 1, ncell_max = 1, n_items = 0;
   int strip = 0;            // B-strip launch (fields per strip), 0: off
   int qcap64 = 0;           // binary64 kernel: LDS queue entries per workgroup
@@ -1179,7 +1181,7 @@ struct MultiSpec {
 // Host work and uploads for one batch.  x/u of each slice are device pointers.
 int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const double *const *dx_in,
                const double *const *du_in, const double *xmax_in, hipStream_t st, bool cull,
-               const MultiSpec *multi = nullptr) {
+               const MultiSpec *multi = nullptr, bool wide = false) {
   // the single pass's 2D form runs every input slice as six plane slices (one joint histogram per
   // invariant, its own value edges); plane t of input slice s writes output cells t, t + 6, ...
   const bool planes = sp2d(sl_in[0].op, sl_in[0].n_val);
@@ -1278,9 +1280,10 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   }
   PLBUF(pl.rec64, ((size_t)pl.total_pts * S64 + 16));
   // + one record (F32 <= 16): the binary32 pair loop requests the record after its last column
-  // (sphere: the binary64 kernel's records, kF64Rec doubles per point, share the buffer)
+  // (sphere: the binary64 difference form's records, kF64Rec doubles per point, share the buffer)
   static_assert(kF64Rec * 2 == rec_f32(kSphere, 2) && kF64Rec * 2 == rec_f32(kSphere, 3), "record sizes");
-  if (mixed || G == kSphere) PLBUF(pl.rec32, ((size_t)pl.total_pts * F32 + 16));
+  const bool rec_f = pl.rec_f = G == kSphere && fast64(J, hist_opk_of(p0));
+  if (mixed || (rec_f && !pl.arena)) PLBUF(pl.rec32, ((size_t)pl.total_pts * F32 + 16));
 
   // ---- spatial sort and culling (binary32 kernel, one-shot calls): started here, so that the device
   // works on it while the tables are built
@@ -1525,7 +1528,8 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     const double large = std::min(std::max(cols / (16.0 * max_blocks), (double)block), 64.0 * block);
     const double small = sp2d(p0.op, p0.n_val) ? std::max(128.0, cols / (64.0 * max_blocks))
                                                : std::max(16.0, sqrt(cols) / 3.0);
-    const int jc = (int)std::min(large, small);
+    // (wide: as few items as there can be, where the allocation-free entry's scratch is short)
+    const int jc = wide ? 64 * block : (int)std::min(large, small);
     const int unit = jc >= block ? block : 16;
     jchunk = (jc + unit - 1) / unit * unit;
   }
@@ -1631,7 +1635,20 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     q.off = total;
     total = (total + q.bytes + 255) & ~(size_t)255;
   }
+  const size_t acells = (size_t)pl.nout * ncell;
+  pl.acc_bytes = 16 * acells + 4 * sizeof(unsigned long long) + 8 * sizeof(int);
+  if (pl.arena) {
+    // Calls that the allocation-free entry took when slices' descriptions were smaller and row tiles
+    // larger (at most a sixteenth of the scratch together) run in parts where they do not fit; and so
+    // do spherical binary64 ones whose second records (64 bytes a point) do not fit beside the rest.
+    const size_t need = ((pl.arena->used + 255) & ~(size_t)255) + total + ((pl.acc_bytes + 255) & ~(size_t)255) +
+                        (mixed ? 1024 * sizeof(Pending) : 0);
+    const size_t more = !mixed && rec_f ? ((size_t)pl.total_pts * F32 + 16) * sizeof(float) : 0;
+    pl.arena->split = need + more > pl.arena->cap && need <= pl.arena->cap + pl.arena->cap / 16;
+  }
   PLBUF(pl.tables, total);
+  PLBUF(pl.acc, pl.acc_bytes);
+  if (!mixed && rec_f && pl.arena) PLBUF(pl.rec32, ((size_t)pl.total_pts * F32 + 16));
   {
     // from page-locked memory, without waiting for it (the allocation-free entry keeps none)
     const bool pinned = !pl.arena && total <= kStageMax;
@@ -1650,9 +1667,6 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   char *tb = pl.tables.p;
   pl.prep = (const PrepSliceHost *)(tb + parts[6].off);
   pl.items64 = (const Item *)(tb + parts[7].off);
-  const size_t acells = (size_t)pl.nout * ncell;
-  pl.acc_bytes = 16 * acells + 4 * sizeof(unsigned long long) + 8 * sizeof(int);
-  PLBUF(pl.acc, pl.acc_bytes);
   pl.acc_s = (double *)pl.acc.p;
   pl.acc_c = (unsigned long long *)(pl.acc_s + acells);
   pl.pcount = pl.acc_c + acells;
@@ -1766,8 +1780,8 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
       zp[nz] = pl.mcounts.p;
       zb[nz++] = (int64_t)sizeof(unsigned long long) * mcells;
     }
-    HIPCHK(launch_prep(pl.G, pl.D, use_mixed, pl.geom_code, pl.prep, pl.n, pl.max_n, pl.rec64.p, pl.rec32.p, nz, zp, zb,
-                       st));
+    HIPCHK(launch_prep(pl.G, pl.D, use_mixed, pl.geom_code, pl.prep, pl.n, pl.max_n, pl.rec64.p,
+                       use_mixed || pl.rec_f ? pl.rec32.p : nullptr, nz, zp, zb, st));
   }
   const bool use_sload = use_mixed && pl.sload;
   const int stage = (use_sload || !use_mixed) ? 0 : pl.tj * pl.F32 * 4;
@@ -2286,8 +2300,8 @@ extern "C" int sf_hist_batch_device_noalloc(sf_ctx *ctx, int32_t n, const sf_pro
   if (n == 0) return SF_OK;
   if (!d_sums || !d_counts) return ctx->fail(SF_E_ARG, "null sums or counts");
   if (!ctx->scratch_ptr) return ctx->fail(SF_E_DEVICE, "the scratch array has no address on this device");
-  // the records alone must fit (checked before any device work; the tables, items, accumulators
-  // and queue are checked as the plan takes them)
+  // the records alone must fit in half of it (checked before any device work; the tables, items,
+  // accumulators, the queue and the binary64 difference form's own records as the plan takes them)
   int64_t pts = 0;
   for (int s = 0; s < n; ++s) pts += sl[s].N;
   const int G = sl[0].geometry == SF_GEOM_FLAT ? kFlat : kSphere;
@@ -2314,31 +2328,45 @@ extern "C" int sf_hist_batch_device_noalloc(sf_ctx *ctx, int32_t n, const sf_pro
                      "sf_hist_batch_device", n, (unsigned long long)(SF_NOALLOC_SCRATCH_BYTES >> 20));
   rc = coord_max(ctx, n, sl, st, 1.0, xmax, (double *)ctx->scratch_ptr);
   if (rc) return rc;
-  Plan &pl = ctx->noalloc;
-  Arena arena{ctx->scratch_ptr, (size_t)SF_NOALLOC_SCRATCH_BYTES, 0};
-  pl.arena = &arena;
-  // no culling: its sort workspace would be another buffer
-  rc = plan_build(ctx, pl, n, sl, px.data(), pu.data(), xmax.data(), st, false);
-  pl.arena = nullptr;
-  if (rc) return rc;
   for (int k = 0; k < 8; ++k) ctx->stats[k] = 0;
-  ctx->stats[0] = pl.total_pairs;
-  ctx->stats[2] = work_items(pl);
-  ctx->stats[3] = std::max(pl.n_items > 0 ? pl.grid : 0, pl.n_units > 0 ? pl.near_grid : 0);
-  ctx->stats[7] = pl.block;
   ctx->ev_pending = false;
-  if (pl.total_pairs == 0) return SF_OK;
-  unsigned long long *dc = (unsigned long long *)d_counts;
-  rc = plan_launch(pl, pl.mixed, d_sums, dc, st, nullptr);
-  if (rc) return rc;
-  if (pl.mixed) {
-    unsigned long long pc = 0;
-    HIPCHK(hipMemcpyAsync(&pc, pl.pcount, sizeof(pc), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    ctx->stats[1] = (int64_t)pc;
-    // the queue overflowed its share of the scratch: the merge was skipped, redo in binary64
-    if ((int64_t)pc > pl.cap) rc = plan_launch(pl, false, d_sums, dc, st, nullptr);
-  }
+  // slices a .. b - 1 in one launch; where they do not fit, in halves, one after the other on the stream
+  const int ncell = out_cells(sl[0]);
+  auto run = [&](auto &&self, int a, int b, bool wide) -> int {
+    Plan &pl = ctx->noalloc;
+    Arena arena{ctx->scratch_ptr, (size_t)SF_NOALLOC_SCRATCH_BYTES, 0};
+    pl.arena = &arena;
+    // no culling: its sort workspace would be another buffer
+    int rc = plan_build(ctx, pl, b - a, sl + a, px.data() + a, pu.data() + a, xmax.data() + a, st, false, nullptr, wide);
+    pl.arena = nullptr;
+    if (rc == SF_E_UNSUPPORTED && arena.split) {
+      if (b - a == 1) return wide ? rc : self(self, a, b, true);
+      const int m = a + (b - a) / 2;
+      rc = self(self, a, m, false);
+      return rc ? rc : self(self, m, b, false);
+    }
+    if (rc) return rc;
+    ctx->stats[0] += pl.total_pairs;
+    ctx->stats[2] += work_items(pl);
+    ctx->stats[3] = std::max<int64_t>(ctx->stats[3], pl.n_items > 0 ? pl.grid : 0);
+    ctx->stats[7] = pl.block;
+    if (pl.total_pairs == 0) return SF_OK;
+    double *ds = d_sums + (size_t)a * ncell;
+    unsigned long long *dc = (unsigned long long *)d_counts + (size_t)a * ncell;
+    rc = plan_launch(pl, pl.mixed, ds, dc, st, nullptr);
+    if (rc) return rc;
+    if (pl.mixed) {
+      unsigned long long pc = 0;
+      HIPCHK(hipMemcpyAsync(&pc, pl.pcount, sizeof(pc), hipMemcpyDeviceToHost, st));
+      HIPCHK(hipStreamSynchronize(st));
+      ctx->stats[1] += (int64_t)pc;
+      // the queue overflowed its share of the scratch: the merge was skipped, redo in binary64
+      if ((int64_t)pc > pl.cap) rc = plan_launch(pl, false, ds, dc, st, nullptr);
+    }
+    return rc;
+  };
+  rc = run(run, 0, n, false);
+  if (!rc) ctx->err.clear();
   return rc;
 }
 

@@ -31,6 +31,9 @@ inline constexpr __host__ __device__ int rec_f32(int G, int D) { return (G == kF
 inline constexpr __host__ __device__ int rec_id(int G, int D) { return (G == kFlat) ? 4 * D + 1 : 15; }
 //   binary64 kernel, sphere (pair64f): P0 P1 P2 2 U0 2 U1 2 U2 ur {2^-12 |u|, id}  (8 doubles)
 inline constexpr int kF64Rec = 8;
+// the binary64 launches that take the difference form (pair64f): every 1D operator and the single
+// pass, and the joint du_L and du_L^2; the other joint operators keep the reference's sequence
+inline constexpr bool fast64(bool J, int opk) { return !J || opk == 1 || opk == 2; }
 template <int G, int D> struct Rec {
   static constexpr int d64 = rec_d64(G, D);
   static constexpr int f32 = rec_f32(G, D);

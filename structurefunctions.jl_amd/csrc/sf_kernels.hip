@@ -1015,9 +1015,6 @@ DEV Row item_row(const Item &w, const Slice &s) {
 // margin of a value decision point, by the exact rules.  Flat keys that are not above 2^-100
 // (coincident points, NaN) also take the exact rules.  A pair that is not counted updates the
 // lane's scratch slot.
-// the binary64 launches that take the difference form (pair64f): every 1D operator and the single
-// pass, and the joint du_L and du_L^2; the other joint operators keep the reference's sequence
-inline constexpr bool fast64(bool J, int opk) { return !J || opk == 1 || opk == 2; }
 // doubles per point of the records it reads: the flat binary64 records, or prep64s's
 template <int G, int D>
 inline constexpr int rec_pair64 = (G == kFlat) ? Rec<G, D>::d64 : kF64Rec;
