@@ -45,7 +45,8 @@ hipError_t launch_eval_math(int fn, int64_t n, const double *a, const double *b,
 size_t cull_workspace_bytes(int64_t N);
 hipError_t launch_cull(const double *x, int64_t N, int W, int D, int geom, double reach, int bits, void *ws,
                        int32_t *perm, double *info, float *gbox, hipStream_t st);
-hipError_t launch_cull_units(const float *gbox, int64_t N, double *info, double reach, int slice, Item *units,
+hipError_t launch_cull_count(const float *gbox, int64_t N, double *info, double reach, int K, hipStream_t st);
+hipError_t launch_cull_units(const float *gbox, int64_t N, double *info, double reach, int K, int slice, Item *units,
                              int64_t n, hipStream_t st);
 int hist_occupancy(int G, int D, bool J, bool mixed, int opk, bool sload, bool fx, int block,
                    size_t smem);
@@ -1087,6 +1088,7 @@ struct CullInfo {
   bool tried = false, active = false;
   double reach = 0;       // largest counted distance in key-space units
   int64_t units = 0;
+  int rstep = 1;          // row blocks of 64 rstep records
 };
 
 // Starts the spatial order, group boxes and number of work units of one slice on the device
@@ -1123,21 +1125,50 @@ int cull_start(sf_ctx *ctx, const sf_problem &p, const double *dx, double xmax, 
   return SF_OK;
 }
 
-// ci.active: whether culling is worth it, from launch_cull's info
-void cull_decide(const sf_problem &p, const double *info, int rows, CullInfo &ci) {
+// Whether culling may be worth it, from launch_cull's info, and whether the units of wide row blocks are
+// to be counted (ci.rstep).  Joint histograms of points on a surface: rows that lie side by side in the
+// spatial order send many lanes to one cell where the reach holds thousands of points, and LDS atomics to one
+// address serialize.  The waves of a block of 1024 rows take rows 16 apart; but the block's box is larger,
+// and more columns are in its reach.  (1D histograms have copies for that.  In space, points as close have
+// boxes that much wider: blocks of 1024 rows took 1.4 to 2.0 times as long at N = 65536.)
+void cull_rows(const sf_problem &p, bool J, const double *info, int rows, CullInfo &ci) {
   if (!ci.tried || p.N < 4 * (int64_t)rows) return;
   if (info[6] != 0.0) return;  // non-finite coordinates: no culling
   // worth it only if the reach is small against the extent
   double ext = 0;
   for (int k = 0; k < 3; ++k) ext = std::max(ext, info[3 + k] - info[k]);
   if (!(info[9] < 0.5 * ext)) return;
-  // ... and units leave out half of the pairs at least: a full unit is 64 x 64 pairs, and whole row
-  // tiles over long column ranges take less per pair
   uint64_t units;
   memcpy(&units, &info[8], sizeof units);
-  if ((double)units * 4096.0 > 0.5 * (double)pairs_of(p.N) || units > (uint64_t)(1 << 30)) return;
   ci.active = true;
-  ci.units = (int64_t)units;
+  ci.units = (int64_t)std::min<uint64_t>(units, 1ull << 31);
+  // (from 4096 columns in reach of a row block on: below, wide blocks do not pay, and counting them would)
+  if (J && p.W == 2 && ci.units > p.N) ci.rstep = kWideRows;
+}
+
+// The row blocks (launch_cull_count's number against launch_cull's), and whether the units leave out
+// enough: most of their pairs are counted, which makes them slower than the pairs of whole tiles.  Measured
+// (flat 2D, 3D, sphere; N = 16384 to 262144; reaches of 0.5 to 35 % of the domain):
+//   wide blocks pay up to 1.5 (fixed-point cells) or 2.0 (binary64 cells) times the units of narrow ones
+//   share of all pairs at which units and whole tiles take as long: 1D 0.75; joint, narrow blocks, 0.4 .. 0.55
+//   (fixed point) and 0.25 .. 0.4 (binary64 cells), in space 0.8; wide blocks 0.63 .. 0.8 (fixed point), and
+//   for binary64 cells from 0.37 at 1.17 times the narrow units over 0.45 (1.35) to 0.7 (2.0)
+// Joint du_L, flat 2D, N = 200000, 40 x 64 bins, binary64 cells, ms, narrow / wide / whole tiles: reach 10 %
+// 6.7 / 5.2 / 19.4, 20 % 22.5 / 14.8 / 19.6, 35 % 54.7 / 34.2 / 20.5; fixed point, 25 %: 15.5 / 11.5 / 18.4.
+void cull_decide(const sf_problem &p, bool J, bool fx, const double *info, CullInfo &ci) {
+  double most = !J ? 0.75 : (p.W == 3 ? 0.75 : (fx ? 0.5 : 0.33));
+  if (ci.rstep > 1) {
+    uint64_t units;
+    memcpy(&units, &info[11], sizeof units);
+    const double times = (double)units / (double)std::max<int64_t>(ci.units, 1);
+    if (times <= (fx ? 1.5 : 2.0)) {
+      ci.units = (int64_t)std::min<uint64_t>(units, 1ull << 31);
+      most = fx ? 0.65 : 0.35 + 0.42 * (times - 1.15);
+    } else {
+      ci.rstep = 1;
+    }
+  }
+  if ((double)ci.units * 4096.0 > most * (double)pairs_of(p.N) || ci.units > (1 << 30)) ci.active = false;
 }
 
 // Stride of the binary32 record order: record k holds point (k * mul) mod N.  Points that the
@@ -1545,11 +1576,25 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     std::vector<double> own(pinned ? 0 : (size_t)n * kCullInfo);
     if (pinned) HIPCHK(ctx->down.acquire(bytes));
     double *info = pinned ? (double *)ctx->down.p : own.data();
-    HIPCHK(hipMemcpyAsync(info, ctx->cull_info.p, bytes, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    auto read = [&]() -> int {
+      HIPCHK(hipMemcpyAsync(info, ctx->cull_info.p, bytes, hipMemcpyDeviceToHost, st));
+      HIPCHK(hipStreamSynchronize(st));
+      return SF_OK;
+    };
+    int rc = read();
+    if (rc) return rc;
+    bool again = false;
+    for (int s = 0; s < n; ++s) {
+      cull_rows(sl[s], J, info + (size_t)s * kCullInfo, block, cinfo[s]);
+      if (!cinfo[s].active || cinfo[s].rstep == 1) continue;
+      HIPCHK(launch_cull_count(pl.gboxes.p + (size_t)grp[s] * 6, sl[s].N, ctx->cull_info.p + (size_t)s * kCullInfo,
+                               cinfo[s].reach, cinfo[s].rstep, st));
+      again = true;
+    }
+    if (again && (rc = read())) return rc;
     int64_t units = 0;
     for (int s = 0; s < n; ++s) {
-      cull_decide(sl[s], info + (size_t)s * kCullInfo, block, cinfo[s]);
+      if (cinfo[s].active) cull_decide(sl[s], J, pl.fx, info + (size_t)s * kCullInfo, cinfo[s]);
       if (units + cinfo[s].units > (1LL << 30)) cinfo[s].active = false;
       if (!cinfo[s].active) continue;
       units += cinfo[s].units;
@@ -1563,7 +1608,7 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
       for (int s = 0; s < n; ++s) {
         if (!cinfo[s].active || cinfo[s].units == 0) continue;
         HIPCHK(launch_cull_units(pl.gboxes.p + (size_t)grp[s] * 6, sl[s].N, ctx->cull_info.p + (size_t)s * kCullInfo,
-                                 cinfo[s].reach, s, pl.units.p + units, cinfo[s].units, st));
+                                 cinfo[s].reach, cinfo[s].rstep, s, pl.units.p + units, cinfo[s].units, st));
         units += cinfo[s].units;
       }
     }

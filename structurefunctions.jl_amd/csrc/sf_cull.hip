@@ -11,7 +11,7 @@
 //   sort_*        stable radix sort of the keys, carrying point indices: the record order
 //   cull_groups   the bounding box of every group of kGroup consecutive records
 //   cull_units    the work units: a wave's 64 rows and one or two column groups within reach
-// The host reads back the slice box and the number of units (80 bytes).
+// The host reads back the slice box and the number of units (kCullInfo words).
 #include <hip/hip_runtime.h>
 
 #include "sf_internal.h"
@@ -291,8 +291,9 @@ __global__ void __launch_bounds__(kCullBlock) cull_groups(const double *kc, cons
     }
 }
 
-// Work units of a slice: row block rb (64 records) with the pair of column groups (64 records) at
-// j0, as far as their boxes are in reach and some column lies above some row.  One wave per row
+// Work units of a slice: row block rb (64 K records) with the pair of column groups (64 records) at
+// j0, as far as their boxes are in reach and some column lies above some row.  The K waves of a row block
+// take its rows K apart (unit k: rows rb 64 K + k + K lane).  One wave per row
 // block and kUnitSpan runs of 64 groups, one group per lane.  The boxes are rounded outwards to
 // binary32 and the limit carries a margin, so no counted pair is lost.  WRITE false: their number is
 // added to *count and the squared limit goes to *lim (both in the slice's info); true: they are
@@ -302,7 +303,7 @@ __global__ void __launch_bounds__(kCullBlock) cull_groups(const double *kc, cons
 constexpr int kUnitSpan = 16;
 template <bool WRITE>
 __global__ void __launch_bounds__(kCullBlock) cull_units(const float *gbox, int64_t N, const double *info,
-                                                         double reach, int slice, Item *units,
+                                                         double reach, int K, int slice, Item *units,
                                                          unsigned long long cap, unsigned long long *count,
                                                          double *lim) {
   constexpr int W = kCullBlock / 64;
@@ -314,32 +315,41 @@ __global__ void __launch_bounds__(kCullBlock) cull_units(const float *gbox, int6
   // coordinates of the slice's magnitude, and the rounding of three binary32 squares and their sum
   const double l = reach * (1.0 + 1e-6) + 1e-13 * fmax(1.0, info[7]);
   const float lim2 = __double2float_ru(l * l * (1.0 + 1e-5) + 1e-30);
-  if (!WRITE && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *lim = l;
+  if (!WRITE && lim && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *lim = l;
   const int64_t rb = (int64_t)blockIdx.x * W + w;
   const int64_t last = (N - 1) / kGroup;
   unsigned mine = 0;
-  if (rb * 64 < N) {
-    const float *a0 = gbox + 6 * (2 * rb), *a1 = gbox + 6 * (2 * rb + 1 < last ? 2 * rb + 1 : last);
+  const int64_t g0 = 2 * K * rb;  // first group of the row block
+  if (rb * 64 * K < N) {
     float lo[3], hi[3];
-    for (int k = 0; k < 3; ++k) {
-      lo[k] = fminf(a0[k], a1[k]);
-      hi[k] = fmaxf(a0[3 + k], a1[3 + k]);
+    {
+      const int64_t ga = g0 + (lane & (2 * K - 1));
+      const float *a = gbox + 6 * (ga < last ? ga : last);
+      for (int k = 0; k < 3; ++k) {
+        lo[k] = a[k];
+        hi[k] = a[3 + k];
+      }
     }
+    for (int o = K; o > 0; o >>= 1)
+      for (int k = 0; k < 3; ++k) {
+        lo[k] = fminf(lo[k], __shfl_xor(lo[k], o));
+        hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], o));
+      }
 #pragma unroll 4  // (loads of several runs in flight)
     for (int t = 0; t < kUnitSpan; ++t) {
       const int64_t g = ((int64_t)blockIdx.y * kUnitSpan + t) * 64 + lane;
       unsigned long long m = 0ull;
-      if ((g | 63) >= 2 * rb && (g & ~63ll) <= last) {  // (the same for the whole wave)
+      if ((g | 63) >= g0 && (g & ~63ll) <= last) {  // (the same for the whole wave)
         const float *b = gbox + 6 * (g < last ? g : last);
         float d2 = 0.f;
         for (int k = 0; k < 3; ++k) {
           const float gap = fmaxf(0.f, fmaxf(b[k] - hi[k], lo[k] - b[3 + k]));
           d2 = __builtin_fmaf(gap, gap, d2);
         }
-        m = __ballot(g <= last && g >= 2 * rb && d2 <= lim2);
+        m = __ballot(g <= last && g >= g0 && d2 <= lim2);
       }
       if (lane == 0) masks[w][t] = m;
-      mine += (unsigned)__popcll((m | (m >> 1)) & 0x5555555555555555ull);
+      mine += (unsigned)K * (unsigned)__popcll((m | (m >> 1)) & 0x5555555555555555ull);
     }
   } else if (lane < kUnitSpan) {
     masks[w][lane] = 0ull;
@@ -359,19 +369,22 @@ __global__ void __launch_bounds__(kCullBlock) cull_units(const float *gbox, int6
       const unsigned long long m = masks[w][t];
       const unsigned long long pairs = (m | (m >> 1)) & 0x5555555555555555ull;
       if ((pairs >> lane) & 1ull) {
-        const unsigned long long k = o + (unsigned)__popcll(pairs & ((1ull << lane) - 1ull));
+        const unsigned long long k = o + (unsigned)K * (unsigned)__popcll(pairs & ((1ull << lane) - 1ull));
         const int64_t g = ((int64_t)blockIdx.y * kUnitSpan + t) * 64 + lane;
         const int64_t j0 = (g + ((m >> lane) & 1ull ? 0 : 1)) * kGroup;
         const int64_t j1 = (g + ((m >> lane) & 2ull ? 2 : 1)) * kGroup;
-        if (k < cap) units[k] = Item{slice, (int32_t)(rb * 64), (int32_t)j0, (int32_t)(j1 < N ? j1 : N)};
+        for (int r = 0; r < K; ++r)
+          if (k + r < cap)
+            units[k + r] = Item{slice, (int32_t)(rb * 64 * K + r) | (K > 1 ? kWideUnit : 0), (int32_t)j0,
+                                (int32_t)(j1 < N ? j1 : N)};
       }
-      o += (unsigned)__popcll(pairs);
+      o += (unsigned)K * (unsigned)__popcll(pairs);
     }
   }
 }
 
-dim3 unit_grid(int64_t N) {
-  const int64_t rows = (N + 63) / 64, groups = (N + kGroup - 1) / kGroup;
+dim3 unit_grid(int64_t N, int K) {
+  const int64_t rows = (N + 64 * K - 1) / (64 * K), groups = (N + kGroup - 1) / kGroup;
   return dim3((unsigned)((rows + kCullBlock / 64 - 1) / (kCullBlock / 64)),
               (unsigned)((groups + 64 * kUnitSpan - 1) / (64 * kUnitSpan)));
 }
@@ -438,13 +451,13 @@ size_t cull_workspace_bytes(int64_t N) {
 // x: the slice's positions (device, point-major, W per point); geom 0 flat, 1 sphere in degrees,
 // 2 sphere in radians; bits: of the Morton key per axis, 8 or 10.  Writes the record order to perm (N
 // entries), to gbox one box per kGroup records (6 floats each), and to info (kCullInfo words) the slice
-// box (8 doubles: lo[3], hi[3], non-finite count, largest |coordinate|), the number of work units
-// within `reach` (an unsigned 64-bit integer), the distance beyond which they were left out, and a
-// zero for launch_cull_units.  ws: cull_workspace_bytes(N) bytes of device memory.
+// box (8 doubles: lo[3], hi[3], non-finite count, largest |coordinate|), the number of work units of row
+// blocks of 64 within `reach` (an unsigned 64-bit integer), the distance beyond which they were left out,
+// and zeros for launch_cull_units and launch_cull_count.  ws: cull_workspace_bytes(N) bytes of device memory.
 hipError_t launch_cull(const double *x, int64_t N, int W, int D, int geom, double reach, int bits, void *ws,
                        int32_t *perm, double *info, float *gbox, hipStream_t st) {
   static_assert(kGroup == 32, "cull_groups reduces over half waves, cull_units takes two groups to 64 rows");
-  if (N < 1 || N > (1LL << 30) || (bits != 8 && bits != 10)) return hipErrorInvalidValue;
+  if (N < 1 || N > kWideUnit || (bits != 8 && bits != 10)) return hipErrorInvalidValue;
   CullWs w;
   cull_ws_layout(N, (char *)ws, w);
   const int nblk = (int)((N + kCullBlock - 1) / kCullBlock);
@@ -468,17 +481,26 @@ hipError_t launch_cull(const double *x, int64_t N, int W, int D, int geom, doubl
   hipLaunchKernelGGL(cull_groups, dim3(nblk), dim3(kCullBlock), 0, st, (const double *)w.kc,
                      (const int32_t *)perm, N, gbox);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(cull_units<false>, unit_grid(N), dim3(kCullBlock), 0, st, (const float *)gbox, N,
-                     (const double *)info, reach, 0, (Item *)nullptr, 0ull, (unsigned long long *)(info + 8),
+  hipLaunchKernelGGL(cull_units<false>, unit_grid(N, 1), dim3(kCullBlock), 0, st, (const float *)gbox, N,
+                     (const double *)info, reach, 1, 0, (Item *)nullptr, 0ull, (unsigned long long *)(info + 8),
                      info + 9);
   return hipGetLastError();
 }
 
-// Writes the slice's n work units (their number and the slice's info from launch_cull) to units.
-hipError_t launch_cull_units(const float *gbox, int64_t N, double *info, double reach, int slice, Item *units,
+// Counts the work units of row blocks of 64 K records (K: kWideRows) into info word 11.
+hipError_t launch_cull_count(const float *gbox, int64_t N, double *info, double reach, int K, hipStream_t st) {
+  static_assert(kWideRows > 1 && kWideRows <= 32 && (kWideRows & (kWideRows - 1)) == 0, "a wave reduces 2 K boxes");
+  hipLaunchKernelGGL(cull_units<false>, unit_grid(N, K), dim3(kCullBlock), 0, st, gbox, N, (const double *)info, reach,
+                     K, 0, (Item *)nullptr, 0ull, (unsigned long long *)(info + 11), (double *)nullptr);
+  return hipGetLastError();
+}
+
+// Writes the slice's n work units (their number and the slice's info from launch_cull, or
+// launch_cull_count) to units.
+hipError_t launch_cull_units(const float *gbox, int64_t N, double *info, double reach, int K, int slice, Item *units,
                              int64_t n, hipStream_t st) {
-  hipLaunchKernelGGL(cull_units<true>, unit_grid(N), dim3(kCullBlock), 0, st, gbox, N, (const double *)info, reach,
-                     slice, units, (unsigned long long)n, (unsigned long long *)(info + 10), (double *)nullptr);
+  hipLaunchKernelGGL(cull_units<true>, unit_grid(N, K), dim3(kCullBlock), 0, st, gbox, N, (const double *)info, reach,
+                     K, slice, units, (unsigned long long)n, (unsigned long long *)(info + 10), (double *)nullptr);
   return hipGetLastError();
 }
 

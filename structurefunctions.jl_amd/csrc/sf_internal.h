@@ -112,7 +112,10 @@ struct Item {
   int32_t i0;       // first row of the i-tile
   int32_t j0, j1;   // column range [j0, j1), j0 >= i0
 };
-// (a culled slice's work unit is an Item of one wave: 64 rows from i0 on, at most 64 columns)
+// A culled slice's work unit is an Item of one wave: 64 rows and at most 64 columns.  The rows lie side by side
+// from i0 on; where kWideUnit is set in i0 (a culled slice has fewer points), kWideRows apart.
+inline constexpr int kWideRows = 16;
+inline constexpr int32_t kWideUnit = 1 << 30;
 
 struct Pending {      // a pair the binary32 kernel could not bin with certainty (binary32 record indices)
   int32_t slice, i, j;
@@ -258,7 +261,7 @@ inline constexpr int kCell32Max = 1024;
 // records per box of a culled slice (its work units hold one or two such groups of columns)
 inline constexpr int kGroup = 32;
 // words (8 bytes) of a slice's culling information: see launch_cull
-inline constexpr int kCullInfo = 11;
+inline constexpr int kCullInfo = 12;
 // largest re-bin queue staged in LDS per workgroup (entries, split evenly between its waves);
 // the host shrinks it where the LDS it takes would cost a workgroup per CU
 inline constexpr int kQueueCap = 8192;

@@ -1288,11 +1288,11 @@ DEV bool near_value_edge(double v, const double *E, int nE, int g) {
 inline constexpr int kManyRare = 48, kManyCols = 4096;
 
 // MANY (with MASK): the form for fields with masked points; only the pairs of the lanes in `want` are
-// evaluated.  Returns the lanes whose pair is left to the reference's
+// evaluated, and zb is the slice's vzero.  Returns the lanes whose pair is left to the reference's
 // sequence.
 template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR, bool MANY>
 DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double *A, int i, int j,
-                 const double *B, double *rn, const double *next, Pending64 &pa, lanes_t want) {
+                 const double *B, double *rn, const double *next, Pending64 &pa, lanes_t want, int zb) {
   constexpr int S = rec_pair64<G, D>;
   constexpr int W = (G == kFlat) ? D : 3;  // space the differences live in
   constexpr int UO = (G == kFlat) ? D : 3; // first velocity word of a record
@@ -1391,8 +1391,8 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
       rare_v |= __builtin_amdgcn_ballot_w64(near_value_edge(v, m.vE, P.n_val + 1, vb0));
     }
     if constexpr (MANY) {
-      zero = s.vzero == kNoZeroBin ? 0ull : zero;
-      vb0 = lane_of(zero) ? s.vzero : vb0;
+      zero = zb == kNoZeroBin ? 0ull : zero;
+      vb0 = lane_of(zero) ? zb : vb0;
       rare_v &= ~(zero | nan);
     }
   } else {
@@ -1495,7 +1495,7 @@ DEV void rare64(const Params &P, const Slice &s, const Smem &m, const double *re
 // (a call with other bits than all ones holds one group).
 template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR, bool MANY>
 DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j, int j1,
-                    const double *__restrict__ rec, unsigned &dm_out, int &jl, unsigned want) {
+                    const double *__restrict__ rec, unsigned &dm_out, int &jl, unsigned want, int slice_id) {
   constexpr int S = rec_pair64<G, D>;
   // the slice offset is wave-uniform by construction; say so, so that the column addresses stay in
   // SGPRs
@@ -1506,6 +1506,8 @@ DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double
   double ra[S], rb[S];
   load_rec64<S>(cp, ra);
   Pending64 pa{m.scr, 0.0, 0.0};
+  int zb = kNoZeroBin;
+  if constexpr (MANY && J) zb = P.slices[slice_id].vzero;
   unsigned dm = 0u;
   while (j < j1) {
     const int je = min(j1, j + 32);
@@ -1516,7 +1518,7 @@ DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double
         wl = __builtin_amdgcn_ballot_w64((int)wb < 0);
         wb += wb;
       }
-      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU, MIR, MANY>(P, s, m, ri, i, jc, B, rn, next, pa, wl));
+      dm = shift_flag(dm, pair64f<G, D, J, OPK, MASK, VU, MIR, MANY>(P, s, m, ri, i, jc, B, rn, next, pa, wl, zb));
     };
     dm = 0u;
     for (; j + 1 < je; j += 2, cp += 2 * S) {
@@ -1542,11 +1544,11 @@ DEV int run_cols64f(const Params &P, const Slice &s, const Smem &m, const double
 // the key table's form and the form of the pair (many) are chosen per column range, not per pair
 template <int G, int D, bool J, int OPK>
 DEV int run_range64f(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j, int je, bool mask,
-                     bool many, unsigned want, const double *__restrict__ rec, unsigned &dm, int &jl) {
+                     bool many, unsigned want, const double *__restrict__ rec, unsigned &dm, int &jl, int slice_id) {
   auto run = [&](auto vu, auto mir) {
-    if (many) return run_cols64f<G, D, J, OPK, true, vu.value, mir.value, true>(P, s, m, ri, i, j, je, rec, dm, jl, want);
-    return mask ? run_cols64f<G, D, J, OPK, true, vu.value, mir.value, false>(P, s, m, ri, i, j, je, rec, dm, jl, ~0u)
-                : run_cols64f<G, D, J, OPK, false, vu.value, mir.value, false>(P, s, m, ri, i, j, je, rec, dm, jl, ~0u);
+    if (many) return run_cols64f<G, D, J, OPK, true, vu.value, mir.value, true>(P, s, m, ri, i, j, je, rec, dm, jl, want, slice_id);
+    return mask ? run_cols64f<G, D, J, OPK, true, vu.value, mir.value, false>(P, s, m, ri, i, j, je, rec, dm, jl, ~0u, slice_id)
+                : run_cols64f<G, D, J, OPK, false, vu.value, mir.value, false>(P, s, m, ri, i, j, je, rec, dm, jl, ~0u, slice_id);
   };
   auto run_vu = [&](auto mir) {
     return (J && s.v_uniform) ? run(std::integral_constant<bool, J>(), mir) : run(std::false_type(), mir);
@@ -1608,7 +1610,7 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
           const bool mask = j < row.jm;
           int je = mask ? row.jm : w.j1;
           if (many > 0) je = min(je, j + many);
-          const int jn = run_range64f<G, D, J, OPK>(P, s, m, ri, row.i, j, je, mask, many > 0, ~0u, rec, dm, jl);
+          const int jn = run_range64f<G, D, J, OPK>(P, s, m, ri, row.i, j, je, mask, many > 0, ~0u, rec, dm, jl, cur);
           if (__ballot(dm != 0u)) {
             unsigned tot = 0u;
             if (many <= 0) (void)wave_prefix((unsigned)__popc(dm), &tot);
@@ -1616,7 +1618,7 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
               many = kManyCols;
               const unsigned want = dm;
               (void)run_range64f<G, D, J, OPK>(P, s, m, ri, row.i, j + ((jl - j) & ~31), jl + 1, true, true, want, rec,
-                                               dm, jl);
+                                               dm, jl, cur);
             }
             rare64<G, D, J, OPK>(P, s, m, rec, dm, row.i, jl);
           }
@@ -2219,18 +2221,20 @@ DEV void queue_wave_flush(const Params &P, const Smem &m, int slice_id, int fiel
 
 // Joint histograms: of the pairs (i, jl - t) whose bits t are set in dm, those of two points at rest.  Their
 // value is zero, which lies on a value edge as often as not, so that masked fields (land, resting water)
-// queued a share of all pairs; but its bin is known (s.vzero).  Counts them and returns the bits of the
+// queued a share of all pairs; but its bin is known (Slice::vzero).  Counts them and returns the bits of the
 // others, and of those whose key is uncertain.  cl: record of column jl.  Joint du_L, sphere, N = 60000, 64 x
 // 64 bins, 30 % of the points at rest: 17.1 ms with their pairs queued, 3.2 now (none at rest: 2.8); fixed point
 // 17.0 and 3.0. The headline call, without such points, takes 0.5 % longer for the test of its queued pairs.
 template <int G, int D, int OPK, bool FX>
 DEV unsigned rest_pairs(const Params &P, const Slice &s, const Smem &m, const float *ri, unsigned dm,
-                        const float4 *cl) {
+                        const float4 *cl, int slice_id) {
   constexpr int F = Rec<G, D>::f32;
   constexpr int NI = (G == kFlat) ? 4 * D : 12;  // the norm's bound: zero at rest only
   constexpr int W = (G == kFlat) ? D : 3;
   const unsigned todo = ri[NI] == 0.f ? dm : 0u;
-  if (__ballot(todo != 0u) == 0ull || s.vzero == kNoZeroBin) return dm;
+  if (__ballot(todo != 0u) == 0ull) return dm;
+  const int vzero = P.slices[slice_id].vzero;  // (read here: not held over the pair loops)
+  if (vzero == kNoZeroBin) return dm;
   for (int t = 0; t < 32; ++t) {
     const bool mine = (todo >> t) & 1u;
     if (__ballot(mine) == 0ull) continue;
@@ -2251,9 +2255,9 @@ DEV unsigned rest_pairs(const Params &P, const Slice &s, const Smem &m, const fl
     const int db0 = ge ? m.blo[c].y + 1 : m.blo[c].y;
     if (!(ge | le) || (unsigned)db0 >= (unsigned)P.n_dist) continue;  // (a NaN distance is in no bin)
     if constexpr (OPK >= 9) atomicAdd(&m.mc[(db0 << m.lmcop) + (int)(__lane_id() & (m.mcop - 1))], 1u);
-    if ((unsigned)s.vzero >= (unsigned)P.n_val) continue;
-    if constexpr (FX) atomicAdd(&m.zc[db0 * kZeroBins + min(max(s.vzero - s.gz, 0), kZeroBins - 1)], 1u);
-    else atomicAdd(&m.hc[s.vzero * m.jv + db0 * m.jd + m.coff], 1u);
+    if ((unsigned)vzero >= (unsigned)P.n_val) continue;
+    if constexpr (FX) atomicAdd(&m.zc[db0 * kZeroBins + min(max(vzero - s.gz, 0), kZeroBins - 1)], 1u);
+    else atomicAdd(&m.hc[vzero * m.jv + db0 * m.jd + m.coff], 1u);
   }
   return dm;
 }
@@ -2287,7 +2291,7 @@ DEV void run_chunk32_vu(const Params &P, const Slice &s, const Smem &m, const fl
       dm = shift_flag(dm, pair32<G, D, J, OPK, MASK, FX, VU, SL>(P, s, m, ri, i, j, ra, rb, cp + R, false, pa, sa));
       ++j;
     }
-    if constexpr (J) dm = rest_pairs<G, D, OPK, FX>(P, s, m, ri, dm, col + (int64_t)(je - 1 - col_j0) * R);
+    if constexpr (J) dm = rest_pairs<G, D, OPK, FX>(P, s, m, ri, dm, col + (int64_t)(je - 1 - col_j0) * R, slice_id);
     queue_deferred(P, m, dm, i, je - 1, slice_id, 0, -1);
   }
   if constexpr (FX) {
@@ -2451,12 +2455,15 @@ __global__ void __launch_bounds__(1024, FX ? 6 : 1) hist32n(Params P, const floa
     while (have && w.slice == cur) {
       cols += w.j1 - w.j0;
       if (cols > budget) break;
-      const int i = w.i0 + lane;
+      // rows of the unit's block: side by side, or kWideRows apart in a block of as many times 64
+      const int step = w.i0 & kWideUnit ? kWideRows : 1, i0 = w.i0 & ~kWideUnit;
+      const int i = i0 + lane * step;
+      const int end = (i0 & -64 * step) + 64 * step;  // of the block
       Row row;
       row.i = i < s.N ? i : kNoRow;
       row.any = true;
       row.rec = i < s.N ? i : (int)(s.N - 1);
-      row.jm = w.i0 + 64 <= __builtin_amdgcn_readfirstlane((int)s.N) ? min(w.j1, w.i0 + 64) : w.j1;
+      row.jm = end <= __builtin_amdgcn_readfirstlane((int)s.N) ? min(w.j1, end) : w.j1;
       float ri[F];
 #pragma unroll
       for (int k = 0; k < F; ++k) ri[k] = rec[(s.pt_off + row.rec) * F + k];
