@@ -31,8 +31,6 @@ hipError_t launch_prep(int G, int D, bool mixed, int geom_code, const void *prep
 hipError_t launch_hist(int G, int D, bool J, bool mixed, bool sload, bool near, const Params &P, int grid,
                        int block, size_t smem, hipStream_t st);
 hipError_t launch_recheck(int G, int D, bool J, const Params &P, int grid, hipStream_t st);
-hipError_t launch_merge(const double *src_s, const unsigned long long *src_c, double *dst_s,
-                        unsigned long long *dst_c, int64_t n, hipStream_t st);
 hipError_t launch_merge_checked(const double *src_s, const unsigned long long *src_c, double *dst_s,
                                 unsigned long long *dst_c, int64_t n,
                                 const unsigned long long *pcount, int64_t cap, int *flag,

@@ -283,13 +283,6 @@ DEV int val_bin64(double v, const double *E, int nE, const Slice &s) {
   return g;
 }
 
-// Full exact evaluation of pair (i, j) of slice s from binary64 records.  Returns the output cell
-// (0-based within the slice) or -1 if the pair is not counted; writes the value.  OPK fixes the
-// operator at compile time (1: {1,0}, 2: {2,0}) with the same operation sequence as the generic
-// functor; 0 dispatches on P.op at run time; 3 is the single pass, which writes du_L to val[0] and
-// |du|^2 to val[1] (flat: _pf_sp_simd_pairs!, serial_single_pass.jl:245-253, du_L =
-// dot(du, dx) * inv(sqrt(r2)); sphere: _sp1d_pairs!, :333-338, du_L = dot(du, e1)); 4 is a plane
-// of the single pass's 2D form: the same du_L and |du|^2, then invariant s.plane as value.
 // Invariant t of the single pass's 2D form from du_L and |du|^2, in the reference's operation
 // order (_sp2d_simd_pairs!, serial_single_pass.jl:906-911): |du|^2, du_L^2, |du|^2 - du_L^2,
 // du_L |du|^2, du_L du_L^2, du_L (|du|^2 - du_L^2).  t is uniform over a slice.
@@ -307,23 +300,19 @@ DEV T sp_invariant(int t, T duL, T dn2) {
   }
 }
 
-DEV int cell32(float key, const Slice &s);
 DEV unsigned cell32_off(float key, const Slice &s);
 DEV int cell32m(float key, const Slice &s);
-template <int G>
-DEV int cell32_any(float key, const Slice &s);
 
-// CERT (sphere): the distance bin is read from the chord^2 cell table of the binary32 kernel
-// (lo, hi, blo: ambiguity interval and bin count per cell) with the binary64 chord^2 |q - p|^2,
-// which is the reference's own |d|^2; the reference's central angle 2 atan2(|d|, |p + q|) is
-// monotone in it, and the table's margins (2^-20 relative and more) exceed the error of both the
-// binary32 rounding of the key and the reference's angle.  Only a pair whose chord^2 lies in a
-// cell's ambiguity interval computes the angle and searches (tab is then the global binary64 key
-// table).  Values are always the reference's operation sequence.
-template <int G, int D, bool J, int OPK = 0, bool CERT = false>
+// Full exact evaluation of pair (i, j) of slice s from binary64 records.  Returns the output cell
+// (0-based within the slice) or -1 if the pair is not counted; writes the value.  OPK fixes the
+// operator at compile time (1: {1,0}, 2: {2,0}) with the same operation sequence as the generic
+// functor; 0 dispatches on P.op at run time; 3 is the single pass, which writes du_L to val[0] and
+// |du|^2 to val[1] (flat: _pf_sp_simd_pairs!, serial_single_pass.jl:245-253, du_L =
+// dot(du, dx) * inv(sqrt(r2)); sphere: _sp1d_pairs!, :333-338, du_L = dot(du, e1)); 4 is a plane
+// of the single pass's 2D form: the same du_L and |du|^2, then invariant s.plane as value.
+template <int G, int D, bool J, int OPK = 0>
 DEV int exact_cell(const Params &P, const Slice &s, const double *A, const double *B,
-                   const Cell *tab, const double *dE, const double *vE, double *val,
-                   const float2 *lohi = nullptr, const int2 *blo_tab = nullptr, int *bins = nullptr) {
+                   const Cell *tab, const double *dE, const double *vE, double *val, int *bins = nullptr) {
   const int nEd = P.n_dist + 1;
   int db;
   double v;
@@ -400,21 +389,8 @@ DEV int exact_cell(const Params &P, const Slice &s, const double *A, const doubl
       v = sf_raw64<D>(P.op, P.nl, P.nt, du, dx, r2);
     }
   } else {
-    SphereFrame f;
-    bool exact_dist = true;
-    if constexpr (CERT) {
-      f = sphere_frame64_noangle(A, B);
-      const float key = (float)sdot<3>(f.d, f.d);
-      const int c = cell32_any<G>(key, s);
-      const float2 lh = lohi[c];
-      exact_dist = (key >= lh.x) & (key <= lh.y);
-      db = (key > lh.y) ? blo_tab[c].x + 1 : blo_tab[c].x;
-      if (exact_dist) f.distance = sphere_distance64(A, B, f.d, P.radius);
-    } else {
-      f = sphere_frame64(A, B, P.radius);
-    }
-    if (exact_dist)
-      db = s.drule.on ? lin_rule_bin(s.drule, f.distance, P.n_dist) : dist_bin64(f.distance, tab, dE, nEd, s);
+    const SphereFrame f = sphere_frame64(A, B, P.radius);
+    db = s.drule.on ? lin_rule_bin(s.drule, f.distance, P.n_dist) : dist_bin64(f.distance, tab, dE, nEd, s);
     if (!f.ok || db < 1 || db > P.n_dist) return -1;
     if (bins) bins[0] = db - 1;
     double du[3];
@@ -935,23 +911,19 @@ DEV void wave_lds_sync() {
 // ---------------------------------------------------------------------------------------------
 // hist64: binary64 pair arithmetic
 // ---------------------------------------------------------------------------------------------
-template <int G, int D, bool J, int OPK, bool MASK>
+// a pair of the batch-leading flat geometry by the reference's sequence (the joint operators without a
+// difference form)
+template <int D, int OPK, bool MASK>
 DEV void pair64(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j,
                 const double *rj) {
   if (MASK && j <= i) return;
-  double v[2] = {0.0, 0.0};
+  double v = 0.0;
   int bins[2] = {0, 0};
-  int c;
-  if constexpr (G == kSphere)
-    c = exact_cell<G, D, J, OPK, true>(P, s, ri, rj, P.cells + s.tab_off, m.dE, m.vE, v, m.lohi, m.blo, bins);
-  else
-    c = exact_cell<G, D, J, OPK>(P, s, ri, rj, m.tab, m.dE, m.vE, v, nullptr, nullptr, bins);
+  const int c = exact_cell<kFlat, D, true, OPK>(P, s, ri, rj, m.tab, m.dE, m.vE, &v, bins);
   // the slot from the bins (no division of c), and a pair that is not counted goes to the lane's
   // scratch slot (never flushed): the update is unconditional, the loop body has no branch here
-  int h = J ? bins[1] * m.jv + bins[0] * m.jd + m.coff : (bins[0] << m.lcop) + (int)(__lane_id() & (m.copies - 1));
-  h = c >= 0 ? h : m.scr;
-  if constexpr (OPK == 3) hist_add_sp(m, h, v[0], v[1]);
-  else hist_add(m, h, v[0]);
+  const int h = bins[1] * m.jv + bins[0] * m.jd + m.coff;
+  hist_add(m, c >= 0 ? h : m.scr, v);
 }
 
 template <int S>
@@ -965,21 +937,21 @@ DEV void load_rec64(const double *__restrict__ p, double *r) {
 // record buffers alternating so that the next column's record is requested before the current
 // pair is evaluated.  The request past the last column reads at most one record beyond the
 // slice: the next slice's first record, or the record array's tail pad.
-template <int G, int D, bool J, int OPK, bool MASK>
+template <int D, int OPK, bool MASK>
 DEV void run_cols64(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j0, int j1,
                     const double *__restrict__ rec) {
-  constexpr int S = Rec<G, D>::d64;
+  constexpr int S = Rec<kFlat, D>::d64;
   const double *col = rec + (int64_t)s.pt_off * S;
   double ra[S], rb[S];
   load_rec64<S>(col + (int64_t)j0 * S, ra);
   int j = j0;
   for (; j + 1 < j1; j += 2) {
     load_rec64<S>(col + (int64_t)(j + 1) * S, rb);
-    pair64<G, D, J, OPK, MASK>(P, s, m, ri, i, j, ra);
+    pair64<D, OPK, MASK>(P, s, m, ri, i, j, ra);
     load_rec64<S>(col + (int64_t)(j + 2) * S, ra);
-    pair64<G, D, J, OPK, MASK>(P, s, m, ri, i, j + 1, rb);
+    pair64<D, OPK, MASK>(P, s, m, ri, i, j + 1, rb);
   }
-  if (j < j1) pair64<G, D, J, OPK, MASK>(P, s, m, ri, i, j, ra);
+  if (j < j1) pair64<D, OPK, MASK>(P, s, m, ri, i, j, ra);
 }
 
 // Row of the work item's tile that this thread owns.  Joint histograms: lane l of wave w takes
@@ -1023,8 +995,14 @@ DEV Row item_row(const Item &w, const Slice &s) {
   return r;
 }
 
-// Sphere, and flat point fields (not the batch-leading pairs): the same pairs as pair64 /
-// exact_cell, with the reference's operation sequence for every value, arranged like the binary32
+// a histogram update that waits for the next pair's table read
+struct Pending64 {
+  int h;
+  double v, w;  // value (single pass: du_L) and |du|^2 (single pass)
+};
+
+// The joint operators without a difference form on the sphere and on flat point fields (batch-leading
+// pairs: run_cols64): the reference's operation sequence for every value, arranged like the binary32
 // kernel's pair.  The distance bin is read from the binary32 key table (chord^2 or r^2: its
 // margins, 2^-20 relative and more, exceed the binary32 rounding of the binary64 key); the
 // previous pair's histogram update is deferred until this pair's table read is in flight (LDS
@@ -1035,16 +1013,7 @@ DEV Row item_row(const Item &w, const Slice &s) {
 // margin of a value decision point, by the exact rules.  Flat keys that are not above 2^-100
 // (coincident points, NaN) also take the exact rules.  A pair that is not counted updates the
 // lane's scratch slot.
-// doubles per point of the records it reads: the flat binary64 records, or prep64s's
-template <int G, int D>
-inline constexpr int rec_pair64 = (G == kFlat) ? Rec<G, D>::d64 : kF64Rec;
-
-struct Pending64 {
-  int h;
-  double v, w;  // value (single pass: du_L) and |du|^2 (single pass)
-};
-
-template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR>
+template <int G, int D, int OPK, bool MASK, bool VU, bool MIR>
 DEV void pair64p(const Params &P, const Slice &s, const Smem &m, const double *A, int i, int j,
                  const double *B, double *rn, const double *next, Pending64 &pa) {
   constexpr int S = Rec<G, D>::d64;
@@ -1067,8 +1036,7 @@ DEV void pair64p(const Params &P, const Slice &s, const Smem &m, const double *A
   const float2 lh = *(const float2 *)((const char *)m.lohi + c);
   const int blo = ((const int2 *)((const char *)m.blo + c))->x;
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (OPK == 3) hist_add_sp(m, pa.h, pa.v, pa.w);
-  else hist_add(m, pa.h, pa.v);
+  hist_add(m, pa.h, pa.v);
   asm volatile("" ::"v"(lh.x), "v"(lh.y), "v"(blo) : "memory");
   // outside [lo, hi] a key is above the edge exactly when key >= lo
   const bool ge = key >= lh.x;
@@ -1077,65 +1045,36 @@ DEV void pair64p(const Params &P, const Slice &s, const Smem &m, const double *A
   int db = ge ? blo + 1 : blo;
   load_rec64<S>(next, rn);
   __builtin_amdgcn_sched_barrier(0);
-  double v, w = 0.0;
+  double v;
   if constexpr (G == kFlat) {
-    // exact_cell's flat point-field values (sf_raw64 and its specialisations)
-    if constexpr (OPK == 3 || OPK == 4) {
-      const double inv_r = 1.0 / __builtin_sqrt(r2);
-      const double duL = sdot<D>(du, dx) * inv_r;
-      const double dn2 = sdot<D>(du, du);
-      if constexpr (OPK == 3) {
-        v = duL;
-        w = dn2;
-      } else {
-        v = sp_invariant(s.plane, duL, dn2);
-      }
-    } else if constexpr (OPK == 2) {
-      const double p = sdot<D>(du, dx);
-      v = p * p / r2;
-    } else if constexpr (OPK == 1) {
-      const double sq = __builtin_sqrt(r2);
-      double rh[D];
-#pragma unroll
-      for (int k = 0; k < D; ++k) rh[k] = dx[k] / sq;
-      v = 1.0 * sdot<D>(du, rh);
+    // exact_cell's flat point-field values
+    if constexpr (OPK == 4) {
+      const double duL = sdot<D>(du, dx) * (1.0 / __builtin_sqrt(r2));
+      v = sp_invariant(s.plane, duL, sdot<D>(du, du));
     } else {
       v = sf_raw64<D>(P.op, P.nl, P.nt, du, dx, r2);
     }
   } else {
     sphere_delta64<D>(f, A, B, du);
     const double rh[3] = {1.0, 0.0, 0.0};
-    if constexpr (OPK == 3) {
-      v = sdot<D>(du, rh);
-      w = sdot<D>(du, du);
-    } else if constexpr (OPK == 4) {
-      v = sp_invariant(s.plane, sdot<D>(du, rh), sdot<D>(du, du));
-    } else if constexpr (OPK == 1) {
-      v = 1.0 * sdot<D>(du, rh);
-    } else if constexpr (OPK == 2) {
-      const double L = sdot<D>(du, rh);
-      v = 1.0 * (L * L);
-    } else {
-      v = op_apply64<D>(P.op, P.nl, P.nt, du, rh);
-    }
+    if constexpr (OPK == 4) v = sp_invariant(s.plane, sdot<D>(du, rh), sdot<D>(du, du));
+    else v = op_apply64<D>(P.op, P.nl, P.nt, du, rh);
   }
   // value bin (1-based).  Uniform value edges (a LinearBinEdges rule or an equally spaced edge
   // vector): read from t = (v - v0) / w in binary32, certified like the binary32 kernel's (the
   // host slack covers the edges' distance from v0 + k w, and the rule's decision points' distance
   // from the edges), with twice its relative term for the rounding of v - v0 to binary32.  Only a
   // value within that margin of a decision point (or non-finite) takes the exact rule or search.
-  int vb = 1;
+  int vb;
   bool amb_v = false;
-  if constexpr (J) {
-    if constexpr (VU) {  // s.v_uniform, chosen once per column range
-      const float t = (float)(v - s.v0) * s.vinvf;
-      const float eps = __builtin_fmaf(9.6e-7f, __builtin_fabsf(t), s.vslack);
-      const float gh = __builtin_floorf(t + eps);
-      amb_v = !(t - eps >= gh);
-      vb = amb_v ? 0 : (int)gh + 1;  // |t| < 2^21 when certain: the conversion is exact
-    } else {
-      vb = s.vrule.on ? lin_rule_bin(s.vrule, v, P.n_val) : val_bin64(v, m.vE, P.n_val + 1, s);
-    }
+  if constexpr (VU) {  // s.v_uniform, chosen once per column range
+    const float t = (float)(v - s.v0) * s.vinvf;
+    const float eps = __builtin_fmaf(9.6e-7f, __builtin_fabsf(t), s.vslack);
+    const float gh = __builtin_floorf(t + eps);
+    amb_v = !(t - eps >= gh);
+    vb = amb_v ? 0 : (int)gh + 1;  // |t| < 2^21 when certain: the conversion is exact
+  } else {
+    vb = s.vrule.on ? lin_rule_bin(s.vrule, v, P.n_val) : val_bin64(v, m.vE, P.n_val + 1, s);
   }
   if (exact_dist | amb_v) {
     if (exact_dist) {
@@ -1149,21 +1088,19 @@ DEV void pair64p(const Params &P, const Slice &s, const Smem &m, const double *A
                         : dist_bin64(r2, P.cells + s.tab_off, m.dE, P.n_dist + 1, s);
       }
     }
-    if (J && amb_v) vb = s.vrule.on ? lin_rule_bin(s.vrule, v, P.n_val) : val_bin64(v, m.vE, P.n_val + 1, s);
+    if (amb_v) vb = s.vrule.on ? lin_rule_bin(s.vrule, v, P.n_val) : val_bin64(v, m.vE, P.n_val + 1, s);
   }
   const bool ok = (G == kSphere) ? f.ok : true;
   const bool add = (!MASK || j > i) & ok & ((unsigned)(db - 1) < (unsigned)P.n_dist) &
-                   (!J || (unsigned)(vb - 1) < (unsigned)P.n_val);
-  const int h = J ? (vb - 1) * m.jv + (db - 1) * m.jd + m.coff
-                  : ((db - 1) << m.lcop) + (int)(__lane_id() & (m.copies - 1));
+                   ((unsigned)(vb - 1) < (unsigned)P.n_val);
+  const int h = (vb - 1) * m.jv + (db - 1) * m.jd + m.coff;
   pa.h = add ? h : m.scr;
   pa.v = v;
-  pa.w = w;
 }
 
 // Columns j0 .. j1 - 1 of one row with pair64p; two record buffers alternate (the request past
 // the last column reads at most one record beyond the slice, as in run_cols64).
-template <int G, int D, bool J, int OPK, bool MASK, bool VU, bool MIR>
+template <int G, int D, int OPK, bool MASK, bool VU, bool MIR>
 DEV void run_cols64pv(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j0, int j1,
                       const double *__restrict__ rec) {
   constexpr int S = Rec<G, D>::d64;
@@ -1173,26 +1110,30 @@ DEV void run_cols64pv(const Params &P, const Slice &s, const Smem &m, const doub
   Pending64 pa{m.scr, 0.0, 0.0};
   int j = j0;
   for (; j + 1 < j1; j += 2) {
-    pair64p<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, col + (int64_t)(j + 1) * S, pa);
-    pair64p<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j + 1, rb, ra, col + (int64_t)(j + 2) * S, pa);
+    pair64p<G, D, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, col + (int64_t)(j + 1) * S, pa);
+    pair64p<G, D, OPK, MASK, VU, MIR>(P, s, m, ri, i, j + 1, rb, ra, col + (int64_t)(j + 2) * S, pa);
   }
-  if (j < j1) pair64p<G, D, J, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, col + (int64_t)(j + 1) * S, pa);
-  if constexpr (OPK == 3) hist_add_sp(m, pa.h, pa.v, pa.w);
-  else hist_add(m, pa.h, pa.v);
+  if (j < j1) pair64p<G, D, OPK, MASK, VU, MIR>(P, s, m, ri, i, j, ra, rb, col + (int64_t)(j + 1) * S, pa);
+  hist_add(m, pa.h, pa.v);
 }
 
 // the value-bin lookup (uniform or exact) and the key table's form are chosen once per column range,
 // not per pair
-template <int G, int D, bool J, int OPK, bool MASK>
+template <int G, int D, int OPK, bool MASK>
 DEV void run_cols64p(const Params &P, const Slice &s, const Smem &m, const double *ri, int i, int j0, int j1,
                      const double *__restrict__ rec) {
+  static_assert(OPK == 0 || OPK == 4, "the other operators have a difference form");
   auto run = [&](auto mir) {
-    if (J && s.v_uniform) run_cols64pv<G, D, J, OPK, MASK, J, mir.value>(P, s, m, ri, i, j0, j1, rec);
-    else run_cols64pv<G, D, J, OPK, MASK, false, mir.value>(P, s, m, ri, i, j0, j1, rec);
+    if (s.v_uniform) run_cols64pv<G, D, OPK, MASK, true, mir.value>(P, s, m, ri, i, j0, j1, rec);
+    else run_cols64pv<G, D, OPK, MASK, false, mir.value>(P, s, m, ri, i, j0, j1, rec);
   };
   if (G == kSphere && s.mir) run(std::integral_constant<bool, G == kSphere>());
   else run(std::false_type());
 }
+
+// doubles per point of the records that the difference form reads: the flat binary64 records, or prep64s's
+template <int G, int D>
+inline constexpr int rec_pair64 = (G == kFlat) ? Rec<G, D>::d64 : kF64Rec;
 
 // ---------------------------------------------------------------------------------------------
 // The binary64 pair in difference form (every 1D operator, and the joint du_L and du_L^2).
@@ -1291,8 +1232,7 @@ DEV int exact_points(const Params &P, const Slice &s, const Smem &m, int i, int 
     A[k] = P.rec64[(s.pt_off + lo) * S + k];
     B[k] = P.rec64[(s.pt_off + hi) * S + k];
   }
-  return exact_cell<G, D, J, (OPK <= 4 ? OPK : 0)>(P, s, A, B, P.cells + s.tab_off, m.dE, m.vE, v, nullptr,
-                                                   nullptr, bins);
+  return exact_cell<G, D, J, (OPK <= 4 ? OPK : 0)>(P, s, A, B, P.cells + s.tab_off, m.dE, m.vE, v, bins);
 }
 
 // whether a searched value edge next to 0-based bin g lies within 2^-34 (relative) of v: the two
@@ -1611,8 +1551,8 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
       if (w.slice != cur) {
         cur = w.slice;
         s = P.slices[cur];
-        // the binary32 key table of certified distance bins (the
-        // binary64 key table is read from global memory by the rare pairs that need it)
+        // the binary32 key table of certified distance bins (the binary64 key table is read from
+        // global memory by the rare pairs that need it)
         load_tables(m, P, s, FAST || G == kSphere || !P.bl);
       }
       since_flush = 0;
@@ -1646,11 +1586,11 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
           j = jn;
         }
       } else if (G == kSphere || !P.bl) {
-        if (w.j0 < row.jm) run_cols64p<G, D, J, OPK, true>(P, s, m, ri, row.i, w.j0, row.jm, rec);
-        if (row.jm < w.j1) run_cols64p<G, D, J, OPK, false>(P, s, m, ri, row.i, max(row.jm, w.j0), w.j1, rec);
-      } else {
-        if (w.j0 < row.jm) run_cols64<G, D, J, OPK, true>(P, s, m, ri, row.i, w.j0, row.jm, rec);
-        if (row.jm < w.j1) run_cols64<G, D, J, OPK, false>(P, s, m, ri, row.i, max(row.jm, w.j0), w.j1, rec);
+        if (w.j0 < row.jm) run_cols64p<G, D, OPK, true>(P, s, m, ri, row.i, w.j0, row.jm, rec);
+        if (row.jm < w.j1) run_cols64p<G, D, OPK, false>(P, s, m, ri, row.i, max(row.jm, w.j0), w.j1, rec);
+      } else if constexpr (G == kFlat) {
+        if (w.j0 < row.jm) run_cols64<D, OPK, true>(P, s, m, ri, row.i, w.j0, row.jm, rec);
+        if (row.jm < w.j1) run_cols64<D, OPK, false>(P, s, m, ri, row.i, max(row.jm, w.j0), w.j1, rec);
       }
     }
   }
@@ -1703,12 +1643,6 @@ DEV int cell32m(float key, const Slice &s) {
   asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(c), "s"(s.mir - 1));
   return key < k1 ? r : 2 * s.mir - 1 - r;
 }
-// either table, off the pair loops' main path
-template <int G>
-DEV int cell32_any(float key, const Slice &s) {
-  return (G == kSphere && s.mir) ? cell32m(key, s) : cell32(key, s);
-}
-
 // value-axis bin from a binary32 value with absolute error bound dv = dva * dvb; sets amb when
 // undecidable.  For uniform edges (VU) dva carries the factor 1 / bin width (the bound in bin
 // widths is then one multiply-add away).  Returns the 0-based value bin g (valid bins 0 .. nE-2;
@@ -2932,15 +2866,6 @@ __global__ void __launch_bounds__(256) recheck_multi(Params P) {
 }
 
 #if SF_PART == 0
-__global__ void merge_out(const double *src_s, const unsigned long long *src_c, double *dst_s,
-                          unsigned long long *dst_c, int64_t n) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) {
-    dst_s[k] += src_s[k];
-    dst_c[k] += src_c[k];
-  }
-}
-
 // merge unless the re-bin queue overflowed (then the accumulators are incomplete: flag it and
 // leave the outputs untouched so the host can redo the call in binary64)
 __global__ void merge_checked(const double *src_s, const unsigned long long *src_c, double *dst_s,
@@ -2968,16 +2893,6 @@ __global__ void derive_sp(double *s, unsigned long long *c, int64_t nbins) {
   col[5] = col[3] - col[4];
   const unsigned long long n = cc[0];
   for (int t = 1; t < kSpRows; ++t) cc[t] = n;
-}
-
-__global__ void zero_u64(unsigned long long *p, int64_t n) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) p[k] = 0ull;
-}
-
-__global__ void zero_f64(double *p, int64_t n) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) p[k] = 0.0;
 }
 
 __global__ void eval_math(int fn, int64_t n, const double *a, const double *b, double *out) {
@@ -3279,13 +3194,6 @@ hipError_t launch_recheck(int G, int D, bool J, const Params &P, int grid, hipSt
   const size_t smem = (size_t)nh * (P.nmom > 1 ? 36 : 12) + 16;
   (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   return hipLaunchKernel(f, dim3(grid), dim3(256), args, smem, st);
-}
-
-hipError_t launch_merge(const double *src_s, const unsigned long long *src_c, double *dst_s,
-                        unsigned long long *dst_c, int64_t n, hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  merge_out<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(src_s, src_c, dst_s, dst_c, n);
-  return hipGetLastError();
 }
 
 hipError_t launch_eval_math(int fn, int64_t n, const double *a, const double *b, double *out,
