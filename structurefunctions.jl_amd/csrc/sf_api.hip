@@ -775,8 +775,9 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
   (void)fill(Flo, Fhi);
   T.crowd = crowd / std::max(top, 1e-300);
   int mir = 0;
-  // (its five instructions a pair cost 4 %, a share of 0.8 % re-binned 40 % and more)
-  if (!flat && p.precision == SF_PREC_FP64 && crowd > 0.004) {
+  // (its five instructions a pair cost 4 %, a share of 0.8 % re-binned 40 % and more; it can be larger
+  // than the plain table by up to 16 KB of LDS, which a histogram of thousands of bins may not leave)
+  if (!flat && p.precision == SF_PREC_FP64 && crowd > 0.004 && nE <= kCell32Max) {
     // mirrored table (cell32m): `mir` cells for keys below 2, the rest by m = 4 - key below 2 downwards.
     // The smallest cells are those of the edge next to zero or next to 4 (keys within 2^-20 of 4 are
     // uncertain anyway: nearly antipodal).

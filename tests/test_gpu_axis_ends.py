@@ -30,3 +30,14 @@ def test_uncertain_share(ctx, geometry, k):
             # for the densest), the nearly coincident and antipodal keys hold 2^-22 of all pairs
             st = ctx.stats()
             assert st["rebinned"] <= (10 * 2.0 ** -19 * len(edges) + 2.0 ** -20) * st["pairs"] + 8
+
+
+def test_thousands_of_bins_near_pi(ctx):
+    # 7800 bins between 3.04 rad and nearly pi: the histogram leaves room for the plain key table only
+    # (7800 x 20 bytes and a table of 10 KB are more than a workgroup's 160 KB)
+    edges = np.linspace(np.pi - 0.1, np.pi - 0.0012, 7801)
+    x, u, _ = field("deg", 2, 1500, 5)
+    os_, oc, oa, og = _oracle.hist(x, u, edges, op=(0, 2, 0), geometry="deg", nthreads=4, with_mag=True)
+    assert oc.sum() > 500
+    gs, gc = gpu_hist(ctx, x, u, edges, (0, 2, 0), geometry="deg", prec="fp64")
+    check(gs, gc, os_, oc, oa, TOL["fp64"], "bins near pi", og=og, mag=MAG["fp64"])
