@@ -853,9 +853,9 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
         s.vinv = (double)(1.0L / w);
         s.v0f = (float)v0;
         s.vinvf = (float)(1.0L / w);
-        // exact product of two binary32 numbers, rounded once: within 2^-24 |v0 / w| of
-        // -v0f / w, which the slack's 4u (1 + |v0 / w|) term covers
-        // 1 / w and of a binary64 value to binary32)
+        // exact product of two binary32 numbers, rounded once; with the roundings of v0 and of
+        // 1 / w to binary32 it is within 3 * 2^-24 |v0 / w| (and terms of second order) of
+        // -v0 / w, which the slack's 4u (1 + |v0 / w|) covers
         s.vtc = (float)(-(double)s.v0f * (double)s.vinvf);
         // slack in t units: edge non-uniformity + rounding of v0 and 1/w in binary32
         const long double u = ldexpl(1.0L, -24);
