@@ -295,7 +295,7 @@ struct Plan {
   Arena *arena = nullptr;  // set: every buffer is taken from this region (no device allocation)
   // fused outputs: 1D operators evaluated with the main (joint) one, their accumulators and the
   // caller's outputs they merge into
-  int n1d = 0, nf = 0, mcopies = 0;
+  int n1d = 0, mcopies = 0;
   DevBuf<double> msums;
   DevBuf<unsigned long long> mcounts;
   double *mdst_s[kMaxFused] = {};
@@ -1253,22 +1253,6 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   pl.ncell = out_cells(p0);  // per input slice
   pl.sp = p0.op == SF_OP_SINGLE_PASS && !planes;
   pl.n1d = multi ? multi->n1d : 0;
-  pl.nf = fused_pad(pl.n1d);
-  if (pl.n1d) {
-    // a NaN distance is told by the value, which is NaN too, unless no output takes the distance; on an
-    // axis whose first or last bin is open it then would be counted, and the kernel of most outputs,
-    // which tests the key, is taken
-    auto takes = [&](int op, int nl, int nt) {
-      const bool norm = op == SF_OP_S2 || (op == SF_OP_FULLVEC && nl == 2);
-      const bool across = op == SF_OP_PROJECTED && nl == 0 && (nt == 1 || nt == 3) && p0.D == 3;
-      return !(op == SF_OP_PROJECTED && nl == 0 && nt == 0) && !(flat && (norm || across));
-    };
-    bool taken = pl.J && takes(p0.op, p0.nl, p0.nt), open = false;
-    for (int k = 0; k < pl.n1d; ++k) taken = taken || takes(multi->op[k], multi->nl[k], multi->nt[k]);
-    for (int s = 0; s < n; ++s)
-      open = open || sl[s].dist_edges[0] < 0.0 || !(sl[s].dist_edges[p0.n_dist] < 1e18);
-    if (!taken && open) pl.nf = kMaxFused;
-  }
   // B-strip: slices that share positions (the auxiliary axes of one field: same x, N, edges) and
   // bin 1D histograms in binary32 evaluate each pair's geometry once for up to kStripMax fields.
   // Opt-in (tuning variant 3): the per-slice 1D kernel with 16 histogram copies outruns it (eight
@@ -1395,7 +1379,6 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   Pk.n_val = p0.n_val;
   Pk.nmom = pl.sp ? 4 : 1;
   Pk.n1d = pl.n1d;
-  Pk.nf = pl.nf;
   const int nmom = Pk.nmom;
   Tuning tn = ctx->tune;
   // the autotuner times one-operator launches; a fused launch (more LDS, more work per pair) keeps
@@ -1448,12 +1431,12 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   if (pl.n1d) {
     mcop = 16;
     while (mcop > 1 && (size_t)smem_layout(p0.n_dist, p0.n_val, ncell_max, stage_bytes, copies, nmom, pl.fx, 0,
-                                           strip, jlayout, pl.nf, mcop).total > ctx->max_smem)
+                                           strip, jlayout, pl.n1d, mcop).total > ctx->max_smem)
       mcop >>= 1;
   }
   pl.mcopies = mcop;
   const SmemLayout L0 = smem_layout(p0.n_dist, p0.n_val, ncell_max, stage_bytes, copies, nmom, pl.fx, 0, strip,
-                                    jlayout, pl.nf, mcop);
+                                    jlayout, pl.n1d, mcop);
   // the binary64 kernel keeps one copy of a joint histogram, and queues the pairs it evaluates by
   // the reference's sequence: kRareQueue entries per wave, fewer (or none: such pairs are then
   // evaluated as they come) where the LDS does not hold them
@@ -1487,7 +1470,7 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   // (3.9 % of the pairs) 34.4 -> 13.6 ms, 50 bins (0.8 %) 10.0 -> 7.3; twelve groups of 3.9 % cost 16.9.
   auto bytes32 = [&](int q) {
     return (size_t)smem_layout(p0.n_dist, p0.n_val, ncell_max, stage_bytes, copies, nmom, pl.fx, q, strip, jlayout,
-                               pl.nf, mcop).total;
+                               pl.n1d, mcop).total;
   };
   auto queue_need = [&](int blk) {
     if (!mixed) return 0;
@@ -1779,7 +1762,6 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   P.bl = (flat && p0.semantics == SF_SEM_BATCH) ? 1 : 0;
   P.strip = strip;
   P.n1d = pl.n1d;
-  P.nf = pl.nf;
   P.mcopies = mcop;
   P.n_slices = pl.nout;
   P.mab_a = P.mab_b = 0;
@@ -1846,7 +1828,7 @@ int plan_launch(Plan &pl, bool use_mixed, double *out_s, unsigned long long *out
   const int stage_mixed = stage * ((use_mixed && pl.strip) ? pl.strip : 1);
   P.stage_bytes = stage_mixed;
   const SmemLayout L = smem_layout(P.n_dist, P.n_val, P.ncell_max, stage_mixed, P.copies, P.nmom, P.fx, P.qcap,
-                                   P.strip, P.jlayout, P.nf, P.mcopies);
+                                   P.strip, P.jlayout, P.n1d, P.mcopies);
   if (ev) HIPCHK(hipEventRecord(ev[0], st));
   if (P.n_items > 0)
     HIPCHK(launch_hist(pl.G, pl.D, pl.J, use_mixed, use_sload, false, P, pl.grid, pl.block, (size_t)L.total, st));

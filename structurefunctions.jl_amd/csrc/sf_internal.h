@@ -159,7 +159,7 @@ struct Params {
   int32_t strip;           // B-strip launch: LDS histograms per workgroup (fields per strip), 0: off
   // fused outputs (one pair evaluation, several operators): n1d 1D histograms besides the joint
   // one (if any); 1D output k of slice s accumulates at msums / mcounts + (k n_slices + s) n_dist
-  int32_t n1d, nf;         // nf: outputs that the kernel evaluates (fused_pad)
+  int32_t n1d;
   int32_t mcopies;         // lane-group copies of each fused 1D histogram (power of two)
   int32_t n_slices;
   int32_t mop[8], mnl[8], mnt[8];

@@ -624,7 +624,7 @@ struct Smem {
 template <bool JT>
 DEV Smem carve(char *base, const Params &P, int stage_bytes) {
   const SmemLayout L = smem_layout(P.n_dist, P.n_val, P.ncell_max, stage_bytes, P.copies, P.nmom, P.fx,
-                                   P.qcap, P.strip, P.jlayout, P.nf, P.mcopies);
+                                   P.qcap, P.strip, P.jlayout, P.n1d, P.mcopies);
   Smem m;
   m.nmom = P.nmom;
   m.fx = P.fx != 0;
@@ -1809,9 +1809,8 @@ DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *
   constexpr int NF = OPK == 9 ? 1 : (OPK == 10 ? 2 : (OPK == 11 ? 4 : (OPK == 12 ? 6 : kMaxFused)));
   constexpr bool needN2 = (OPK == 0) || MULTI || SP || SP2;
   // operators that do not take the distance: |du|^2, and on the flat geometry the horizontal transverse
-  // component (fused outputs of such operators alone take the kernel of kMaxFused outputs, see plan_build)
-  constexpr bool NAN_KEY = OPK == 0 || (MULTI && NF == kMaxFused) ||
-                           (G == kFlat && (SP2 || (D == 3 && (OPK == 6 || OPK == 8))));
+  // component; fused outputs may all be such
+  constexpr bool NAN_KEY = OPK == 0 || MULTI || (G == kFlat && (SP2 || (D == 3 && (OPK == 6 || OPK == 8))));
   const int nb = P.n_dist;
   lanes_t amb, amb_d;
   float key, L = 0.f, T = 0.f, tn2 = 0.f, n2 = 0.f, amp = 1.0f, umax;
@@ -3128,7 +3127,7 @@ static const void *pick_hist(int G, int D, bool J, bool mixed, int opk, bool sl,
 }
 
 static int opk_of(const Params &P) {
-  if (P.n1d > 0) return fused_opk(P.nf);
+  if (P.n1d > 0) return fused_opk(P.n1d);
   if (sp2d(P.op, P.n_val)) return 4;
   if (P.nmom > 1) return 3;
   if (P.op == 0 && P.nl == 1 && P.nt == 0) return 1;

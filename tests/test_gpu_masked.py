@@ -125,3 +125,24 @@ def test_masked_fused(ctx, geometry, D, ops):
             check(sums[k], counts[k], os_, oc, oa, TOL["mixed"], f"{geometry} {op}", og=og, mag=MAG["mixed"])
             gs, gc = gpu_hist(ctx, x, u, de, op, geometry=geometry, prec="mixed")
             check(gs.reshape(-1), gc.reshape(-1), os_, oc, oa, TOL["mixed"], f"{geometry} {op}", og=og, mag=MAG["mixed"])
+
+
+def test_masked_fused_many_bins(ctx):
+    """4500 bins with an open end: 90 KB of LDS for one fused output (eight would need 340 of 160)."""
+    x, u, edges = field("flat", 2, 500, 43)
+    x, u = mask(x, u, "nowhere", 0.2, False, 1)
+    x[0, ::7] *= -1.0
+    de = np.append(np.linspace(0.0, edges[-1], 4500), np.inf)
+    p = _native.SfProblem()
+    xc, uc = np.asfortranarray(x), np.asfortranarray(u)
+    p.D, p.W, p.N = uc.shape[0], xc.shape[0], 500
+    p.x, p.u = xc.ctypes.data, uc.ctypes.data
+    p.geometry, p.radius = _oracle.GEOM["flat"], 1.0
+    p.n_dist, p.dist_edges = len(de) - 1, de.ctypes.data
+    p.precision, p.count_bits = 1, 64
+    o = _native.SfOutput()
+    o.op, o.nl, o.nt = 1, 0, 0
+    sums, counts = np.zeros(len(de) - 1), np.zeros(len(de) - 1, dtype=np.uint64)
+    ctx.hist_multi([p], [o], [sums], [counts])
+    os_, oc, oa, og = _oracle.hist(x, u, de, op=(1, 0, 0), geometry="flat", nthreads=4, with_mag=True)
+    check(sums, counts, os_, oc, oa, TOL["mixed"], "4500 bins", og=og, mag=MAG["mixed"])
