@@ -861,7 +861,10 @@ void build_tables(const sf_problem &p, double xmax, SliceTables &T) {
         const long double u = ldexpl(1.0L, -24);
         s.vslack = round_up_f(dev + 4.0L * u * (1.0L + fabsl((long double)v0 / w)) + 4.0L * u * nv + 1e-6L +
                               rule_slack(p.val_rule) / w);
-        s.vslackt = round_up_f((long double)s.vslack + 4.8e-7L * (nv + 2));
+        // a value in range has |t| < nv + 1: the rounding of t and of t + eps, t - eps (u |t| each, of which
+        // two meet an edge).  Twice this (8u |t| at its largest) left a quarter more pairs to the re-bin
+        // where the values crowd at an edge in the middle of the axis
+        s.vslackt = round_up_f((long double)s.vslack + 4.0L * u * (nv + 2));
         // one margin for every value in range (|t| < nv + 1): 16u |t| covers the rounding of the
         // multiply-add, of the value and of the sums vtc + margin and t - floor(t)
         const long double eps = (long double)s.vslack + 24.0L * u * (nv + 2) + 4.0L * u * fabsl((long double)s.vtc);

@@ -1,0 +1,30 @@
+"""Binary32 joint calls over uniform value edges: the share of pairs left to the re-bin, against the pairs
+whose exact value lies within the margin that the binary32 value and its bin number need."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import gpu_hist
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nv,half", [(512, 4.0), (1024, 4.0), (256, 2.0)])
+def test_share_near_uniform_value_edges(ctx, nv, half):
+    rng = np.random.default_rng(nv)
+    n = 1500
+    x = rng.uniform(0, 1, (2, n))
+    u = rng.normal(size=(2, n))
+    ve = np.linspace(-half, half, nv + 1)  # an edge at zero, where the values crowd; exact in binary32
+    gpu_hist(ctx, x, u, np.array([1e-6, 2.0]), (0, 1, 0), vedges=ve, prec="mixed")
+    st = ctx.stats()
+    i, j = np.triu_indices(n, 1)
+    dx, du = x[:, j] - x[:, i], u[:, j] - u[:, i]
+    w = 2 * half / nv
+    t = ((du * dx).sum(0) / np.sqrt((dx * dx).sum(0)) + half) / w
+    unit = 2.0 ** -24
+    norm = np.sqrt((u * u).sum(0))
+    value = 16 * unit * (norm[i] + norm[j]) / w  # the value's bound, in bins
+    edges = 4 * unit * (1 + half / w) + 4 * unit * nv + 1e-6  # v0, 1 / w and -v0 / w in binary32
+    bins = 4 * unit * (nv + 2)  # the bin number and its two offsets
+    want = np.count_nonzero(np.abs(t - np.rint(t)) <= value + edges + bins)
+    assert st["rebinned"] <= 1.03 * want + 10
