@@ -1475,15 +1475,30 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     return (size_t)smem_layout(p0.n_dist, p0.n_val, ncell_max, stage_bytes, copies, nmom, pl.fx, q, strip, jlayout,
                                pl.n1d, mcop).total;
   };
+  // Third-order operators: their values crowd at zero (a cube's density grows as v^(-2/3)), and where the
+  // axis has an edge there, up to 5 % of the pairs are uncertain on the sphere (cubes; du_L^2 du_T 2.5 %)
+  // and 2.4 % on flat fields.  Every reservation in the global queue takes its counter 12 ns, so that a wave
+  // needs room for three groups of 32 columns: 160 entries where they cost no threads per CU, for cubes
+  // on the sphere 300 at any price.  Kernel ms with room for 32 / now, sphere, N = 40000: du_T^3, 64 x 64 bins,
+  // binary32 4.81 (two workgroups of 512) / 2.19 (one of 1024); fixed point, 48 x 64 bins, du_T^3 4.87 / 1.87,
+  // du_L^2 du_T 4.83 / 1.73.  Flat 2D du_L^3, binary32, 64 x 64: 2.22 / 1.80; with one workgroup of 1024
+  // in place of two of 768 it would be 2.26 for 1.70 (fixed point).
+  bool third = false;
+  if (J && ((p0.op == SF_OP_PROJECTED && p0.nl + p0.nt == 3) || p0.op == SF_OP_S3 || p0.op == SF_OP_L1T2COMP))
+    for (int s = 0; s < n && !third; ++s)
+      for (int k = 0; k <= p0.n_val && !third; ++k)
+        third = std::fabs(sl[s].val_edges[k]) * p0.n_val < 0.0625 * (sl[s].val_edges[p0.n_val] - sl[s].val_edges[0]);
+  const bool cubes = third && G == kSphere && p0.op == SF_OP_PROJECTED && (p0.nl == 3 || p0.nt == 3);
+  double room = cubes ? 300.0 : (third ? 160.0 : 32.0);
   auto queue_need = [&](int blk) {
     if (!mixed) return 0;
     // (32 entries a wave at least: a size that leaves no room for a queue beside one workgroup more per CU
     // had every queued pair wait for the global counter, fixed point, 48 x 80 bins 2.25 -> 4.27 ms)
     const double each = crowd > 0.001 ? 2048.0 * crowd : 0.0;
-    const double wave = std::max(32.0, std::max(4.0 * each, std::min(12.0 * each, 160.0)));
+    const double wave = std::max(room, std::max(4.0 * each, std::min(12.0 * each, 160.0)));
     int q = 64;
-    while (q < wave * (blk / 64) && q < kQueueCap) q *= 2;
-    while (q > 0 && bytes32(q) > ctx->max_smem) q = q > 64 ? q / 2 : 0;
+    while (q < wave * (blk / 64) && q < kQueueCap) q = third ? q + 64 : 2 * q;
+    while (q > 0 && bytes32(q) > ctx->max_smem) q = q > 64 ? q / 128 * 64 : 0;
     return q;
   };
   auto resident = [&](int blk) {  // workgroups of blk threads per CU
@@ -1497,12 +1512,23 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     // 768, fixed point, N = 98304, flat 2D: 4.71 / 4.93 ms at 40 x 64 bins, 4.91 / 5.06 at 20 x 32; two of
     // 512 against one of 1024, sphere, N = 65536, 40 x 64 bins: binary64 3.64 / 4.04, binary32 3.10 /
     // 3.34; fused, 40 x 48: 10.1 / 10.6.  64 x 96 bins keep two of 768 (fixed point) and one of 1024.
-    int most = 0;
-    for (const int blk : {512, 768, 1024}) {
-      const int threads = resident(blk) * blk;
-      if (threads > most) {
-        most = threads;
-        block = blk;
+    auto most_threads = [&] {
+      int most = 0;
+      for (const int blk : {512, 768, 1024}) {
+        const int threads = resident(blk) * blk;
+        if (threads > most) {
+          most = threads;
+          block = blk;
+        }
+      }
+      return most;
+    };
+    const int threads = most_threads();
+    if (third && !cubes) {
+      room = 32.0;
+      if (most_threads() <= threads) {
+        room = 160.0;
+        (void)most_threads();
       }
     }
   }
@@ -1525,6 +1551,7 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
   if (mixed) {
     for (int q = kQueueCap; q >= 64 && qcap == 0; q >>= 1)
       if (bytes32(q) <= ctx->max_smem && occupancy(block, bytes32(q)) >= bpc) qcap = q;
+    qcap = std::max(qcap, queue_need(block));
   }
   if (t_bpc) bpc = std::min(bpc, t_bpc);
   const int max_blocks = bpc * ctx->n_cu;

@@ -1,8 +1,10 @@
 """Binary32 joint calls over uniform value edges: the share of pairs left to the re-bin, against the pairs
-whose exact value lies within the margin that the binary32 value and its bin number need."""
+whose exact value lies within the margin that the binary32 value and its bin number need, and the time that
+their queue takes where it is large."""
 import numpy as np
 import pytest
 
+from sfamd import synthetic
 from test_gpu_parity import gpu_hist
 
 pytestmark = pytest.mark.gpu
@@ -28,3 +30,25 @@ def test_share_near_uniform_value_edges(ctx, nv, half):
     bins = 4 * unit * (nv + 2)  # the bin number and its two offsets
     want = np.count_nonzero(np.abs(t - np.rint(t)) <= value + edges + bins)
     assert st["rebinned"] <= 1.03 * want + 10
+
+
+@pytest.mark.parametrize("op,nd,nv,half,prec", [((0, 0, 3), 64, 64, 4.0, "mixed"), ((0, 3, 0), 64, 64, 0.5, "mixed"),
+                                                ((0, 0, 3), 48, 64, 4.0, "fixed"), ((0, 2, 1), 48, 64, 0.5, "fixed")])
+def test_third_order_queue(ctx, op, nd, nv, half, prec):
+    # 2 to 5 % of the pairs are queued: their reservations in the global queue must not bound the kernel
+    x, u, de, _ = synthetic.config4(N=40000)
+    m = 2.0 * float(np.sum(np.var(u, axis=1)))
+    de = np.geomspace(de[0], np.pi, nd + 1)
+
+    def kernel_us(op, half):
+        t = []
+        for _ in range(4):
+            gpu_hist(ctx, x, u, de, op, geometry="deg", vedges=np.linspace(-half, half, nv + 1), prec=prec)
+            st = ctx.stats()
+            t.append(st["hist_ns"])
+        return min(t), st["rebinned"] / st["pairs"]
+
+    plain, few = kernel_us((0, 0, 1), 2.0 * m ** 0.5)
+    cube, many = kernel_us(op, half * m ** 1.5)
+    assert few < 0.005 and many > 0.01
+    assert cube <= 1.7 * plain
