@@ -48,7 +48,7 @@ hipError_t launch_cull_units(const float *gbox, int64_t N, double *info, double 
                              int64_t n, hipStream_t st);
 int hist_occupancy(int G, int D, bool J, bool mixed, int opk, bool sload, bool fx, int block,
                    size_t smem);
-int hist_opk(const Params &P);
+int hist_opk(const Params &P, int G, bool mixed);
 int strip_occupancy(int G, int D, int opk, int block, size_t smem);
 struct PrepSliceHost {
   const double *x, *u;
@@ -340,7 +340,7 @@ int hist_opk_of(const sf_problem &p0) {
   Pk.nt = p0.nt;
   Pk.n_val = p0.n_val;
   Pk.nmom = (p0.op == SF_OP_SINGLE_PASS && p0.n_val == 0) ? 4 : 1;
-  return hist_opk(Pk);
+  return hist_opk(Pk, -1, true);
 }
 TuneKey tune_key(const sf_problem &p0, int64_t input_pairs) {
   int lg = 0;
@@ -1458,8 +1458,8 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
                      "histogram of %d cells needs %d bytes of LDS; the device allows %zu per workgroup",
                      ncell, std::max(L0.total, L64.total), ctx->max_smem);
   auto occupancy = [&](int blk, size_t bytes) {
-    const int nb = strip ? strip_occupancy(G, D, hist_opk(Pk), blk, bytes)
-                         : hist_occupancy(G, D, J, mixed, hist_opk(Pk), sload, pl.fx, blk, bytes);
+    const int nb = strip ? strip_occupancy(G, D, hist_opk(Pk, G, mixed), blk, bytes)
+                         : hist_occupancy(G, D, J, mixed, hist_opk(Pk, G, mixed), sload, pl.fx, blk, bytes);
     // LDS is handed out in units of 1280 bytes, which the runtime's figure leaves out (max_smem is a
     // CU's: 128 of them): a re-bin queue sized to the last byte had cost a workgroup per CU (flat 3D
     // du_L^2, 100 bins, N = 98304, 512 threads: 4.94 ms, now 4.24)

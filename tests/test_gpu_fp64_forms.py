@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import _oracle
-from test_gpu_parity import gpu_hist
+from test_gpu_parity import MAG, TOL, check, gpu_hist
 
 pytestmark = pytest.mark.gpu
 VE = np.linspace(-3, 3, 31)
@@ -98,3 +98,25 @@ def test_non_finite_velocities(ctx, geometry):
         gs, gc = gs.reshape(want.shape), gc.reshape(want.shape)
         assert np.array_equal(gc, cnt)
         assert np.array_equal(np.isnan(gs), np.isnan(want)) and np.array_equal(np.isinf(gs), np.isinf(want))
+
+
+@pytest.mark.parametrize("D", [2, 3])
+def test_squared_increment_takes_no_direction(ctx, D):
+    # |du|^2 (S2, FullVector{2}) of flat fields forms no du_L: its kernel is not slower than du_L^2's
+    rng = np.random.default_rng(D)
+    x, u = rng.uniform(size=(D, 30000)), rng.normal(size=(D, 30000))
+    edges = np.geomspace(1e-2, 1.9, 49)
+
+    def kernel_ns(op):
+        t = []
+        for _ in range(5):
+            gpu_hist(ctx, x, u, edges, op)
+            t.append(ctx.stats()["hist_ns"])
+        return min(t)
+
+    square = kernel_ns((0, 2, 0))
+    assert kernel_ns((1, 0, 0)) <= square and kernel_ns((5, 2, 0)) <= square
+    for op in ((1, 0, 0), (5, 2, 0)):
+        os_, oc, oa, og = _oracle.hist(x[:, :3001], u[:, :3001], edges, op=op, geometry="flat", nthreads=4, with_mag=True)
+        gs, gc = gpu_hist(ctx, x[:, :3001], u[:, :3001], edges, op)
+        check(gs, gc, os_, oc, oa, TOL["fp64"], f"{D}D {op}", og=og, mag=MAG["fp64"])
