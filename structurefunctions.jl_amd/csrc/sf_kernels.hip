@@ -1690,11 +1690,11 @@ DEV int val_bin32(float v, float dva, float dvb, const Slice &s, const float *E3
       if (E32[mid] < v) lo = mid + 1; else hi = mid;
     }
   }
-  // nearest edges must be farther than the error bound (edges rounded to binary32: slack)
+  // nearest edges must be farther than the error bound (edges rounded to binary32: slack; NaN: undecidable)
   const float gap = __builtin_fmaf(dva, dvb, __builtin_fmaf(s.vslack, __builtin_fabsf(v), s.vabs)) + 1e-37f;
   bool near = false;
-  if (lo > 0 && v - E32[lo - 1] <= gap) near = true;
-  if (lo < nE && E32[lo] - v <= gap) near = true;
+  if (lo > 0 && !(v - E32[lo - 1] > gap)) near = true;
+  if (lo < nE && !(E32[lo] - v > gap)) near = true;
   amb |= __builtin_amdgcn_ballot_w64(near);
   gf = (float)(lo - 1);
   return lo - 1;
@@ -1816,8 +1816,9 @@ DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *
   constexpr int NF = OPK == 9 ? 1 : (OPK == 10 ? 2 : (OPK == 11 ? 4 : (OPK == 12 ? 6 : kMaxFused)));
   constexpr bool needN2 = (OPK == 0) || MULTI || SP || SP2;
   // operators that do not take the distance: |du|^2, and on the flat geometry the horizontal transverse
-  // component; fused outputs may all be such
-  constexpr bool NAN_KEY = OPK == 0 || MULTI || (G == kFlat && (SP2 || (D == 3 && (OPK == 6 || OPK == 8))));
+  // component; fused outputs may all be such (joint histograms: the margin of the value is NaN; an operator
+  // chosen at run time: its finiteness test takes the key, 2 to 6 % less than two scalar operations here)
+  constexpr bool NAN_KEY = MULTI || (!J && G == kFlat && D == 3 && (OPK == 6 || OPK == 8));
   const int nb = P.n_dist;
   lanes_t amb, amb_d;
   float key, L = 0.f, T = 0.f, tn2 = 0.f, n2 = 0.f, amp = 1.0f, umax;
@@ -2027,6 +2028,8 @@ DEV lanes_t pair32(const Params &P, const Slice &s, const Smem &m, const float *
       // integer and the bits are kFxBase + q (no conversion needed)
       pa.q = __float_as_uint(__builtin_fmaf(v, s.vsf, __builtin_fmaf(-gf, s.fxc1, s.fxc0)));
     }
+  } else if constexpr (OPK == 0) {
+    amb |= lanes_nlt(__builtin_fmaf(key, 0.0f, __builtin_fabsf(v)), __builtin_inff());
   } else if constexpr (!SP) {
     amb |= lanes_nlt(__builtin_fabsf(v), __builtin_inff());
   }

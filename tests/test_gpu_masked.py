@@ -146,3 +146,27 @@ def test_masked_fused_many_bins(ctx):
     ctx.hist_multi([p], [o], [sums], [counts])
     os_, oc, oa, og = _oracle.hist(x, u, de, op=(1, 0, 0), geometry="flat", nthreads=4, with_mag=True)
     check(sums, counts, os_, oc, oa, TOL["mixed"], "4500 bins", og=og, mag=MAG["mixed"])
+
+
+@pytest.mark.parametrize("geometry,D", [("flat", 2), ("flat", 3), ("deg", 2), ("deg", 3)])
+@pytest.mark.parametrize("prec", ["fp64", "mixed", "fixed"])
+def test_nowhere_open_axes(ctx, geometry, D, prec):
+    """NaN positions of either sign on axes with open ends: operators that take the distance and that do not."""
+    x, u, edges = field(geometry, D, 500, 61)
+    x, u = mask(x, u, "nowhere", 0.2, False, 1)
+    x[0, ::7] *= -1.0
+    x[0, 3::11] = -np.nan
+    p = "mixed" if prec == "fixed" else prec
+    for de in (np.append(edges, np.inf), np.concatenate([[-np.inf, 0.0], edges, [np.inf]])):
+        for op in ((0, 0, 0), (0, 0, 1), (0, 0, 2), (0, 0, 3), (0, 1, 2), (1, 0, 0), (2, 0, 0), (3, 0, 0), (4, 0, 0), (5, 1, 0),
+                   (5, 2, 0), (5, 3, 0)):
+            for ve in (None, np.array([-np.inf, 0.0, np.inf]), np.linspace(-4, 4, 24)):
+                if prec == "fixed" and ve is None:
+                    continue
+                os_, oc, oa, og = _oracle.hist(x, u, de, op=op, geometry=geometry, vedges=ve, nthreads=8, with_mag=True)
+                gs, gc = gpu_hist(ctx, x, u, de, op, geometry=geometry, vedges=ve, prec=prec)
+                og = np.where(np.isfinite(og), og, 0.0)
+                mag = MAG[p] + (16 * 2.0 ** -53 / 1e-4 if prec == "fp64" else 0.0)
+                if prec == "fixed":  # 2^-22 value bins a pair
+                    og = og + oc * 8.0 / 23 * 2.0 ** -22 / mag
+                check(gs, gc, os_, oc, oa, TOL[p], f"{geometry} D={D} {op} {prec}", og=og, mag=mag)
