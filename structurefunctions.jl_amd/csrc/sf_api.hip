@@ -1499,7 +1499,28 @@ int plan_build(sf_ctx *ctx, Plan &pl, int n_in, const sf_problem *sl_in, const d
     int q = 64;
     while (q < wave * (blk / 64) && q < kQueueCap) q = third ? q + 64 : 2 * q;
     while (q > 0 && bytes32(q) > ctx->max_smem) q = q > 64 ? q / 128 * 64 : 0;
-    return q;
+    if (third || each == 0.0 || q == 0) return q;
+    // Fewer where these cost more threads than their reservations: a pair takes about 0.6 + 10 / w ps
+    // with w waves on each CU (joint twice that), and a reservation for G groups 12 ns / 2048 G.  A
+    // group as large as all that is left for the queue gains nothing by it.  Four groups' room at any
+    // price (one workgroup per CU) / now: flat 3D, linear, 150 bins, N = 60000, 2.3 % of the pairs, 8.1 / 4.8 ms;
+    // sphere, 200 bins, 51 %, done again in binary64 with the same shape, 51.2 / 34.4 ms.
+    int best = 0;
+    double least = 1e300;
+    int most = 0;
+    for (int r = 32 * (blk / 64); r <= q; r *= 2) {
+      const int w = occupancy(blk, bytes32(r)) * (blk / 64);
+      most = std::max(most, w);
+      if (2 * w < most || w == 0) break;
+      // (flat: the crowded keys are the largest ones, which few pairs have; 5 % at most)
+      const double groups = std::max(1.0, floor(r / (blk / 64) / (G == kFlat ? std::min(each, 102.4) : each)));
+      const double t = std::max((J ? 2.0 : 1.0) * (0.6 + 10.0 / w), 6.0 / groups);
+      if (t < least) {
+        least = t;
+        best = r;
+      }
+    }
+    return best > 0 ? best : q;
   };
   auto resident = [&](int blk) {  // workgroups of blk threads per CU
     return std::max(1, occupancy(blk, mixed ? bytes32(queue_need(blk))

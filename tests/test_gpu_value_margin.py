@@ -1,6 +1,6 @@
 """Binary32 joint calls over uniform value edges: the share of pairs left to the re-bin, against the pairs
 whose exact value lies within the margin that the binary32 value and its bin number need, and the time that
-their queue takes where it is large."""
+their queue takes where it is large (value edges at zero, distance bins that share cells of the key table)."""
 import numpy as np
 import pytest
 
@@ -52,3 +52,21 @@ def test_third_order_queue(ctx, op, nd, nv, half, prec):
     cube, many = kernel_us(op, half * m ** 1.5)
     assert few < 0.005 and many > 0.01
     assert cube <= 1.7 * plain
+
+
+def test_crowded_axis_keeps_its_threads(ctx):
+    # a linear axis whose largest keys share cells, on points that have few such distances: room for their
+    # pairs in the queue must not cost most of the threads
+    rng = np.random.default_rng(4)
+    n = 18000
+    x = np.cumsum(rng.normal(scale=0.002, size=(2, n)), axis=1) % 1.0
+    u = rng.normal(size=(2, n))
+
+    def kernel_ns(nd):
+        t = []
+        for _ in range(6):
+            gpu_hist(ctx, x, u, np.linspace(0.0, np.sqrt(2), nd + 1), (0, 2, 0), prec="mixed")
+            t.append(ctx.stats()["hist_ns"])
+        return min(t)
+
+    assert kernel_ns(162) <= 2.0 * kernel_ns(60)
