@@ -1180,6 +1180,12 @@ inline constexpr int rec_pair64 = (G == kFlat) ? Rec<G, D>::d64 : kF64Rec;
 // rest 3.8); 30 % at rest: 14.1, 4.0 (9.1); 10 % of the velocities NaN: 33.6, 4.0 (8.5); 1D du_L^2, 10 % NaN:
 // 23.9, 3.1 (7.4).  Fewer rare pairs than kManyRare in a group (2 % of it) are better queued: those of a
 // joint du_L^2 whose first edge is zero, 0.8 %, took 0.82 ms and 0.94 with this form (N = 30011).
+// In 1D it also bins pairs of uncertain keys (cells of the key table that hold several edges) by the
+// reference's distance, where kBinHere lanes have one; their value needs no more than that.  Where it
+// leaves most of the rare pairs all the same, the wave keeps off it for as many columns.  N = 60000, linear bins:
+// sphere 300 bins 24.1 ms by the queue, 18.0 (22.0 before the difference form), 600 30.4 and 18.4 (22.7); flat
+// 3D 300 8.4 and 6.3 (5.7), 600 10.9 and 5.9 (6.0); 150 bins, 2.5 % uncertain, stay with the queue.  Edge
+// vectors take a walk: flat 2D 300 10.2 and 10.1 (8.9), 600 15.9 and 12.7 (11.6).
 // ---------------------------------------------------------------------------------------------
 DEV double rsqrt64(double x) {
   const double y = __builtin_amdgcn_rsq(x);
@@ -1247,6 +1253,7 @@ DEV bool near_value_edge(double v, const double *E, int nE, int g) {
 }
 
 inline constexpr int kManyRare = 48, kManyCols = 4096;
+inline constexpr int kBinHere = 12;
 
 // MANY (with MASK): the form for fields with masked points; only the pairs of the lanes in `want` are
 // evaluated, and zb is the slice's vzero.  Returns the lanes whose pair is left to the reference's
@@ -1277,8 +1284,8 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
   asm volatile("" ::"v"(lh.x), "v"(lh.y), "v"(bm1) : "memory");
   // a key outside [lo, hi] is above the edge exactly when it is not below lo; a NaN key is uncertain
   const lanes_t ge = lanes_nlt(key, lh.x);
-  const lanes_t rare_d = ge & lanes_ngt(key, lh.y);
-  const int db0 = lane_of(ge) ? bm1 + 1 : bm1;
+  lanes_t rare_d = ge & lanes_ngt(key, lh.y);
+  int db0 = lane_of(ge) ? bm1 + 1 : bm1;
   double e2 = 0.0;
   if constexpr (G == kSphere) {
     double e[3];
@@ -1373,6 +1380,25 @@ DEV lanes_t pair64f(const Params &P, const Slice &s, const Smem &m, const double
         if constexpr (D == 3) q += __builtin_fabs(du[2]);
         rare_v &= ~lanes_nan(q);
       }
+    }
+  }
+  if constexpr (MANY && !J) {
+    // uncertain distance bins, by the reference's distance (not of nearly coincident or antipodal points)
+    const lanes_t here = rare_d & want & lanes_lt(G == kFlat ? __builtin_fmaxf(1e-29f, 0x1p14f * s.xerr * s.xerr) : 0x1p-42f, key) &
+                         (G == kFlat ? ~0ull : lanes_lt(key, 4.0f - 0x1p-18f));
+    if (__popcll(here) >= kBinHere) {
+      if (lane_of(here)) {
+        double r;
+        if constexpr (G == kSphere) {
+          r = sphere_distance64(A, B, d, P.radius);
+        } else {
+          r = sdot<D>(d, d);
+          if (P.bl || s.drule.on) r = __builtin_sqrt(r);  // (else the edges' squares)
+        }
+        db0 = (s.drule.on ? lin_rule_bin(s.drule, r, P.n_dist)
+                          : dist_bin64(r, P.cells + s.tab_off, m.dE, P.n_dist + 1, s)) - 1;
+      }
+      rare_d &= ~here;
     }
   }
   const lanes_t in_d = lanes_below(db0, P.n_dist);
@@ -1533,7 +1559,7 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
   __shared__ int s_item;
   const int B = blockDim.x;
   int cur = -1;
-  int many = 0;  // columns that the wave still runs in the form for fields with masked points
+  int many = 0;  // columns that the wave still runs in the form for fields with masked points (below 0: not in it)
   Slice s{};
   unsigned long long since_flush = 0;
   zero_hist(m);
@@ -1580,16 +1606,18 @@ __global__ void __launch_bounds__(1024) hist64(Params P, const double *__restric
           const int jn = run_range64f<G, D, J, OPK>(P, s, m, ri, row.i, j, je, mask, many > 0, ~0u, rec, dm, jl, cur);
           if (__ballot(dm != 0u)) {
             unsigned tot = 0u;
-            if (many <= 0) (void)wave_prefix((unsigned)__popc(dm), &tot);
+            if (many == 0) (void)wave_prefix((unsigned)__popc(dm), &tot);
             if (tot >= kManyRare) {
-              many = kManyCols;
               const unsigned want = dm;
               (void)run_range64f<G, D, J, OPK>(P, s, m, ri, row.i, j + ((jl - j) & ~31), jl + 1, true, true, want, rec,
                                                dm, jl, cur);
+              unsigned left = 0u;  // not worth its instructions where most of the pairs are left
+              if (__ballot(dm != 0u)) (void)wave_prefix((unsigned)__popc(dm), &left);
+              many = 2 * left > tot ? -kManyCols : kManyCols;
             }
             rare64<G, D, J, OPK>(P, s, m, rec, dm, row.i, jl);
           }
-          many -= jn - j;
+          many = many > 0 ? max(many - (jn - j), 0) : min(many + (jn - j), 0);
           j = jn;
         }
       } else if (G == kSphere || !P.bl) {

@@ -4,10 +4,14 @@ Counts are bit-identical to the oracle's.  Sums: two binary64 sequences of a pai
 2^-53 of the velocities, divided by the sine of the separation on the sphere; the tolerance is
 1e-12 of sum |value| plus 16 * 2^-53 / sin of sum ||du||^order (16 roundings of operands no larger
 than the velocities, sin the smallest sine among the case's pairs)."""
+import time
+
 import numpy as np
 import pytest
 
 import _oracle
+import sfamd
+from sfamd import bins
 from test_gpu_parity import MAG, TOL, check, gpu_hist
 
 pytestmark = pytest.mark.gpu
@@ -120,3 +124,41 @@ def test_squared_increment_takes_no_direction(ctx, D):
         os_, oc, oa, og = _oracle.hist(x[:, :3001], u[:, :3001], edges, op=op, geometry="flat", nthreads=4, with_mag=True)
         gs, gc = gpu_hist(ctx, x[:, :3001], u[:, :3001], edges, op)
         check(gs, gc, os_, oc, oa, TOL["fp64"], f"{D}D {op}", og=og, mag=MAG["fp64"])
+
+
+@pytest.mark.parametrize("geometry", ["flat2", "flat3", "deg"])
+def test_crowded_axis(ctx, geometry):
+    # thousands of bins in the key table's cells: most pairs' distance bins are uncertain, on linear
+    # axes, axes of unequal bins and open ones
+    rng = np.random.default_rng(8)
+    x, u, _ = _field(geometry, 2500, 8)
+    top = np.pi if geometry == "deg" else np.sqrt(x.shape[0])
+    geo = "deg" if geometry == "deg" else "flat"
+    for de in (np.linspace(0.0, top, 1501), np.sort(rng.uniform(0.2, top, 900)),
+               np.concatenate([[-np.inf, 0.0], np.sort(rng.uniform(0.0, top, 700)), [np.inf]])):
+        for op in ((0, 2, 0), (0, 3, 0), (0, 0, 1), (1, 0, 0), (2, 0, 0)):
+            os_, oc, oa, og = _oracle.hist(x, u, de, op=op, geometry=geo, nthreads=8, with_mag=True)
+            gs, gc = gpu_hist(ctx, x, u, de, op, geometry=geo)
+            check(gs, gc, os_, oc, oa, TOL["fp64"], f"{geometry} {op}", og=og, mag=16 * 2.0 ** -53 / 1e-4)
+
+    # the linear rule, and the time of a call with 600 bins by it against 60
+    be = sfamd.MI355XBackend(0, "fp64")
+
+    def call(x, u, nd):
+        kw = dict(distance_metric=sfamd.Haversine(1.0)) if geometry == "deg" else {}
+        return sfamd.calculate_structure_function(sfamd.L2SF, x, u, bins.LinearBinEdges(0.0, top, nd + 1), np.uint64,
+                                                  backend=be, output_type=sfamd.StructureFunctionSumsAndCounts, **kw)
+
+    _, oc, _ = _oracle.hist(x, u, bins.LinearBinEdges(0.0, top, 1501), op=(0, 2, 0), geometry=geo)
+    assert np.array_equal(np.asarray(call(x, u, 1500).counts).astype(np.uint64), oc)
+    big = _field(geometry, 60000, 9)
+
+    def seconds(nd):
+        t = []
+        for _ in range(4):
+            t0 = time.perf_counter()
+            call(big[0], big[1], nd)
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    assert seconds(600) <= (9.0 if geometry == "deg" else 3.8) * seconds(60)
