@@ -218,7 +218,8 @@ int sf_hist_multi(sf_ctx *ctx, int32_t n_slices, const sf_problem *slices, int32
  * re-bin queue) is carved from one static device array of SF_NOALLOC_SCRATCH_BYTES per device,
  * held until the process ends.  Limits: the records of all slices must fit in half of it (about
  * 400 000 points for the sphere in a binary32 precision, 700 000 in binary64) and the rest of the
- * call in the remainder, else SF_E_UNSUPPORTED is returned; the re-bin queue gets whatever is left,
+ * call in the remainder, else SF_E_UNSUPPORTED is returned (a batch that does not fit in one launch
+ * with all of its work buffers runs in parts, one after the other); the re-bin queue gets whatever is left,
  * and a call that overflows it is redone with the binary64 kernel (slower, same results); no tile
  * culling.  Every call on a device shares the array and leaves its contents behind (what must
  * start at zero is cleared by each call): calls that overlap in time on one device race, so

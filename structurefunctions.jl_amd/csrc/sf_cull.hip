@@ -11,6 +11,7 @@
 //   sort_*        stable radix sort of the keys, carrying point indices: the record order
 //   cull_groups   the bounding box of every group of kGroup consecutive records
 //   cull_units    the work units: a wave's 64 rows and one or two column groups within reach
+//                 (launch_cull_count: their number alone, for wide row blocks)
 // The host reads back the slice box and the number of units (kCullInfo words).
 #include <hip/hip_runtime.h>
 

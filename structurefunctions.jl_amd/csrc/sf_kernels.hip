@@ -1146,9 +1146,11 @@ inline constexpr int rec_pair64 = (G == kFlat) ? Rec<G, D>::d64 : kF64Rec;
 // All of it in binary64, 1 / |dx| and 1 / sin from the hardware's estimate with one third-order
 // step (its error is the last multiply-add's rounding).  The reference's sequence forms the frame
 // of every pair (on the sphere two tangent vectors, four projections on the local bases, a square
-// root and a division: 92 binary64 operations); this one takes 19 and the reciprocal square root,
-// and its rounding errors are no larger: differences of nearby points are exact here, where the
-// reference subtracts two projections of the full velocities.
+// root and a division: 92 binary64 operations); this one takes 19 and the reciprocal square root.
+// Differences of nearby points are exact here, where the reference subtracts two projections of the full
+// velocities; its errors stay in the last bits all the same, not always below the sequence's: bins' sums
+// against extended precision, 2-norm, sequence / this: flat 3D du_L 8.3e-16 / 3.5e-16, du_L^2 1.7e-16 / 4.5e-16
+// (N = 777); sphere, 2500 points, du_L 1.0e-15 / 1.4e-15, du_L^3 0.9e-15 / 1.5e-15.
 //
 // What bounds it: the vector ALU, where a binary64 add or multiply-add takes 4.5 cycles per wave,
 // a binary32 multiply-add 4 and a binary32 add 2.5 (so splitting values into binary32 pairs saves
