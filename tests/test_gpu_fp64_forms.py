@@ -12,7 +12,8 @@ import pytest
 import _oracle
 import sfamd
 from sfamd import bins
-from test_gpu_parity import MAG, TOL, check, gpu_hist
+from test_gpu_parity import gpu_hist
+from test_gpu_parity import MAG, TOL, check
 
 pytestmark = pytest.mark.gpu
 VE = np.linspace(-3, 3, 31)
